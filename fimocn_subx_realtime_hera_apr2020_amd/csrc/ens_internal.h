@@ -128,6 +128,9 @@ void ens_launch_trdp(const EnsGrid &g, const EnsState &s, hipStream_t st);
 void ens_launch_hystat_init(const EnsGrid &g, const EnsState &s, hipStream_t st);
 void ens_launch_convert_member(const EnsGrid &g, const EnsState &s, int member, const DevState &src,
                                hipStream_t st);
+// count fields of n values: FP32 ones 'stride' apart to consecutive FP64 ones, and back
+void ens_launch_widen(const float *src, double *dst, size_t n, size_t stride, int count, hipStream_t st);
+void ens_launch_narrow(const double *src, float *dst, size_t n, size_t stride, int count, hipStream_t st);
 void ens_launch_globsum(const EnsGrid &g, const EnsState &s, double *part64, float *part32, int nblocks,
                         hipStream_t st);
 

@@ -991,6 +991,19 @@ __global__ void __launch_bounds__(256) k_e_convert(EnsGrid g, EnsState s, int m,
   }
 }
 
+// fields between their FP32 arrays and the FP64 staging member (one grid row
+// per field): what the host reads and writes is FP64
+__global__ void __launch_bounds__(256) k_e_widen(const float *src, double *dst, size_t n, size_t stride) {
+  src += blockIdx.y * stride;
+  dst += blockIdx.y * n;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = (double)src[i];
+}
+__global__ void __launch_bounds__(256) k_e_narrow(const double *src, float *dst, size_t n, size_t stride) {
+  src += blockIdx.y * n;
+  dst += blockIdx.y * stride;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = (float)src[i];
+}
+
 // ---------------------------------------------------------------------------
 // globsum (globsum.F90:70-101) per member: FP64 block partials, and FP32
 // Kahan-compensated partials (value + compensation) of the same sums.
@@ -1121,6 +1134,16 @@ void ens_launch_hystat_init(const EnsGrid &g, const EnsState &s, hipStream_t st)
 void ens_launch_convert_member(const EnsGrid &g, const EnsState &s, int member, const DevState &src,
                                hipStream_t st) {
   k_e_convert<<<2048, 256, 0, st>>>(g, s, member, src);
+}
+static dim3 field_grid(size_t n, int count) {
+  const size_t b = (n + 255) / 256;
+  return dim3((unsigned)(b < 2048 ? b : 2048), count);
+}
+void ens_launch_widen(const float *src, double *dst, size_t n, size_t stride, int count, hipStream_t st) {
+  k_e_widen<<<field_grid(n, count), 256, 0, st>>>(src, dst, n, stride);
+}
+void ens_launch_narrow(const double *src, float *dst, size_t n, size_t stride, int count, hipStream_t st) {
+  k_e_narrow<<<field_grid(n, count), 256, 0, st>>>(src, dst, n, stride);
 }
 void ens_launch_globsum(const EnsGrid &g, const EnsState &s, double *part64, float *part32, int nblocks,
                         hipStream_t st) {

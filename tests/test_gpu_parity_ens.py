@@ -664,3 +664,23 @@ def test_fused_tracer_fct_launch_shapes_agree():
         for m in range(2):
             for n in ref[m]:
                 assert np.array_equal(ref[m][n], f[m][n]), (tile, m, n)
+
+
+@pytest.mark.parametrize("ntra, ntrb", [(1, 3), (4, 3), (2, 4), (3, 7)])
+def test_class_b_load_and_download_in_chunks(ntra, ntrb):
+    """Class-B tracers travel up to ntra at a time through the FP64 staging
+    member: what comes back is what went in, rounded once to FP32, for counts
+    below, at a multiple of and above ntra, and the other members' stay."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, state
+    g = fimhip.icos_grid(2)
+    th, ds = state.vertical_tables(38)
+    e = fimhip.Ensemble(g, 3, 38, ntra, DT, th, ds)
+    try:
+        e.set_class_b(ntrb, 6)
+        trb = np.random.default_rng(5).uniform(-1.0, 1.0, (3, ntrb, g.nip, 38))
+        for m in (2, 0, 1):
+            e.load_class_b(m, trb[m])
+        for m in range(3):
+            assert np.array_equal(e.download(m, "trb"), trb[m].astype(np.float32).astype(np.float64)), m
+    finally:
+        e.close()
