@@ -2,10 +2,9 @@
 //
 // regrid_1d (207-512) with restp_1d (792-890), equilb (1282-1437) and
 // inflate (893-1007), and remap_1d (515-789) with pcwise (1010-1279), run one
-// wavefront per column (lane = level) with the column in LDS; at 64 levels
-// the inherently serial sweeps (equilb, inflate, the theta redistribution)
-// run in separate kernels one thread per column with the column in
-// registers.  The lateral interface smoothing dffusn_lev (dffusn.F90:37-58)
+// wavefront per column (lane = level) with the column in LDS; the inherently
+// serial sweeps (equilb, inflate, the theta redistribution) run in separate
+// kernels one thread per column with the column in registers.  The lateral interface smoothing dffusn_lev (dffusn.F90:37-58)
 // is a cell-level kernel.  Loop orders and operation orders are those of the
 // reference.  Columns a land/sea mask marks as land are left as they are.
 #include "fimhip_internal.h"
@@ -61,32 +60,6 @@ __device__ void restp_1d(const double *thold, const double *pkold, int kold, dou
 __device__ __forceinline__ double cushn(double arg, double arg1) {
   double m = dmin(arg, 2. * arg1);
   return .25 * (m * m) / arg1 + dmax(arg, 2. * arg1) - arg1;
-}
-
-__device__ void equilb(const double *thet, double *pnew, int kk, double slak, int k0 = 3) {
-  for (int k = k0; k <= kk - 2; k++) {
-    if (pnew[k - 3] > pnew[0] - THIN) continue;
-    double dp1 = pnew[k - 3] - pnew[k - 2];
-    double dp2 = pnew[k - 2] - pnew[k - 1];
-    double dp3 = pnew[k - 1] - pnew[k];
-    double dp4 = pnew[k] - pnew[k + 1];
-    double dp5 = pnew[k + 1] - pnew[k + 2];
-    double th2 = thet[k - 2], th3 = thet[k - 1], th4 = thet[k];
-    if (dp2 > dp1 && dp4 > dp5) {
-      double goal = .5 * (dp3 + dmin(dp2, dp4));
-      if (dp2 > goal && dp4 > goal) {
-        double dis3 = dmin(dp2 - goal, goal - dp3) * slak;
-        double dis4 = dmin(dp4 - goal, goal - dp3) * slak;
-        if (th3 > th2 && th4 > th3) {
-          double ratio = (th4 - th3) / (th3 - th2);
-          if (ratio > 1.) dis4 = dis3 / ratio;
-          else dis3 = dis4 * ratio;
-        }
-        pnew[k - 1] = pnew[k - 1] + dis3;
-        pnew[k] = pnew[k] - dis4;
-      }
-    }
-  }
 }
 
 // dffusn_lev(exsmo, smoo_coeff, nvlp1, kbl+2, nvl): reads the regridded Exner
@@ -149,15 +122,13 @@ __global__ void __launch_bounds__(256) k_dffusn_lev(HybCols<V> s) {
 //    previous one stopped, which for non-decreasing targets is found by a
 //    binary search, so each lane integrates its own layer in the reference
 //    order (a lane-0 sweep takes over for non-monotone targets);
-//  * the excol fix and equilb change nothing unless their condition holds on
-//    the unmodified column somewhere; lane 0 then runs the sweep from the
-//    first such level;
+//  * the excol fix changes nothing unless its condition holds on the
+//    unmodified column somewhere; lane 0 then runs the sweep;
 //  * the two fill sweeps of pcwise: a cell's update ignores its neighbour
 //    whenever neighbour*1e-22 is provably below half an ulp of the cell's own
 //    term (bounded by the running maximum of the column); the remaining
 //    chains are resolved neighbour by neighbour in sweep order;
-//  * inflate, the top-of-column loop and the theta redistribution run on
-//    lane 0.
+//  * the top-of-column loop runs on lane 0.
 constexpr int HW = 4;   // columns (wavefronts) per block
 
 __device__ __forceinline__ void wsync() {
@@ -250,63 +221,6 @@ __device__ __forceinline__ float w_max_all(float x) {
   x = dpp_fmax<DPP_BCAST31, 0xc>(x);
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
-__device__ __forceinline__ int w_min_int(int x) {
-  for (int d = 1; d < 64; d <<= 1) x = min(x, __shfl_xor(x, d, 64));
-  return x;
-}
-
-// inflate (hybgen.F90:893-1007) for one column on lane 0, the per-level
-// constants prepared beforehand by all lanes: dp0b[k-1] = rd*dpsig(k)/p1000*
-// shrink (k = 1..nvl-1) and tap[k] = 1/(1+tq**2), tq = (nvl-k)/4 (k = 2..nvl),
-// each formed by the same operations as in inflate().
-__device__ void inflate_w(const double *dp0b, const double *tap, int nvl, double extop, double *exner) {
-  double dpsum = 0.;
-  int last = 1;
-  for (int k = 1; k <= nvl - 1; k++) {
-    double dp0 = dp0b[k - 1];
-    dpsum = dpsum + dp0;
-    const double exold = exner[k];
-    if (k <= KBL) {
-      last = k + 1;
-      exner[k] = exner[k - 1] - dp0;
-    } else {
-      if (k > last) {
-        const double p2 = ldexp(1., k - last);
-        dp0 = dp0 / dmin(10., 1.25 * p2);
-        dp0 = dmax(dp0, RD * 100. / P1000);
-      }
-      const double dp1 = cushn(dmax(0., exner[k - 1] - dmin(exold, exner[0] - dpsum)), dp0);
-      if (exner[k - 1] - dp1 < exold - THIN) {
-        if (k == last) last = k + 1;
-        exner[k] = dmax(extop, exner[k - 1] - dp1);
-      }
-    }
-  }
-  for (int k = nvl; k >= 2; k--) {
-    double q = exner[k - 1] / CP;
-    q = q * q * sqrt(q);
-    const double dp0 = RD * THKTOP / P1000 * tap[k] / q;
-    const double exold = exner[k - 1];
-    const double dp1 = cushn(dmax(0., exold - exner[k]), dp0);
-    if (exner[k] + dp1 > exold + THIN) exner[k - 1] = exner[k] + dp1;
-    if (exner[k - 1] < exner[k - 2] - dp0) break;
-  }
-}
-
-// all lanes: the per-level constants of inflate_w for surface pressure psurf
-__device__ __forceinline__ void inflate_prep(const double *dpsig, int nvl, double psurf, double *dp0b, double *tap,
-                                             int lane) {
-  const double top = .2;
-  const double shrink = dmin(1., (psurf / P1000 - top) / (1. - top));
-  for (int k = 1 + lane; k <= nvl; k += 64) {
-    if (k <= nvl - 1) dp0b[k - 1] = RD * ldc(dpsig, k - 1) / P1000 * shrink;
-    if (k >= 2) {
-      const double tq = .25 * (double)(nvl - k);
-      tap[k] = 1. / (1. + tq * tq);
-    }
-  }
-}
-
 // true when y*1e-22 cannot move t, for every |y| <= bound (|y*1e-22| < |t|*2^-55,
 // with margin for the growth of the bound along a sweep)
 __device__ __forceinline__ bool absorbs(double t, double bound) {
@@ -544,11 +458,13 @@ __device__ float pcwise_wf(int kk, const PcwGeomF &gm, float a, int lane) {
   return y;
 }
 
-// regrid_1d (hybgen.F90:207-512), one wavefront per column
-// With SPLIT the column-serial equilb and inflate are left to
-// k_regrid_tail, which runs them one thread per column with the column in
-// registers; the Exner function after the heat diffusion goes to sdot.
-template <typename V, bool SPLIT>
+// regrid_1d (hybgen.F90:207-512), one wavefront per column, up to the heat
+// diffusion; the Exner function goes to sdot.  The column-serial equilb and
+// inflate are left to k_regrid_tail, which runs them one thread per column with
+// the column in registers, at every layer count: on lane 0 of each column's
+// wavefront they leave 63 lanes idle (G6 x 50, FP64: 390 us with them on
+// lane 0, 101 us for the two kernels).
+template <typename V>
 __global__ void __launch_bounds__(64 * HW) k_regrid_w(HybCols<V> s, const StepCtl *ctl, int its) {
   __shared__ double sh[HW][7][LMAX];
   const int ncol = s.ncol, nvl = s.nvl, nvlp1 = nvl + 1;
@@ -566,8 +482,6 @@ __global__ void __launch_bounds__(64 * HW) k_regrid_w(HybCols<V> s, const StepCt
   const double tolrnce = 0.001;
   for (int k = lane; k < nvl; k += 64) thcol[k] = (double)TR(s.tr, 0, col, k);
   for (int k = lane; k < nvlp1; k += 64) excol[k] = L2(s.ex, col, k);
-  const double psurf = L2(s.pr, col, 0);
-  const double eqlb_slak = .1 * (double)its / (10. + (double)its);
   wsync();
   {
     bool t = false;
@@ -699,41 +613,16 @@ __global__ void __launch_bounds__(64 * HW) k_regrid_w(HybCols<V> s, const StepCt
     for (int k = 2 + lane; k <= nvlp1; k += 64) ev = ev || (exnew[k - 1] > exnew[k - 2] + THIN);
     if (!wany(ev)) break;
   }
-  if (SPLIT) {
-    for (int k = lane; k < nvlp1; k += 64) L2(s.sdot, col, k) = exnew[k];
-    return;
-  }
-  // equilb from the first level where it would move an interface
-  {
-    int first = 1 << 30;
-    for (int k = 3 + lane; k <= nvl - 2; k += 64) {
-      if (exnew[k - 3] > exnew[0] - THIN) continue;
-      const double dp1 = exnew[k - 3] - exnew[k - 2], dp2 = exnew[k - 2] - exnew[k - 1];
-      const double dp3 = exnew[k - 1] - exnew[k], dp4 = exnew[k] - exnew[k + 1], dp5 = exnew[k + 1] - exnew[k + 2];
-      if (dp2 > dp1 && dp4 > dp5) {
-        const double goal = .5 * (dp3 + dmin(dp2, dp4));
-        if (dp2 > goal && dp4 > goal) first = min(first, k);
-      }
-    }
-    first = w_min_int(first);
-    if (first <= nvl - 2) {
-      if (lane == 0) equilb(thnew, exnew, nvl, eqlb_slak, first);
-      wsync();
-    }
-  }
-  inflate_prep(s.dpsig, nvl, psurf, heatfx, oldth, lane);
-  wsync();
-  if (lane == 0) inflate_w(heatfx, oldth, nvl, CP * fim_pow(PTOP / P1000, RD / CP), exnew);
-  wsync();
-  for (int k = lane; k < nvlp1; k += 64) L2(s.sdot, col, k) = exnew[k];   // pre-smoothing Exner, kept in sdot
+  for (int k = lane; k < nvlp1; k += 64) L2(s.sdot, col, k) = exnew[k];
 }
 
-// remap_1d (hybgen.F90:515-789), one wavefront per column
-// With SPLIT, inflate has been applied to exsmo by k_remap_inflate, and the
-// theta redistribution is left to k_remap_theta: the remapped theta goes to
-// thbuf and the layer depths in p**(kappa+1), max(pk1new(k)-pk1new(k+1),
-// pk1new(1)*1e-6), to exsmo.
-template <typename V, bool SPLIT>
+// remap_1d (hybgen.F90:515-789), one wavefront per column.  inflate has been
+// applied to exsmo by k_remap_inflate, and the theta redistribution is left to
+// k_remap_theta (one thread per column, as k_regrid_tail; G6 x 50, FP64:
+// 440 us with both on lane 0, 216 us for the three kernels): the remapped
+// theta goes to thbuf and the layer depths in p**(kappa+1),
+// max(pk1new(k)-pk1new(k+1), pk1new(1)*1e-6), to exsmo.
+template <typename V>
 __global__ void __launch_bounds__(64 * HW) k_remap_w(HybCols<V> s, const StepCtl *ctl, int its) {
   __shared__ double sh[HW][7][LMAX];
   const int ncol = s.ncol, nvl = s.nvl, nvlp1 = nvl + 1, ntra = s.ntra;
@@ -747,7 +636,6 @@ __global__ void __launch_bounds__(64 * HW) k_remap_w(HybCols<V> s, const StepCtl
   if (ctl) its = load_ctl(ctl).its;
   double *prcol = sh[c][0], *pk1col = sh[c][1], *exnew = sh[c][2], *prnew = sh[c][3], *pk1new = sh[c][4],
          *th1 = sh[c][5], *exold = sh[c][6];
-  const double *targt = s.thetac;
   const double small = 1.e-6;
   for (int k = lane; k < nvlp1; k += 64) {
     const double eo = L2(s.ex, col, k);
@@ -756,11 +644,6 @@ __global__ void __launch_bounds__(64 * HW) k_remap_w(HybCols<V> s, const StepCtl
     prcol[k] = p;
     exnew[k] = L2(s.exsmo, col, k);
     pk1col[k] = eo * p / CP;
-  }
-  if (!SPLIT) {
-    inflate_prep(s.dpsig, nvl, L2(s.pr, col, 0), prnew, pk1new, lane);
-    wsync();
-    if (lane == 0) inflate_w(prnew, pk1new, nvl, CP * fim_pow(PTOP / P1000, RD / CP), exnew);
   }
   wsync();
   for (int k = lane; k < nvlp1; k += 64) {
@@ -827,29 +710,11 @@ __global__ void __launch_bounds__(64 * HW) k_remap_w(HybCols<V> s, const StepCtl
     if (live) th1[lane] = y;
   }
   wsync();
-  if (SPLIT) {
-    for (int k = lane; k < nvl; k += 64) {
-      C2(s.thbuf, col, k) = th1[k];
-      L2(s.exsmo, col, k) = dmax(pk1new[k] - pk1new[k + 1], pk1new[0] * small);
-    }
-  } else if (lane == 0) {
-    for (int k = nvl; k >= 3; k--) {
-      double dplo = dmax(pk1new[k - 2] - pk1new[k - 1], pk1new[0] * small);
-      double dpup = dmax(pk1new[k - 1] - pk1new[k], pk1new[0] * small);
-      double tha = th1[k - 2], thb = th1[k - 1];
-      double devilo = (tha - ldc(targt, k - 2)) * dplo;
-      double deviup = (thb - ldc(targt, k - 1)) * dpup;
-      if (deviup > 0. && devilo < 0.) {
-        th1[k - 2] = tha + dmin(deviup, -devilo) / dplo;
-        th1[k - 1] = thb - dmin(deviup, -devilo) / dpup;
-      } else if (deviup < 0. && devilo > 0.) {
-        th1[k - 2] = tha - dmin(devilo, -deviup) / dplo;
-        th1[k - 1] = thb + dmin(devilo, -deviup) / dpup;
-      }
-    }
+  for (int k = lane; k < nvl; k += 64) {
+    C2(s.thbuf, col, k) = th1[k];
+    L2(s.exsmo, col, k) = dmax(pk1new[k] - pk1new[k + 1], pk1new[0] * small);
   }
   wsync();
-  if (!SPLIT && lane < nvl) TR(s.tr, 0, col, lane) = (V)th1[lane];
   // exnew(k) = min over exnew(0..k): the reference's top-down monotonicity fix
   {
     const double m = w_prefix_min(lane < nvlp1 ? exnew[lane] : 1.e300, lane);
@@ -870,14 +735,16 @@ __global__ void __launch_bounds__(64 * HW) k_remap_w(HybCols<V> s, const StepCtl
 
 // ===========================================================================
 // The column-serial sweeps of hybgen, one thread per column with the column
-// in registers (NVL levels, every loop unrolled so each array index is a
-// compile-time constant), for the split form of the wave kernels above.  The
-// operations are those of equilb, inflate and the theta redistribution of
-// remap_1d, in the same order.
-template <int NVL>
-__device__ __forceinline__ void equilb_r(const double *targt, double *pnew, double slak) {
+// in registers (up to NVL levels, every loop unrolled so each array index is a
+// compile-time constant).  The operations are those of equilb, inflate and the
+// theta redistribution of remap_1d, in the same order.  nvl is a constant too
+// at NVL levels; below, the same kernels test it once per level, a scalar
+// branch.
+template <int NVL, bool FULL>
+__device__ __forceinline__ void equilb_r(const double *targt, int nvl, double *pnew, double slak) {
 #pragma unroll
   for (int k = 3; k <= NVL - 2; k++) {
+    if (!FULL && k > nvl - 2) continue;
     if (pnew[k - 3] > pnew[0] - THIN) continue;
     const double dp1 = pnew[k - 3] - pnew[k - 2];
     const double dp2 = pnew[k - 2] - pnew[k - 1];
@@ -902,14 +769,15 @@ __device__ __forceinline__ void equilb_r(const double *targt, double *pnew, doub
   }
 }
 
-template <int NVL>
-__device__ __forceinline__ void inflate_r(const double *dpsig, double psurf, double extop, double *exner) {
+template <int NVL, bool FULL>
+__device__ __forceinline__ void inflate_r(const double *dpsig, int nvl, double psurf, double extop, double *exner) {
   double dpsum = 0.;
   const double top = .2;
   const double shrink = dmin(1., (psurf / P1000 - top) / (1. - top));
   int last = 1;
 #pragma unroll
   for (int k = 1; k <= NVL - 1; k++) {
+    if (!FULL && k > nvl - 1) continue;
     double dp0 = RD * ldc(dpsig, k - 1) / P1000 * shrink;
     dpsum = dpsum + dp0;
     const double exold = exner[k];
@@ -929,50 +797,55 @@ __device__ __forceinline__ void inflate_r(const double *dpsig, double psurf, dou
       }
     }
   }
+  bool done = false;
 #pragma unroll
   for (int k = NVL; k >= 2; k--) {
+    if (done || (!FULL && k > nvl)) continue;
     double q = exner[k - 1] / CP;
     q = q * q * sqrt(q);
-    const double tq = .25 * (double)(NVL - k);
+    const double tq = .25 * (double)((FULL ? NVL : nvl) - k);
     const double tap = 1. / (1. + tq * tq);
     const double dp0 = RD * THKTOP / P1000 * tap / q;
     const double exold = exner[k - 1];
     const double dp1 = cushn(dmax(0., exold - exner[k]), dp0);
     if (exner[k] + dp1 > exold + THIN) exner[k - 1] = exner[k] + dp1;
-    if (exner[k - 1] < exner[k - 2] - dp0) break;
+    done = exner[k - 1] < exner[k - 2] - dp0;
   }
 }
 
 // equilb + inflate after the wave part of regrid_1d (Exner function in sdot)
-template <int NVL, typename V>
+template <int NVL, bool FULL, typename V>
 __global__ void __launch_bounds__(64) k_regrid_tail(HybCols<V> s, const StepCtl *ctl, int its, double extop) {
-  const int nvl = NVL, nvlp1 = NVL + 1;
+  const int nvl = FULL ? NVL : s.nvl, nvlp1 = nvl + 1;
   const int col = blockIdx.x * 64 + threadIdx.x;
   if (col >= s.ncol || (s.wet && !s.wet[col])) return;
   if (ctl) its = load_ctl(ctl).its;
   double ex[NVL + 1];
 #pragma unroll
-  for (int k = 0; k <= NVL; k++) ex[k] = L2(s.sdot, col, k);
+  for (int k = 0; k <= NVL; k++)
+    if (k <= nvl) ex[k] = L2(s.sdot, col, k);
   const double psurf = L2(s.pr, col, 0);
-  equilb_r<NVL>(s.thetac, ex, .1 * (double)its / (10. + (double)its));
-  inflate_r<NVL>(s.dpsig, psurf, extop, ex);
+  equilb_r<NVL, FULL>(s.thetac, nvl, ex, .1 * (double)its / (10. + (double)its));
+  inflate_r<NVL, FULL>(s.dpsig, nvl, psurf, extop, ex);
 #pragma unroll
-  for (int k = 0; k <= NVL; k++) L2(s.sdot, col, k) = ex[k];
-  (void)nvl;
+  for (int k = 0; k <= NVL; k++)
+    if (k <= nvl) L2(s.sdot, col, k) = ex[k];
 }
 
 // inflate of the smoothed Exner function at the start of remap_1d (in place)
-template <int NVL, typename V>
+template <int NVL, bool FULL, typename V>
 __global__ void __launch_bounds__(64) k_remap_inflate(HybCols<V> s, double extop) {
-  const int nvlp1 = NVL + 1;
+  const int nvl = FULL ? NVL : s.nvl, nvlp1 = nvl + 1;
   const int col = blockIdx.x * 64 + threadIdx.x;
   if (col >= s.ncol || (s.wet && !s.wet[col])) return;
   double ex[NVL + 1];
 #pragma unroll
-  for (int k = 0; k <= NVL; k++) ex[k] = L2(s.exsmo, col, k);
-  inflate_r<NVL>(s.dpsig, L2(s.pr, col, 0), extop, ex);
+  for (int k = 0; k <= NVL; k++)
+    if (k <= nvl) ex[k] = L2(s.exsmo, col, k);
+  inflate_r<NVL, FULL>(s.dpsig, nvl, L2(s.pr, col, 0), extop, ex);
 #pragma unroll
-  for (int k = 0; k <= NVL; k++) L2(s.exsmo, col, k) = ex[k];
+  for (int k = 0; k <= NVL; k++)
+    if (k <= nvl) L2(s.exsmo, col, k) = ex[k];
 }
 
 // one exchange of the theta redistribution of remap_1d (hybgen.F90:515-789,
@@ -998,13 +871,13 @@ __device__ __forceinline__ void theta_pair(double &tha, double &thb, double dplo
 // carries the upper layer of the pair that straddles two chunks, and the
 // result goes back to column-major tracer 1 through an LDS tile, so every
 // global access is coalesced.
-template <int NVL, typename V>
+template <int NVL, bool FULL, typename V>
 __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
-  constexpr int CH = 16, NCH = NVL / CH;
-  static_assert(NVL % CH == 0, "whole chunks");
+  constexpr int CH = 16;
   __shared__ double sth[CH][65], sdl[CH][65];
   __shared__ V sout[CH + 1][65];   // levels k0 .. k0+CH of the chunk being finished
-  const int nvl = NVL, nvlp1 = NVL + 1, ncol = s.ncol;
+  const int nvl = FULL ? NVL : s.nvl, nvlp1 = nvl + 1, ncol = s.ncol;
+  const int NCH = (nvl + CH - 1) / CH;   // the top chunk may be a part of one
   const int lane = threadIdx.x, c0 = blockIdx.x * 64;
   const int sl = lane & 15, sj = lane >> 4;
   double cth = 0., cdl = 0.;   // level k0+CH (the chunk above): theta still to be finalised, layer depth
@@ -1015,8 +888,9 @@ __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
     for (int i = 0; i < 16; i++) {
       const int c = i * 4 + sj;
       const int cc = min(c0 + c, ncol - 1);   // a partial last tile repeats its last column
-      sth[sl][c] = C2(s.thbuf, cc, k0 + sl);
-      sdl[sl][c] = L2(s.exsmo, cc, k0 + sl);
+      const int lev = FULL ? k0 + sl : min(k0 + sl, nvl - 1);   // levels above the column are not used
+      sth[sl][c] = C2(s.thbuf, cc, lev);
+      sdl[sl][c] = L2(s.exsmo, cc, lev);
     }
     wsync();
     double th[CH], dl[CH];
@@ -1032,6 +906,7 @@ __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
 #pragma unroll
     for (int j = CH - 2; j >= 0; j--) {
       if (k0 + j < 1) break;
+      if (!FULL && k0 + j + 1 > nvl - 1) continue;
       theta_pair(th[j], th[j + 1], dl[j], dl[j + 1], ldc(s.thetac, k0 + j), ldc(s.thetac, k0 + j + 1));
     }
     // levels k0+1 .. k0+CH-1 are final; k0 is carried (final in the bottom chunk)
@@ -1045,34 +920,29 @@ __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
 #pragma unroll
     for (int i = 0; i < 16; i++) {
       const int c = i * 4 + sj;
-      if (c0 + c < ncol && lev < NVL && (!s.wet || s.wet[c0 + c])) TR(s.tr, 0, c0 + c, lev) = sout[1 + sl][c];
+      if (c0 + c < ncol && lev < nvl && (!s.wet || s.wet[c0 + c])) TR(s.tr, 0, c0 + c, lev) = sout[1 + sl][c];
     }
     if (ch == 0 && c0 + lane < ncol && (!s.wet || s.wet[c0 + lane])) TR(s.tr, 0, c0 + lane, 0) = sout[0][lane];
     wsync();
   }
-  (void)nvl;
-  (void)nvlp1;
 }
 
 template <typename V>
 void launch_hybgen_cols(const HybCols<V> &h, const StepCtl *ctl, int its, hipStream_t st, hipEvent_t winds_ready) {
   const dim3 wg((h.ncol + HW - 1) / HW), wb(64, HW);
-  if (h.nvl == NVL_MAX && h.thbuf) {
-    const dim3 tg((h.ncol + 63) / 64), tb(64);
-    const double extop = CP * fim_pow(PTOP / P1000, RD / CP);
-    KT_LAUNCH("k_regrid", st, (k_regrid_w<V, true><<<wg, wb, 0, st>>>(h, ctl, its)));
-    KT_LAUNCH("k_regrid_tail", st, (k_regrid_tail<NVL_MAX, V><<<tg, tb, 0, st>>>(h, ctl, its, extop)));
-    KT_LAUNCH("k_dffusn_lev", st, k_dffusn_lev<V><<<(h.ncol + 3) / 4, dim3(64, 4), 0, st>>>(h));
-    KT_LAUNCH("k_remap_inflate", st, (k_remap_inflate<NVL_MAX, V><<<tg, tb, 0, st>>>(h, extop)));
-    if (winds_ready) (void)hipStreamWaitEvent(st, winds_ready, 0);
-    KT_LAUNCH("k_remap", st, (k_remap_w<V, true><<<wg, wb, 0, st>>>(h, ctl, its)));
-    KT_LAUNCH("k_remap_theta", st, (k_remap_theta<NVL_MAX, V><<<tg, tb, 0, st>>>(h)));
-    return;
-  }
-  KT_LAUNCH("k_regrid", st, (k_regrid_w<V, false><<<wg, wb, 0, st>>>(h, ctl, its)));
+  const dim3 tg((h.ncol + 63) / 64), tb(64);
+  const double extop = CP * fim_pow(PTOP / P1000, RD / CP);
+  const bool full = h.nvl == NVL_MAX;
+  KT_LAUNCH("k_regrid", st, (k_regrid_w<V><<<wg, wb, 0, st>>>(h, ctl, its)));
+  if (full) KT_LAUNCH("k_regrid_tail", st, (k_regrid_tail<NVL_MAX, true, V><<<tg, tb, 0, st>>>(h, ctl, its, extop)));
+  else KT_LAUNCH("k_regrid_tail", st, (k_regrid_tail<NVL_MAX, false, V><<<tg, tb, 0, st>>>(h, ctl, its, extop)));
   KT_LAUNCH("k_dffusn_lev", st, k_dffusn_lev<V><<<(h.ncol + 3) / 4, dim3(64, 4), 0, st>>>(h));
+  if (full) KT_LAUNCH("k_remap_inflate", st, (k_remap_inflate<NVL_MAX, true, V><<<tg, tb, 0, st>>>(h, extop)));
+  else KT_LAUNCH("k_remap_inflate", st, (k_remap_inflate<NVL_MAX, false, V><<<tg, tb, 0, st>>>(h, extop)));
   if (winds_ready) (void)hipStreamWaitEvent(st, winds_ready, 0);
-  KT_LAUNCH("k_remap", st, (k_remap_w<V, false><<<wg, wb, 0, st>>>(h, ctl, its)));
+  KT_LAUNCH("k_remap", st, (k_remap_w<V><<<wg, wb, 0, st>>>(h, ctl, its)));
+  if (full) KT_LAUNCH("k_remap_theta", st, (k_remap_theta<NVL_MAX, true, V><<<tg, tb, 0, st>>>(h)));
+  else KT_LAUNCH("k_remap_theta", st, (k_remap_theta<NVL_MAX, false, V><<<tg, tb, 0, st>>>(h)));
 }
 template void launch_hybgen_cols<float>(const HybCols<float> &, const StepCtl *, int, hipStream_t, hipEvent_t);
 

@@ -98,15 +98,16 @@ __global__ void __launch_bounds__(64 * BC) k_eb_w(EnsGrid g, EnsState s, EnsClas
 
 // fct3d.F90:127-140: massless cells filled from the layers above and below,
 // one thread per column and class-B tracer, the column in registers, loads
-// and stores staged through LDS in chunks of 16 levels.  Needs nvl == NVL.
-template <int NVL>
-__global__ void __launch_bounds__(64) k_eb_fill(EnsState s, EnsClassB b) {
+// and stores staged through LDS in chunks of 16 levels; below NVL levels the
+// layer count is tested once per level.
+template <int NVL, bool FULL>
+__global__ void __launch_bounds__(64) k_eb_fill(int nvl_, EnsState s, EnsClassB b) {
   constexpr int CH = 16, NCH = NVL / CH;
   static_assert(NVL % CH == 0, "whole chunks");
   __shared__ float sf[CH][65];
   __shared__ double sth[CH][65];
   if (!b_active(s, b.dtratio)) return;
-  const int nvl = NVL, ncol = s.ncol;
+  const int nvl = FULL ? NVL : nvl_, ncol = s.ncol;
   const int lane = threadIdx.x, c0 = blockIdx.x * 64, n = blockIdx.y;
   const float *trb = b.trb + (size_t)n * ncol * nvl;
   float *fld = b.fld + (size_t)n * ncol * nvl;
@@ -114,10 +115,11 @@ __global__ void __launch_bounds__(64) k_eb_fill(EnsState s, EnsClassB b) {
 #pragma unroll
   for (int ch = NCH - 1; ch >= 0; ch--) {
     const int k0 = ch * CH;
+    if (!FULL && k0 >= nvl) continue;
     __syncthreads();
     for (int i = 0; i < 16; i++) {
       const int cc = i * 4 + (lane >> 4), kk = lane & 15, gc = c0 + cc;
-      const bool in = gc < ncol;
+      const bool in = gc < ncol && (FULL || k0 + kk < nvl);
       sf[kk][cc] = in ? trb[(size_t)gc * nvl + k0 + kk] : 0.f;
       sth[kk][cc] = in ? b.dpinit[(size_t)gc * nvl + k0 + kk] : 1.;
     }
@@ -125,26 +127,29 @@ __global__ void __launch_bounds__(64) k_eb_fill(EnsState s, EnsClassB b) {
 #pragma unroll
     for (int kk = CH - 1; kk >= 0; kk--) {
       const int k = k0 + kk;
-      if (k == NVL - 1) {
+      if (!FULL && k >= nvl) continue;
+      if (k == (FULL ? NVL : nvl) - 1) {
         x[k] = sf[kk][lane];
       } else {
         const float t = (float)sth[kk][lane];
-        x[k] = (sf[kk][lane] * t + x[k + 1] * ONEMU) / (t + ONEMU);
+        x[k] = (sf[kk][lane] * t + x[k + 1 < NVL ? k + 1 : k] * ONEMU) / (t + ONEMU);
       }
     }
   }
 #pragma unroll
   for (int ch = 0; ch < NCH; ch++) {
     const int k0 = ch * CH;
+    if (!FULL && k0 >= nvl) continue;
     __syncthreads();
     for (int i = 0; i < 16; i++) {
       const int cc = i * 4 + (lane >> 4), kk = lane & 15, gc = c0 + cc;
-      sth[kk][cc] = gc < ncol ? b.dpinit[(size_t)gc * nvl + k0 + kk] : 1.;
+      sth[kk][cc] = gc < ncol && (FULL || k0 + kk < nvl) ? b.dpinit[(size_t)gc * nvl + k0 + kk] : 1.;
     }
     __syncthreads();
 #pragma unroll
     for (int kk = 0; kk < CH; kk++) {
       const int k = k0 + kk;
+      if (!FULL && k >= nvl) continue;
       if (k > 0) {
         const float t = (float)sth[kk][lane];
         x[k] = (x[k] * t + x[k - 1] * ONEMU) / (t + ONEMU);
@@ -154,15 +159,13 @@ __global__ void __launch_bounds__(64) k_eb_fill(EnsState s, EnsClassB b) {
     __syncthreads();
     for (int i = 0; i < 16; i++) {
       const int cc = i * 4 + (lane >> 4), kk = lane & 15, gc = c0 + cc;
-      if (gc < ncol) fld[(size_t)gc * nvl + k0 + kk] = sf[kk][cc];
+      if (gc < ncol && (FULL || k0 + kk < nvl)) fld[(size_t)gc * nvl + k0 + kk] = sf[kk][cc];
     }
   }
 }
 
-// fct3d.F90:141-260: (the massless-cell sweeps in lane 0 unless FILLED),
-// the parabolic fit of each layer and the vertical tracer flux over the
-// upstream slab
-template <bool FILLED>
+// fct3d.F90:141-260: the parabolic fit of each layer and the vertical tracer
+// flux over the upstream slab
 __global__ void __launch_bounds__(64 * BC) k_eb_vert(EnsGrid g, EnsState s, EnsClassB b) {
   __shared__ float sf[BC][NVL_MAX], sth[BC][NVL_MAX];
   __shared__ float sa[BC][NVL_MAX], sb[BC][NVL_MAX], sc[BC][NVL_MAX];
@@ -172,17 +175,12 @@ __global__ void __launch_bounds__(64 * BC) k_eb_vert(EnsGrid g, EnsState s, EnsC
   const int col = blockIdx.y * nip + ipn;
   const bool live = ipn < nip && k < nvl;       // every wave of the block reaches the barriers
   if (live) {
-    sf[c][k] = FILLED ? BTR(b.fld, n, col, k) : BTR(b.trb, n, col, k);
+    sf[c][k] = BTR(b.fld, n, col, k);
     sth[c][k] = (float)BC2(b.dpinit, col, k);
   }
   __syncthreads();
   float *f = sf[c];
   const float *th = sth[c];
-  if (!FILLED && k == 0 && ipn < nip) {
-    for (int kk = nvl - 2; kk >= 0; kk--) f[kk] = (f[kk] * th[kk] + f[kk + 1] * ONEMU) / (th[kk] + ONEMU);
-    for (int kk = 1; kk < nvl; kk++) f[kk] = (f[kk] * th[kk] + f[kk - 1] * ONEMU) / (th[kk] + ONEMU);
-  }
-  __syncthreads();
   if (live) {
     float a = f[k], bb = 0.f, cc = 0.f;
     if (k > 0 && k < nvl - 1) {
@@ -253,7 +251,6 @@ __global__ void __launch_bounds__(64 * BC) k_eb_vert(EnsGrid g, EnsState s, EnsC
     vfx = wk * amount / slab;
   }
   BTR(b.vfx, n, col, k) = vfx;
-  if (!FILLED) BTR(b.fld, n, col, k) = f[k];
 }
 
 // fct3d.F90:276-370: low-order and antidiffusive fluxes, local bounds, the
@@ -349,12 +346,10 @@ void ens_launch_class_b_step(const EnsGrid &g, const EnsState &s, const EnsClass
   const dim3 gt((g.d.nip + BC - 1) / BC, s.members, b.ntrb);
   KT_LAUNCH("eb_transp1", st, k_eb_transp1<<<gr, bl, 0, st>>>(g, s, b));
   KT_LAUNCH("eb_w", st, k_eb_w<<<gr, bl, 0, st>>>(g, s, b));
-  if (g.d.nvl == NVL_MAX) {
-    KT_LAUNCH("eb_fill", st, k_eb_fill<NVL_MAX><<<dim3((s.ncol + 63) / 64, b.ntrb), 64, 0, st>>>(s, b));
-    KT_LAUNCH("eb_vert", st, k_eb_vert<true><<<gt, bl, 0, st>>>(g, s, b));
-  } else {
-    KT_LAUNCH("eb_vert", st, k_eb_vert<false><<<gt, bl, 0, st>>>(g, s, b));
-  }
+  const dim3 fg((s.ncol + 63) / 64, b.ntrb);
+  if (g.d.nvl == NVL_MAX) KT_LAUNCH("eb_fill", st, (k_eb_fill<NVL_MAX, true><<<fg, 64, 0, st>>>(g.d.nvl, s, b)));
+  else KT_LAUNCH("eb_fill", st, (k_eb_fill<NVL_MAX, false><<<fg, 64, 0, st>>>(g.d.nvl, s, b)));
+  KT_LAUNCH("eb_vert", st, k_eb_vert<<<gt, bl, 0, st>>>(g, s, b));
   KT_LAUNCH("eb_lo", st, k_eb_lo<<<gt, bl, 0, st>>>(g, s, b));
   KT_LAUNCH("eb_clip", st, k_eb_clip<<<gt, bl, 0, st>>>(g, s, b));
   KT_LAUNCH("eb_transp0", st, k_eb_transp0<<<gr, bl, 0, st>>>(g, s, b, 0));

@@ -508,9 +508,8 @@ def test_restart_round_trip_then_steps_match_checker_bitwise(case, tmp_path):
 
 @pytest.mark.parametrize("flux_scheme,ntrb", [(1, 0), (2, 2)])
 def test_forty_layers_steps_match_checker_bitwise(oracle_lib, flux_scheme, ntrb):
-    """40 layers (the kernels' paths for nvl below the wavefront width: hybgen
-    with its serial sweeps in the column's wavefront, the fct3d sweeps in
-    lane 0): start-up plus 9 full steps identical to the checker."""
+    """40 layers (the kernels' paths for nvl below the wavefront width):
+    start-up plus 9 full steps identical to the checker."""
     from fimocn_subx_realtime_hera_apr2020_amd import fimhip
     from helpers import seeded_case
     O = oracle_lib
@@ -722,3 +721,34 @@ def test_r4_dropins_are_the_r8_path_rounded(case):
         assert a[0].value == np.float32(DT * 23. / 12.)
     finally:
         inst.close()
+
+
+@pytest.mark.parametrize("nvl", [10, 15, 17, 31, 32, 33, 47, 49, 63])
+def test_ragged_layer_counts_match_checker_bitwise(oracle_lib, nvl):
+    """Layer counts at the edges of the column kernels' 16-level chunks
+    (hybgen's and fct3d's serial sweeps, one thread per column): start-up plus
+    6 full steps with class-B transport every 2 steps, identical to the
+    checker."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip
+    from helpers import seeded_case
+    O = oracle_lib
+    g, st, th, ds = seeded_case(2, nvl=nvl, ntra=2)
+    st["trb"] = np.ascontiguousarray(_class_b_case(g, nvl=nvl, ntrb=2)["trb"])
+    print("case: G2 nvl=%d ntra=2 ntrb=2 6 full steps" % nvl, flush=True)
+    o = O.OracleRun(O.grid_arrays(g, nvl, DT, th, ds), nvl, 2, DT, pow_kind=1, ntrb=2, dtratio=2)
+    o.load(st)
+    o.init(True)
+    m = fimhip.Model(g, nvl, 2, DT, th, ds)
+    try:
+        m.set_class_b(2, 2)
+        m.load(st)
+        m.init_state(True)
+        for its in range(1, 7):
+            m.step(its, 0)
+            o.step(its, 0)
+        m.sync()
+        for f in ("us", "vs", "dp", "pr", "ex", "ph", "mp", "tr", "trdp", "ws", "sdot", "trb"):
+            got = m.download(f)
+            assert _same(got, o.a[f]), (f, rel_l2(got, o.a[f]))
+    finally:
+        m.close()
