@@ -96,21 +96,18 @@ def class_b_kernel_bytes(B):
     return {k: 8 * n for k, n in v.items()}
 
 
-def ens_kernel_bytes(T, fused=False):
+def ens_kernel_bytes(T):
     """The same for the mixed-precision kernels (4 B per FP32 value, 8 B per
-    FP64 value; inputs shared by the tracers of one launch counted once).
-    With the fused tracer transport edgvar3 reconstructs the thickness only."""
+    FP64 value; inputs shared by the tracers of one launch counted once)."""
     return {
         "e_edgvar1": 20 + 36,                # us vs tr1 (f32) pr (f64) -> normal wind edges, pressure gradient, step-start theta (f32)
-        # dp (f64) -> dp_edg; tracers 2..T -> trc_edg (the fused transport forms those itself)
-        "e_edgvar3": 32 if fused else 32 + 28 * (T - 1),
+        "e_edgvar3": 32,                     # dp -> its edge reconstructions
         "e_cnuity12": 104,                   # normal wind and dp edges, dp, dplo(of,vof) -> massfx, antifx, dplo, delp_lo, sums
         "e_cnuity3": 44,                     # in/outflow sums, delp_lo, dp, dp_tdcy(of,vof) -> r+, r-
         "e_cnuity45": 164,                   # antifx r+- massfx dp_tdcy dp pr pressure gradient u v -> massfx dp_tdcy dp pr ex omega
         "e_massadv1": 104,                   # normal wind and dp edges, dp, dp_tdcy(of,vof) -> q_star edges, q_min/max_out
         "e_massadv2": 156,                   # normal wind, q_star, bounds, dp_tdcy, dp, pressure gradient, u v -> massfx dp_tdcy dp pr ex omega
-        "e_trcadv1": 8 + 80 * T,             # massfx dp; per tracer trc_edg (not theta's) tr trdp trl -> antiflx trl lo sums
-        "e_trcadv2": 8 + 40 * T,
+        "e_trcadv12": 32 + 68 * T,           # massfx dp; per tracer tr trdp trl trc(of,vof) -> antiflx trl bounds r+ r-
         "e_trcadv3": 8 + 68 * T,
         "e_trc_fct": 32 + 40 * T,            # massfx dp; per tracer tr trdp trl(of,vof) trc(of,vof) -> tr trdp trl trc
         "e_momtum": 80,                      # u v dp ex mp, step-start theta, tendencies -> relvor tendency u2 v2
@@ -389,7 +386,7 @@ def run_ens(a, grid, th, ds, fimhip):
     prof = e.profile_report()
     e.profile(False)
     cells = M * grid.nip * a.nvl
-    kb = ens_kernel_bytes(a.ntra, e.fused())
+    kb = ens_kernel_bytes(a.ntra)
     value = cells * a.steps / wall
     b_step = ens_step_bytes(a.ntra, a.mode)
     tr_of = (lambda k: pmc_traffic(k, "ens16", a)) if a.mode == 0 else None

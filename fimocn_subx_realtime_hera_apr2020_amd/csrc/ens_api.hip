@@ -49,11 +49,12 @@ struct fimhip_ens {
   int graph_modes[2] = {-1, -1};
   KTimer *kt = nullptr;
   // the tracer FCT as one kernel over patches with recomputed halo rings
-  // (fct_tiles.hip), or as the three-kernel chain with edgvar3's tracer
-  // reconstructions in HBM; both give the same bits.  The chain is the
+  // (fct_tiles.hip), or as the
+  // chain of two (trcadv12, trcadv3); both give the same bits.  The chain is the
   // default (faster at 16 members x G7 x 64 on MI355X); the autotuner keeps
   // whichever form measures faster
   bool fused = false;
+  HostGrid hg;                       // neighbour tables, for the fused form's patches
 };
 
 static void drop_graph(fimhip_ens *e) {
@@ -104,6 +105,7 @@ extern "C" int fimhip_ens_create(const fimhip_grid_desc *gd, int members, int de
   e->lat.assign(gd->lat, gd->lat + nip);
   e->lon.assign(gd->lon, gd->lon + nip);
   for (int k = 0; k < EK_NKERNELS; k++) e->tile[k] = 2;   // 4 columns per block, no swizzle
+  e->tile[EK_TRCADV12] = 4;      // 8 wavefronts per block, XCD-contiguous order
   e->tile[EK_TRCFCT] = 4;        // 32 levels and 16 wavefronts per block, XCD-contiguous order
   if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&e->stream) != hipSuccess) {
     delete e;
@@ -137,9 +139,9 @@ extern "C" int fimhip_ens_create(const fimhip_grid_desc *gd, int members, int de
       {&s.tr_alt, cz * ntra}, {&s.trdp_alt, cz * ntra},
       {&s.u_tdcy, 3 * cz}, {&s.v_tdcy, 3 * cz}, {&s.dpl_tdcy, 3 * cz}, {&s.trc_tdcy, 3 * cz * ntra},
       {&s.trl_tdcy, 3 * cz * ntra}, {&s.massfx, ez}, {&s.ws, cz}, {&s.relvor, cz},
-      {&s.vn_edg, ez}, {&s.dp_edg, ez}, {&s.pgx, cz}, {&s.pgy, cz}, {&s.trc_edg, ez * (ntra > 1 ? ntra - 1 : 1)}, {&s.th0, cz},
+      {&s.vn_edg, ez}, {&s.dp_edg, ez}, {&s.pgx, cz}, {&s.pgy, cz}, {&s.th0, cz},
       {&s.antifx, ez}, {&s.delp_lo, cz}, {&s.r_plus, cz}, {&s.r_mnus, cz}, {&s.antiflx, ez * ntra},
-      {&s.trcr_lo, cz * ntra}, {&s.trmax, cz * ntra}, {&s.trmin, cz * ntra}, {&s.tr_rp, cz * ntra},
+      {&s.trmax, cz * ntra}, {&s.trmin, cz * ntra}, {&s.tr_rp, cz * ntra},
       {&s.tr_rm, cz * ntra}};
   struct { double **p; size_t n; } f64[] = {
       {&s.dp, cz}, {&s.pr, lz}, {&s.ex, lz}, {&s.ph, lz}, {&s.mp, cz}, {&s.sdot, lz}, {&s.exsmo, lz},
@@ -150,12 +152,16 @@ extern "C" int fimhip_ens_create(const fimhip_grid_desc *gd, int members, int de
     if ((r = a.alloc(x.p, x.n))) { fimhip_ens_destroy(e); return r; }
   if ((r = a.alloc(&s.ctl, 1))) { fimhip_ens_destroy(e); return r; }
   {
-    TileHost th;
-    if ((r = ens_build_tiles(hg, nip, th)) || (r = ens_upload_tiles(a, th, g.tiles))) {
+    TileHost t;
+    if ((r = ens_build_tiles(hg, nip, TRC_LIMITS, t)) || (r = ens_upload_tiles(a, t, g.ptiles)) ||
+        (r = ens_make_core(a, t, g))) {
       fimhip_ens_destroy(e);
       return r;
     }
   }
+  e->hg.prox.swap(hg.prox);
+  e->hg.proxs.swap(hg.proxs);
+  e->hg.nprox.swap(hg.nprox);
   // staging member (FP64, plain layout)
   const size_t mcz = (size_t)nip * nvl, mlz = (size_t)nip * (nvl + 1);
   DevState &t = e->stage;
@@ -274,7 +280,6 @@ extern "C" int fimhip_ens_init_state(fimhip_ens *e, int init_hybgen) {
 static void enqueue_step(fimhip_ens *e, int mode, bool side) {
   const EnsGrid &g = e->g;
   EnsState s = e->s;
-  s.edg3_ntr = e->fused ? 0 : e->ntra - 1;
   hipStream_t st = e->stream, sd = e->side;
   ens_launch_abstart(s, e->dt, st);
   if (side) {
@@ -300,7 +305,8 @@ static void enqueue_step(fimhip_ens *e, int mode, bool side) {
     std::swap(s.tr, s.tr_alt);         // the rest of the step works on the new tracers
     std::swap(s.trdp, s.trdp_alt);
   } else {
-    for (int k = EK_TRCADV1; k <= EK_TRCADV3; k++) ens_launch(k, e->tile[k], g, s, st);
+    ens_launch(EK_TRCADV12, e->tile[EK_TRCADV12], g, s, st);
+    ens_launch(EK_TRCADV3, e->tile[EK_TRCADV3], g, s, st);
   }
   // momtum needs nothing of the tracer transport; it runs beside hybgen's
   // column kernels up to the remap (latency-bound, so the two share the
@@ -357,8 +363,21 @@ extern "C" int fimhip_ens_step(fimhip_ens *e, int nsteps, int mode) {
   return FIMHIP_OK;
 }
 
+// the fused form's patches, built when it is first asked for
+static int need_fused_tiles(fimhip_ens *e) {
+  if (e->g.tiles.npatch) return 0;
+  TileHost t;
+  int r = ens_build_tiles(e->hg, e->nip, FCT_LIMITS, t);
+  return r ? r : ens_upload_tiles(e->arena, t, e->g.tiles);
+}
+
 extern "C" int fimhip_ens_set_fused(fimhip_ens *e, int on) {
   if (!e) return FIMHIP_EINVAL;
+  HIPCHK(hipSetDevice(e->device));
+  if (on) {
+    const int r = need_fused_tiles(e);
+    if (r) return r;
+  }
   if (e->fused != (on != 0)) drop_graph(e);
   e->fused = on != 0;
   return FIMHIP_OK;
@@ -582,15 +601,15 @@ extern "C" int fimhip_ens_get_tile(const fimhip_ens *e, int kernel) {
 // Autotuner: for each launch shape in turn, every kernel runs with that
 // shape for 'reps' steps of the given mode under event timing; each kernel
 // then keeps the shape with the least mean time.  Both forms of the tracer
-// transport are swept (the three-kernel chain with edgvar3's tracer
-// reconstructions, then the fused kernel with edgvar3 for the thickness only),
-// and the form whose transport kernels sum to less time is kept.  The steps
-// advance the state, so callers re-create or reload it afterwards.  times
-// (optional) receives EK_NKERNELS x ENS_NTILES mean milliseconds (edgvar3's
-// row from the form kept).
+// transport are swept (trcadv12 and trcadv3, then the fused kernel), and the
+// form whose transport kernels sum to less time is kept.  The steps advance
+// the state, so callers re-create or reload it afterwards.  times (optional)
+// receives EK_NKERNELS x ENS_NTILES mean milliseconds.
 extern "C" int fimhip_ens_autotune(fimhip_ens *e, int mode, int reps, double *times) {
   if (!e || reps < 1 || (mode != 0 && mode != 1)) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(e->device));
+  const int rt = need_fused_tiles(e);
+  if (rt) return rt;
   const int nt = EK_NKERNELS * ENS_NTILES;
   std::vector<double> best[2], tab[2];
   std::vector<int> pick[2];
@@ -618,13 +637,11 @@ extern "C" int fimhip_ens_autotune(fimhip_ens *e, int mode, int reps, double *ti
     }
   }
   e->kt = saved;
-  const double chain = best[0][EK_EDGVAR3] + best[0][EK_TRCADV1] + best[0][EK_TRCADV2] + best[0][EK_TRCADV3];
-  const double fused = best[1][EK_EDGVAR3] + best[1][EK_TRCFCT];
+  const double chain = best[0][EK_TRCADV12] + best[0][EK_TRCADV3], fused = best[1][EK_TRCFCT];
   const int fsel = fused < chain ? 1 : 0;
   e->fused = fsel == 1;
   for (int k = 0; k < EK_NKERNELS; k++) {
-    // edgvar3 does different work in the two forms; the other kernels the same
-    const int f = (k == EK_EDGVAR3 || best[fsel][k] <= best[1 - fsel][k]) ? fsel : 1 - fsel;
+    const int f = best[fsel][k] <= best[1 - fsel][k] ? fsel : 1 - fsel;
     e->tile[k] = pick[f][k];
     if (times)
       for (int t = 0; t < ENS_NTILES; t++) times[k * ENS_NTILES + t] = tab[f][k * ENS_NTILES + t];

@@ -17,9 +17,8 @@
 // index col = member * nip + cell (ncol = members * nip):
 //   cell (nvl, ncol)   level (nvl+1, ncol)   edge (nvl, 6, ncol)
 //   tracer (nvl, ncol, ntra)   AB (nvl, ncol, 3)   tracer AB (nvl, ncol, 3, ntra)
-//   tracer edge (nvl, 6, ncol, ntra - 1) for tracers 2..ntra (theta's edge
-//   values are formed where they are used); the mass flux keeps only the
-//   current slot.
+// (the tracers' edge values are formed where they are used); the mass flux
+// keeps only the current slot.
 #pragma once
 #include <array>
 #include <vector>
@@ -38,11 +37,15 @@ struct Arena;
 // neighbours 4-5 and its edge count (8 bits each); the neighbours' indices of
 // the shared edges, proxs (4 bits each).  The local indices are set for
 // rings 0-2 only.
+constexpr int CORE_ROW = 108;
 struct EnsTiles {
   int npatch;
   const int *off;      // (npatch + 1) first tile cell of each patch
   const int4 *cnt;     // (npatch) n0, n1, n2, n3
   const int4 *ent;
+  const int *core_row; // (CORE_ROW, nip), see k_core_rows in fct_tiles.hip
+  bool cyclic;         // every cell's slots run around it in the same sense
+  int r_max, lo_max;   // most cells of a patch in rings 0-1 and 0-2
 };
 
 // FP32 copies of the grid metrics (the reference stores them in FP32).
@@ -51,6 +54,7 @@ struct EnsGrid {
   const float *cs, *sn, *svc, *sve, *sideln, *hfcoef;
   const float *area, *rarea, *corio, *grndspd, *dfflen;
   EnsTiles tiles;            // the patch partition of the fused tracer FCT
+  EnsTiles ptiles;           // and that of trcadv12, with its core rows
 };
 
 struct EnsState {
@@ -63,13 +67,12 @@ struct EnsState {
   double *dp_tdcy;
   float *trc_tdcy, *trl_tdcy;
   float *massfx, *ws, *relvor;
-  float *vn_edg, *dp_edg, *trc_edg;   // vn_edg: normal edge wind; trc_edg: tracers 2..ntra
+  float *vn_edg, *dp_edg;             // vn_edg: normal edge wind
   float *pgx, *pgy;                   // the edge-pressure line integrals of cnuity5 (per cell-level)
   float *th0;                                  // theta at the start of the step
   float *antifx, *delp_lo, *r_plus, *r_mnus;
-  float *antiflx, *trcr_lo, *trmax, *trmin, *tr_rp, *tr_rm;
+  float *antiflx, *trmax, *trmin, *tr_rp, *tr_rm;
   StepCtl *ctl;
-  int edg3_ntr;                       // tracers 2..edg3_ntr+1 reconstructed by edgvar3 (0: thickness only)
   // Land/sea mask per column (0 = land), or null (every column wet).  An edge
   // carries mass and tracer flux only if both of its cells are wet (as the
   // ocean's continuity gates its fluxes, hycom_cnuity.F90:100-125); a land
@@ -88,8 +91,8 @@ inline int tile_cols(int t) { return 1 << (t & 3); }
 inline bool tile_swz(int t) { return (t >> 2) & 1; }
 
 enum EnsKernel {
-  EK_EDGVAR1 = 0, EK_EDGVAR3, EK_CNUITY12, EK_CNUITY3, EK_CNUITY45, EK_TRCADV1, EK_TRCADV2,
-  EK_TRCADV3, EK_MOMTUM, EK_HYSTAT, EK_MASSADV1, EK_MASSADV2, EK_TRCFCT, EK_NKERNELS
+  EK_EDGVAR1 = 0, EK_EDGVAR3, EK_CNUITY12, EK_CNUITY3, EK_CNUITY45, EK_TRCADV12, EK_TRCADV3,
+  EK_MOMTUM, EK_HYSTAT, EK_MASSADV1, EK_MASSADV2, EK_TRCFCT, EK_NKERNELS
 };
 extern const char *const ens_kernel_names[EK_NKERNELS];
 
@@ -116,9 +119,14 @@ struct TileHost {
   std::vector<int> off;
   std::vector<std::array<int, 4>> cnt, ent;
 };
-int ens_build_tiles(const HostGrid &h, int nip, TileHost &out);
+struct TileLimits { int core, r, lo, tile; };  // most cells in the core, rings 0-1, 0-2, 0-3
+constexpr TileLimits TRC_LIMITS = {48, 84, 124, 1 << 30};   // trcadv12's patches: three blocks per CU
+constexpr TileLimits FCT_LIMITS = {FCT_CORE_MAX, FCT_R_MAX, FCT_LO_MAX, FCT_TILE_MAX};
+int ens_build_tiles(const HostGrid &h, int nip, const TileLimits &lim, TileHost &out);
 int ens_upload_tiles(Arena &a, const TileHost &t, EnsTiles &d);
+int ens_make_core(Arena &a, const TileHost &t, EnsGrid &g);   // g.ptiles' core rows
 // the fused tracer FCT: reads s.tr / s.trdp, writes s.tr_alt / s.trdp_alt
+void ens_launch_trcadv12(int tile, const EnsGrid &g, const EnsState &s, hipStream_t st);
 void ens_launch_trc_fct(int tile, const EnsGrid &g, const EnsState &s, hipStream_t st);
 
 void ens_launch_abstart(const EnsState &s, double dt, hipStream_t st);

@@ -27,6 +27,7 @@
 // update in the same launch, so the kernel reads one buffer and writes the
 // other of a pair (the instance alternates them every step).
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "ens_internal.h"
@@ -38,12 +39,12 @@ namespace fimhip {
 // host: patches and their halo rings
 //
 // Patches grow breadth-first from the lowest unassigned cell over unassigned
-// cells, up to FCT_CORE_MAX cells; the three rings around the patch are the
+// cells, up to lim.core cells; the three rings around the patch are the
 // cells at neighbour distance 1, 2 and 3 from it, each ring in index order.
 // A patch whose rings would exceed the LDS tile gives up its last cells.
 // On the IJ-ordered icosahedral grids this gives compact, roughly hexagonal
 // patches (the three rings hold about twice the core's cells).
-int ens_build_tiles(const HostGrid &h, int nip, TileHost &out) {
+int ens_build_tiles(const HostGrid &h, int nip, const TileLimits &lim, TileHost &out) {
   std::vector<int> asg(nip, -1), mark(nip, -1);
   out.off.assign(1, 0);
   out.cnt.clear();
@@ -56,12 +57,12 @@ int ens_build_tiles(const HostGrid &h, int nip, TileHost &out) {
     q.assign(1, seed);
     ++stamp;
     mark[seed] = stamp;
-    for (size_t qi = 0; qi < q.size() && (int)core.size() < FCT_CORE_MAX; qi++) {
+    for (size_t qi = 0; qi < q.size() && (int)core.size() < lim.core; qi++) {
       const int c = q[qi];
       int nb[NPP];
       for (int e = 0; e < NPP; e++) nb[e] = h.prox[(size_t)c * NPP + e];
       std::sort(nb, nb + NPP);
-      for (int e = 0; e < NPP && (int)core.size() < FCT_CORE_MAX; e++) {
+      for (int e = 0; e < NPP && (int)core.size() < lim.core; e++) {
         const int x = nb[e];
         if (asg[x] >= 0 || mark[x] == stamp) continue;
         mark[x] = stamp;
@@ -85,7 +86,7 @@ int ens_build_tiles(const HostGrid &h, int nip, TileHost &out) {
       }
       const int n0 = (int)ring[0].size(), n1 = n0 + (int)ring[1].size(), n2 = n1 + (int)ring[2].size(),
                 n3 = n2 + (int)ring[3].size();
-      if (n1 <= FCT_R_MAX && n2 <= FCT_LO_MAX && n3 <= FCT_TILE_MAX) {
+      if (n1 <= lim.r && n2 <= lim.lo && n3 <= lim.tile) {
         // local indices of the tile cells, and the neighbour table of rings 0-2
         std::vector<int> cells;
         for (int r = 0; r < 4; r++) cells.insert(cells.end(), ring[r].begin(), ring[r].end());
@@ -128,7 +129,7 @@ int ens_upload_tiles(Arena &a, const TileHost &t, EnsTiles &d) {
   d.off = off;
   d.cnt = c;
   d.ent = e;
-  return FIMHIP_OK;
+  return hipStreamSynchronize(a.stream) == hipSuccess ? FIMHIP_OK : FIMHIP_EHIP;   // the host tables go out of scope
 }
 
 }  // namespace fimhip
@@ -145,7 +146,7 @@ extern "C" int fimhip_ens_patches(const fimhip_grid_desc *gd, int *sizes, int *c
   int r = host_grid_prepare(gd, h);
   if (r) return r;
   TileHost t;
-  if ((r = ens_build_tiles(h, gd->nip, t))) return r;
+  if ((r = ens_build_tiles(h, gd->nip, FCT_LIMITS, t))) return r;
   sizes[0] = (int)t.cnt.size();
   sizes[1] = (int)t.ent.size();
   if (cnt) {
@@ -206,6 +207,13 @@ __device__ __forceinline__ float fct_theta_edge(float thi, float thx, float tht,
   if (nbt > nbl) { const float t = ta; ta = tb; tb = t; }
   return (2.f * (thi + thx) + ta + tb) * (1.f / 6.f);
 }
+
+// The donor-cell value of an edge with mass flux m out of the cell: the
+// low-order flux is m * upwind, and the antidiffusive flux m * (te - upwind),
+// each one rounding on both sides of the edge (the reference forms
+// .5*((m+|m|)*t - (|m|-m)*tx), the same product, and the difference of the two
+// fluxes).
+__device__ __forceinline__ float fct_upwind(float m, float ti, float tx) { return m >= 0.f ? ti : tx; }
 
 __device__ __forceinline__ float fct_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
@@ -282,17 +290,14 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
   for (int e = 0; e < NP; e++) v[e] = Str[l[e] * 64 + lane];
   const float rar = ldc(g.rarea, cell);
   const float a1 = (float)c.ab1, a2 = (float)c.ab2, a3 = (float)c.ab3;
-  float acc = 0.f, mx = ti, mn = ti, fl[NP];
+  float acc = 0.f, mx = ti, mn = ti;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
     mx = fmaxf(mx, v[e]);
     mn = fminf(mn, v[e]);
   }
 #pragma unroll
-  for (int e = 0; e < NP; e++) {
-    fl[e] = .5f * ((m[e] + fabsf(m[e])) * ti - (fabsf(m[e]) - m[e]) * v[e]);
-    acc = acc + fl[e];
-  }
+  for (int e = 0; e < NP; e++) acc = acc + m[e] * fct_upwind(m[e], ti, v[e]);
   const float tlo = -acc * rar;
   const float lo = tdp0 + a1 * tlo + a2 * tlo_of + a3 * tlo_vof;
   mx = fmaxf(0.f, mx);
@@ -317,9 +322,9 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
     for (int j = 0; j < NP; j++) d[j] = v[j] - ti;
 #pragma unroll
     for (int e = 0; e < NP; e++) {
-      float ac = 0.f;
+      float ac = 0.f;      // both cells' sums start at the shared edge's slot
 #pragma unroll
-      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[j], FHF(cell, e, j), ac);
+      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[(e + j) % NP], FHF(cell, e, (e + j) % NP), ac);
       const float eo = ti + ac;
       const int4 ex = Sent[l[e]];
       const int xcell = uni(ex.x), xs = uni(eslot(en, e)), xnp = uni(enp(ex));
@@ -327,7 +332,8 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
       float ax = 0.f;
 #pragma unroll
       for (int j = 0; j < NPP; j++) {
-        if (j < xnp) ax = __builtin_fmaf(Str[uni(lnb(ex, j)) * 64 + lane] - tx, FHF(xcell, xs, j), ax);
+        const int jj = xs + j < xnp ? xs + j : xs + j - xnp;
+        if (j < xnp) ax = __builtin_fmaf(Str[uni(lnb(ex, jj)) * 64 + lane] - tx, FHF(xcell, xs, jj), ax);
       }
       const float en_ = tx + ax;
       te[e] = .5f * (eo + en_);
@@ -336,7 +342,7 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
   float sp = 0.f, sm = 0.f;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
-    const float a = m[e] * te[e] - fl[e];
+    const float a = m[e] * (te[e] - fct_upwind(m[e], ti, v[e]));
     a_out[e] = a;
     sp = sp - fminf(0.f, a);
     sm = sm + fmaxf(0.f, a);
@@ -578,6 +584,330 @@ void ens_launch_trc_fct(int tile, const EnsGrid &g, const EnsState &s, hipStream
   if (tg == 4) launch_fct_tg<4>(tile, g, s, st);
   else if (tg == 2) launch_fct_tg<2>(tile, g, s, st);
   else launch_fct_tg<1>(tile, g, s, st);
+}
+
+// ---------------------------------------------------------------------------
+// trcadv1 and trcadv2 of the tracer transport's chain as one kernel over
+// patches, with edgvar3's tracer reconstructions formed on the way
+// (trcadv_compute.F90:19-240, edgvar3.F90:65-132): a block takes one patch of
+// one member for one tracer, lane = level.  It stages the tracer of rings 0-2
+// in LDS, forms the bounded low-order tracer of rings 0-1 (kept in LDS; the
+// core's tendency is stored), then, after a barrier, the core's two-sided
+// edge values, antidiffusive fluxes (stored for trcadv3) and their sums, the
+// local bounds and the limiter ratios.  Each cell's operations are those of
+// the fused kernel above, in the same order, so the two forms of the
+// transport have the same bits.
+//
+// What bounds it: HBM traffic, 304 B per cell-level for 4 tracers plus the
+// halo, nearly half of it writes, at 4.6 TB/s (a large copy reaches 4.75).  As
+// three kernels (edgvar3's reconstructions stored and read back, the
+// low-order tracer stored, the mass flux read twice) it moved 620 B.  8
+// members x G7 x 64 x 4 tracers: 9.75 -> 7.20 ms; 16 x G5: 1.20 -> 0.94 ms; G6
+// with 20 tracers: 1.65 -> 1.18 ms; 3 x G4 x 38 x 3 tracers: 42 -> 40 us.
+// What got it there:
+//  * the cells' coefficients and stencil offsets come one row per cell by a
+//    vector load, a cell ahead, and are handed out by v_readlane: as scalar
+//    loads they missed the scalar cache and each batch waited about 1500
+//    cycles (9.0 ms);
+//  * of a neighbour's six stencil cells three are in registers (the cell
+//    itself and the two cells at the edge's ends);
+//  * the mass fluxes and tendencies are loaded two cells ahead;
+//  * every tracer and member of a patch runs in turn on one XCD, whose L2
+//    then holds the patch's rows and mass fluxes (8.0 ms in block order);
+//  * patches of up to 48 cells, 84 in rings 0-1 and 124 in rings 0-2, so that
+//    three blocks of 8 wavefronts fit a CU's LDS (cores of 64: two blocks, 8.1
+//    ms; of 32: 7.7 ms; four blocks at 64 VGPRs: 8.0 ms, spills).
+
+// a tile entry of the wavefront's j-th cell, which lane j holds
+__device__ __forceinline__ int4 wave_ent(const int4 &ev, int j) {
+  return make_int4(__builtin_amdgcn_readlane(ev.x, j), __builtin_amdgcn_readlane(ev.y, j),
+                   __builtin_amdgcn_readlane(ev.z, j), __builtin_amdgcn_readlane(ev.w, j));
+}
+
+struct TileInA {
+  float m[NPP], tdp0, lo_of, lo_vof;
+  double dp;
+};
+__device__ __forceinline__ TileInA tile_load_a(const EnsState &s, const StepCtl &c, int nvl, int col, size_t toff,
+                                               size_t aoff, int k) {
+  const int ncol = s.ncol;
+  TileInA r;
+#pragma unroll
+  for (int e = 0; e < NPP; e++) r.m[e] = EE(s.massfx, col, e, k);
+  r.tdp0 = TRV(s.trdp, col);
+  r.lo_of = TAB(s.trl_tdcy, c.of - 1, col);
+  r.lo_vof = TAB(s.trl_tdcy, c.vof - 1, col);
+  r.dp = EC(s.dp, col, k);
+  return r;
+}
+struct TileInB {
+  float m[NPP], to, tv;
+  double dp;
+};
+__device__ __forceinline__ TileInB tile_load_b(const EnsState &s, const StepCtl &c, int nvl, int col, size_t aoff,
+                                               int k) {
+  const int ncol = s.ncol;
+  TileInB r;
+#pragma unroll
+  for (int e = 0; e < NPP; e++) r.m[e] = EE(s.massfx, col, e, k);
+  r.to = TAB(s.trc_tdcy, c.of - 1, col);
+  r.tv = TAB(s.trc_tdcy, c.vof - 1, col);
+  r.dp = EC(s.dp, col, k);
+  return r;
+}
+// LDS value of tile cell l at the lane's level
+__device__ __forceinline__ float lds_at(const float *a, int byte_off, int k) {
+  return *(const float *)((const char *)a + byte_off + 4 * k);
+}
+
+template <int NP>
+__device__ __forceinline__ float tile_lo(const StepCtl &c, const int4 &en, int i, int k, float rar, const TileInA &in,
+                                         const float *Str, float *Slo) {
+  float v[NP];
+  const float rdp = fct_rcp(fmaxf(1.e-11f, (float)in.dp));
+  const float ti = Str[i * 64 + k];
+#pragma unroll
+  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, lnb(en, e) << 8, k);
+  const float a1 = (float)c.ab1, a2 = (float)c.ab2, a3 = (float)c.ab3;
+  float acc = 0.f, mx = ti, mn = ti;
+#pragma unroll
+  for (int e = 0; e < NP; e++) {
+    mx = fmaxf(mx, v[e]);
+    mn = fminf(mn, v[e]);
+    acc = acc + in.m[e] * fct_upwind(in.m[e], ti, v[e]);
+  }
+  const float tlo = -acc * rar;
+  const float lo = in.tdp0 + a1 * tlo + a2 * in.lo_of + a3 * in.lo_vof;
+  Slo[i * 64 + k] = fmaxf(fmaxf(0.f, mn), fminf(fmaxf(0.f, mx), lo * rdp));
+  return tlo;
+}
+
+// word w of a core row that the wavefront holds two words a lane
+__device__ __forceinline__ int row_i(const int2 &row, int w) {
+  return __builtin_amdgcn_readlane(w & 1 ? row.y : row.x, w >> 1);
+}
+__device__ __forceinline__ float row_f(const int2 &row, int w) { return __int_as_float(row_i(row, w)); }
+
+template <int NP, bool CYC>
+__device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, const StepCtl &c, int cell, int i, int t,
+                                          int col, size_t toff, int k, float area, const int2 &row, const TileInB &in,
+                                          const float *Str, const float *Slo) {
+  const int nvl = g.d.nvl, ncol = s.ncol;
+  float v[NP], te[NP];
+  const float dp = (float)in.dp;
+  const float ti = Str[i * 64 + k], lo = Slo[i * 64 + k];
+#pragma unroll
+  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, 102 + e), k);
+  if (t == 0) {
+#pragma unroll
+    for (int e = 0; e < NP; e++) {
+      const int et = (e + NP - 1) % NP, el = (e + 1) % NP;
+      te[e] = fct_theta_edge(ti, v[e], v[et], v[el], ldc(g.d.prox, cell * NPP + et), ldc(g.d.prox, cell * NPP + el));
+    }
+  } else {
+    float d[NP];
+#pragma unroll
+    for (int j = 0; j < NP; j++) d[j] = v[j] - ti;
+#pragma unroll
+    for (int e = 0; e < NP; e++) {
+      float ac = 0.f, ax = 0.f;
+#pragma unroll
+      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[(e + j) % NP], row_f(row, e * NPP + (e + j) % NP), ac);
+      ax = -d[e] * row_f(row, 36 + e * NPP);
+#pragma unroll
+      for (int r = 1; r < NPP; r++) {
+        const float n = CYC && r == 1 ? v[(e + NP - 1) % NP]
+                        : CYC && r == NPP - 1 ? v[(e + 1) % NP]
+                                              : lds_at(Str, row_i(row, 72 + e * (NPP - 1) + r - 1), k);
+        ax = __builtin_fmaf(n - v[e], row_f(row, 36 + e * NPP + r), ax);
+      }
+      te[e] = .5f * ((ti + ac) + (v[e] + ax));
+    }
+  }
+  float sp = 0.f, sm = 0.f, mx = ti, mn = ti;
+#pragma unroll
+  for (int e = 0; e < NP; e++) {
+    const float m = in.m[e];
+    const float a = m * (te[e] - fct_upwind(m, ti, v[e]));
+    __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
+    sp = sp - fminf(0.f, a);
+    sm = sm + fmaxf(0.f, a);
+    mx = fmaxf(mx, v[e]);
+    mn = fminf(mn, v[e]);
+  }
+  mx = fmaxf(fmaxf(0.f, mx), lo);
+  mn = fminf(fmaxf(0.f, mn), lo);
+#pragma unroll
+  for (int e = 0; e < NP; e++) {
+    const float x = lds_at(Slo, row_i(row, 102 + e), k);
+    mx = fmaxf(mx, x);
+    mn = fminf(mn, x);
+  }
+  mx = fmaxf(0.f, mx);
+  mn = fmaxf(0.f, mn);
+  __builtin_nontemporal_store(mx, &TRV(s.trmax, col));
+  __builtin_nontemporal_store(mn, &TRV(s.trmin, col));
+  const float a2 = (float)c.ab2, a3 = (float)c.ab3, ra1 = (float)(1. / c.ab1) * area;
+  const float qp = ((mx - lo) * dp - (a2 * fminf(0.f, in.to) + a3 * fmaxf(0.f, in.tv))) * ra1;
+  const float qm = ((lo - mn) * dp + (a2 * fmaxf(0.f, in.to) + a3 * fminf(0.f, in.tv))) * ra1;
+  __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qp * fct_rcp(fmaxf(sp, 1.e-11f)))), &TRV(s.tr_rp, col));
+  __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qm * fct_rcp(fmaxf(sm, 1.e-11f)))), &TRV(s.tr_rm, col));
+}
+
+template <int NW, bool SWZ, bool CYC>
+__global__ void __launch_bounds__(64 * NW) k_e_trcadv12(EnsGrid g, EnsState s) {
+  extern __shared__ float lds[];       // the tracer of rings 0-2, the low-order tracer of rings 0-1
+  const int nvl = g.d.nvl, nip = g.d.nip, ncol = s.ncol, ntra = g.d.ntra;
+  const int w = uni(threadIdx.y), k = threadIdx.x;
+  const EnsTiles &ts = g.ptiles;
+  float *Str = lds, *Slo = lds + ts.lo_max * 64;
+  const int tm = ntra * s.members;
+  int p, r;
+  if (SWZ) {
+    const int q = blockIdx.x >> 3, per = (ts.npatch + 7) >> 3;
+    p = (blockIdx.x & 7) * per + q / tm;
+    r = q % tm;
+  } else {
+    p = blockIdx.x / tm;
+    r = blockIdx.x % tm;
+  }
+  if (p >= ts.npatch) return;          // the whole block: before any barrier
+  const int mem = r / ntra, t = r % ntra;
+  const bool live = k < nvl;
+  const int base = mem * nip;
+  const int4 cn = ldc4(ts.cnt, p);
+  const int off = ldc(ts.off, p);
+  const int n0 = cn.x, n1 = cn.y, n2 = cn.z;
+  const StepCtl c = load_ctl(s.ctl);
+  // lane j holds the entry of the wavefront's j-th tile cell (every lane loads, also above nvl)
+  const int4 ev = ts.ent[off + min(w + k * NW, n2 - 1)];
+  const int kc = live ? k : 0;
+  const size_t toff = (size_t)t * ncol * nvl + kc, aoff = (size_t)t * 3 * ncol * nvl + kc;
+  constexpr int J0 = (FCT_LO_MAX + NW - 1) / NW;
+  static_assert(J0 <= 64, "one lane per cell of a wavefront");
+  {
+    float v[J0];
+#pragma unroll
+    for (int j = 0; j < J0; j++)
+      if (w + j * NW < n2) v[j] = TRV(s.tr, base + __builtin_amdgcn_readlane(ev.x, j));
+#pragma unroll
+    for (int j = 0; j < J0; j++)
+      if (w + j * NW < n2) Str[(w + j * NW) * 64 + k] = v[j];
+  }
+  // areas of the wavefront's cells, one a lane; stage A's inputs two cells ahead, stage B's one
+  const float arl = g.area[ev.x], rarl = g.rarea[ev.x];
+  auto lane_f = [](float x, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j)); };
+  auto load_a = [&](int j) {
+    return tile_load_a(s, c, nvl, base + __builtin_amdgcn_readlane(ev.x, min(j, (n1 - 1 - w) / NW)), toff, aoff, kc);
+  };
+  TileInA a0 = load_a(0), a1 = load_a(1);
+  __syncthreads();
+  for (int i = w, j = 0; i < n1; i += NW, j++) {
+    const int4 en = wave_ent(ev, j);
+    const TileInA a2 = load_a(j + 2);
+    const float rar = lane_f(rarl, j);
+    const float tlo = enp(en) == 6 ? tile_lo<6>(c, en, i, k, rar, a0, Str, Slo) : tile_lo<5>(c, en, i, k, rar, a0, Str, Slo);
+    if (i < n0 && live) __builtin_nontemporal_store(tlo, &TAB(s.trl_tdcy, c.nf - 1, base + en.x));
+    a0 = a1;
+    a1 = a2;
+  }
+  const int jl = w < n0 ? (n0 - 1 - w) / NW : 0;
+  auto load_row = [&](int j) {
+    return ((const int2 *)ts.core_row)[(size_t)__builtin_amdgcn_readlane(ev.x, min(j, jl)) * (CORE_ROW / 2) + min(k, CORE_ROW / 2 - 1)];
+  };
+  auto load_b = [&](int j) {
+    return tile_load_b(s, c, nvl, base + __builtin_amdgcn_readlane(ev.x, min(j, jl)), aoff, kc);
+  };
+  TileInB cb = load_b(0);
+  int2 row = load_row(0);
+  __syncthreads();
+  for (int i = w, j = 0; i < n0; i += NW, j++) {
+    const int cell = __builtin_amdgcn_readlane(ev.x, j), z = __builtin_amdgcn_readlane(ev.z, j);
+    const TileInB nb = load_b(j + 1);
+    const int2 nrow = load_row(j + 1);
+    const float area = lane_f(arl, j);
+    if (live) {
+      if (((z >> 16) & 0xff) == 6) tile_flux<6, CYC>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
+      else tile_flux<5, CYC>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
+    }
+    cb = nb;
+    row = nrow;
+  }
+}
+
+// tile & 1: 8 or 16 wavefronts per block; tile & 4: each XCD takes a
+// contiguous eighth of the patches, every tracer of a patch in turn
+void ens_launch_trcadv12(int tile, const EnsGrid &g, const EnsState &s, hipStream_t st) {
+  const int np = g.ptiles.npatch, tm = g.d.ntra * s.members;
+  const dim3 swz((np + 7) / 8 * 8 * tm), lin(np * tm);
+  const size_t sh = (size_t)(g.ptiles.lo_max + g.ptiles.r_max) * 64 * sizeof(float);
+  auto run = [&](auto cyc) {
+    constexpr bool C = decltype(cyc)::value;
+    switch (tile & 5) {
+      case 0: k_e_trcadv12<8, false, C><<<lin, dim3(64, 8), sh, st>>>(g, s); break;
+      case 1: k_e_trcadv12<16, false, C><<<lin, dim3(64, 16), sh, st>>>(g, s); break;
+      case 4: k_e_trcadv12<8, true, C><<<swz, dim3(64, 8), sh, st>>>(g, s); break;
+      default: k_e_trcadv12<16, true, C><<<swz, dim3(64, 16), sh, st>>>(g, s); break;
+    }
+  };
+  if (g.ptiles.cyclic) run(std::true_type{});
+  else run(std::false_type{});
+}
+
+// Per cell, as the core of its patch, what the two-sided reconstructions of
+// its edges need, one row of CORE_ROW words that a wavefront reads with one
+// load and hands out lane by lane: 0-35 the cell's own coefficients (edge,
+// stencil cell), 36-71 the neighbours' of the shared edges, each sum starting
+// at the shared edge's slot, 72-101 the LDS byte offsets (256 per tile cell)
+// of the neighbours' stencil cells after the first (which is the cell itself),
+// 102-107 those of the neighbours.  A pentagon's missing stencil cell is the
+// neighbour itself with coefficient 0, before the last.  Clears *cyclic unless
+// the slots of all cells run around them in one sense: then the second and
+// last cells of a neighbour's stencil are the cell's own neighbours of slots
+// e-1 and e+1.  One block per patch, one thread per core cell and edge.
+__global__ void __launch_bounds__(256) k_core_rows(EnsGrid g, EnsTiles ts, int *rows, int *cyclic) {
+  const int p = blockIdx.x, n0 = ts.cnt[p].x;
+  const int4 *ent = ts.ent + ts.off[p];
+  for (int q = threadIdx.x; q < n0 * NPP; q += blockDim.x) {
+    const int e = q % NPP;
+    const int4 en = ent[q / NPP];
+    const int c = en.x, np = enp(en), l = lnb(en, e);
+    const int4 ex = ent[l];
+    const int x = ex.x, nx = enp(ex), xs = eslot(en, e);
+    int *row = rows + (size_t)c * CORE_ROW;
+    row[102 + e] = 256 * l;
+    for (int r = 0; r < NPP; r++) {
+      row[e * NPP + r] = __float_as_int(g.hfcoef[((size_t)c * NPP + e) * NPP + r]);
+      const bool in = nx == NPP || r != NPP - 2;
+      const int j = (xs + (r < NPP - 1 ? r : nx - 1)) % nx;
+      row[36 + e * NPP + r] = in ? __float_as_int(g.hfcoef[((size_t)x * NPP + xs) * NPP + j]) : 0;
+      if (r > 0) row[72 + e * (NPP - 1) + r - 1] = 256 * (in ? lnb(ex, j) : l);
+      const int want = r == 1 ? (e + np - 1) % np : (e + 1) % np;
+      if (e < np && (r == 1 || r == NPP - 1) &&
+          g.d.prox[(size_t)x * NPP + j] != g.d.prox[(size_t)c * NPP + want])
+        *cyclic = 0;
+    }
+  }
+}
+
+int ens_make_core(Arena &a, const TileHost &t, EnsGrid &g) {
+  EnsTiles &d = g.ptiles;
+  d.r_max = d.lo_max = 0;
+  for (auto &c : t.cnt) {
+    d.r_max = std::max(d.r_max, c[1]);
+    d.lo_max = std::max(d.lo_max, c[2]);
+  }
+  int *rows = nullptr, *flag = nullptr, cyclic = 1;
+  int r;
+  if ((r = a.alloc(&rows, (size_t)g.d.nip * CORE_ROW)) || (r = a.upload(&flag, std::vector<int>(1, 1)))) return r;
+  k_core_rows<<<d.npatch, 256, 0, a.stream>>>(g, d, rows, flag);
+  if (hipGetLastError() != hipSuccess ||
+      hipMemcpyAsync(&cyclic, flag, sizeof cyclic, hipMemcpyDeviceToHost, a.stream) != hipSuccess ||
+      hipStreamSynchronize(a.stream) != hipSuccess)
+    return FIMHIP_EHIP;
+  d.core_row = rows;
+  d.cyclic = cyclic != 0;
+  return FIMHIP_OK;
 }
 
 }  // namespace fimhip

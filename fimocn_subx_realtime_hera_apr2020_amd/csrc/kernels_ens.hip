@@ -14,7 +14,7 @@ namespace fimhip {
 
 const char *const ens_kernel_names[EK_NKERNELS] = {
     "e_edgvar1", "e_edgvar3", "e_cnuity12", "e_cnuity3", "e_cnuity45",
-    "e_trcadv1", "e_trcadv2", "e_trcadv3", "e_momtum", "e_hystat", "e_massadv1", "e_massadv2", "e_trc_fct"};
+    "e_trcadv12", "e_trcadv3", "e_momtum", "e_hystat", "e_massadv1", "e_massadv2", "e_trc_fct"};
 
 #define EC(a, col, k) (a)[(size_t)(col) * nvl + (k)]
 #define EL(a, col, k) (a)[(size_t)(col) * nvlp1 + (k)]
@@ -195,55 +195,28 @@ __global__ void __launch_bounds__(64 * COLS) __attribute__((amdgpu_waves_per_eu(
 }
 
 // edgvar3 (edgvar3.F90:65-110, edgvalEval): this cell's least-squares
-// reconstruction of each edge.  The two-sided average of edgvar3.F90:111-132
-// is formed by the readers (cnuity, trcadv) from both cells' values; the
-// tracers' sums are fused multiply-adds in stencil order, as the fused tracer
-// transport forms them for both cells of an edge.  The
-// thickness is reconstructed as a deviation from the cell's own value, the
-// differences taken in FP64.
+// reconstruction of the thickness on each edge, as a deviation from the
+// cell's own value, the differences taken in FP64.  The two-sided average of
+// edgvar3.F90:111-132 is formed by cnuity from both cells' values; the tracers'
+// edge values are formed where they are used (trcadv12).
 template <int NP>
 __device__ __forceinline__ void e_edgvar3_col(const EnsGrid &g, const EnsState &s, int ipn, int base, int k) {
-  const int nvl = g.d.nvl, ncol = s.ncol;
+  const int nvl = g.d.nvl;
   const int col = base + ipn;
-  float hf[NP][NP];
-  int nb[NP];
+  float d[NP], out[NP];
+  const double b0 = EC(s.dp, col, k);
+#pragma unroll
+  for (int j = 0; j < NP; j++) d[j] = (float)(EC(s.dp, base + GPROX(ipn, j), k) - b0);
 #pragma unroll
   for (int i = 0; i < NP; i++) {
-    nb[i] = base + GPROX(ipn, i);
+    float acc = 0.f;
 #pragma unroll
-    for (int j = 0; j < NP; j++) hf[i][j] = FHF(ipn, i, j);
+    for (int j = 0; j < NP; j++) acc = acc + d[j] * FHF(ipn, i, j);
+    out[i] = (float)(b0 + (double)acc);
   }
-  float d[NP], out[NP];
-  {
-    const double b0 = EC(s.dp, col, k);
 #pragma unroll
-    for (int j = 0; j < NP; j++) d[j] = (float)(EC(s.dp, nb[j], k) - b0);
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < NP; j++) acc = acc + d[j] * hf[i][j];
-      out[i] = (float)(b0 + (double)acc);
-    }
-#pragma unroll
-    for (int i = 0; i < NP; i++) __builtin_nontemporal_store(out[i], &EE(s.dp_edg, col, i, k));
-    if (NP < NPP) __builtin_nontemporal_store(0.f, &EE(s.dp_edg, col, NPP - 1, k));
-  }
-  for (int f = 1; f <= s.edg3_ntr; f++) {
-    const float b0 = ETR(s.tr, f, col, k);
-#pragma unroll
-    for (int j = 0; j < NP; j++) d[j] = ETR(s.tr, f, nb[j], k) - b0;
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < NP; j++) acc = __builtin_fmaf(d[j], hf[i][j], acc);
-      out[i] = b0 + acc;
-    }
-#pragma unroll
-    for (int i = 0; i < NP; i++) __builtin_nontemporal_store(out[i], &ETE(s.trc_edg, f - 1, col, i, k));
-    if (NP < NPP) __builtin_nontemporal_store(0.f, &ETE(s.trc_edg, f - 1, col, NPP - 1, k));
-  }
+  for (int i = 0; i < NP; i++) __builtin_nontemporal_store(out[i], &EE(s.dp_edg, col, i, k));
+  if (NP < NPP) __builtin_nontemporal_store(0.f, &EE(s.dp_edg, col, NPP - 1, k));
 }
 
 template <int COLS, bool SWZ>
@@ -561,144 +534,13 @@ __global__ void __launch_bounds__(64 * COLS) k_e_massadv2(EnsGrid g, EnsState s)
 }
 
 // ---------------------------------------------------------------------------
-// trcadv1-3 (trcadv_compute.F90:19-315), every tracer of a column in one
-// thread, so the mass fluxes and the thickness are read once.  The final mass
-// flux is antisymmetric, so the neighbour's flux through the shared edge is
-// the negated own one.  Tracer edge values are the same bits on both sides
-// of an edge: tracer 1 from the edge-symmetric stencil (e_theta_edge, formed
-// here from the tracer values this kernel loads anyway), the others as the
-// average of both cells' reconstructions (stored by edgvar3; forming the
-// neighbour's here from its ring instead measured 7 ms slower at 16 x G7 x
-// 64 than the stored values; forming the cell's own one here from the
-// neighbour values already loaded saved no time either: 81 VGPRs instead of
-// 63, occupancy 5 instead of 7).  trcadv1 leaves trcadv2's sums of the
-// antidiffusive out- and inflows in tr_rp/tr_rm, and trcadv2 forms the local
-// bounds of trcadv1 again from the tracer values instead of reading them.
-
-template <int NP>
-__device__ __forceinline__ void e_trcadv1_col(const EnsGrid &g, const EnsState &s, const StepCtl &c, int ipn,
-                                              int base, int k) {
-  const int nvl = g.d.nvl, ncol = s.ncol, ntra = g.d.ntra;
-  const int nf = c.nf - 1, of = c.of - 1, vof = c.vof - 1;
-  const int col = base + ipn;
-  const float thshld = 1.e-11f;
-  float m[NP];
-  int xs[NP];
-#pragma unroll
-  for (int e = 0; e < NP; e++) {
-    xs[e] = base + GPROX(ipn, e);
-    m[e] = EE(s.massfx, col, e, k);
-  }
-  const float rdp = frcp(fmaxf(thshld, (float)EC(s.dp, col, k))), rar = GF(rarea, ipn);
-  const float a1 = (float)c.ab1, a2 = (float)c.ab2, a3 = (float)c.ab3;
-  for (int t = 0; t < ntra; t++) {
-    // every load of this tracer before its first store
-    const float *trf = s.tr + (size_t)t * ncol * nvl;
-    const float ti = trf[(size_t)col * nvl + k];
-    float v[NP], te[NP];
-#pragma unroll
-    for (int e = 0; e < NP; e++) v[e] = trf[(size_t)xs[e] * nvl + k];
-    const float tdp0 = ETR(s.trdp, t, col, k), tlo_of = ETAB(s.trl_tdcy, t, of, col, k);
-    const float tlo_vof = ETAB(s.trl_tdcy, t, vof, col, k);
-    if (t == 0) {
-#pragma unroll
-      for (int e = 0; e < NP; e++) {
-        const int et = (e + NP - 1) % NP, el = (e + 1) % NP;
-        te[e] = e_theta_edge(ti, v[e], v[et], v[el], xs[et], xs[el]);
-      }
-    } else {
-      float eo[NP], en[NP];
-#pragma unroll
-      for (int e = 0; e < NP; e++) {
-        eo[e] = ETE(s.trc_edg, t - 1, col, e, k);
-        en[e] = ETE(s.trc_edg, t - 1, xs[e], GPROXS(ipn, e), k);
-      }
-#pragma unroll
-      for (int e = 0; e < NP; e++) te[e] = .5f * (eo[e] + en[e]);
-    }
-    float acc = 0.f, sp = 0.f, sm = 0.f, mx = ti, mn = ti;
-#pragma unroll
-    for (int e = 0; e < NP; e++) {
-      mx = fmaxf(mx, v[e]);
-      mn = fminf(mn, v[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < NP; e++) {
-      const float fl = .5f * ((m[e] + fabsf(m[e])) * ti - (fabsf(m[e]) - m[e]) * v[e]);
-      const float a = m[e] * te[e] - fl;
-      __builtin_nontemporal_store(a, &ETE(s.antiflx, t, col, e, k));
-      sp = sp - fminf(0.f, a);
-      sm = sm + fmaxf(0.f, a);
-      acc = acc + fl;
-    }
-    if (NP < NPP) __builtin_nontemporal_store(0.f, &ETE(s.antiflx, t, col, NPP - 1, k));
-    const float tlo = -acc * rar;
-    __builtin_nontemporal_store(tlo, &ETAB(s.trl_tdcy, t, nf, col, k));
-    const float lo = tdp0 + a1 * tlo + a2 * tlo_of + a3 * tlo_vof;
-    mx = fmaxf(0.f, mx);
-    mn = fmaxf(0.f, mn);
-    __builtin_nontemporal_store(fmaxf(mn, fminf(mx, lo * rdp)), &ETR(s.trcr_lo, t, col, k));
-    __builtin_nontemporal_store(sp, &ETR(s.tr_rp, t, col, k));
-    __builtin_nontemporal_store(sm, &ETR(s.tr_rm, t, col, k));
-  }
-}
-
-template <int COLS, bool SWZ>
-__global__ void __launch_bounds__(64 * COLS) k_e_trcadv1(EnsGrid g, EnsState s) {
-  const int nip = g.d.nip, nvl = g.d.nvl;
-  const int k = threadIdx.x, ipn = tile_cell<COLS, SWZ>();
-  if (ipn >= nip || k >= nvl) return;
-  const StepCtl c = load_ctl(s.ctl);
-  const int base = blockIdx.y * nip;
-  if (GNP(ipn) == 6) e_trcadv1_col<6>(g, s, c, ipn, base, k);
-  else e_trcadv1_col<5>(g, s, c, ipn, base, k);
-}
-
-template <int COLS, bool SWZ>
-__global__ void __launch_bounds__(64 * COLS) k_e_trcadv2(EnsGrid g, EnsState s) {
-  const int nip = g.d.nip, nvl = g.d.nvl, ncol = s.ncol, ntra = g.d.ntra;
-  const int k = threadIdx.x, ipn = tile_cell<COLS, SWZ>();
-  if (ipn >= nip || k >= nvl) return;
-  const StepCtl c = load_ctl(s.ctl);
-  const int of = c.of - 1, vof = c.vof - 1;
-  const int base = blockIdx.y * nip, col = base + ipn;
-  const float thshld = 1.e-11f;
-  int xs[NPP];
-#pragma unroll
-  for (int e = 0; e < NPP; e++) xs[e] = base + GPROX(ipn, e);
-  const float dp = (float)EC(s.dp, col, k), area = GF(area, ipn);
-  const float a2 = (float)c.ab2, a3 = (float)c.ab3, ra1 = (float)(1. / c.ab1) * area;
-  for (int t = 0; t < ntra; t++) {
-    const float sp = ETR(s.tr_rp, t, col, k), sm = ETR(s.tr_rm, t, col, k);
-    const float ti = ETR(s.tr, t, col, k), lo = ETR(s.trcr_lo, t, col, k);
-    float mx = ti, mn = ti;
-#pragma unroll
-    for (int e = 0; e < NPP; e++) {
-      const float v = ETR(s.tr, t, xs[e], k);
-      mx = fmaxf(mx, v);
-      mn = fminf(mn, v);
-    }
-    mx = fmaxf(fmaxf(0.f, mx), lo);
-    mn = fminf(fmaxf(0.f, mn), lo);
-#pragma unroll
-    for (int e = 0; e < NPP; e++) {
-      const float v = ETR(s.trcr_lo, t, xs[e], k);
-      mx = fmaxf(mx, v);
-      mn = fminf(mn, v);
-    }
-    mx = fmaxf(0.f, mx);
-    mn = fmaxf(0.f, mn);
-    __builtin_nontemporal_store(mx, &ETR(s.trmax, t, col, k));
-    __builtin_nontemporal_store(mn, &ETR(s.trmin, t, col, k));
-    const float to = ETAB(s.trc_tdcy, t, of, col, k), tv = ETAB(s.trc_tdcy, t, vof, col, k);
-    const float qp = ((mx - lo) * dp - (a2 * fminf(0.f, to) + a3 * fmaxf(0.f, tv))) * ra1;
-    const float qm = ((lo - mn) * dp + (a2 * fmaxf(0.f, to) + a3 * fminf(0.f, tv))) * ra1;
-    __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qp * frcp(fmaxf(sp, thshld)))), &ETR(s.tr_rp, t, col, k));
-    __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qm * frcp(fmaxf(sm, thshld)))), &ETR(s.tr_rm, t, col, k));
-  }
-}
-
-// trcadv3: the limiter's neighbour value is gathered through a per-lane
+// trcadv3 (trcadv_compute.F90:242-315), every tracer of a column in one
+// thread, on the antidiffusive fluxes, limiter ratios, bounds and low-order
+// tendency that trcadv12 (fct_tiles.hip) leaves.  The final mass flux is
+// antisymmetric and tracer edge values are the same bits on both sides of an
+// edge, so the tracer fluxes cancel exactly across it.
+//
+// The limiter's neighbour value is gathered through a per-lane
 // address (R+ or R- of the neighbour by the sign of the flux) and every load
 // of a tracer is issued before the first is used.
 template <int NP>
@@ -1107,8 +949,7 @@ void ens_launch(int kernel, int tile, const EnsGrid &g, const EnsState &s, hipSt
     case EK_CNUITY12: ENS_DISPATCH(k_e_cnuity12, 1); break;
     case EK_CNUITY3: ENS_DISPATCH(k_e_cnuity3, 1); break;
     case EK_CNUITY45: ENS_DISPATCH(k_e_cnuity45, 1); break;
-    case EK_TRCADV1: ENS_DISPATCH(k_e_trcadv1, 1); break;
-    case EK_TRCADV2: ENS_DISPATCH(k_e_trcadv2, 1); break;
+    case EK_TRCADV12: ens_launch_trcadv12(tile, g, s, st); break;
     case EK_TRCADV3: ENS_DISPATCH(k_e_trcadv3, 1); break;
     case EK_MOMTUM: ENS_DISPATCH(k_e_momtum, 1); break;
     case EK_MASSADV1: ENS_DISPATCH(k_e_massadv1, 1); break;

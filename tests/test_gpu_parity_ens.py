@@ -607,8 +607,8 @@ def test_class_b_fp32_form_against_fp64():
 ])
 def test_fused_tracer_fct_equals_stage_chain(level, nvl, members, steps, mode, scheme, graph):
     """The tracer transport as one kernel over patches with recomputed halo
-    rings gives the bytes of the three-kernel chain with edgvar3's tracer
-    reconstructions in device memory, for every field of every member."""
+    rings gives the bytes of the chain of trcadv12 and trcadv3, for every field
+    of every member."""
     from fimocn_subx_realtime_hera_apr2020_amd import fimhip, state
     g = fimhip.icos_grid(level)
     th, ds = state.vertical_tables(nvl)
@@ -684,3 +684,90 @@ def test_class_b_load_and_download_in_chunks(ntra, ntrb):
             assert np.array_equal(e.download(m, "trb"), trb[m].astype(np.float32).astype(np.float64)), m
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("level, nvl, ntra, tile", [(1, 16, 1, 1), (2, 64, 2, 0), (3, 38, 5, 5), (4, 63, 3, 1),
+                                                    (4, 17, 4, 4), (5, 64, 1, 5)])
+def test_trcadv12_shapes_and_ragged_sizes_equal_the_fused_form(level, nvl, ntra, tile):
+    """trcadv12's patches (48 cells) and the fused form's (64 cells) cut the grid
+    differently, and its launch shapes order and divide the patches differently:
+    the tracers have the same bytes, for one tracer (theta alone) upwards and
+    layer counts below the wavefront's width."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, state
+    g = fimhip.icos_grid(level)
+    th, ds = state.vertical_tables(nvl)
+    out = []
+    for fused in (False, True):
+        e = fimhip.Ensemble(g, 2, nvl, ntra, DT, th, ds)
+        try:
+            e.set_fused(fused)
+            if not fused:
+                e.set_tiles({"e_trcadv12": tile})
+            for m in range(2):
+                e.synth(m, seed=20240601, synth_member=m, flags=FLAGS)
+            e.init_state(False)
+            e.step(4, 1)
+            e.sync()
+            out.append([{n: e.download(m, n) for n in ("tr", "trdp", "dp")} for m in range(2)])
+        finally:
+            e.close()
+    for m in range(2):
+        for n in out[0][m]:
+            assert np.array_equal(out[0][m][n], out[1][m][n]), (m, n)
+
+
+def _turned(g, seed=None):
+    """The same grid with every cell's slots in the opposite sense, or (seed)
+    each cell's slots started at another neighbour or turned at random."""
+    import dataclasses
+    P, S, n = g.prox.astype(int) - 1, g.proxs.astype(int) - 1, g.nprox.astype(int)
+    r = np.random.default_rng(seed)
+    perm = np.tile(np.arange(6), (g.nip, 1))           # new slot -> old slot
+    turn = np.ones(g.nip, bool) if seed is None else r.random(g.nip) < 0.5
+    for c in range(g.nip):
+        o = np.arange(n[c])
+        if turn[c]:
+            o = o[::-1]
+        if seed is not None:
+            o = np.roll(o, r.integers(n[c]))
+        perm[c, :n[c]] = o
+    back = np.argsort(perm, axis=1)                    # old slot -> new slot
+    i = np.arange(g.nip)[:, None]
+    S2 = S.copy()
+    for c in range(g.nip):
+        S2[c, :n[c]] = [back[P[c, e], S[c, e]] for e in perm[c, :n[c]]]
+    cs, sn = g.cs[i, perm].copy(), g.sn[i, perm].copy()
+    for a in (cs, sn):                                 # trailing and leading stencil cells change places
+        a[turn] = a[turn][:, :, [0, 1, 3, 2]]
+    return dataclasses.replace(
+        g, prox=(P[i, perm] + 1).astype(np.int32), proxs=(S2 + 1).astype(np.int32), cs=cs, sn=sn,
+        sidevec_c=g.sidevec_c[i, perm].copy(), sidevec_e=g.sidevec_e[i, perm].copy(),
+        sideln=g.sideln[i, perm].copy(), rprox_ln=g.rprox_ln[i, perm].copy(),
+        hfcoef=g.hfcoef[i[:, :, None], perm[:, :, None], perm[:, None, :]].copy())
+
+
+@pytest.mark.parametrize("seed", [None, 3])
+def test_tracer_transport_on_grids_with_other_slot_orders(seed):
+    """A grid's neighbour slots may run around a cell in either sense (seed
+    None: all reversed) or in a mixture of senses, where the two-sided
+    reconstruction takes every stencil cell from the neighbour's own list:
+    the transport agrees with the generator's order to FP32 rounding (sums in
+    another order; four steps of values near 1: 1e-6 of each field's norm)
+    and with the fused form on the same grid bit for bit."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip
+    g, th, ds = _grid(3)
+    out = []
+    for gr, fused in ((g, False), (_turned(g, seed), False), (_turned(g, seed), True)):
+        e = fimhip.Ensemble(gr, 1, NVL, NTRA, DT, th, ds)
+        try:
+            e.set_fused(fused)
+            e.synth(0, seed=20240601, flags=1)
+            e.init_state(False)
+            e.step(4, 1)
+            e.sync()
+            out.append({n: e.download(0, n) for n in ("tr", "trdp", "dp")})
+        finally:
+            e.close()
+    for n in out[0]:
+        assert rel_l2(out[1][n], out[0][n]) < 1e-6, n
+        assert np.array_equal(out[1][n], out[2][n]), n
