@@ -55,21 +55,22 @@ SEED = 20240601
 
 
 def plain_kernel_bytes(T):
-    """Compulsory HBM bytes per cell-level of each FP64 kernel launch: the
-    distinct array elements it must read plus those it writes (8 B each)."""
+    """Compulsory HBM bytes per cell-level of each FP64 kernel launch of the
+    device-resident step: the distinct array elements it must read plus those
+    it writes (8 B each)."""
     v = {
-        "k_edgvar1": 5 + 36,                 # us vs pr mp tr1 -> u v lp mont uvsq trc1 on 6 edges
-        "k_edgvar3": 7 * T,                  # dp, tracers 2..T -> 6 edge values each
-        "k_cnuity12": 18 + 3 + 6 + 6 + 2,    # u/v/dp edges, dp, dplo(of,vof) -> massfx, antifx, dplo, delp_lo
-        "k_cnuity3": 6 + 4 + 2,              # antifx, delp_lo, dp, dp_tdcy(of,vof) -> r+, r-
-        "k_cnuity45": 27 + 11,               # antifx r+- massfx dplo dptdcy dp pr lp_edg u v -> massfx dptdcy dp pr ex omega
-        "k_massadv1": 12 + 6 + 1 + 2 + 6 + 2,   # u/v/dp edges, dp, dp_tdcy(of,vof) -> limited dp edges, q_min/max_out
-        "k_massadv2": 12 + 2 + 6 + 2 + 1 + 6 + 2 + 6 + 6 + 1 + 1 + 1 + 1 + 1,
-        # u/v/dp edges, q_min/max_out, dp_tdcy(of,vof), dp, lp_edg, u, v -> dp edges, massfx, dp_tdcy, dp, pr, ex, omega
-        "k_trcadv1": 27 * T,
-        "k_trcadv2": 16 * T,
-        "k_trcadv3": 18 * T,
-        "k_momtum": 3 + 1 + 30 + 4 + 5,
+        "k_edgvar1": 4 + 15,                 # us vs pr mp -> normal wind, Montgomery + kinetic energy edges, dpdx dpdy, vorticity
+        "k_edgvar3": 7,                      # dp -> 6 edge values
+        "k_cnuity12": 12 + 3 + 12 + 4,       # normal wind and dp edges, dp, dplo(of,vof) -> massfx, antifx, dplo, delp_lo, sums
+        "k_cnuity3": 6 + 2,                  # sums, delp_lo, dp, dp_tdcy(of,vof) -> r+, r-
+        "k_cnuity45": 22 + 11,               # antifx r+- massfx dplo dptdcy dp dpdx dpdy u v -> massfx dptdcy dp pr ex omega
+        "k_massadv1": 12 + 1 + 2 + 6 + 2,    # normal wind and dp edges, dp, dp_tdcy(of,vof) -> limited dp edges, q_min/max_out
+        "k_massadv2": 12 + 2 + 2 + 1 + 4 + 12 + 5,
+        # normal wind, limited edges, q_min/max_out, dp_tdcy(of,vof), dp, dpdx, dpdy, u, v -> dp edges, massfx, dp_tdcy, dp, pr, ex, omega
+        "k_trcadv1": 7 + 14 * T,             # massfx dp; per tracer tr trdp trl(of,vof) -> antiflx trl lo sums
+        "k_trcadv2": 1 + 10 * T,             # dp; per tracer tr lo sums trc(of,vof) -> bounds r+ r-
+        "k_trcadv3": 1 + 16 * T,             # dp; per tracer antiflx r+- bounds trl trc(of,vof) trdp -> trc tr
+        "k_momtum": 5 + 6 + 1 + 4 + 4,       # u v dp ex theta, energy edges, vorticity, tendencies -> tendencies u2 v2
         "k_regrid": 3,                       # theta, Exner -> Exner (sdot)
         "k_regrid_tail": 2,                  # Exner in sdot, in place
         "k_dffusn_lev": 2,

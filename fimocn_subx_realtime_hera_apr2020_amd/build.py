@@ -16,7 +16,7 @@ CSRC = os.path.join(PKG, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(PKG, "libfimhip.so")
 
-SOURCES = ["fimhip_api.hip", "kernels_plain.hip", "transp3d.hip", "hybgen.hip", "ens_api.hip", "kernels_ens.hip",
+SOURCES = ["fimhip_api.hip", "kernels_plain.hip", "trc_patch.hip", "transp3d.hip", "hybgen.hip", "ens_api.hip", "kernels_ens.hip",
            "transp3d_ens.hip", "fct_tiles.hip", "hycom_cnuity.hip",
            "hycom_edgvar.hip", "hycom_momtum.hip", "hycom_transp.hip", "hycom_hybgen.hip"]
 HOST_SOURCES = ["grid.cpp", "lsq_svd.cpp"]      # host-only C++ (g++)

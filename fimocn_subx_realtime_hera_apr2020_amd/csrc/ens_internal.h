@@ -119,11 +119,15 @@ struct TileHost {
   std::vector<int> off;
   std::vector<std::array<int, 4>> cnt, ent;
 };
-struct TileLimits { int core, r, lo, tile; };  // most cells in the core, rings 0-1, 0-2, 0-3
-constexpr TileLimits TRC_LIMITS = {48, 84, 124, 1 << 30};   // trcadv12's patches: three blocks per CU
-constexpr TileLimits FCT_LIMITS = {FCT_CORE_MAX, FCT_R_MAX, FCT_LO_MAX, FCT_TILE_MAX};
+struct TileLimits { int rings, core, r, lo, tile; };  // rings; most cells in the core, rings 0-1, 0-2, 0-3
+constexpr TileLimits TRC_LIMITS = {2, 48, 84, 124, 124};   // trcadv12's patches: three blocks per CU
+constexpr TileLimits TRC64_LIMITS = {2, 44, 80, 120, 120}; // the FP64 step's trcadv1
+constexpr TileLimits FCT_LIMITS = {3, FCT_CORE_MAX, FCT_R_MAX, FCT_LO_MAX, FCT_TILE_MAX};
 int ens_build_tiles(const HostGrid &h, int nip, const TileLimits &lim, TileHost &out);
 int ens_upload_tiles(Arena &a, const TileHost &t, EnsTiles &d);
+// the FP64 step's patches of at most 'core' cells and their rows (trc_patch.hip)
+int patch_tables(Arena &a, const HostGrid &h, const DevGrid &g, int core, EnsTiles &ts);
+void launch_patch_trcadv1(const DevGrid &g, const DevState &s, const EnsTiles &ts, const AB &ab, hipStream_t st);
 int ens_make_core(Arena &a, const TileHost &t, EnsGrid &g);   // g.ptiles' core rows
 // the fused tracer FCT: reads s.tr / s.trdp, writes s.tr_alt / s.trdp_alt
 void ens_launch_trcadv12(int tile, const EnsGrid &g, const EnsState &s, hipStream_t st);

@@ -39,8 +39,8 @@ namespace fimhip {
 // host: patches and their halo rings
 //
 // Patches grow breadth-first from the lowest unassigned cell over unassigned
-// cells, up to lim.core cells; the three rings around the patch are the
-// cells at neighbour distance 1, 2 and 3 from it, each ring in index order.
+// cells, up to lim.core cells; the lim.rings (2 or 3) rings around the patch are
+// the cells at neighbour distance 1, 2 and 3 from it, each ring in index order.
 // A patch whose rings would exceed the LDS tile gives up its last cells.
 // On the IJ-ordered icosahedral grids this gives compact, roughly hexagonal
 // patches (the three rings hold about twice the core's cells).
@@ -49,70 +49,66 @@ int ens_build_tiles(const HostGrid &h, int nip, const TileLimits &lim, TileHost 
   out.off.assign(1, 0);
   out.cnt.clear();
   out.ent.clear();
-  std::vector<int> core, ring[4], q;
-  int stamp = 0;
+  out.ent.reserve((size_t)nip * (lim.rings + 1));
+  std::vector<int> cells, q;           // the patch's core, then its rings
+  int stamp = 0, n[4];
   for (int seed = 0; seed < nip; seed++) {
     if (asg[seed] >= 0) continue;
-    core.assign(1, seed);
+    cells.assign(1, seed);
     q.assign(1, seed);
     ++stamp;
     mark[seed] = stamp;
-    for (size_t qi = 0; qi < q.size() && (int)core.size() < lim.core; qi++) {
+    for (size_t qi = 0; qi < q.size() && (int)cells.size() < lim.core; qi++) {
       const int c = q[qi];
       int nb[NPP];
       for (int e = 0; e < NPP; e++) nb[e] = h.prox[(size_t)c * NPP + e];
       std::sort(nb, nb + NPP);
-      for (int e = 0; e < NPP && (int)core.size() < lim.core; e++) {
+      for (int e = 0; e < NPP && (int)cells.size() < lim.core; e++) {
         const int x = nb[e];
         if (asg[x] >= 0 || mark[x] == stamp) continue;
         mark[x] = stamp;
-        core.push_back(x);
+        cells.push_back(x);
         q.push_back(x);
       }
     }
     for (;;) {
       // rings by distance from the core
       ++stamp;
-      for (int c : core) mark[c] = stamp;
-      ring[0] = core;
-      for (int r = 1; r <= 3; r++) {
-        ring[r].clear();
-        for (int c : ring[r - 1])
+      for (int c : cells) mark[c] = stamp;
+      n[0] = (int)cells.size();
+      for (int r = 1; r <= lim.rings; r++) {
+        for (int i = r == 1 ? 0 : n[r - 2]; i < n[r - 1]; i++)
           for (int e = 0; e < NPP; e++) {
-            const int x = h.prox[(size_t)c * NPP + e];
-            if (mark[x] != stamp) { mark[x] = stamp; ring[r].push_back(x); }
+            const int x = h.prox[(size_t)cells[i] * NPP + e];
+            if (mark[x] != stamp) { mark[x] = stamp; cells.push_back(x); }
           }
-        std::sort(ring[r].begin(), ring[r].end());
+        std::sort(cells.begin() + n[r - 1], cells.end());
+        n[r] = (int)cells.size();
       }
-      const int n0 = (int)ring[0].size(), n1 = n0 + (int)ring[1].size(), n2 = n1 + (int)ring[2].size(),
-                n3 = n2 + (int)ring[3].size();
-      if (n1 <= lim.r && n2 <= lim.lo && n3 <= lim.tile) {
-        // local indices of the tile cells, and the neighbour table of rings 0-2
-        std::vector<int> cells;
-        for (int r = 0; r < 4; r++) cells.insert(cells.end(), ring[r].begin(), ring[r].end());
-        for (int i = 0; i < n3; i++) mark[cells[i]] = -2 - i;       // local index i, encoded
-        for (int i = 0; i < n3; i++) {
-          const int c = cells[i];
-          int nbl[NPP] = {0, 0, 0, 0, 0, 0}, sl = 0;
-          if (i < n2)
-            for (int e = 0; e < NPP; e++) {
-              const int m = mark[h.prox[(size_t)c * NPP + e]];
-              if (m > -2) return FIMHIP_EINVAL;        // a ring-2 cell's neighbour outside the tile
-              nbl[e] = -2 - m;
-            }
-          for (int e = 0; e < NPP; e++) sl |= h.proxs[(size_t)c * NPP + e] << (4 * e);
-          out.ent.push_back({c, nbl[0] | nbl[1] << 8 | nbl[2] << 16 | nbl[3] << 24,
-                             nbl[4] | nbl[5] << 8 | h.nprox[c] << 16, sl});
-        }
-        for (int i = 0; i < n3; i++) mark[cells[i]] = 0;
-        for (int c : core) asg[c] = (int)out.cnt.size();
-        out.cnt.push_back({n0, n1, n2, n3});
-        out.off.push_back((int)out.ent.size());
-        break;
-      }
-      if (core.size() == 1) return FIMHIP_EINVAL;     // one cell's rings exceed the tile
-      core.pop_back();
+      if (lim.rings < 3) n[3] = n[2];
+      if (n[1] <= lim.r && n[2] <= lim.lo && n[3] <= lim.tile) break;
+      if (n[0] == 1) return FIMHIP_EINVAL;     // one cell's rings exceed the tile
+      cells.resize(n[0] - 1);
     }
+    // local indices of the tile cells, and the neighbour table of all but the last ring
+    for (int i = 0; i < n[3]; i++) mark[cells[i]] = -2 - i;       // local index i, encoded
+    for (int i = 0; i < n[3]; i++) {
+      const int c = cells[i];
+      int nbl[NPP] = {0, 0, 0, 0, 0, 0}, sl = 0;
+      if (i < n[lim.rings - 1])
+        for (int e = 0; e < NPP; e++) {
+          const int m = mark[h.prox[(size_t)c * NPP + e]];
+          if (m > -2) return FIMHIP_EINVAL;        // a neighbour outside the tile
+          nbl[e] = -2 - m;
+        }
+      for (int e = 0; e < NPP; e++) sl |= h.proxs[(size_t)c * NPP + e] << (4 * e);
+      out.ent.push_back({c, nbl[0] | nbl[1] << 8 | nbl[2] << 16 | nbl[3] << 24,
+                         nbl[4] | nbl[5] << 8 | h.nprox[c] << 16, sl});
+    }
+    for (int i = 0; i < n[3]; i++) mark[cells[i]] = 0;
+    for (int i = 0; i < n[0]; i++) asg[cells[i]] = (int)out.cnt.size();
+    out.cnt.push_back({n[0], n[1], n[2], n[3]});
+    out.off.push_back((int)out.ent.size());
   }
   return FIMHIP_OK;
 }

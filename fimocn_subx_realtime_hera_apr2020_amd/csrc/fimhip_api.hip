@@ -6,13 +6,14 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "fimhip.h"
-#include "fimhip_internal.h"
+#include "ens_internal.h"
 #include "fim_pow.h"
 #include "synth.h"
 #include "host_common.h"
@@ -53,6 +54,12 @@ struct fimhip_ctx {
   int flux_conserv_schm = 1;         // 1 = cnuity (FCT), 2 = mass_adv
   int dtratio = 6;                   // class-B / class-A time step ratio
   DevClassB cb{};                    // class-B tracer transport (cb.ntrb = 0: off)
+  // Set after fimhip_step, which does not store edgvar1's edge fields and the
+  // tracers' reconstructions: they are formed, from the arrays of the step's start, when they are asked for
+  // or before something else writes what they are formed from.
+  bool edges_due = false;
+  struct { double *us, *vs, *pr, *mp, *tr; } start{};
+  EnsTiles tiles{};                  // patches of trcadv1 in fimhip_step
 };
 
 // dyn_init.F90:125 taper for smoo_coeff
@@ -101,22 +108,21 @@ int host_grid_prepare(const fimhip_grid_desc *gd, HostGrid &h) {
 
 int dev_grid_upload(Arena &a, const fimhip_grid_desc *gd, const HostGrid &h, DevGrid &g) {
   const int nip = gd->nip, nvl = gd->nvl;
-  auto vec = [](const double *p, size_t n) { return std::vector<double>(p, p + n); };
   g.nip = nip; g.nvl = nvl; g.ntra = gd->ntra; g.dt = gd->dt;
   int *dprox, *dproxs, *dnprox;
   double *dcs, *dsn, *dsvc, *dsve, *dsideln, *dhf, *darea, *drarea, *dcorio, *dgrnd, *ddff, *dsmoo, *dth, *dds;
   int r = 0;
   if ((r = a.upload(&dprox, h.prox)) || (r = a.upload(&dproxs, h.proxs)) || (r = a.upload(&dnprox, h.nprox)) ||
-      (r = a.upload(&dcs, vec(gd->cs, (size_t)nip * NPP * 4))) ||
-      (r = a.upload(&dsn, vec(gd->sn, (size_t)nip * NPP * 4))) ||
-      (r = a.upload(&dsvc, vec(gd->sidevec_c, (size_t)nip * NPP * 2))) ||
-      (r = a.upload(&dsve, vec(gd->sidevec_e, (size_t)nip * NPP * 2))) ||
-      (r = a.upload(&dsideln, vec(gd->sideln, (size_t)nip * NPP))) ||
-      (r = a.upload(&dhf, vec(gd->hfcoef, (size_t)nip * NPP * NPP))) ||
-      (r = a.upload(&darea, vec(gd->area, nip))) || (r = a.upload(&drarea, h.rarea)) ||
+      (r = a.upload(&dcs, gd->cs, (size_t)nip * NPP * 4)) ||
+      (r = a.upload(&dsn, gd->sn, (size_t)nip * NPP * 4)) ||
+      (r = a.upload(&dsvc, gd->sidevec_c, (size_t)nip * NPP * 2)) ||
+      (r = a.upload(&dsve, gd->sidevec_e, (size_t)nip * NPP * 2)) ||
+      (r = a.upload(&dsideln, gd->sideln, (size_t)nip * NPP)) ||
+      (r = a.upload(&dhf, gd->hfcoef, (size_t)nip * NPP * NPP)) ||
+      (r = a.upload(&darea, gd->area, nip)) || (r = a.upload(&drarea, h.rarea)) ||
       (r = a.upload(&dcorio, h.corio)) || (r = a.upload(&dgrnd, h.grndspd)) ||
       (r = a.upload(&ddff, h.dfflen)) || (r = a.upload(&dsmoo, h.smoo)) ||
-      (r = a.upload(&dth, vec(gd->thetac, nvl))) || (r = a.upload(&dds, vec(gd->dpsig, nvl))))
+      (r = a.upload(&dth, gd->thetac, nvl)) || (r = a.upload(&dds, gd->dpsig, nvl)))
     return r;
   g.prox = dprox; g.proxs = dproxs; g.nprox = dnprox;
   g.cs = dcs; g.sn = dsn; g.svc = dsvc; g.sve = dsve; g.sideln = dsideln; g.hfcoef = dhf;
@@ -162,9 +168,14 @@ extern "C" int fimhip_create(const fimhip_grid_desc *gd, int device, fimhip_ctx 
       {&s.mont_edg, ez}, {&s.uvsq_edg, ez}, {&s.trc_edg, ez * ntra}, {&s.antifx, ez}, {&s.delp_lo, cz},
       {&s.r_plus, cz}, {&s.r_mnus, cz}, {&s.antiflx, ez * ntra}, {&s.trcr_lo, cz * ntra},
       {&s.trmax, cz * ntra}, {&s.trmin, cz * ntra}, {&s.tr_rp, cz * ntra}, {&s.tr_rm, cz * ntra},
-      {&s.u2, cz}, {&s.v2, cz}, {&s.exsmo, lz}, {&s.thbuf, cz}};
+      {&s.u2, cz}, {&s.v2, cz}, {&s.exsmo, lz}, {&s.thbuf, cz}, {&s.vn, ez}, {&s.bke, ez}, {&s.pgx, cz},
+      {&s.pgy, cz}, {&s.dp_alt, cz}, {&s.pr_alt, lz}, {&s.mp_alt, cz}, {&s.tr_alt, cz * ntra}};
   for (auto &a : arrs)
     if ((r = c->arena.alloc(a.p, a.n))) { fimhip_destroy(c); return r; }
+  // patches of 44 cells, smaller where those would leave CUs without a block
+  // (trcadv1 at G3 x 4 tracers: 25 us with 44, 12 us with 12; at G4 29 and 28)
+  const int core = (int)std::max(12LL, (long long)nip * ntra / 600);
+  if ((r = patch_tables(c->arena, hg, c->g, core, c->tiles))) { fimhip_destroy(c); return r; }
   c->gsum_blocks = GSUM_BLOCKS;
   if ((r = c->arena.alloc(&c->gsum_partial, (size_t)c->gsum_blocks * (1 + ntra)))) { fimhip_destroy(c); return r; }
   if (hipStreamSynchronize(c->stream) != hipSuccess) { fimhip_destroy(c); return FIMHIP_EHIP; }
@@ -316,6 +327,30 @@ extern "C" long long fimhip_field_size(const fimhip_ctx *c, int f) {
   return FIMHIP_EINVAL;
 }
 
+// edgvar1's edge fields of the last fimhip_step (u_edg, v_edg, lp_edg,
+// mont_edg, uvsq_edg and trc_edg)
+static void form_edges(fimhip_ctx *c) {
+  if (!c->edges_due) return;
+  c->edges_due = false;
+  DevState t = c->s;
+  t.us = c->start.us; t.vs = c->start.vs; t.pr = c->start.pr; t.mp = c->start.mp; t.tr = c->start.tr;
+  launch_edgvar1(c->g, t, c->stream);
+  if (c->ntra > 1) step_own_edges(c->g, t, 1, c->ntra, c->stream);
+}
+static bool edge_field(int f) {
+  return f == FIMHIP_U_EDG || f == FIMHIP_V_EDG || f == FIMHIP_LP_EDG || f == FIMHIP_MONT_EDG ||
+         f == FIMHIP_UVSQ_EDG || f == FIMHIP_TRC_EDG;
+}
+// before field f is written (f < 0: any field): after a step of the transport
+// alone the winds and the Montgomery potential are still those of its start
+static void before_write(fimhip_ctx *c, int f) {
+  if (!c->edges_due) return;
+  const DevState &s = c->s;
+  const bool us = c->start.us == s.us, vs = c->start.vs == s.vs, mp = c->start.mp == s.mp;
+  if (f < 0 ? us || vs || mp : edge_field(f) || (f == FIMHIP_US && us) || (f == FIMHIP_VS && vs) || (f == FIMHIP_MP && mp))
+    form_edges(c);
+}
+
 static int h2d(fimhip_ctx *c, int f, const double *h) {
   if (!h) return FIMHIP_EINVAL;
   double **p = field_ptr(c, f);
@@ -362,6 +397,7 @@ static int ab_out(fimhip_ctx *c, int f, double *h) { return ab_slot(c, f, h, c->
 extern "C" int fimhip_upload(fimhip_ctx *c, int f, const double *h) {
   if (!c || f < 0 || f >= FIMHIP_NFIELDS) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  before_write(c, f);
   int r = h2d(c, f, h);
   if (r) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -371,6 +407,7 @@ extern "C" int fimhip_upload(fimhip_ctx *c, int f, const double *h) {
 extern "C" int fimhip_download(fimhip_ctx *c, int f, double *h) {
   if (!c || f < 0 || f >= FIMHIP_NFIELDS) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  if (edge_field(f)) form_edges(c);
   int r = d2h(c, f, h);
   if (r) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -395,6 +432,7 @@ extern "C" int fimhip_edgvar1_r8(fimhip_ctx *c, int its, const double *u_vel, co
   (void)its; (void)delp; (void)exner; (void)geop; (void)dp_edg; (void)geop_edg;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_US, u_vel)); TRY(h2d(c, FIMHIP_VS, v_vel)); TRY(h2d(c, FIMHIP_PR, pres));
   TRY(h2d(c, FIMHIP_MP, montg)); TRY(h2d(c, FIMHIP_TR, tracr));
   // trc_edg is intent(out) for tracer 1 only; the other tracers pass through
@@ -415,9 +453,10 @@ extern "C" int fimhip_edgvar3_r8(fimhip_ctx *c, int its, const double *u_vel, co
   (void)u_edg; (void)v_edg; (void)lp_edg; (void)geop_edg; (void)mont_edg; (void)uvsq_edg;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_DP, delp)); TRY(h2d(c, FIMHIP_TR, tracr));
   TRY(h2d(c, FIMHIP_TRC_EDG, trc_edg));   // tracer 1 edges pass through
-  launch_edgvar3(c->g, c->s, c->stream, true);
+  launch_edgvar3(c->g, c->s, c->stream);
   TRY(d2h(c, FIMHIP_DP_EDG, dp_edg)); TRY(d2h(c, FIMHIP_TRC_EDG, trc_edg));
   return finish(c);
 }
@@ -430,12 +469,13 @@ extern "C" int fimhip_cnuity_r8(fimhip_ctx *c, int its, const double *u_velo, co
   (void)its; (void)timing;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_US, u_velo)); TRY(h2d(c, FIMHIP_VS, v_velo)); TRY(h2d(c, FIMHIP_U_EDG, u_edg));
   TRY(h2d(c, FIMHIP_V_EDG, v_edg)); TRY(h2d(c, FIMHIP_DP_EDG, dp_edg)); TRY(h2d(c, FIMHIP_LP_EDG, lp_edg));
   TRY(h2d(c, FIMHIP_DP, delp)); TRY(h2d(c, FIMHIP_PR, pres)); TRY(h2d(c, FIMHIP_EX, exner));
   TRY(ab_in(c, FIMHIP_DP_TDCY, dp_tndcy)); TRY(ab_in(c, FIMHIP_DPL_TDCY, dplo_tndcy));
   TRY(ab_nf_in(c, FIMHIP_MASSFX, massfx));     // a pentagon's sixth edge passes through
-  launch_cnuity(c->g, c->s, c->ab, c->stream, true);
+  launch_cnuity(c->g, c->s, c->ab, c->stream);
   TRY(d2h(c, FIMHIP_DP, delp)); TRY(d2h(c, FIMHIP_PR, pres)); TRY(d2h(c, FIMHIP_EX, exner));
   TRY(ab_out(c, FIMHIP_DP_TDCY, dp_tndcy)); TRY(ab_out(c, FIMHIP_DPL_TDCY, dplo_tndcy));
   TRY(ab_out(c, FIMHIP_MASSFX, massfx)); TRY(d2h(c, FIMHIP_WS, omega));
@@ -449,11 +489,12 @@ extern "C" int fimhip_mass_adv_r8(fimhip_ctx *c, int its, const double *u_velo, 
   (void)its; (void)timing;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_US, u_velo)); TRY(h2d(c, FIMHIP_VS, v_velo)); TRY(h2d(c, FIMHIP_U_EDG, u_edg));
   TRY(h2d(c, FIMHIP_V_EDG, v_edg)); TRY(h2d(c, FIMHIP_DP_EDG, dp_edg)); TRY(h2d(c, FIMHIP_LP_EDG, lp_edg));
   TRY(h2d(c, FIMHIP_DP, delp)); TRY(h2d(c, FIMHIP_PR, pres)); TRY(h2d(c, FIMHIP_EX, exner));
   TRY(ab_in(c, FIMHIP_DP_TDCY, dp_tndcy)); TRY(ab_nf_in(c, FIMHIP_MASSFX, massfx));
-  launch_mass_adv(c->g, c->s, c->ab, c->stream, true);
+  launch_mass_adv(c->g, c->s, c->ab, c->stream);
   TRY(d2h(c, FIMHIP_DP_EDG, dp_edg)); TRY(d2h(c, FIMHIP_DP, delp)); TRY(d2h(c, FIMHIP_PR, pres));
   TRY(d2h(c, FIMHIP_EX, exner)); TRY(ab_out(c, FIMHIP_DP_TDCY, dp_tndcy)); TRY(ab_out(c, FIMHIP_MASSFX, massfx));
   TRY(d2h(c, FIMHIP_WS, omega));
@@ -466,6 +507,7 @@ extern "C" int fimhip_transp0_r8(fimhip_ctx *c, int its, double *cumufx, const d
   (void)its;
   if (!c || c->cb.ntrb < 1) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_DP, dp3d));
   launch_transp0(c->g, c->s, c->cb, c->stream);
   TRY(d2h(c, FIMHIP_CUMUFX, cumufx)); TRY(d2h(c, FIMHIP_DPINIT, dpinit));
@@ -477,6 +519,7 @@ extern "C" int fimhip_transp1_r8(fimhip_ctx *c, int its, int nf, int of, int vof
   (void)its;
   if (!c || c->cb.ntrb < 1 || nf < 1 || nf > 3 || of < 1 || of > 3 || vof < 1 || vof > 3) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_CUMUFX, cumufx)); TRY(h2d(c, FIMHIP_MASSFX, massfx));
   launch_transp1(c->g, c->s, c->cb, AB{nf, of, vof, adbash1, adbash2, adbash3}, c->stream);
   TRY(d2h(c, FIMHIP_CUMUFX, cumufx));
@@ -488,6 +531,7 @@ extern "C" int fimhip_transp2_r8(fimhip_ctx *c, int its, double *tracr, const do
   (void)its; (void)timing;
   if (!c || c->cb.ntrb < 1 || !tracr) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   const size_t tz = (size_t)c->nip * c->nvl * c->cb.ntrb;
   double *trb_host = tracr + (size_t)c->nip * c->nvl * c->ntra;
   HIPCHK(hipMemcpyAsync(c->cb.trb, trb_host, tz * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -503,10 +547,11 @@ extern "C" int fimhip_trcadv_r8(fimhip_ctx *c, int its, const double *trcr_edg, 
   (void)its; (void)timing;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_TRC_EDG, trcr_edg)); TRY(h2d(c, FIMHIP_TR, tracr)); TRY(h2d(c, FIMHIP_TRDP, trcdp));
   TRY(ab_in(c, FIMHIP_TRC_TDCY, trc_tdcy)); TRY(ab_in(c, FIMHIP_TRL_TDCY, trclo_tdcy));
   TRY(ab_nf_in(c, FIMHIP_MASSFX, massfx)); TRY(h2d(c, FIMHIP_DP, delp));
-  launch_trcadv(c->g, c->s, c->ab, c->stream, true);
+  launch_trcadv(c->g, c->s, c->ab, c->stream);
   TRY(d2h(c, FIMHIP_TR, tracr)); TRY(d2h(c, FIMHIP_TRDP, trcdp));
   TRY(ab_out(c, FIMHIP_TRC_TDCY, trc_tdcy)); TRY(ab_out(c, FIMHIP_TRL_TDCY, trclo_tdcy));
   return finish(c);
@@ -519,6 +564,7 @@ extern "C" int fimhip_momtum_r8(fimhip_ctx *c, int its, double *u_velo, double *
   (void)its; (void)geop_edg;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_US, u_velo)); TRY(h2d(c, FIMHIP_VS, v_velo)); TRY(h2d(c, FIMHIP_EX, exner));
   TRY(h2d(c, FIMHIP_U_EDG, u_edg)); TRY(h2d(c, FIMHIP_V_EDG, v_edg)); TRY(h2d(c, FIMHIP_TRC_EDG, trcr_edg));
   TRY(h2d(c, FIMHIP_MONT_EDG, mont_edg)); TRY(h2d(c, FIMHIP_UVSQ_EDG, uvsq_edg));
@@ -535,6 +581,7 @@ extern "C" int fimhip_hybgen_r8(fimhip_ctx *c, int its, const double *targt, dou
   (void)timing;
   if (!c || !targt) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   HIPCHK(hipMemcpyAsync((void *)c->g.thetac, targt, c->nvl * sizeof(double), hipMemcpyHostToDevice, c->stream));
   TRY(h2d(c, FIMHIP_US, us3d)); TRY(h2d(c, FIMHIP_VS, vs3d)); TRY(h2d(c, FIMHIP_TR, tr3d));
   TRY(h2d(c, FIMHIP_EX, ex3d)); TRY(h2d(c, FIMHIP_DP, dp3d)); TRY(h2d(c, FIMHIP_PR, pr3d));
@@ -549,6 +596,7 @@ extern "C" int fimhip_hystat_r8(fimhip_ctx *c, int its, double *ph3d, const doub
                                 const double *dp3d, double *tr3d, double *trdp, double *psrf, double *ptdcy) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  form_edges(c);
   TRY(h2d(c, FIMHIP_PH, ph3d)); TRY(h2d(c, FIMHIP_EX, ex3d)); TRY(h2d(c, FIMHIP_DP, dp3d));
   TRY(h2d(c, FIMHIP_TR, tr3d)); TRY(h2d(c, FIMHIP_PSRF, psrf)); TRY(h2d(c, FIMHIP_PTDCY, ptdcy));
   launch_hystat(c->g, c->s, its, c->stream);
@@ -734,6 +782,7 @@ extern "C" int fimhip_transp2_r4(fimhip_ctx *c, int its, float *tracr, float *cu
 extern "C" int fimhip_init_state(fimhip_ctx *c, int init_hybgen) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  before_write(c, -1);
   launch_trdp(c->g, c->s, c->stream);
   if (init_hybgen) {
     launch_hybgen(c->g, c->s, 0, c->stream);
@@ -762,10 +811,12 @@ extern "C" int fimhip_step(fimhip_ctx *c, int its, int mode) {
     ~TimerScope() { g_ktimer = nullptr; }
   } scope(c->kt);
   ab_rotate(c->ab, its, c->dt);
-  launch_edgvar1(c->g, c->s, c->stream);
-  launch_edgvar3(c->g, c->s, c->stream, false);
-  if (c->flux_conserv_schm == 2) launch_mass_adv(c->g, c->s, c->ab, c->stream, false);
-  else launch_cnuity(c->g, c->s, c->ab, c->stream, false);
+  const DevState &s = c->s;
+  c->start = {s.us, s.vs, s.pr, s.mp, s.tr};
+  c->edges_due = true;
+  step_edges(c->g, s, mode == 0, c->stream);
+  step_own_edges(c->g, s, 0, 1, c->stream);
+  step_continuity(c->g, c->s, c->ab, c->flux_conserv_schm == 2, c->stream);
   if (c->cb.ntrb > 0) {             // dyn_run.F90:388-405
     launch_transp1(c->g, c->s, c->cb, c->ab, c->stream);
     if (its % c->dtratio == 0) {
@@ -773,11 +824,11 @@ extern "C" int fimhip_step(fimhip_ctx *c, int its, int mode) {
       launch_transp0(c->g, c->s, c->cb, c->stream);
     }
   }
-  launch_trcadv(c->g, c->s, c->ab, c->stream, false);
+  step_tracers(c->g, c->s, c->tiles, c->ab, mode == 1, c->stream);
   if (mode == 0) {
-    launch_momtum(c->g, c->s, c->ab, c->stream);
+    step_momtum(c->g, c->s, c->start.tr, c->ab, c->stream);
     launch_hybgen(c->g, c->s, its, c->stream);
-    launch_hystat(c->g, c->s, its, c->stream);
+    step_hystat(c->g, c->s, its, c->stream);
   }
   HIPCHK(hipGetLastError());
   return FIMHIP_OK;
@@ -990,6 +1041,7 @@ int synth_into(int nip, int nvl, int ntra, const double *lat, const double *lon,
 extern "C" int fimhip_synth_device(fimhip_ctx *c, unsigned long long seed, int member, int flags) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  before_write(c, -1);
   return synth_into(c->nip, c->nvl, c->ntra, c->lat.data(), c->lon.data(), seed, member, flags, c->s, c->stream);
 }
 

@@ -66,6 +66,12 @@ struct DevState {
   double *antifx, *delp_lo, *r_plus, *r_mnus;
   double *antiflx, *trcr_lo, *trmax, *trmin, *tr_rp, *tr_rm;   // per tracer
   double *u2, *v2, *exsmo, *thbuf;
+  // the device-resident step: the normal edge wind, Montgomery potential plus
+  // kinetic energy on the edges, the edge-pressure line integrals, and the
+  // buffers that alternate with dp, pr, mp and tr, so that the values of a
+  // step's start stay until the next step
+  double *vn, *bke, *pgx, *pgy;
+  double *dp_alt, *pr_alt, *mp_alt, *tr_alt;
 };
 
 // Class-B tracer transport state (transp3d.F90, fct3d.F90): the tracers
@@ -136,16 +142,27 @@ void kt_end(hipStream_t st);
 
 // launch helpers (kernels_plain.hip)
 void launch_edgvar1(const DevGrid &g, const DevState &s, hipStream_t st);
-// two_sided: edgvar3 stores the two-sided edge averages (the drop-in entries'
-// arrays); false: each cell's own reconstructions, averaged by the readers
-// (the device-resident step).  Results are the same bits either way.
-void launch_edgvar3(const DevGrid &g, const DevState &s, hipStream_t st, bool two_sided);
-void launch_cnuity(const DevGrid &g, const DevState &s, const AB &ab, hipStream_t st, bool two_sided);
-void launch_mass_adv(const DevGrid &g, const DevState &s, const AB &ab, hipStream_t st, bool two_sided);
+// the drop-in entries: edgvar3 stores the two-sided edge averages
+void launch_edgvar3(const DevGrid &g, const DevState &s, hipStream_t st);
+void launch_cnuity(const DevGrid &g, const DevState &s, const AB &ab, hipStream_t st);
+void launch_mass_adv(const DevGrid &g, const DevState &s, const AB &ab, hipStream_t st);
+// the device-resident step's forms of the same routines (the same bits of
+// every state field).  step_edges keeps what the step itself reads instead of
+// the reference's six edge arrays; step_own_edges stores each cell's own
+// reconstructions.  step_continuity and step_tracers advance s.dp and s.pr, and
+// s.tr, into their other buffers; last: a step without hystat, which would
+// form the tracer mass again.
+void step_edges(const DevGrid &g, const DevState &s, bool momentum, hipStream_t st);
+void step_own_edges(const DevGrid &g, const DevState &s, int f0, int f1, hipStream_t st);
+void step_continuity(const DevGrid &g, DevState &s, const AB &ab, bool mass_adv, hipStream_t st);
+struct EnsTiles;
+void step_tracers(const DevGrid &g, DevState &s, const EnsTiles &ts, const AB &ab, bool last, hipStream_t st);
+void step_momtum(const DevGrid &g, DevState &s, const double *theta_start, const AB &ab, hipStream_t st);
+void step_hystat(const DevGrid &g, DevState &s, int its, hipStream_t st);
 void launch_transp0(const DevGrid &g, const DevState &s, const DevClassB &b, hipStream_t st);
 void launch_transp1(const DevGrid &g, const DevState &s, const DevClassB &b, const AB &ab, hipStream_t st);
 void launch_transp2(const DevGrid &g, const DevState &s, const DevClassB &b, hipStream_t st);
-void launch_trcadv(const DevGrid &g, const DevState &s, const AB &ab, hipStream_t st, bool two_sided);
+void launch_trcadv(const DevGrid &g, const DevState &s, const AB &ab, hipStream_t st);
 void launch_momtum(const DevGrid &g, DevState &s, const AB &ab, hipStream_t st);
 void launch_hybgen(const DevGrid &g, const DevState &s, int its, hipStream_t st);
 void launch_hystat(const DevGrid &g, const DevState &s, int its, hipStream_t st);

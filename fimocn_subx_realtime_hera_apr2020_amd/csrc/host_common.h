@@ -44,13 +44,14 @@ struct Arena {
   template <class T>
   int alloc(T **p, size_t n) { return raw((void **)p, n * sizeof(T)); }
   template <class T>
-  int upload(T **p, const std::vector<T> &h) {
-    int r = alloc(p, h.size());
+  int upload(T **p, const T *h, size_t n) {
+    int r = alloc(p, n);
     if (r) return r;
-    if (hipMemcpyAsync(*p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, stream) != hipSuccess)
-      return FIMHIP_EHIP;
+    if (hipMemcpyAsync(*p, h, n * sizeof(T), hipMemcpyHostToDevice, stream) != hipSuccess) return FIMHIP_EHIP;
     return 0;
   }
+  template <class T>
+  int upload(T **p, const std::vector<T> &h) { return upload(p, h.data(), h.size()); }
   void release() {
     for (void *p : allocs) (void)hipFree(p);
     allocs.clear();

@@ -175,7 +175,8 @@ enum {
    what the reference's arrays hold.  After fimhip_step, DP_EDG and TRC_EDG
    (tracers 2..ntra) hold each cell's own reconstructions (the step's readers
    form the two-sided averages), except that DP_EDG holds mass_adv's final
-   edge depths under flux_conserv_schm = 2. */
+   edge depths under flux_conserv_schm = 2.  The step does not store the
+   others and TRC_EDG; they are formed when they are downloaded. */
 /* number of doubles of a field */
 long long fimhip_field_size(const fimhip_ctx *ctx, int field);
 int fimhip_upload(fimhip_ctx *ctx, int field, const double *host);

@@ -752,3 +752,54 @@ def test_ragged_layer_counts_match_checker_bitwise(oracle_lib, nvl):
             assert _same(got, o.a[f]), (f, rel_l2(got, o.a[f]))
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("mode,flux_scheme,nvl", [(0, 1, 64), (1, 1, 64), (0, 2, 33), (1, 2, 64)])
+def test_edge_fields_formed_when_asked_for(oracle_lib, mode, flux_scheme, nvl):
+    """fimhip_step stores none of edgvar1's edge fields; a download after it
+    returns the ones of that step, whatever was written in between: fields
+    uploaded over the step's (after transport alone the winds and Montgomery
+    potential of its start are the current ones), another seeded state, the
+    start-up, or the routines on host arrays."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip
+    from helpers import seeded_case
+    O = oracle_lib
+    g, st, th, ds = seeded_case(3, nvl=nvl)
+    o = O.OracleRun(O.grid_arrays(g, nvl, DT, th, ds), nvl, NTRA, DT, pow_kind=1, flux_scheme=flux_scheme)
+    o.load(st)
+    o.init(True)
+    for its in (1, 2, 3):
+        o.step(its, mode)
+    edges = ("u_edg", "v_edg", "lp_edg", "mont_edg", "uvsq_edg")
+
+    def same_edges(m):
+        live = (np.arange(6)[None, :] < g.nprox[:, None])[:, :, None]
+        for f in edges:
+            assert _same(m.download(f) * live, o.a[f].reshape(m.shape(f)) * live), f
+        assert _same(m.download("trc_edg")[0] * live, o.a["trc_edg"].reshape(m.shape("trc_edg"))[0] * live)
+
+    def then(m, what):
+        if what == "upload":
+            for f in ("us", "vs", "mp", "pr", "tr"):
+                m.upload(f, m.download(f) + 1.)
+        elif what == "synth":
+            m.synth(seed=5)
+            m.init_state(True)
+        elif what == "hystat":
+            z = {f: m.download(f) for f in ("ph", "ex", "mp", "dp", "tr", "trdp", "psrf", "ptdcy")}
+            m.hystat(3, *[z[f] for f in ("ph", "ex", "mp", "dp", "tr", "trdp", "psrf", "ptdcy")])
+        elif what == "edge":
+            m.upload("v_edg", m.download("v_edg"))
+
+    for what in ("nothing", "upload", "synth", "hystat", "edge"):
+        m = fimhip.Model(g, nvl, NTRA, DT, th, ds)
+        try:
+            m.set_flux_scheme(flux_scheme)
+            m.load(st)
+            m.init_state(True)
+            for its in (1, 2, 3):
+                m.step(its, mode)
+            then(m, what)
+            same_edges(m)
+        finally:
+            m.close()
