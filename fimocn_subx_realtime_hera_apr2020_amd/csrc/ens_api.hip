@@ -45,9 +45,11 @@ struct fimhip_ens {
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // one captured step per buffer parity (the fused tracer FCT reads tr/trdp
   // and writes tr_alt/trdp_alt, and the instance swaps them after the step)
-  hipGraph_t graph[2] = {nullptr, nullptr};
-  hipGraphExec_t exec[2] = {nullptr, nullptr};
-  int graph_modes[2] = {-1, -1};
+  // and, with class-B tracers, for the steps that move them and the others
+  hipGraph_t graph[4] = {};
+  hipGraphExec_t exec[4] = {};
+  int graph_modes[4] = {-1, -1, -1, -1};
+  int its = 0;                       // steps since init_state, as the device counts them
   KTimer *kt = nullptr;
   // the tracer FCT as one kernel over patches with recomputed halo rings
   // (fct_tiles.hip), or as the
@@ -59,7 +61,7 @@ struct fimhip_ens {
 };
 
 static void drop_graph(fimhip_ens *e) {
-  for (int p = 0; p < 2; p++) {
+  for (int p = 0; p < 4; p++) {
     if (e->exec[p]) (void)hipGraphExecDestroy(e->exec[p]);
     if (e->graph[p]) (void)hipGraphDestroy(e->graph[p]);
     e->exec[p] = nullptr;
@@ -266,6 +268,7 @@ extern "C" int fimhip_ens_init_state(fimhip_ens *e, int init_hybgen) {
   HIPCHK(hipMemsetAsync(s.trc_tdcy, 0, 3 * cz * e->ntra * 4, e->stream));
   HIPCHK(hipMemsetAsync(s.trl_tdcy, 0, 3 * cz * e->ntra * 4, e->stream));
   HIPCHK(hipMemsetAsync(s.massfx, 0, cz * NPP * 4, e->stream));
+  e->its = 0;
   StepCtl c{0, 0, 2, 1, 0., 0., 0.};
   HIPCHK(hipMemcpyAsync(s.ctl, &c, sizeof c, hipMemcpyHostToDevice, e->stream));
   if (e->cb.ntrb > 0) {            // dyn_init.F90:1096-1098
@@ -282,7 +285,8 @@ extern "C" int fimhip_ens_init_state(fimhip_ens *e, int init_hybgen) {
 // and hybgen up to remap_1d (the first reader of its winds): momtum reads only
 // what cnuity and edgvar1 left and writes only what remap_1d and the next
 // step read.
-static void enqueue_step(fimhip_ens *e, int mode, bool side) {
+// move_b: a step that moves the class-B tracers (dyn_run.F90:396)
+static void enqueue_step(fimhip_ens *e, int mode, bool side, bool move_b) {
   const EnsGrid &g = e->g;
   EnsState s = e->s;
   hipStream_t st = e->stream, sd = e->side;
@@ -304,7 +308,7 @@ static void enqueue_step(fimhip_ens *e, int mode, bool side) {
   } else {
     for (int k = EK_CNUITY12; k <= EK_CNUITY45; k++) ens_launch(k, e->tile[k], g, s, st);
   }
-  if (e->cb.ntrb > 0) ens_launch_class_b_step(g, s, e->cb, st);   // dyn_run.F90:388-405
+  if (e->cb.ntrb > 0) ens_launch_class_b_step(g, s, e->cb, move_b, st);   // dyn_run.F90:388-405
   if (e->fused) {
     ens_launch(EK_TRCFCT, e->tile[EK_TRCFCT], g, s, st);
     std::swap(s.tr, s.tr_alt);         // the rest of the step works on the new tracers
@@ -333,7 +337,8 @@ static void enqueue_step(fimhip_ens *e, int mode, bool side) {
 
 // one step enqueued directly (no graph), the tracer buffers swapped after it
 static void step_once(fimhip_ens *e, int mode, bool side) {
-  enqueue_step(e, mode, side);
+  e->its++;
+  enqueue_step(e, mode, side, e->cb.ntrb > 0 && e->its % e->cb.dtratio == 0);
   if (e->fused) swap_tracer_buffers(e);
 }
 
@@ -354,15 +359,17 @@ extern "C" int fimhip_ens_step(fimhip_ens *e, int nsteps, int mode) {
   }
   for (int i = 0; i < nsteps; i++) {
     // the buffer parity of this step: which of the pair holds the tracers
-    const int p = (e->fused && e->s.tr > e->s.tr_alt) ? 1 : 0;
+    const bool move_b = e->cb.ntrb > 0 && (e->its + 1) % e->cb.dtratio == 0;
+    const int p = ((e->fused && e->s.tr > e->s.tr_alt) ? 1 : 0) + (move_b ? 2 : 0);
     if (e->graph_modes[p] != mode) {
       HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-      enqueue_step(e, mode, e->overlap);
+      enqueue_step(e, mode, e->overlap, move_b);
       HIPCHK(hipStreamEndCapture(e->stream, &e->graph[p]));
       HIPCHK(hipGraphInstantiate(&e->exec[p], e->graph[p], nullptr, nullptr, 0));
       e->graph_modes[p] = mode;
     }
     HIPCHK(hipGraphLaunch(e->exec[p], e->stream));
+    e->its++;
     if (e->fused) swap_tracer_buffers(e);
   }
   return FIMHIP_OK;

@@ -108,7 +108,7 @@ struct EnsClassB {
   float *fld, *vfx, *fmx, *fmn, *fld1, *flp, *fln, *uan;
 };
 void ens_launch_class_b_init(const EnsGrid &g, const EnsState &s, const EnsClassB &b, hipStream_t st);
-void ens_launch_class_b_step(const EnsGrid &g, const EnsState &s, const EnsClassB &b, hipStream_t st);
+void ens_launch_class_b_step(const EnsGrid &g, const EnsState &s, const EnsClassB &b, bool move, hipStream_t st);
 
 // Sizes of the fused tracer FCT's patches (its LDS tile).
 constexpr int FCT_CORE_MAX = 64;               // core cells of a patch

@@ -10,9 +10,10 @@
 // antidiffusive fluxes and the clipped fluxes are too, and the class-B tracer
 // mass moves between cells without loss (fct3d's own clipping aside).
 //
-// The step is captured once as a graph: whether a step moves the class-B
-// tracers (its % dtratio == 0, dyn_run.F90:396) is decided on the device from
-// the step counter, and the transport kernels of other steps return at once.
+// A step that moves the class-B tracers (its % dtratio == 0, dyn_run.F90:396)
+// and one that does not are captured as two graphs; the host counts the steps
+// as the device does.  (Launched every step and returning at once on the
+// device's count, 3 x G4 x 38 layers took 332 us a step where it takes 320.)
 // Mapping: one wavefront per column (lane = level), blockIdx.y = member,
 // blockIdx.z = class-B tracer; the massless-cell sweeps one thread per column.
 #include "ens_internal.h"
@@ -35,17 +36,11 @@ constexpr float ATHIRD = 1.f / 3.f, EPSIL = 1.e-11f, ONEMU = 1.e-6f;
 __device__ __forceinline__ int b_cell() {
   return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * BC + threadIdx.y));
 }
-// a step that moves the class-B tracers (dyn_run.F90:396)
-__device__ __forceinline__ bool b_active(const EnsState &s, int dtratio) {
-  return load_ctl(s.ctl).its % dtratio == 0;
-}
-
-// transp0 (transp3d.F90:22-41); unconditional at start-up
-__global__ void __launch_bounds__(64 * BC) k_eb_transp0(EnsGrid g, EnsState s, EnsClassB b, int always) {
+// transp0 (transp3d.F90:22-41)
+__global__ void __launch_bounds__(64 * BC) k_eb_transp0(EnsGrid g, EnsState s, EnsClassB b) {
   const int nip = g.d.nip, nvl = g.d.nvl;
   const int k = threadIdx.x, ipn = b_cell();
   if (ipn >= nip || k >= nvl) return;
-  if (!always && !b_active(s, b.dtratio)) return;
   const int col = blockIdx.y * nip + ipn;
   BC2(b.dpinit, col, k) = BC2(s.dp, col, k);
 #pragma unroll
@@ -79,7 +74,6 @@ __global__ void __launch_bounds__(64 * BC) k_eb_w(EnsGrid g, EnsState s, EnsClas
   const int nip = g.d.nip, nvl = g.d.nvl;
   const int k = threadIdx.x, ipn = b_cell();
   if (ipn >= nip) return;
-  if (!b_active(s, b.dtratio)) return;
   const int col = blockIdx.y * nip + ipn;
   const bool live = k < nvl;
   double vdv = 0.;
@@ -106,7 +100,6 @@ __global__ void __launch_bounds__(64) k_eb_fill(int nvl_, EnsState s, EnsClassB 
   static_assert(NVL % CH == 0, "whole chunks");
   __shared__ float sf[CH][65];
   __shared__ double sth[CH][65];
-  if (!b_active(s, b.dtratio)) return;
   const int nvl = FULL ? NVL : nvl_, ncol = s.ncol;
   const int lane = threadIdx.x, c0 = blockIdx.x * 64, n = blockIdx.y;
   const float *trb = b.trb + (size_t)n * ncol * nvl;
@@ -171,7 +164,6 @@ __global__ void __launch_bounds__(64 * BC) k_eb_vert(EnsGrid g, EnsState s, EnsC
   __shared__ float sa[BC][NVL_MAX], sb[BC][NVL_MAX], sc[BC][NVL_MAX];
   const int nip = g.d.nip, nvl = g.d.nvl, ncol = s.ncol;
   const int k = threadIdx.x, c = threadIdx.y, ipn = b_cell(), n = blockIdx.z;
-  if (!b_active(s, b.dtratio)) return;         // the same for every wave of the grid
   const int col = blockIdx.y * nip + ipn;
   const bool live = ipn < nip && k < nvl;       // every wave of the block reaches the barriers
   if (live) {
@@ -259,7 +251,6 @@ __global__ void __launch_bounds__(64 * BC) k_eb_lo(EnsGrid g, EnsState s, EnsCla
   const int nip = g.d.nip, nvl = g.d.nvl, ncol = s.ncol;
   const int k = threadIdx.x, ipn = b_cell(), n = blockIdx.z;
   if (ipn >= nip || k >= nvl) return;
-  if (!b_active(s, b.dtratio)) return;
   const int base = blockIdx.y * nip, col = base + ipn;
   const int np = BNP(ipn);
   const float fl = BTR(b.fld, n, col, k);
@@ -312,7 +303,6 @@ __global__ void __launch_bounds__(64 * BC) k_eb_clip(EnsGrid g, EnsState s, EnsC
   const int nip = g.d.nip, nvl = g.d.nvl, ncol = s.ncol;
   const int k = threadIdx.x, ipn = b_cell(), n = blockIdx.z;
   if (ipn >= nip || k >= nvl) return;
-  if (!b_active(s, b.dtratio)) return;
   const int base = blockIdx.y * nip, col = base + ipn;
   const int np = BNP(ipn);
   const float lp = BTR(b.flp, n, col, k), ln = BTR(b.fln, n, col, k);
@@ -336,15 +326,16 @@ __global__ void __launch_bounds__(64 * BC) k_eb_clip(EnsGrid g, EnsState s, EnsC
 
 void ens_launch_class_b_init(const EnsGrid &g, const EnsState &s, const EnsClassB &b, hipStream_t st) {
   const dim3 gr((g.d.nip + BC - 1) / BC, s.members), bl(64, BC);
-  k_eb_transp0<<<gr, bl, 0, st>>>(g, s, b, 1);
+  k_eb_transp0<<<gr, bl, 0, st>>>(g, s, b);
 }
 
 // transp1 every step; transp2 (w, fct3d) and transp0 on the steps that move
-// the class-B tracers (decided on the device)
-void ens_launch_class_b_step(const EnsGrid &g, const EnsState &s, const EnsClassB &b, hipStream_t st) {
+// the class-B tracers
+void ens_launch_class_b_step(const EnsGrid &g, const EnsState &s, const EnsClassB &b, bool move, hipStream_t st) {
   const dim3 gr((g.d.nip + BC - 1) / BC, s.members), bl(64, BC);
   const dim3 gt((g.d.nip + BC - 1) / BC, s.members, b.ntrb);
   KT_LAUNCH("eb_transp1", st, k_eb_transp1<<<gr, bl, 0, st>>>(g, s, b));
+  if (!move) return;
   KT_LAUNCH("eb_w", st, k_eb_w<<<gr, bl, 0, st>>>(g, s, b));
   const dim3 fg((s.ncol + 63) / 64, b.ntrb);
   if (g.d.nvl == NVL_MAX) KT_LAUNCH("eb_fill", st, (k_eb_fill<NVL_MAX, true><<<fg, 64, 0, st>>>(g.d.nvl, s, b)));
@@ -352,7 +343,7 @@ void ens_launch_class_b_step(const EnsGrid &g, const EnsState &s, const EnsClass
   KT_LAUNCH("eb_vert", st, k_eb_vert<<<gt, bl, 0, st>>>(g, s, b));
   KT_LAUNCH("eb_lo", st, k_eb_lo<<<gt, bl, 0, st>>>(g, s, b));
   KT_LAUNCH("eb_clip", st, k_eb_clip<<<gt, bl, 0, st>>>(g, s, b));
-  KT_LAUNCH("eb_transp0", st, k_eb_transp0<<<gr, bl, 0, st>>>(g, s, b, 0));
+  KT_LAUNCH("eb_transp0", st, k_eb_transp0<<<gr, bl, 0, st>>>(g, s, b));
 }
 
 }  // namespace fimhip
