@@ -616,35 +616,40 @@ def run_uneven(a, th, ds, fimhip):
 # HBM bytes each kernel of the ocean continuity equation must move per ocean
 # cell-level (FP64: edge arrays 6 x 8 B, cell arrays 8 B; a neighbour's value
 # counted once; per-cell grid tables and the clipped-flux sums left out)
-HYC_KERNEL_BYTES = {"hyc_flux": 352, "hyc_lowsum": 144, "hyc_limits": 48, "hyc_clip": 184, "hyc_recover": 128,
-                    "hyc_del2p": 16, "hyc_bolus": 80, "hyc_bclip": 88, "hyc_final": 248, "hyc_check": 48}
+HYC_KERNEL_BYTES = {
+    "hyc_normal": 6 * 48,                       # um vm un vn -> the edges' normal velocities (uploaded edges only)
+    "hyc_flux": 3 * 48 + 16 + 2 * 48 + 24,      # normal velocities, dpm_edg, dp (2) -> fluxes, dp_lo, flux sums
+    "hyc_limits": 48, "hyc_clip": 48 + 32, "hyc_recover": 24, "hyc_del2p": 16, "hyc_bolus": 32, "hyc_bclip": 40,
+    "hyc_final": 5 * 48 + 48 + 32,              # fluxes mssfx_avg, ratios, stages' dp -> massflx mssfx_avg dp pres
+    "hyc_check": 48}
 # what a step must read and write at least per ocean cell-level: um, vm, un,
 # vn, dpm_edg and mssfx_avg in, massflx and mssfx_avg out (8 edge arrays), dp
 # at both leapfrog levels and pres in and out
 HYC_STEP_BYTES = 8 * 48 + 2 * 24
 # the same for the edge interpolation's kernels (neighbour values counted once)
 HYC_EDG_KERNEL_BYTES = {
-    # one launch per level: uclin vclin -> u, v edges; the first also dp ->
-    # pres and u, v edges -> uvsq (both counted half, the mean per launch)
-    "hyc_uvedge": 8 * 2 + 2 * 48 + 8 + 24,
-    "hyc_edgint": 8 + 8 + 16 + 50 + 3 * 48,    # dp pres montg spcifv -> pr_edg dp_edg mont spcv
+    "hyc_vnorm": 32 + 8 + 8 + 2 * 48,          # u v (2 levels) dp -> pres, normal velocities
+    "hyc_edgint": 8 + 48,                      # dp -> dp_edg
     "hyc_janjic": 8 + 8 + 8 + 48,              # pres geop spcifv -> geop_edg
+    # the public arrays, when one is asked for; one launch per level: uclin
+    # vclin -> u, v edges; the first also dp -> pres and u, v edges -> uvsq
+    # (both counted half, the mean per launch)
+    "hyc_uvedge": 8 * 2 + 2 * 48 + 8 + 24,
+    "hyc_edgint_full": 8 + 8 + 16 + 50 + 3 * 48,    # dp pres montg spcifv -> pr_edg dp_edg mont spcv
 }
 HYC_MOM_KERNEL_BYTES = {
-    "hyc_mom_pgf": 16 + 8 + 3 * 48 + 8 + 8 + 16,     # dp (2 levels) u v (new) mont uvsq spcv edges pres -> pres gradx grady
-    "hyc_del4": 16 + 16,                            # u v (new) -> their del4prep
-    "hyc_dissip": 16 + 8 + 16,                      # del4prep u v, dp -> dissipation tendencies
-    "hyc_mom_upd": 96 + 16 + 32 + 16 + 8 + 8 + 32,  # um vm edges, tendencies, u v (2 levels), grad, pres, dp -> u v
+    "hyc_mom_pgf": 32 + 24 + 16 + 8 + 48,           # u v dp (2 levels, old dp) montg spcifv -> pres and six cell arrays
+    "hyc_mom_pgf_edg": 16 + 16 + 5 * 48 + 8 + 48,   # the same from uploaded um vm mont uvsq spcv
+    "hyc_mom_upd": 16 + 8 + 8 + 32 + 32 + 32,       # del4prep u v, dp, pres, u v (2 levels), four cell arrays -> u v
 }
 # bclin_edgvar, cnuity and momtum: in u, v and dp (2 levels), pres, montg,
 # spcifv, mssfx_avg; out u, v (2 levels), dp, pres, massflx, mssfx_avg (the
 # edge values stay inside)
 HYC_OCEAN_STEP_BYTES = (32 + 16 + 8 + 16 + 48) + (32 + 16 + 8 + 48 + 48)
-# bclin_edgvar then cnuity: in uclin, vclin and dp (2 levels), pres, montg,
-# spcifv, mssfx_avg; out the edge values the ocean step goes on to read (um,
-# vm, un, vn, dp_edg, mont_edg, uvsq_edg, spcv_edg on 6 edges, pr_edg on 6
-# edges x kdm+1 interfaces), massflx, mssfx_avg, dp (2 levels) and pres
-HYC_CHAIN_BYTES = (32 + 16 + 8 + 16 + 48) + (8 * 48 + 50) + (2 * 48 + 16 + 8)
+# bclin_edgvar then cnuity: in uclin, vclin and dp (2 levels), pres,
+# mssfx_avg; out massflx, mssfx_avg, dp (2 levels) and pres (the edge values
+# stay inside until one is asked for)
+HYC_CHAIN_BYTES = (32 + 16 + 8 + 48) + (2 * 48 + 16 + 8)
 
 # the tracer transport's kernels with nfld = 2 + numtr tracers: the bytes one
 # launch must move per ocean cell-level (the fct3d kernels run all tracers in

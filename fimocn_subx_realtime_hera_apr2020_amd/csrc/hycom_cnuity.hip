@@ -17,20 +17,32 @@
 // so that each XCD works on a contiguous eighth of the cells and neighbour
 // rows are found in its L2.  A kernel boundary stands wherever a stage reads
 // a neighbour's value that the previous stage writes:
-//   hyc_flux     low/high-order edge fluxes, each edge's pair once (98-159)
-//   hyc_lowsum   low-order thickness, pressure, in/outflow sums of the
-//                antidiffusive fluxes                           (169-265)
+//   hyc_normal   the edges' normal velocities from uploaded edge velocities
+//                (fimhip_ocn_edgvar leaves them formed)
+//   hyc_flux     low/high-order edge fluxes (98-159), low-order thickness and
+//                the in/outflow sums of the antidiffusive fluxes (169-265)
 //   hyc_limits   local bounds and limiter ratios              (269-300)
-//   hyc_clip     limited antidiffusive fluxes and update      (315-393)
+//   hyc_clip     thickness after the limited antidiffusive fluxes, the
+//                clipped parts' column sums                    (315-393)
 //   hyc_recover  the clipped flux as a barotropic correction and its
-//                thickness update; dp from pres, del2p's own part (434-548)
+//                thickness update; dp from pres               (434-548)
 //   hyc_del2p    the biharmonic del2p from the neighbours     (553-603)
-//   hyc_bolus    interface-slope bolus fluxes, outflow ratios (605-683)
-//   hyc_bclip    limited bolus fluxes and their update        (685-776)
-//   hyc_final    the clipped bolus correction, the mass-flux average, the
+//   hyc_bolus    the ratio of each layer to its interface-slope bolus outflow
+//                (biharmonic form only)                       (605-683)
+//   hyc_bclip    clipped bolus fluxes and update              (685-776)
+//   hyc_final    the edge mass flux of all stages, the mass-flux average, the
 //                leapfrog time smoothing, the bottom pressure (778-954)
-// The thickness after the antidiffusive update goes to its own array (dpc),
-// which hyc_recover reads at the neighbours while it writes the new level.
+// All of these are bound by memory, and an edge array (six values per cell
+// and layer) is six times a cell array, so only three are kept between the
+// kernels: the low-order flux, the antidiffusive flux and, at the end, the
+// mass flux.  The mass flux of the stages in between is not updated in
+// memory: hyc_final forms the limited flux and both barotropic corrections
+// again from cell values, and the bolus flux is formed by each kernel that
+// reads it.  (With every stage's flux in memory, and the fluxes' sums in a
+// kernel of their own, G7 x 32 layers took 1.46 ms a step in these kernels;
+// this takes 1.24.)
+// A stage's thickness has an array of its own where the next stage reads it
+// at the neighbours.
 // The duplicate-flux check (chkdup) compares each pair of edge fluxes once
 // and sets a flag; the global mass and its drift correction (glob2d) are
 // summed on the host in cell order, as the reference does serially.
@@ -47,74 +59,30 @@ namespace hyc {
 namespace {
 
 
-// the high- and low-order fluxes of one edge seen from the cell whose values
-// are 'a' (its edge ea) towards the cell 'b' (its edge eb)  (98-159)
-struct EdgeFlux {
-  double anti, low;
-};
-__device__ __forceinline__ EdgeFlux edge_flux(const HycGrid &g, const HycState &s, const double *dpm,
-                                              const double *dpn, int kdm, int a, int ea, int b, int eb, int k,
-                                              double dtleap) {
-  double valu1 = HSVE(a, ea, 1) * HE(s.um, a, ea, k) - HSVE(a, ea, 0) * HE(s.vm, a, ea, k);
-  double valu2 = HSVE(b, eb, 1) * HE(s.um, b, eb, k) - HSVE(b, eb, 0) * HE(s.vm, b, eb, k);
-  const double outgom = .5 * (valu1 - valu2);
-  valu1 = g.rsideln[a * NPP + ea] * dtleap * g.rprox_ln[a * NPP + ea];
-  valu2 = g.rsideln[b * NPP + eb] * dtleap * g.rprox_ln[b * NPP + eb];
-  const double q = hmin(fabs(outgom) * .5 * (valu1 + valu2), 1.);
-  const double dpedg = .5 * (HE(s.dpm_edg, a, ea, k) + HE(s.dpm_edg, b, eb, k));
-  double hi = outgom >= 0. ? dpedg * (1. - q) + HC(dpm, a, k) * q : dpedg * (1. - q) + HC(dpm, b, k) * q;
-  hi = hi * outgom;
-  valu1 = HSVE(a, ea, 1) * HE(s.un, a, ea, k) - HSVE(a, ea, 0) * HE(s.vn, a, ea, k);
-  valu2 = HSVE(b, eb, 1) * HE(s.un, b, eb, k) - HSVE(b, eb, 0) * HE(s.vn, b, eb, k);
-  const double outgon = .5 * (valu1 - valu2);
-  const double lo = outgon >= 0. ? outgon * HC(dpn, a, k) : outgon * HC(dpn, b, k);
-  return EdgeFlux{hi - lo, lo};
-}
-
-// the edge fluxes, each pair of an edge's two sides once: the cell of lower
-// index evaluates the reference's expression from both sides (the same
-// operations with the two cells' roles exchanged) and writes both
+// the normal velocities of the ocean's edges from the edge velocities (98-106)
 template <int LPC>
-__global__ void __launch_bounds__(256) hyc_flux(HycGrid g, HycState s, int leapm, int leapn, double dtleap) {
-  const int kdm = g.kdm, nip = g.nip;
-  const Col<LPC> c = hcol<LPC>(nip);
+__global__ void __launch_bounds__(256) hyc_normal(HycGrid g, HycState s) {
+  const int kdm = g.kdm;
+  const Col<LPC> c = hcol<LPC>(g.nip);
   if (!c.ok || c.k >= kdm) return;
   const int i = c.i, k = c.k;
-  const int ci = g.cinfo[i];
-  int ix[NPP], ex[NPP];
+  if (!ci_wet(g.cinfo[i])) return;
 #pragma unroll
   for (int e = 0; e < NPP; e++) {
-    ix[e] = g.prox[i * NPP + e];
-    ex[e] = g.proxs[i * NPP + e];
-  }
-  if (!ci_wet(ci)) {      // (the work array of antidiffusive fluxes is never read on land)
-#pragma unroll
-    for (int e = 0; e < NPP; e++) HE(s.massflx, i, e, k) = H_LAND;
-    return;
-  }
-  const double *dpm = s.dp + (size_t)(leapm - 1) * nip * kdm, *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
-  const int np = ci_np(ci);
-#pragma unroll
-  for (int e = 0; e < NPP; e++) {
-    const bool open = ci_open(ci, e);
-    if (open && i < ix[e]) {
-      const EdgeFlux fa = edge_flux(g, s, dpm, dpn, kdm, i, e, ix[e], ex[e], k, dtleap);
-      const EdgeFlux fb = edge_flux(g, s, dpm, dpn, kdm, ix[e], ex[e], i, e, k, dtleap);
-      __builtin_nontemporal_store(fa.anti, &HE(s.antiflx, i, e, k));
-      __builtin_nontemporal_store(fa.low, &HE(s.massflx, i, e, k));
-      __builtin_nontemporal_store(fb.anti, &HE(s.antiflx, ix[e], ex[e], k));
-      __builtin_nontemporal_store(fb.low, &HE(s.massflx, ix[e], ex[e], k));
-    } else if (!open) {      // an edge to land carries no flux; a pentagon's sixth slot is land-valued
-      HE(s.antiflx, i, e, k) = HE(s.massflx, i, e, k) = e < np ? 0. : H_LAND;
-    }
+    HE(s.vnm, i, e, k) = HSVE(i, e, 1) * HE(s.um, i, e, k) - HSVE(i, e, 0) * HE(s.vm, i, e, k);
+    HE(s.vnn, i, e, k) = HSVE(i, e, 1) * HE(s.un, i, e, k) - HSVE(i, e, 0) * HE(s.vn, i, e, k);
   }
 }
 
-// low-order thickness, pressure and the in/outflow sums of the antidiffusive
-// fluxes (169-265)
+// the edge fluxes, every cell its own six (the expression of either side of
+// an edge is the other's with the roles exchanged), and their sums.  Bound by
+// memory: three edge arrays read at the cell and its neighbours' matching
+// edges, two written; forming each pair once, by the cell of lower index,
+// would read less from the caches and not from HBM, and would need the sums
+// in a second pass over both fluxes.
 template <int LPC>
-__global__ void __launch_bounds__(256) hyc_lowsum(HycGrid g, HycState s, int leapn, double dtleap) {
-  __shared__ double sh[256 / LPC][LPC + 1];
+__global__ void __launch_bounds__(256) hyc_flux(HycGrid g, HycState s, int leapm, int leapn, double dtleap) {
+  __shared__ double scf[256 / LPC][NPP];
   const int kdm = g.kdm, nip = g.nip;
   const Col<LPC> c = hcol<LPC>(nip);
   if (!c.ok) return;
@@ -122,41 +90,75 @@ __global__ void __launch_bounds__(256) hyc_lowsum(HycGrid g, HycState s, int lea
   const bool live = k < kdm;
   const int kk = live ? k : 0;
   const int ci = g.cinfo[i];
-  if (!ci_wet(ci)) {
-    if (live) {
-      __builtin_nontemporal_store(0., &HC(s.dp_lo, i, k));
-      __builtin_nontemporal_store(H_EPSIL, &HC(s.flxplus, i, k));
-      __builtin_nontemporal_store(-H_EPSIL, &HC(s.flxmnus, i, k));
-    }
-    return;
-  }
-  const double *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
-  const int np = ci_np(ci);
-  double mf[NPP], af[NPP];
+  int ix[NPP], ex[NPP];
 #pragma unroll
   for (int e = 0; e < NPP; e++) {
-    mf[e] = HE(s.massflx, i, e, kk);
-    af[e] = HE(s.antiflx, i, e, kk);
+    ix[e] = g.prox[i * NPP + e];
+    ex[e] = g.proxs[i * NPP + e];
   }
-  const double d = HC(dpn, i, kk);
-  double flx = 0.;
+  if (!ci_wet(ci)) {      // (no work array is read on land)
+    if (live)
 #pragma unroll
-  for (int e = 0; e < NPP; e++)
-    if (e < np) flx = flx + mf[e];
-  if (live) __builtin_nontemporal_store(d, &HC(s.dpold, i, k));
-  const double p = col_pres(sh[c.cc], live ? d : 0., HP(i, 0), k, kdm);
+      for (int e = 0; e < NPP; e++) __builtin_nontemporal_store(H_LAND, &HE(s.massflx, i, e, k));
+    return;
+  }
+  const double *dpm = s.dp + (size_t)(leapm - 1) * nip * kdm, *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
+  const int np = ci_np(ci);
+  const double mi = HC(dpm, i, kk), d = HC(dpn, i, kk);
+  // lane e: the sum of both sides' time step over the length scale of edge e
+  if (k < NPP) {
+    const int x = g.prox[i * NPP + k] * NPP + g.proxs[i * NPP + k], a = i * NPP + k;
+    scf[c.cc][k] = g.rsideln[a] * dtleap * g.rprox_ln[a] + g.rsideln[x] * dtleap * g.rprox_ln[x];
+  }
+  wave_sync();
+  double flx = 0., fp = H_EPSIL, fm = -H_EPSIL;
+  // two edges at a time: the six would hold 62 values in flight, and 12
+  // waves a compute unit are too few for the loads' latency
+  constexpr int HF = 2;
+#pragma unroll
+  for (int e0 = 0; e0 < NPP; e0 += HF) {
+    double va[HF], vb[HF], na[HF], nb[HF], da[HF], db[HF], mx[HF], nx[HF];
+#pragma unroll
+    for (int h = 0; h < HF; h++) {
+      const int e = e0 + h;
+      va[h] = HE(s.vnm, i, e, kk);
+      vb[h] = HE(s.vnm, ix[e], ex[e], kk);
+      da[h] = HE(s.dpm_edg, i, e, kk);
+      db[h] = HE(s.dpm_edg, ix[e], ex[e], kk);
+      mx[h] = HC(dpm, ix[e], kk);
+      na[h] = HE(s.vnn, i, e, kk);
+      nb[h] = HE(s.vnn, ix[e], ex[e], kk);
+      nx[h] = HC(dpn, ix[e], kk);
+    }
+#pragma unroll
+    for (int h = 0; h < HF; h++) {
+      const int e = e0 + h;
+      const bool open = ci_open(ci, e);
+      const double outgom = .5 * (va[h] - vb[h]);
+      const double q = hmin(fabs(outgom) * .5 * scf[c.cc][e], 1.);
+      const double dpedg = .5 * (da[h] + db[h]);
+      double hi = dpedg * (1. - q) + (outgom >= 0. ? mi : mx[h]) * q;
+      hi = hi * outgom;
+      const double outgon = .5 * (na[h] - nb[h]);
+      const double lo = outgon * (outgon >= 0. ? d : nx[h]);
+      const double anti = hi - lo;
+      // an edge to land carries no flux; a pentagon's sixth slot is land-valued
+      if (live) {
+        __builtin_nontemporal_store(open ? lo : e < np ? 0. : H_LAND, &HE(s.massflx, i, e, k));
+        if (open) __builtin_nontemporal_store(anti, &HE(s.antiflx, i, e, k));
+      }
+      if (open) {
+        flx = flx + lo;
+        if (anti >= 0.) fp = fp + anti;
+        else fm = fm + anti;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if (!live) return;
-  __builtin_nontemporal_store(p, &HP(i, k + 1));
   double lo = d - flx * g.rarea[i] * dtleap;
   if (lo < 0. && lo + H_ONECM > 0.) lo = 0.;
   __builtin_nontemporal_store(lo, &HC(s.dp_lo, i, k));
-  double fp = H_EPSIL, fm = -H_EPSIL;
-#pragma unroll
-  for (int e = 0; e < NPP; e++) {
-    if (e >= np) break;
-    if (af[e] >= 0.) fp = fp + af[e];
-    else fm = fm + af[e];
-  }
   __builtin_nontemporal_store(fp, &HC(s.flxplus, i, k));
   __builtin_nontemporal_store(fm, &HC(s.flxmnus, i, k));
 }
@@ -171,10 +173,7 @@ __global__ void __launch_bounds__(256) hyc_limits(HycGrid g, HycState s, int lea
   int nb[NPP];      // neighbours, loaded before the mask is tested
 #pragma unroll
   for (int e = 0; e < NPP; e++) nb[e] = g.prox[i * NPP + e];
-  if (!ci_wet(ci)) {
-    HC(s.rplus, i, k) = HC(s.rmnus, i, k) = 0.;
-    return;
-  }
+  if (!ci_wet(ci)) return;
   const double *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
   const double lo = HC(s.dp_lo, i, k), dn = HC(dpn, i, k);
   double dpmax = hmax(lo, dn), dpmin = hmin(lo, dn);
@@ -190,6 +189,21 @@ __global__ void __launch_bounds__(256) hyc_limits(HycGrid g, HycState s, int lea
   dpmin = hmax(0., dpmin);
   __builtin_nontemporal_store((lo - dpmin) * g.area[i] / (dtleap * HC(s.flxplus, i, k)), &HC(s.rmnus, i, k));
   __builtin_nontemporal_store((lo - dpmax) * g.area[i] / (dtleap * HC(s.flxmnus, i, k)), &HC(s.rplus, i, k));
+}
+
+// the limiter of an edge's antidiffusive flux a towards a neighbour with the
+// ratios rpx, rmx (315-336)
+__device__ __forceinline__ double anti_clip(double a, double rpi, double rmi, double rpx, double rmx) {
+  return a >= 0. ? hmin(hmin(1., rmi), rpx) : hmin(hmin(1., rpi), rmx);
+}
+// the barotropic flux that returns an edge's clipped sum cl (434-453): upstream,
+// by the layer's share of the column; that of the bolus fluxes (778-795) forms
+// its product in another order
+__device__ __forceinline__ double baro_flux(double cl, double di, double rpi, double dx, double rpx) {
+  return cl > 0. ? cl * (di * rpi) : (cl < 0. ? cl * (dx * rpx) : 0.);
+}
+__device__ __forceinline__ double baro_flux_b(double cl, double di, double rpi, double dx, double rpx) {
+  return cl > 0. ? cl * di * rpi : (cl < 0. ? cl * dx * rpx : 0.);
 }
 
 template <int LPC>
@@ -209,20 +223,16 @@ __global__ void __launch_bounds__(256) hyc_clip(HycGrid g, HycState s, double dt
     if (k < NPP) s.clippd[i * NPP + k] = 0.;
     return;
   }
-  const int np = ci_np(ci);
   const double rmi = HC(s.rmnus, i, kk), rpi = HC(s.rplus, i, kk);
   double part[NPP], flx = 0.;
 #pragma unroll
   for (int e = 0; e < NPP; e++) {
     const int ix = nb[e];
-    const double a = HE(s.antiflx, i, e, kk), mfv = HE(s.massflx, i, e, kk);
-    const double rpx = HC(s.rplus, ix, kk), rmx = HC(s.rmnus, ix, kk);
-    const double clip = a >= 0. ? hmin(hmin(1., rmi), rpx) : hmin(hmin(1., rpi), rmx);
+    const double a = HE(s.antiflx, i, e, kk);
+    const double clip = anti_clip(a, rpi, rmi, HC(s.rplus, ix, kk), HC(s.rmnus, ix, kk));
     const bool open = ci_open(ci, e);
-    const double ac = a * clip;
     part[e] = open && live ? a * (1. - clip) : 0.;
-    if (open && live) __builtin_nontemporal_store(mfv + ac, &HE(s.massflx, i, e, k));
-    if (e < np) flx = flx + (open ? ac : a);    // a closed edge's antidiffusive flux is 0
+    flx = open ? flx + a * clip : flx;
   }
   const double cl = col_sums6<LPC>(sh[c.cc], part, k, kdm);
   if (k < NPP) s.clippd[i * NPP + k] = cl;
@@ -233,16 +243,14 @@ __global__ void __launch_bounds__(256) hyc_clip(HycGrid g, HycState s, double dt
     __builtin_nontemporal_store(d, &HC(s.dpc, i, k));
   }
   const double p = col_pres(sh[c.cc][0], d, HP(i, 0), k, kdm);
-  if (live) __builtin_nontemporal_store(p, &HP(i, k + 1));
   if (k == kdm - 1) s.rpbot[i] = 1. / p;
 }
 
 // the clipped fluxes back as an upstream barotropic correction and its
 // thickness update (434-491); with interface smoothing, dp again from the
-// interface pressures and del2p's own part (508-548)
+// interface pressures (508-548)
 template <int LPC>
-__global__ void __launch_bounds__(256) hyc_recover(HycGrid g, HycState s, int leapn, double dtleap, int smooth,
-                                                   double biharm) {
+__global__ void __launch_bounds__(256) hyc_recover(HycGrid g, HycState s, double dtleap, int smooth) {
   __shared__ double sh[256 / LPC][LPC + 1];
   const int kdm = g.kdm, nip = g.nip;
   const Col<LPC> c = hcol<LPC>(nip);
@@ -254,23 +262,14 @@ __global__ void __launch_bounds__(256) hyc_recover(HycGrid g, HycState s, int le
   int nb[NPP];      // neighbours, loaded before the mask is tested
 #pragma unroll
   for (int e = 0; e < NPP; e++) nb[e] = g.prox[i * NPP + e];
-  if (!ci_wet(ci)) {
-    if (smooth && live) __builtin_nontemporal_store(biharm == 0. && k >= 1 ? HP(i, k) : H_LAND, &HC(s.del2p, i, k));
-    return;
-  }
-  double *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
+  if (!ci_wet(ci)) return;
   const double dci = HC(s.dpc, i, kk), rpi = s.rpbot[i];
   double flx = 0.;
 #pragma unroll
   for (int e = 0; e < NPP; e++) {
     const int ix = nb[e];
-    const double cl = s.clippd[i * NPP + e], dcx = HC(s.dpc, ix, kk), rpx = s.rpbot[ix];
-    const double mfv = HE(s.massflx, i, e, kk);
-    const double q = cl > 0. ? cl * (dci * rpi) : (cl < 0. ? cl * (dcx * rpx) : 0.);
-    if (ci_open(ci, e)) {
-      flx = flx + q;
-      if (live) __builtin_nontemporal_store(mfv + q, &HE(s.massflx, i, e, k));
-    }
+    const double q = baro_flux(s.clippd[i * NPP + e], dci, rpi, HC(s.dpc, ix, kk), s.rpbot[ix]);
+    flx = ci_open(ci, e) ? flx + q : flx;
   }
   double d = 0.;
   if (live) {
@@ -279,17 +278,11 @@ __global__ void __launch_bounds__(256) hyc_recover(HycGrid g, HycState s, int le
   }
   const double p0 = HP(i, 0);
   const double p = col_pres(sh[c.cc], d, p0, k, kdm);
-  if (live) __builtin_nontemporal_store(p, &HP(i, k + 1));
-  if (smooth) {
-    const double pa = __shfl_up(p, 1, LPC);
-    const double pk = k > 0 ? pa : p0;         // the interface above layer k
-    if (live) {
-      __builtin_nontemporal_store(p - pk, &HC(dpn, i, k));
-      __builtin_nontemporal_store(biharm == 0. && k >= 1 ? pk : H_LAND, &HC(s.del2p, i, k));
-    }
-  } else if (live) {
-    __builtin_nontemporal_store(d, &HC(dpn, i, k));
-  }
+  const double pa = __shfl_up(p, 1, LPC);
+  const double pk = k > 0 ? pa : p0;         // the interface above layer k
+  if (!live) return;
+  __builtin_nontemporal_store(p, &HP(i, k + 1));
+  __builtin_nontemporal_store(smooth ? p - pk : d, &HC(s.dpr, i, k));
 }
 
 template <int LPC>
@@ -319,56 +312,75 @@ __global__ void __launch_bounds__(256) hyc_del2p(HycGrid g, HycState s, double b
   __builtin_nontemporal_store(biharm * sum / (double)ncount + (1. - biharm) * pi, &HC(s.del2p, i, k));
 }
 
-// bolus fluxes (605-646; the antidiffusive-flux array holds them) and, for
-// the biharmonic form, the ratio of each layer's mass to its outflow (664-683)
+// The bolus fluxes of a cell's six edges at lane k's layer (605-646): the
+// flux of each interface between two layers, limited to what either side
+// holds below it, and the layer's as the difference of its two interfaces'.
+// del2p is the interface pressure itself unless the form is biharmonic.
+// ed: a few LDS words per edge, filled here by lane e of the column with what
+// the neighbour's column has one of (each lane loading them for itself costs
+// the column a load per edge and value)
 template <int LPC>
-__global__ void __launch_bounds__(256) hyc_bolus(HycGrid g, HycState s, int leapn, double dtleap, double thkdff,
-                                                 double biharm) {
+__device__ __forceinline__ void bolus_fluxes(const HycGrid &g, const HycState &s, int i, int ci, const int (&nb)[NPP],
+                                             int k, double dtleap, double thkdff, double biharm,
+                                             double (*ed)[NPP], double (&f)[NPP]) {
+  const int kdm = g.kdm;
+  const int kk = k < kdm ? k : 0;
+  double pxk[NPP], dx[NPP];
+#pragma unroll
+  for (int e = 0; e < NPP; e++) {
+    pxk[e] = HP(nb[e], kk);
+    dx[e] = biharm > 0. ? HC(s.del2p, nb[e], kk) : 0.;
+  }
+  if (k < NPP) {
+    const int x = g.prox[i * NPP + k];
+    ed[0][k] = HP(x, kdm);
+    ed[1][k] = g.area[x];
+    ed[2][k] = (double)ci_np(g.cinfo[x]);
+    ed[3][k] = g.sideln[i * NPP + k];
+  }
+  const double pik = HP(i, kk), pbi = HP(i, kdm);
+  const double di = biharm > 0. ? HC(s.del2p, i, kk) : pik;
+  const double flxmn = -((pbi - pik) * g.area[i] / (double)ci_np(ci));
+  wave_sync();
+#pragma unroll
+  for (int e = 0; e < NPP; e++) {
+    // the limited flux of interface k (between layers k-1 and k), lanes 1..kdm-1
+    const double q = dtleap * thkdff * (di - (biharm > 0. ? dx[e] : pxk[e])) * ed[3][e];
+    const double flxmx = (ed[0][e] - pxk[e]) * ed[1][e] / ed[2][e];
+    const double b = k >= 1 && k < kdm ? hmin(flxmx * .999, hmax(flxmn * .999, q)) : 0.;
+    // layer k's flux: interface k+1's minus interface k's (0 above the top),
+    // the bottom layer minus interface kdm-1's
+    const double bn = __shfl_down(b, 1, LPC);
+    f[e] = ci_open(ci, e) ? (k < kdm - 1 ? bn - b : -b) : 0.;
+  }
+}
+
+// the ratio of each layer's mass to its bolus outflow (664-683)
+template <int LPC>
+__global__ void __launch_bounds__(256) hyc_bolus(HycGrid g, HycState s, double dtleap, double thkdff, double biharm) {
+  __shared__ double sed[256 / LPC][4][NPP];
   const int kdm = g.kdm, nip = g.nip;
   const Col<LPC> c = hcol<LPC>(nip);
   if (!c.ok) return;
   const int i = c.i, k = c.k;
-  const bool live = k < kdm;
-  const int kk = live ? k : 0;
   const int ci = g.cinfo[i];
   int nb[NPP];      // neighbours, loaded before the mask is tested
 #pragma unroll
   for (int e = 0; e < NPP; e++) nb[e] = g.prox[i * NPP + e];
-  if (!ci_wet(ci)) return;      // the bolus fluxes of land are never read
-  const int np = ci_np(ci);
-  const double pik = HP(i, kk), pbi = HP(i, kdm), di = HC(s.del2p, i, kk), ai = g.area[i];
-  double fp = H_EPSIL;
+  if (!ci_wet(ci)) return;
+  const double dr = HC(s.dpr, i, k < kdm ? k : 0);
+  double f[NPP], fp = H_EPSIL;
+  bolus_fluxes<LPC>(g, s, i, ci, nb, k, dtleap, thkdff, biharm, sed[c.cc], f);
 #pragma unroll
-  for (int e = 0; e < NPP; e++) {
-    const int ix = nb[e];
-    const double dx = HC(s.del2p, ix, kk), pxk = HP(ix, kk), pbx = HP(ix, kdm), ax = g.area[ix];
-    const int npx = ci_np(g.cinfo[ix]);
-    const double sl = g.sideln[i * NPP + e];
-    // the limited flux of interface k (between layers k-1 and k), lanes 1..kdm-1
-    double b = 0.;
-    if (live && k >= 1) {
-      const double q = dtleap * thkdff * (di - dx) * sl;
-      const double flxmx = (pbx - pxk) * ax / (double)npx;
-      const double flxmn = -((pbi - pik) * ai / (double)np);
-      b = hmin(flxmx * .999, hmax(flxmn * .999, q));
-    }
-    // layer k's flux: interface k+1's minus interface k's (0 above the top),
-    // the bottom layer minus interface kdm-1's
-    const double bn = __shfl_down(b, 1, LPC);
-    double f = k < kdm - 1 ? bn - b : -b;
-    f = ci_open(ci, e) ? f : 0.;
-    if (live) __builtin_nontemporal_store(f, &HE(s.antiflx, i, e, k));
-    if (biharm > 0. && e < np) fp = fp + hmax(0., f);
-  }
-  if (biharm > 0. && live) {
-    const double *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
-    __builtin_nontemporal_store(HC(dpn, i, k) * ai / fp, &HC(s.rmnus, i, k));
-  }
+  for (int e = 0; e < NPP; e++)
+    if (e < ci_np(ci)) fp = fp + hmax(0., f[e]);
+  if (k < kdm) __builtin_nontemporal_store(dr * g.area[i] / fp, &HC(s.brat, i, k));
 }
 
 template <int LPC>
-__global__ void __launch_bounds__(256) hyc_bclip(HycGrid g, HycState s, int leapn, double biharm, double masscor) {
-  __shared__ double sh[256 / LPC][NPP][LPC + 1];
+__global__ void __launch_bounds__(256) hyc_bclip(HycGrid g, HycState s, double dtleap, double thkdff, double biharm,
+                                                 double masscor) {
+  __shared__ double sh[256 / LPC][NPP][LPC + 1], sed[256 / LPC][4][NPP];
   const int kdm = g.kdm, nip = g.nip;
   const Col<LPC> c = hcol<LPC>(nip);
   if (!c.ok) return;
@@ -380,20 +392,19 @@ __global__ void __launch_bounds__(256) hyc_bclip(HycGrid g, HycState s, int leap
 #pragma unroll
   for (int e = 0; e < NPP; e++) nb[e] = g.prox[i * NPP + e];
   if (!ci_wet(ci)) {
-    if (biharm > 0. && k < NPP) s.clippd[i * NPP + k] = 0.;
+    if (biharm > 0. && k < NPP) s.clippb[i * NPP + k] = 0.;
     return;
   }
   const int np = ci_np(ci);
-  const double rmi = HC(s.rmnus, i, kk);
-  double part[NPP], flx = 0.;
+  const double p0 = HP(i, 0), dr = HC(s.dpr, i, kk);
+  double f[NPP], part[NPP], flx = 0.;
+  bolus_fluxes<LPC>(g, s, i, ci, nb, k, dtleap, thkdff, biharm, sed[c.cc], f);
+  const double rmi = HC(s.brat, i, kk);
 #pragma unroll
   for (int e = 0; e < NPP; e++) {
-    const int ix = nb[e];
-    double b = HE(s.antiflx, i, e, kk);
-    const double rmx = HC(s.rmnus, ix, kk);
-    double pt = 0.;
+    double b = f[e], pt = 0.;
     if (biharm > 0.) {
-      const double clip = b > 0. ? hmin(1., rmi) : hmin(1., rmx);
+      const double clip = b > 0. ? hmin(1., rmi) : hmin(1., HC(s.brat, nb[e], kk));
       const bool doit = ci_open(ci, e) && b != 0.;
       pt = doit ? b * (1. - clip) : 0.;
       b = doit ? b * clip : b;
@@ -403,26 +414,28 @@ __global__ void __launch_bounds__(256) hyc_bclip(HycGrid g, HycState s, int leap
   }
   if (biharm > 0.) {
     const double cl = col_sums6<LPC>(sh[c.cc], part, k, kdm);
-    if (k < NPP) s.clippd[i * NPP + k] = cl;
+    if (k < NPP) s.clippb[i * NPP + k] = cl;
   }
   double d = 0.;
-  double *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
   if (live) {
-    d = HC(dpn, i, k) - flx * g.rarea[i];
+    d = dr - flx * g.rarea[i];
     if (d < 0. && d + H_ONECM > 0.) d = 0.;
     d = d * (1. + masscor);
-    __builtin_nontemporal_store(d, &HC(dpn, i, k));
     __builtin_nontemporal_store(d, &HC(s.dptmp, i, k));
   }
-  const double p = col_pres(sh[c.cc][0], d, HP(i, 0), k, kdm);
-  if (live) __builtin_nontemporal_store(p, &HP(i, k + 1));
-  if (k == kdm - 1) s.rpbot[i] = 1. / p;
+  // (the interfaces themselves are read at the neighbours by this kernel:
+  // hyc_final stores the new ones)
+  const double p = col_pres(sh[c.cc][0], d, p0, k, kdm);
+  if (k == kdm - 1) s.rpbotb[i] = 1. / p;
 }
 
+// The mass flux of all stages, from the low-order and antidiffusive fluxes and
+// the stages' cell values, and the last thickness.  Bound by memory: three
+// edge arrays read and two written.
 template <int LPC>
-__global__ void __launch_bounds__(256) hyc_final(HycGrid g, HycState s, int leapm, int leapn, double dtleap,
+__global__ void __launch_bounds__(256, 4) hyc_final(HycGrid g, HycState s, int leapm, int leapn, double dtleap,
                                                  int smooth, double biharm) {
-  __shared__ double sh[256 / LPC][LPC + 1];
+  __shared__ double sh[256 / LPC][LPC + 1], sed[256 / LPC][4][NPP];
   const int kdm = g.kdm, nip = g.nip;
   const Col<LPC> c = hcol<LPC>(nip);
   if (!c.ok) return;
@@ -439,37 +452,79 @@ __global__ void __launch_bounds__(256) hyc_final(HycGrid g, HycState s, int leap
   }
   double *dpm = s.dp + (size_t)(leapm - 1) * nip * kdm, *dpn = s.dp + (size_t)(leapn - 1) * nip * kdm;
   const int np = ci_np(ci);
+  const double p0 = HP(i, 0);
+  const double rmi = HC(s.rmnus, i, kk), rpi = HC(s.rplus, i, kk);
+  const double dci = HC(s.dpc, i, kk), rbi = s.rpbot[i];
+  // lane e: what edge e's two columns have one of
+  double (*ed)[NPP] = sed[c.cc];
+  if (k < NPP) {
+    const int x = g.prox[i * NPP + k];
+    ed[0][k] = s.clippd[i * NPP + k];
+    ed[1][k] = s.rpbot[x];
+    ed[2][k] = s.clippb[i * NPP + k];
+    ed[3][k] = s.rpbotb[x];
+  }
+  wave_sync();
   double mf[NPP];
+  constexpr int HF = 3;      // three edges at a time in registers, for more waves in flight
 #pragma unroll
-  for (int e = 0; e < NPP; e++) mf[e] = HE(s.massflx, i, e, kk);
-  double dn = HC(dpn, i, kk);
+  for (int e0 = 0; e0 < NPP; e0 += HF) {
+    double af[HF], rpx[HF], rmx[HF], dcx[HF];
+#pragma unroll
+    for (int h = 0; h < HF; h++) {
+      const int e = e0 + h;
+      mf[e] = HE(s.massflx, i, e, kk);
+      af[h] = HE(s.antiflx, i, e, kk);
+      rpx[h] = HC(s.rplus, nb[e], kk);
+      rmx[h] = HC(s.rmnus, nb[e], kk);
+      dcx[h] = HC(s.dpc, nb[e], kk);
+    }
+#pragma unroll
+    for (int h = 0; h < HF; h++) {
+      const int e = e0 + h;
+      const double clip = anti_clip(af[h], rpi, rmi, rpx[h], rmx[h]);
+      const double q = baro_flux(ed[0][e], dci, rbi, dcx[h], ed[1][e]);
+      mf[e] = ci_open(ci, e) ? mf[e] + af[h] * clip + q : mf[e];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  double dn = HC(smooth ? s.dptmp : s.dpr, i, kk), av[NPP];
+  const double dold = HC(dpn, i, kk), dm = HC(dpm, i, kk);
+#pragma unroll
+  for (int e = 0; e < NPP; e++) av[e] = smooth ? HE(s.mssfx_avg, i, e, kk) : 0.;
   if (smooth && biharm > 0.) {
     const double dtinv = 1. / dtleap;
-    const double dti = HC(s.dptmp, i, kk), rpi = s.rpbot[i];
+    const double dti = dn, rci = s.rpbotb[i];
     double flx = 0.;
 #pragma unroll
     for (int e = 0; e < NPP; e++) {
       const int ix = nb[e];
-      const double cl = s.clippd[i * NPP + e], dtx = HC(s.dptmp, ix, kk), rpx = s.rpbot[ix];
-      const double q = cl > 0. ? cl * dti * rpi : (cl < 0. ? cl * dtx * rpx : 0.);
+      const double q = baro_flux_b(ed[2][e], dti, rci, HC(s.dptmp, ix, kk), ed[3][e]);
       if (e < np) {
         flx = flx + q;
         mf[e] = mf[e] + q * dtinv;
-        if (live) __builtin_nontemporal_store(mf[e], &HE(s.massflx, i, e, k));
       }
     }
     dn = dn - flx * g.rarea[i];
-    if (live) __builtin_nontemporal_store(dn, &HC(dpn, i, k));
-    const double p = col_pres(sh[c.cc], live ? dn : 0., HP(i, 0), k, kdm);
-    if (live) __builtin_nontemporal_store(p, &HP(i, k + 1));
+  }
+  double pb = 0.;
+  if (smooth) {
+    pb = col_pres(sh[c.cc], live ? dn : 0., p0, k, kdm);
+    if (live) __builtin_nontemporal_store(pb, &HP(i, k + 1));
+  } else if (k == kdm - 1) {
+    pb = HP(i, kdm);
   }
   if (!live) return;
-  if (smooth)
 #pragma unroll
-    for (int e = 0; e < NPP; e++)
-      if (e < np) __builtin_nontemporal_store(HE(s.mssfx_avg, i, e, k) + mf[e], &HE(s.mssfx_avg, i, e, k));
-  __builtin_nontemporal_store(H_ASSLDP * (HC(s.dpold, i, k) + dn) + (1. - H_ASSLDP - H_ASSLDP) * HC(dpm, i, k), &HC(dpm, i, k));
-  if (k == kdm - 1) s.aux[i] = HP(i, kdm);
+  for (int e = 0; e < NPP; e++)
+    if (e < np) {
+      __builtin_nontemporal_store(mf[e], &HE(s.massflx, i, e, k));
+      if (smooth) __builtin_nontemporal_store(av[e] + mf[e], &HE(s.mssfx_avg, i, e, k));
+    }
+  __builtin_nontemporal_store(dn, &HC(dpn, i, k));
+  __builtin_nontemporal_store(dm, &HC(s.dpe, i, k));
+  __builtin_nontemporal_store(H_ASSLDP * (dold + dn) + (1. - H_ASSLDP - H_ASSLDP) * dm, &HC(dpm, i, k));
+  if (k == kdm - 1) s.aux[i] = pb;
 }
 
 // duplicate edge fluxes must be equal and opposite bit for bit (chkdup); the
@@ -600,18 +655,21 @@ extern "C" int fimhip_ocn_create(const fimhip_grid_desc *gd, const double *rprox
   double *um, *vm, *un, *vn, *dpe;
   struct { double **p; size_t n; } arrs[] = {
       {&um, ez}, {&vm, ez}, {&un, ez}, {&vn, ez}, {&dpe, ez}, {&s.dp, 2 * cz}, {&s.pres, (size_t)nip * (kdm + 1)},
-      {&s.massflx, ez}, {&s.mssfx_avg, ez}, {&s.antiflx, ez}, {&s.dp_lo, cz}, {&s.dpold, cz}, {&s.flxplus, cz},
-      {&s.flxmnus, cz}, {&s.rplus, cz}, {&s.rmnus, cz}, {&s.del2p, cz}, {&s.dptmp, cz}, {&s.dpc, cz},
-      {&s.clippd, (size_t)nip * NPP}, {&s.rpbot, (size_t)nip}, {&s.aux, (size_t)nip},
+      {&s.massflx, ez}, {&s.mssfx_avg, ez}, {&s.antiflx, ez}, {&s.vnm, ez}, {&s.vnn, ez}, {&s.dp_lo, cz},
+      {&s.dpc, cz}, {&s.dpr, cz}, {&s.flxplus, cz}, {&s.flxmnus, cz}, {&s.rplus, cz}, {&s.rmnus, cz},
+      {&s.del2p, cz}, {&s.dptmp, cz}, {&s.brat, cz}, {&s.clippd, (size_t)nip * NPP}, {&s.clippb, (size_t)nip * NPP},
+      {&s.rpbot, (size_t)nip}, {&s.rpbotb, (size_t)nip}, {&s.aux, (size_t)nip}, {&s.dpe, cz},
+      {&s.pbe, (size_t)nip}, {&s.p0e, (size_t)nip}, {&o->pres_f, (size_t)nip * (kdm + 1)},
       // the edge interpolation's inputs and outputs
-      {&o->ed.uclin, 2 * cz}, {&o->ed.vclin, 2 * cz}, {&o->ed.utrop, (size_t)nip * 3}, {&o->ed.vtrop, (size_t)nip * 3},
+      {&o->ed.uclin, 2 * cz}, {&o->ed.vclin, 2 * cz}, {&o->ed.uclin_alt, 2 * cz}, {&o->ed.vclin_alt, 2 * cz},
+      {&o->ed.utrop, (size_t)nip * 3}, {&o->ed.vtrop, (size_t)nip * 3},
       {&o->ed.geop, (size_t)nip * (kdm + 1)}, {&o->ed.montg, cz}, {&o->ed.spcifv, cz},
       {&o->ed.pr_edg, (size_t)nip * NPP * (kdm + 1)}, {&o->ed.geop_edg, ez}, {&o->ed.mont_edg, ez},
       {&o->ed.uvsq_edg, ez}, {&o->ed.spcv_edg, ez},
       // the momentum equation's forcing and work arrays
       {&o->mo.taux, (size_t)nip}, {&o->mo.tauy, (size_t)nip}, {&o->mo.ustarb, (size_t)nip},
-      {&o->mo.drag, (size_t)nip}, {&o->mo.dpbot, (size_t)nip}, {&o->mo.gradx, cz}, {&o->mo.grady, cz},
-      {&o->mo.d4u, cz}, {&o->mo.d4v, cz}, {&o->mo.du, cz}, {&o->mo.dv, cz},
+      {&o->mo.drag, (size_t)nip}, {&o->mo.dpbot, (size_t)nip}, {&o->mo.d4u, cz}, {&o->mo.d4v, cz},
+      {&o->mo.gradx, cz}, {&o->mo.grady, cz}, {&o->mo.relvor, cz}, {&o->mo.visc, cz},
       // the tracers and density the transport and the grid generator share
       {&o->tr.temp, cz}, {&o->tr.saln, cz}, {&o->hy.dens, cz}};
   for (auto &a : arrs)
@@ -688,24 +746,58 @@ extern "C" long long fimhip_ocn_field_size(const fimhip_ocn *o, int f) {
   return (long long)n;
 }
 
+// an edge array that fimhip_ocn_edgvar leaves to be formed
+static bool lazy_edge(int f) {
+  return f == FIMHIP_OCN_UM_EDG || f == FIMHIP_OCN_VM_EDG || f == FIMHIP_OCN_UN_EDG || f == FIMHIP_OCN_VN_EDG ||
+         f == FIMHIP_OCN_DPM_EDG || f == FIMHIP_OCN_PR_EDG || f == FIMHIP_OCN_MONT_EDG ||
+         f == FIMHIP_OCN_UVSQ_EDG || f == FIMHIP_OCN_SPCV_EDG;
+}
+
+int ocn_put(fimhip_ocn *o, int f, const double *h) {
+  size_t n = 0;
+  const double *d0 = ocn_field(o, f, &n);
+  if (!d0) return FIMHIP_EINVAL;
+  const bool uv = f == FIMHIP_OCN_UCLIN || f == FIMHIP_OCN_VCLIN;
+  // the values the due edge arrays are formed from: the velocities until
+  // momtum has moved them to the other pair, the thickness until cnuity has
+  // kept its copy
+  const bool source = f == FIMHIP_OCN_UTROP || f == FIMHIP_OCN_VTROP || f == FIMHIP_OCN_MONTG ||
+                      f == FIMHIP_OCN_SPCIFV || (uv && !o->e_uv_old) || (f == FIMHIP_OCN_DP && !o->e_dp_old);
+  if (lazy_edge(f) || source) {
+    const int r = ocn_form_edges(o);
+    if (r) return r;
+  }
+  HIPCHK(hipMemcpyAsync(ocn_field(o, f, &n), h, n * sizeof(double), hipMemcpyHostToDevice, o->stream));
+  if (uv) o->alt_stale = true;
+  return FIMHIP_OK;
+}
+
+int ocn_get(fimhip_ocn *o, int f, double *h) {
+  size_t n = 0;
+  const double *d = ocn_field(o, f, &n);
+  if (!d) return FIMHIP_EINVAL;
+  if (lazy_edge(f)) {
+    const int r = ocn_form_edges(o);
+    if (r) return r;
+  }
+  HIPCHK(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, o->stream));
+  return FIMHIP_OK;
+}
+
 extern "C" int fimhip_ocn_upload(fimhip_ocn *o, int f, const double *h) {
   if (!o || !h) return FIMHIP_EINVAL;
-  size_t n = 0;
-  double *d = ocn_field(o, f, &n);
-  if (!d) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
-  HIPCHK(hipMemcpyAsync(d, h, n * sizeof(double), hipMemcpyHostToDevice, o->stream));
+  const int r = ocn_put(o, f, h);
+  if (r) return r;
   HIPCHK(hipStreamSynchronize(o->stream));
   return FIMHIP_OK;
 }
 
 extern "C" int fimhip_ocn_download(fimhip_ocn *o, int f, double *h) {
   if (!o || !h) return FIMHIP_EINVAL;
-  size_t n = 0;
-  double *d = ocn_field(o, f, &n);
-  if (!d) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
-  HIPCHK(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, o->stream));
+  const int r = ocn_get(o, f, h);
+  if (r) return r;
   HIPCHK(hipStreamSynchronize(o->stream));
   return FIMHIP_OK;
 }
@@ -718,15 +810,17 @@ static void ocn_kernels(fimhip_ocn *o, int leapm, int leapn) {
   const dim3 grid(ocn_blocks(o, LPC)), blk(256);     // a multiple of 8 blocks: see hcol
   const double dt = o->dtleap;
   const int smooth = o->thkdff != 0.;
+  if (!o->edges_due) KT_LAUNCH("hyc_normal", st, hyc_normal<LPC><<<grid, blk, 0, st>>>(g, s));
   KT_LAUNCH("hyc_flux", st, hyc_flux<LPC><<<grid, blk, 0, st>>>(g, s, leapm, leapn, dt));
-  KT_LAUNCH("hyc_lowsum", st, hyc_lowsum<LPC><<<grid, blk, 0, st>>>(g, s, leapn, dt));
   KT_LAUNCH("hyc_limits", st, hyc_limits<LPC><<<grid, blk, 0, st>>>(g, s, leapn, dt));
   KT_LAUNCH("hyc_clip", st, hyc_clip<LPC><<<grid, blk, 0, st>>>(g, s, dt));
-  KT_LAUNCH("hyc_recover", st, hyc_recover<LPC><<<grid, blk, 0, st>>>(g, s, leapn, dt, smooth, o->biharm));
+  KT_LAUNCH("hyc_recover", st, hyc_recover<LPC><<<grid, blk, 0, st>>>(g, s, dt, smooth));
   if (smooth) {
-    if (o->biharm > 0.) KT_LAUNCH("hyc_del2p", st, hyc_del2p<LPC><<<grid, blk, 0, st>>>(g, s, o->biharm));
-    KT_LAUNCH("hyc_bolus", st, hyc_bolus<LPC><<<grid, blk, 0, st>>>(g, s, leapn, dt, o->thkdff, o->biharm));
-    KT_LAUNCH("hyc_bclip", st, hyc_bclip<LPC><<<grid, blk, 0, st>>>(g, s, leapn, o->biharm, o->masscor));
+    if (o->biharm > 0.) {
+      KT_LAUNCH("hyc_del2p", st, hyc_del2p<LPC><<<grid, blk, 0, st>>>(g, s, o->biharm));
+      KT_LAUNCH("hyc_bolus", st, hyc_bolus<LPC><<<grid, blk, 0, st>>>(g, s, dt, o->thkdff, o->biharm));
+    }
+    KT_LAUNCH("hyc_bclip", st, hyc_bclip<LPC><<<grid, blk, 0, st>>>(g, s, dt, o->thkdff, o->biharm, o->masscor));
   }
   KT_LAUNCH("hyc_final", st, hyc_final<LPC><<<grid, blk, 0, st>>>(g, s, leapm, leapn, dt, smooth, o->biharm));
   KT_LAUNCH("hyc_check", st, hyc_check<LPC><<<grid, blk, 0, st>>>(g, s));
@@ -736,10 +830,17 @@ static void ocn_kernels(fimhip_ocn *o, int leapm, int leapn) {
 static int ocn_launch(fimhip_ocn *o, int nstep, int leapm, int leapn) {
   if (nstep < 1 || leapm < 1 || leapm > 2 || leapn < 1 || leapn > 2 || leapm == leapn) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
+  // the step keeps the thickness at level leapm for the due edge arrays: a
+  // second step, or another level, is a step on the arrays themselves
+  if (o->e_dp_old || leapm != o->e_leapm) {
+    const int r = ocn_form_edges(o);
+    if (r) return r;
+  }
   HIPCHK(hipMemsetAsync(o->s.flag, 0, sizeof(int), o->stream));
   g_ktimer = o->kt;
   if (o->kdm <= 32) ocn_kernels<32>(o, leapm, leapn);
   else ocn_kernels<64>(o, leapm, leapn);
+  o->e_dp_old = true;
   g_ktimer = nullptr;
   HIPCHK(hipGetLastError());
   // the drift correction of the total mass, at the first step and every 10
@@ -780,19 +881,16 @@ extern "C" int fimhip_ocn_cnuity_r8(fimhip_ocn *o, int nstep, int leapm, int lea
   const double *in[] = {um_edg, vm_edg, un_edg, vn_edg, dpm_edg, dp, pres, massflx, mssfx_avg};
   const int fi[] = {FIMHIP_OCN_UM_EDG, FIMHIP_OCN_VM_EDG, FIMHIP_OCN_UN_EDG, FIMHIP_OCN_VN_EDG, FIMHIP_OCN_DPM_EDG,
                     FIMHIP_OCN_DP, FIMHIP_OCN_PRES, FIMHIP_OCN_MASSFLX, FIMHIP_OCN_MSSFX_AVG};
-  for (int j = 0; j < 9; j++) {
-    size_t n = 0;
-    double *d = ocn_field(o, fi[j], &n);
-    HIPCHK(hipMemcpyAsync(d, in[j], n * sizeof(double), hipMemcpyHostToDevice, o->stream));
-  }
-  const int r = ocn_launch(o, nstep, leapm, leapn);
+  int r = 0;
+  for (int j = 0; j < 9; j++)
+    if ((r = ocn_put(o, fi[j], in[j]))) return r;
+  r = ocn_launch(o, nstep, leapm, leapn);
   if (r && r != FIMHIP_EDUP) return r;
   double *outp[] = {dp, pres, massflx, mssfx_avg};
   const int fo[] = {FIMHIP_OCN_DP, FIMHIP_OCN_PRES, FIMHIP_OCN_MASSFLX, FIMHIP_OCN_MSSFX_AVG};
   for (int j = 0; j < 4; j++) {
-    size_t n = 0;
-    double *d = ocn_field(o, fo[j], &n);
-    HIPCHK(hipMemcpyAsync(outp[j], d, n * sizeof(double), hipMemcpyDeviceToHost, o->stream));
+    const int e = ocn_get(o, fo[j], outp[j]);
+    if (e) return e;
   }
   HIPCHK(hipStreamSynchronize(o->stream));
   return r;

@@ -533,6 +533,11 @@ static int hyb_launch(fimhip_ocn *o, int leap, int with_tracers) {
   if (leap < 1 || leap > 2 || !o->hy.cols || !(o->mo.batrop > 0.)) return FIMHIP_EINVAL;
   if (with_tracers && o->tr.numtr <= 0) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
+  // the thickness and the velocities are written in place
+  if (!o->e_dp_old || !o->e_uv_old) {
+    const int r = ocn_form_edges(o);
+    if (r) return r;
+  }
   const size_t cz = (size_t)o->nip * o->kdm;
   HycHyb h{};
   h.cols = o->hy.cols;
@@ -618,19 +623,12 @@ extern "C" int fimhip_ocn_hybgn1_r8(fimhip_ocn *o, int nstep, int leap, const do
   const int fi[] = {FIMHIP_OCN_DENS, FIMHIP_OCN_DP, FIMHIP_OCN_PRES, FIMHIP_OCN_TEMP, FIMHIP_OCN_SALN,
                     FIMHIP_OCN_UCLIN, FIMHIP_OCN_VCLIN, FIMHIP_OCN_PASSV};
   const int nio = passv_tr ? 8 : 7;
-  for (int j = 0; j < nio; j++) {
-    size_t n = 0;
-    double *d = ocn_field(o, fi[j], &n);
-    if (!d) return FIMHIP_EINVAL;
-    HIPCHK(hipMemcpyAsync(d, io[j], n * sizeof(double), hipMemcpyHostToDevice, o->stream));
-  }
-  const int r = hyb_launch(o, leap, passv_tr ? 1 : 0);
-  if (r) return r;
-  for (int j = 0; j < nio; j++) {
-    size_t n = 0;
-    double *d = ocn_field(o, fi[j], &n);
-    HIPCHK(hipMemcpyAsync(io[j], d, n * sizeof(double), hipMemcpyDeviceToHost, o->stream));
-  }
+  int r = 0;
+  for (int j = 0; j < nio; j++)
+    if ((r = ocn_put(o, fi[j], io[j]))) return r;
+  if ((r = hyb_launch(o, leap, passv_tr ? 1 : 0))) return r;
+  for (int j = 0; j < nio; j++)
+    if ((r = ocn_get(o, fi[j], io[j]))) return r;
   HIPCHK(hipStreamSynchronize(o->stream));
   return FIMHIP_OK;
 }

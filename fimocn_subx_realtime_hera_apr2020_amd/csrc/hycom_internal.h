@@ -33,9 +33,17 @@ struct HycGrid {
 struct HycState {
   double *um, *vm, *un, *vn, *dpm_edg;
   double *dp, *pres, *massflx, *mssfx_avg;
-  // work arrays
-  double *antiflx, *dp_lo, *dpold, *dpc, *flxplus, *flxmnus, *rplus, *rmnus, *del2p, *dptmp;
-  double *clippd, *rpbot, *aux;
+  // work arrays: the edges' normal velocities at both levels (6 per cell);
+  // the stages' thicknesses (dpc clipped, dpr recovered, dptmp after the bolus
+  // fluxes), the limiter ratios, the bolus ratio; the clipped column sums and
+  // reciprocal bottom pressures of the antidiffusive and the bolus fluxes
+  double *vnm, *vnn, *antiflx;
+  double *dp_lo, *dpc, *dpr, *flxplus, *flxmnus, *rplus, *rmnus, *del2p, *dptmp, *brat;
+  double *clippd, *clippb, *rpbot, *rpbotb, *aux;
+  // what the edge interpolation saw, kept for momtum and for a later reader of
+  // its arrays: the mid-time thickness (kdm,nip; copied when the leapfrog
+  // filter replaces it), its bottom and the top interface (nip)
+  double *dpe, *pbe, *p0e;
   int *flag;
 };
 
@@ -44,6 +52,9 @@ __device__ __forceinline__ double hmax(double a, double b) { return a > b ? a : 
 __device__ __forceinline__ int ci_np(int ci) { return ci & 7; }
 __device__ __forceinline__ bool ci_wet(int ci) { return (ci >> 3) & 1; }
 __device__ __forceinline__ bool ci_open(int ci, int e) { return (ci >> (4 + e)) & 1; }
+// a hexagon of the ocean with six ocean neighbours: most cells, and a constant
+// word, with which the edges' expressions lose their selections on the coast
+constexpr int CI_SEA = 6 | 8 | 0x3f0;
 
 // the column of the lane (i, its slot cc in the block) and the lane's layer k;
 // the host pads the grid to a multiple of 8 blocks, and block b, which the
@@ -73,29 +84,60 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// pres(k+1) = pres(k) + d(k), k = 0..kdm-1, from pres(0) = p0: every lane forms
-// the whole chain in layer order and keeps the interface below its layer
+// The column's sequential chains.  One lane of the column runs a chain in
+// layer order over a row the column's lanes put in LDS (every lane running it
+// and keeping its own layer's value takes three more instructions a layer);
+// the row is read eight layers ahead of the sums that replace them, so that
+// the chain waits for LDS once in eight additions.  Lanes from kdm on put
+// zeros.
+constexpr int CHK = 8;
+// row(k) = p0 + row(0) + ... + row(k), in place
+__device__ __forceinline__ void row_chain(double *row, double p0, int kdm) {
+  double prev = p0, b[CHK];
+#pragma unroll
+  for (int j = 0; j < CHK; j++) b[j] = row[j];
+  for (int j0 = 0; j0 < kdm; j0 += CHK) {
+    double o[CHK];
+#pragma unroll
+    for (int j = 0; j < CHK; j++) o[j] = prev = prev + b[j];
+    const int nx = j0 + CHK < kdm ? j0 + CHK : j0;
+#pragma unroll
+    for (int j = 0; j < CHK; j++) b[j] = row[nx + j];
+#pragma unroll
+    for (int j = 0; j < CHK; j++) row[j0 + j] = o[j];
+  }
+}
+// the sum of the row from 0 on
+__device__ __forceinline__ double row_sum(const double *row, int kdm) {
+  double acc = 0.;
+  for (int j0 = 0; j0 < kdm; j0 += CHK) {
+    double b[CHK];
+#pragma unroll
+    for (int j = 0; j < CHK; j++) b[j] = row[j0 + j];
+#pragma unroll
+    for (int j = 0; j < CHK; j++) acc = acc + b[j];
+  }
+  return acc;
+}
+// pres(k+1) = pres(k) + d(k), k = 0..kdm-1, from pres(0) = p0: each lane keeps
+// the interface below its layer
 __device__ __forceinline__ double col_pres(double *buf, double d, double p0, int k, int kdm) {
   buf[k] = d;
   wave_sync();
-  double prev = p0, mine = 0.;
-  for (int j = 0; j < kdm; j++) {
-    prev = prev + buf[j];
-    if (j == k) mine = prev;
-  }
+  if (k == 0) row_chain(buf, p0, kdm);
+  wave_sync();
+  const double mine = buf[k];
   wave_sync();
   return mine;
 }
-// the six sums over the column's layers, in layer order from 0, of part[e]:
-// lane e < NPP of the column returns edge e's
+// the six sums over the column's layers, in layer order from 0, of part[e]
+// (0 in the lanes from kdm on): lane e < NPP of the column returns edge e's
 template <int LPC>
 __device__ __forceinline__ double col_sums6(double (*buf)[LPC + 1], const double *part, int k, int kdm) {
 #pragma unroll
   for (int e = 0; e < NPP; e++) buf[e][k] = part[e];
   wave_sync();
-  double acc = 0.;
-  if (k < NPP)
-    for (int j = 0; j < kdm; j++) acc = acc + buf[k][j];
+  const double acc = k < NPP ? row_sum(buf[k], kdm) : 0.;
   wave_sync();
   return acc;
 }
@@ -103,6 +145,7 @@ __device__ __forceinline__ double col_sums6(double (*buf)[LPC + 1], const double
 // the arrays of the edge interpolation (hycom_edgvar.F90 bclin_edgvar)
 struct HycEdg {
   double *uclin, *vclin, *utrop, *vtrop, *geop, *montg, *spcifv;
+  double *uclin_alt, *vclin_alt;   // momtum writes the new velocities here and the pairs are swapped
   double *pr_edg, *geop_edg, *mont_edg, *uvsq_edg, *spcv_edg;
 };
 
@@ -113,7 +156,9 @@ struct HycMom {
   const double *corio, *meshsz;   // omegx2*sin(lat) (dyn_init.F90:753), sqrt(area) (hycom_init.F90:327)
   double *taux, *tauy, *ustarb;   // (nip)
   double *drag, *dpbot;           // (nip): bottom drag; bottom of dissip's pressure column
-  double *gradx, *grady, *d4u, *d4v, *du, *dv;   // (kdm,nip)
+  // (kdm,nip): del4prep's velocities, the pressure force, the vorticity, the
+  // eddy viscosity
+  double *d4u, *d4v, *gradx, *grady, *relvor, *visc;
   double batrop, veldff, smagcf;
 };
 
@@ -160,13 +205,30 @@ struct fimhip_ocn {
   fimhip::hyc::HycTr tr{};
   fimhip::hyc::HycHybState hy{};
   bool janjic = false;               // janjic_ocn (fimnamelist.F90:246)
+  // fimhip_ocn_edgvar forms only what cnuity and momtum read (the edges'
+  // normal velocities and thickness); the public edge arrays follow when one
+  // of them is asked for, from the values of that call:
+  bool edges_due = false;            // the public edge arrays are older than the last edgvar
+  int e_leapm = 0, e_leapn = 0;      // its levels
+  bool e_dp_old = false;             // cnuity has run since: its mid-time thickness is in s.dpe
+  bool e_uv_old = false;             // momtum has run since: its velocities are in the alt pair
+  bool alt_stale = false;            // the alt pair's land values miss an upload
+  double *pres_f = nullptr;          // (kdm+1,nip) interfaces of the forming
   std::vector<int> wet;
   std::vector<double> area;
   fimhip::KTimer *kt = nullptr;              // non-null while profiling
 };
 
-// the device array of a FIMHIP_OCN_* field and its element count
+// the device array of a FIMHIP_OCN_* field and its element count; nullptr for
+// a field the instance does not have
 double *ocn_field(fimhip_ocn *o, int f, size_t *n);
+// the public edge arrays, if they are due (hycom_edgvar.hip)
+int ocn_form_edges(fimhip_ocn *o);
+// a whole field to or from the host on the instance's stream, with the edge
+// arrays formed first where the transfer would read them or replace what they
+// are formed from
+int ocn_put(fimhip_ocn *o, int f, const double *h);
+int ocn_get(fimhip_ocn *o, int f, double *h);
 // blocks of a launch over all cells with LPC lanes per column (a multiple of 8)
 inline unsigned ocn_blocks(const fimhip_ocn *o, int lpc) {
   const int cpb = 256 / lpc;

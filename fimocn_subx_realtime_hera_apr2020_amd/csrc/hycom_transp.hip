@@ -597,21 +597,6 @@ extern "C" int fimhip_ocn_transp2(fimhip_ocn *o, int leapn) {
   return tr2_launch(o, o->s.dp + (size_t)(leapn - 1) * o->nip * o->kdm);
 }
 
-static int ocn_put(fimhip_ocn *o, int f, const double *h) {
-  size_t n = 0;
-  double *d = ocn_field(o, f, &n);
-  if (!d) return FIMHIP_EINVAL;
-  HIPCHK(hipMemcpyAsync(d, h, n * sizeof(double), hipMemcpyHostToDevice, o->stream));
-  return FIMHIP_OK;
-}
-static int ocn_get(fimhip_ocn *o, int f, double *h) {
-  size_t n = 0;
-  double *d = ocn_field(o, f, &n);
-  if (!d) return FIMHIP_EINVAL;
-  HIPCHK(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, o->stream));
-  return FIMHIP_OK;
-}
-
 extern "C" int fimhip_ocn_transp0_r8(fimhip_ocn *o, int nstep, int leapn, double *cumuflx, const double *dp,
                                     double *dpinit) {
   (void)nstep;

@@ -433,7 +433,9 @@ int fimhip_ocn_edgvar_r8(fimhip_ocn *ocn, int nstep, int leapm, int leapn, const
                          double *pr_edg, double *geop_edg, double *mont_edg, double *uvsq_edg, double *spcv_edg);
 /* the same on the device-resident arrays, asynchronous (fimhip_ocn_cnuity
  * and the downloads wait for it); its edge values are those
- * fimhip_ocn_cnuity reads (dp_edg is FIMHIP_OCN_DPM_EDG) */
+ * fimhip_ocn_cnuity and fimhip_ocn_momtum use (dp_edg is
+ * FIMHIP_OCN_DPM_EDG); the arrays themselves are formed when one is
+ * downloaded */
 int fimhip_ocn_edgvar(fimhip_ocn *ocn, int leapm, int leapn);
 /* hycom_momtum.F90:16 momtum(nstep, leapm, leapn, utrop, vtrop, uclin, vclin,
  * um_edg, vm_edg, geop_edg, mont_edg, uvsq_edg, spcv_edg, taux, tauy, ubforc,

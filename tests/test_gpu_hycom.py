@@ -616,3 +616,65 @@ def test_ocean_interval_resident_matches_checker(oracle_lib, level, kdm):
         assert o.mass == h.mass
     finally:
         o.close()
+
+
+@pytest.mark.parametrize("kdm", [16, 48])
+@pytest.mark.parametrize("janjic", [False, True])
+@pytest.mark.parametrize("then", ["edgvar", "cnuity", "momtum", "momtum first", "hybgn1", "upload", "upload early",
+                                  "momtum twice", "cnuity twice", "other levels"])
+def test_edge_arrays_formed_when_asked_for(oracle_lib, then, janjic, kdm):
+    """fimhip_ocn_edgvar leaves the public edge arrays to be formed when one is
+    asked for: they are those of its own call whatever ran or was uploaded
+    since, and what runs next uses them."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, ocean
+    print("case: G3 x %d, edge arrays after %s, janjic %s" % (kdm, then, janjic), flush=True)
+    g = _grid(3)
+    case = ocean.hycom_ocean_case(g, kdm=kdm, seed=97, numtr=1)
+    h = oracle_lib.HycomCnuity(g, case)
+    o = fimhip.Ocean(g, kdm, case["wet"], case["dtleap"])
+    try:
+        o.set_janjic(janjic)
+        o.set_momtum(case["batrop"], case["veldff"], case["smagcf"])
+        o.set_transport(1, case["temdff"])
+        o.set_hybgen(case["targt"], case["salmin"], case["dpmin"], case["latij"])
+        for n in fimhip.OCN_MOMTUM_FIELDS + ["temp", "saln", "dens", "passv", "cumuflx", "dpinit"]:
+            o.upload(n, case[n])
+
+        def both(*ops):
+            for op, st, m, n in ops:
+                if op == "edgvar":
+                    h.edgvar(g, m, n, janjic)
+                    o.step_edgvar(m, n)
+                elif op == "cnuity":
+                    assert h.step(st, m, n) == 0
+                    o.step(st, m, n)
+                else:
+                    h.momtum(g, m, n, janjic)
+                    o.step_momtum(m, n)
+
+        e, c, mo = ("edgvar", 1, 2, 1), ("cnuity", 1, 2, 1), ("momtum", 1, 2, 1)
+        both(*{"edgvar": [e], "cnuity": [e, c], "momtum": [e, c, mo], "momtum first": [e, mo], "hybgn1": [e, c, mo],
+               "upload": [e, c, mo], "upload early": [e, c], "momtum twice": [e, c, mo, ("momtum", 1, 1, 2)],
+               "cnuity twice": [e, c, ("cnuity", 2, 1, 2)],
+               "other levels": [e, ("cnuity", 1, 1, 2), ("momtum", 1, 1, 2)]}[then])
+        if then == "hybgn1":
+            oracle_lib.hycom_interval_op(h, "hybgn1", 1)
+            o.step_hybgn1(1)
+        elif then.startswith("upload"):
+            for n in ("uclin", "vclin", "utrop", "montg", "spcifv"):
+                h.e[n][...] = .5 * np.asarray(case[n]).reshape(h.e[n].shape)
+                o.upload(n, h.e[n])
+            for n in ("dp", "pres"):
+                h.a[n][...] = np.asarray(case[n]).reshape(h.a[n].shape)
+                o.upload(n, h.a[n])
+        got = {n: o.download(n) for n in EDG_CHECK[:5] + tuple(h.EDG_OUT)}
+        got["pres"] = o.download("pres")
+        _edg_same(h, got, then)
+        both(c, mo)                 # on the arrays themselves
+        both(("edgvar", 2, 1, 2), ("cnuity", 2, 1, 2), ("momtum", 2, 1, 2))
+        for n in ARRAYS:
+            assert _same(o.download(n), h.a[n]), n
+        for n in ("uclin", "vclin", "ustarb"):
+            assert _same(o.download(n), h.e[n]), n
+    finally:
+        o.close()
