@@ -108,8 +108,8 @@ def ens_kernel_bytes(T):
         "e_cnuity45": 164,                   # antifx r+- massfx dp_tdcy dp pr pressure gradient u v -> massfx dp_tdcy dp pr ex omega
         "e_massadv1": 104,                   # normal wind and dp edges, dp, dp_tdcy(of,vof) -> q_star edges, q_min/max_out
         "e_massadv2": 156,                   # normal wind, q_star, bounds, dp_tdcy, dp, pressure gradient, u v -> massfx dp_tdcy dp pr ex omega
-        "e_trcadv12": 32 + 68 * T,           # massfx dp; per tracer tr trdp trl trc(of,vof) -> antiflx trl bounds r+ r-
-        "e_trcadv3": 8 + 68 * T,
+        "e_trcadv12": 32 + 56 * T,           # massfx dp; per tracer tr trdp trl trc(of,vof) -> antiflx trl bounds r+ r-
+        "e_trcadv3": 8 + 52 * T,             # (and 4 T of tracer mass out on transport-only steps)
         "e_trc_fct": 32 + 40 * T,            # massfx dp; per tracer tr trdp trl(of,vof) trc(of,vof) -> tr trdp trl trc
         "e_momtum": 80,                      # u v dp ex mp, step-start theta, tendencies -> relvor tendency u2 v2
         "k_regrid": 20,

@@ -289,6 +289,7 @@ extern "C" int fimhip_ens_init_state(fimhip_ens *e, int init_hybgen) {
 static void enqueue_step(fimhip_ens *e, int mode, bool side, bool move_b) {
   const EnsGrid &g = e->g;
   EnsState s = e->s;
+  s.keep_trdp = mode == 1;
   hipStream_t st = e->stream, sd = e->side;
   ens_launch_abstart(s, e->dt, st);
   if (side) {

@@ -60,6 +60,7 @@ struct EnsGrid {
 struct EnsState {
   int members, ncol;
   float *us, *vs, *u2, *v2;
+  int keep_trdp;                     // the tracer mass trcadv3 forms is read again (transport-only steps; otherwise hystat writes it)
   float *tr_alt, *trdp_alt;          // the other buffer of tr / trdp (the fused FCT writes it)
   double *dp, *pr, *ex, *ph, *mp, *sdot, *exsmo, *psrf, *ptdcy, *thbuf;
   float *tr, *trdp;

@@ -589,17 +589,18 @@ void ens_launch_trc_fct(int tile, const EnsGrid &g, const EnsState &s, hipStream
 // one member for one tracer, lane = level.  It stages the tracer of rings 0-2
 // in LDS, forms the bounded low-order tracer of rings 0-1 (kept in LDS; the
 // core's tendency is stored), then, after a barrier, the core's two-sided
-// edge values, antidiffusive fluxes (stored for trcadv3) and their sums, the
+// edge values, antidiffusive fluxes (stored for trcadv3 by the edge's cell of
+// lower index) and their sums, the
 // local bounds and the limiter ratios.  Each cell's operations are those of
 // the fused kernel above, in the same order, so the two forms of the
 // transport have the same bits.
 //
-// What bounds it: HBM traffic, 304 B per cell-level for 4 tracers plus the
-// halo, nearly half of it writes, at 4.6 TB/s (a large copy reaches 4.75).  As
+// What bounds it: HBM traffic, 256 B per cell-level for 4 tracers plus the
+// halo, half of it writes, at 4.4 TB/s (a large copy reaches 4.75).  As
 // three kernels (edgvar3's reconstructions stored and read back, the
 // low-order tracer stored, the mass flux read twice) it moved 620 B.  8
-// members x G7 x 64 x 4 tracers: 9.75 -> 7.20 ms; 16 x G5: 1.20 -> 0.94 ms; G6
-// with 20 tracers: 1.65 -> 1.18 ms; 3 x G4 x 38 x 3 tracers: 42 -> 40 us.
+// members x G7 x 64 x 4 tracers: 9.75 -> 6.7 ms; 16 x G5: 1.20 -> 0.87 ms; G6
+// with 20 tracers: 1.65 -> 1.07 ms; 3 x G4 x 38 x 3 tracers: 42 -> 40 us.
 // What got it there:
 //  * the cells' coefficients and stencil offsets come one row per cell by a
 //    vector load, a cell ahead, and are handed out by v_readlane: as scalar
@@ -693,7 +694,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   const float dp = (float)in.dp;
   const float ti = Str[i * 64 + k], lo = Slo[i * 64 + k];
 #pragma unroll
-  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, 102 + e), k);
+  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, 102 + e) & ~1, k);
   if (t == 0) {
 #pragma unroll
     for (int e = 0; e < NP; e++) {
@@ -725,7 +726,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   for (int e = 0; e < NP; e++) {
     const float m = in.m[e];
     const float a = m * (te[e] - fct_upwind(m, ti, v[e]));
-    __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
+    if (row_i(row, 102 + e) & 1) __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
     sp = sp - fminf(0.f, a);
     sm = sm + fmaxf(0.f, a);
     mx = fmaxf(mx, v[e]);
@@ -735,7 +736,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   mn = fminf(fmaxf(0.f, mn), lo);
 #pragma unroll
   for (int e = 0; e < NP; e++) {
-    const float x = lds_at(Slo, row_i(row, 102 + e), k);
+    const float x = lds_at(Slo, row_i(row, 102 + e) & ~1, k);
     mx = fmaxf(mx, x);
     mn = fminf(mn, x);
   }
@@ -856,7 +857,8 @@ void ens_launch_trcadv12(int tile, const EnsGrid &g, const EnsState &s, hipStrea
 // stencil cell), 36-71 the neighbours' of the shared edges, each sum starting
 // at the shared edge's slot, 72-101 the LDS byte offsets (256 per tile cell)
 // of the neighbours' stencil cells after the first (which is the cell itself),
-// 102-107 those of the neighbours.  A pentagon's missing stencil cell is the
+// 102-107 those of the neighbours, with bit 0 set where the cell stores the
+// edge's antidiffusive flux (it has the lower index).  A pentagon's missing stencil cell is the
 // neighbour itself with coefficient 0, before the last.  Clears *cyclic unless
 // the slots of all cells run around them in one sense: then the second and
 // last cells of a neighbour's stencil are the cell's own neighbours of slots
@@ -871,7 +873,7 @@ __global__ void __launch_bounds__(256) k_core_rows(EnsGrid g, EnsTiles ts, int *
     const int4 ex = ent[l];
     const int x = ex.x, nx = enp(ex), xs = eslot(en, e);
     int *row = rows + (size_t)c * CORE_ROW;
-    row[102 + e] = 256 * l;
+    row[102 + e] = 256 * l | (c < x);
     for (int r = 0; r < NPP; r++) {
       row[e * NPP + r] = __float_as_int(g.hfcoef[((size_t)c * NPP + e) * NPP + r]);
       const bool in = nx == NPP || r != NPP - 2;

@@ -538,7 +538,12 @@ __global__ void __launch_bounds__(64 * COLS) k_e_massadv2(EnsGrid g, EnsState s)
 // thread, on the antidiffusive fluxes, limiter ratios, bounds and low-order
 // tendency that trcadv12 (fct_tiles.hip) leaves.  The final mass flux is
 // antisymmetric and tracer edge values are the same bits on both sides of an
-// edge, so the tracer fluxes cancel exactly across it.
+// edge, so the tracer fluxes cancel exactly across it, and one of the two
+// sides' fluxes, which are each other's negative, is all that is stored: the
+// cell of lower index's.  Bound by memory: half the fluxes written there and
+// read here took trcadv12 from 7.2 to 6.7 ms and this kernel from 4.6 to 3.7 ms
+// at 8 members x G7 x 64 layers x 4 tracers (0.3 of it by leaving out the
+// tracer mass where hystat writes it again).
 //
 // The limiter's neighbour value is gathered through a per-lane
 // address (R+ or R- of the neighbour by the sign of the flux) and every load
@@ -550,9 +555,17 @@ __device__ __forceinline__ void e_trcadv3_col(const EnsGrid &g, const EnsState &
   const int nf = c.nf - 1, of = c.of - 1, vof = c.vof - 1;
   const int col = base + ipn;
   const float thshld = 1.e-11f;
-  int xs[NP];
+  // the row of each edge's flux, at the edge's cell of lower index, and the
+  // sign it has seen from here
+  int xs[NP], row[NP];
+  float sg[NP];
 #pragma unroll
-  for (int e = 0; e < NP; e++) xs[e] = base + GPROX(ipn, e);
+  for (int e = 0; e < NP; e++) {
+    const int x = GPROX(ipn, e);
+    xs[e] = base + x;
+    row[e] = ipn < x ? col * NPP + e : xs[e] * NPP + GPROXS(ipn, e);
+    sg[e] = ipn < x ? 1.f : -1.f;
+  }
   const float rdp = frcp(fmaxf(thshld, (float)EC(s.dp, col, k))), rar = GF(rarea, ipn);
   const float a1 = (float)c.ab1, a2 = (float)c.ab2, a3 = (float)c.ab3;
   for (int t = 0; t < ntra; t++) {
@@ -563,7 +576,7 @@ __device__ __forceinline__ void e_trcadv3_col(const EnsGrid &g, const EnsState &
     const float tmn = ETR(s.trmin, t, col, k), tmx = ETR(s.trmax, t, col, k);
     float a[NP], r[NP];
 #pragma unroll
-    for (int e = 0; e < NP; e++) a[e] = ETE(s.antiflx, t, col, e, k);
+    for (int e = 0; e < NP; e++) a[e] = sg[e] * s.antiflx[(tb * NPP + row[e]) * nvl + k];
 #pragma unroll
     for (int e = 0; e < NP; e++) {
       const float *src = a[e] >= 0.f ? s.tr_rp : s.tr_rm;
@@ -576,7 +589,7 @@ __device__ __forceinline__ void e_trcadv3_col(const EnsGrid &g, const EnsState &
     const float tt = trl + at;
     const float tdp = tdp0 + a1 * tt + a2 * tco + a3 * tcv;
     __builtin_nontemporal_store(tt, &ETAB(s.trc_tdcy, t, nf, col, k));
-    __builtin_nontemporal_store(tdp, &ETR(s.trdp, t, col, k));
+    if (s.keep_trdp) __builtin_nontemporal_store(tdp, &ETR(s.trdp, t, col, k));
     if (col_wet(s.wet, col)) __builtin_nontemporal_store(fmaxf(tmn, fminf(tmx, tdp * rdp)), &ETR(s.tr, t, col, k));   // land keeps its tracers
   }
 }
