@@ -880,51 +880,83 @@ __device__ __forceinline__ KPair kp_merge(KPair a, KPair b) {  // a + b, compens
   return r;
 }
 
+// One wavefront per column, lane = level, four tracers (and with the first
+// four the mass) per pass over the thickness, each lane its own partial sums
+// over the columns of its wavefront.  Bound by memory: one read of the
+// thickness and the tracers.  (A thread per column, one sum a pass, read 256
+// bytes apart and the thickness once per tracer: 8 members x G7 x 64 layers x
+// 4 tracers took 10.7 ms, this takes 0.43.)
+template <int NT>
+__device__ __forceinline__ void e_globsum_pass(const EnsGrid &g, const EnsState &s, int t0, bool mass, double (&a)[NT + 1],
+                                               KPair (&kp)[NT + 1]) {
+  const int nip = g.d.nip, nvl = g.d.nvl, ntra = g.d.ntra, ncol = s.ncol;
+  const int k = threadIdx.x & 63, m = blockIdx.y;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (k >= nvl) return;
+  constexpr int UN = 2;      // columns in flight
+  const int stride = gridDim.x * 4;
+  for (int i0 = blockIdx.x * 4 + w; i0 < nip; i0 += UN * stride) {
+    double dp[UN];
+    float tr[UN][NT];
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      const int col = m * nip + min(i0 + u * stride, nip - 1);
+      dp[u] = EC(s.dp, col, k);
+#pragma unroll
+      for (int j = 0; j < NT; j++) tr[u][j] = ETR(s.tr, min(t0 + j, ntra - 1), col, k);
+    }
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      const int ipn = i0 + u * stride;
+      if (ipn >= nip) break;
+      const double v = ldc(g.d.area, ipn) * dp[u];
+      const float vf = GF(area, ipn) * (float)dp[u];
+      if (mass) {
+        a[NT] = a[NT] + v;
+        kp[NT] = kp_add(kp[NT], vf);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        a[j] = a[j] + v * (double)tr[u][j];
+        kp[j] = kp_add(kp[j], vf * tr[u][j]);
+      }
+    }
+  }
+}
 __global__ void __launch_bounds__(256) k_e_globsum(EnsGrid g, EnsState s, double *p64, float *p32) {
   __shared__ double sh[256];
   __shared__ float shs[256], shc[256];
-  const int nip = g.d.nip, nvl = g.d.nvl, ntra = g.d.ntra, ncol = s.ncol;
-  const int m = blockIdx.y, nb = gridDim.x;
-  for (int q = 0; q <= ntra; q++) {
-    double acc = 0.;
-    KPair kp{0.f, 0.f};
-    for (int ipn = blockIdx.x * 256 + threadIdx.x; ipn < nip; ipn += nb * 256) {
-      const int col = m * nip + ipn;
-      double colsum = 0.;
-      for (int k = 0; k < nvl; k++) {
-        const double dp = EC(s.dp, col, k);
-        double v = g.d.area[ipn] * dp;
-        float vf = GF(area, ipn) * (float)dp;
-        if (q > 0) {
-          const float tr = ETR(s.tr, q - 1, col, k);
-          v = v * (double)tr;
-          vf = vf * tr;
+  const int ntra = g.d.ntra, m = blockIdx.y, nb = gridDim.x;
+  constexpr int NT = 4;
+  for (int t0 = 0; t0 < ntra; t0 += NT) {
+    double a[NT + 1] = {};
+    KPair kp[NT + 1] = {};
+    e_globsum_pass<NT>(g, s, t0, t0 == 0, a, kp);
+#pragma unroll
+    for (int j = 0; j <= NT; j++) {
+      const int q = j == NT ? 0 : t0 + j + 1;      // 0: the mass
+      if (q > ntra || (j == NT && t0 > 0)) continue;
+      sh[threadIdx.x] = a[j];
+      shs[threadIdx.x] = kp[j].s;
+      shc[threadIdx.x] = kp[j].c;
+      __syncthreads();
+      for (int w = 128; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+          sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + w];
+          KPair r = kp_merge(KPair{shs[threadIdx.x], shc[threadIdx.x]}, KPair{shs[threadIdx.x + w], shc[threadIdx.x + w]});
+          shs[threadIdx.x] = r.s;
+          shc[threadIdx.x] = r.c;
         }
-        colsum = colsum + v;
-        kp = kp_add(kp, vf);
+        __syncthreads();
       }
-      acc = acc + colsum;
-    }
-    sh[threadIdx.x] = acc;
-    shs[threadIdx.x] = kp.s;
-    shc[threadIdx.x] = kp.c;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if (threadIdx.x < w) {
-        sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + w];
-        KPair r = kp_merge(KPair{shs[threadIdx.x], shc[threadIdx.x]}, KPair{shs[threadIdx.x + w], shc[threadIdx.x + w]});
-        shs[threadIdx.x] = r.s;
-        shc[threadIdx.x] = r.c;
+      if (threadIdx.x == 0) {
+        const size_t o = ((size_t)m * (ntra + 1) + q) * nb + blockIdx.x;
+        p64[o] = sh[0];
+        p32[2 * o] = shs[0];
+        p32[2 * o + 1] = shc[0];
       }
       __syncthreads();
     }
-    if (threadIdx.x == 0) {
-      const size_t o = ((size_t)m * (ntra + 1) + q) * nb + blockIdx.x;
-      p64[o] = sh[0];
-      p32[2 * o] = shs[0];
-      p32[2 * o + 1] = shc[0];
-    }
-    __syncthreads();
   }
 }
 
