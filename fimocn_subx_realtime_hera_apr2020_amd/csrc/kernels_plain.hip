@@ -599,15 +599,19 @@ __global__ void __launch_bounds__(256) k_momtum(DevGrid g, DevState s, AB ab) {
 
 // ---------------------------------------------------------------------------
 // hystat.F90:23-115 (column part), one wavefront per column: the column is
-// staged in LDS with coalesced loads, lane 0 runs the serial surface-pressure
+// staged in LDS with coalesced loads, one lane runs the serial surface-pressure
 // and Montgomery-potential sums in the reference order (in batches of CHN
 // levels, as update_pres_col), and every lane then forms its level's
-// geopotential.  mp_out may be another array than s.mp.
+// geopotential.  The block's COLS sums run side by side in one wavefront: LDS
+// instructions bound the kernel, and a wavefront's instruction serves COLS
+// columns for the price of one (a lane in each wavefront: 284 us at G7 x 64
+// layers; this 162).  mp_out may be another array than s.mp.
 __global__ void __launch_bounds__(256) k_hystat(DevGrid g, DevState s, double *mp_out, int its) {
+  // an odd row length: the columns of a sum's lanes lie in different banks
   __shared__ double sh_ex[COLS][NVL_MAX + 1];
-  __shared__ double sh_th[COLS][NVL_MAX];
-  __shared__ double sh_dp[COLS][NVL_MAX];
-  __shared__ double sh_mp[COLS][NVL_MAX];
+  __shared__ double sh_th[COLS][NVL_MAX + 1];
+  __shared__ double sh_dp[COLS][NVL_MAX + 1];
+  __shared__ double sh_mp[COLS][NVL_MAX + 1];
   const int nip = g.nip, nvl = g.nvl, nvlp1 = nvl + 1;
   const int k = threadIdx.x, c = threadIdx.y;
   const int ipn = wave_col();
@@ -620,28 +624,29 @@ __global__ void __launch_bounds__(256) k_hystat(DevGrid g, DevState s, double *m
     }
   }
   __syncthreads();
-  if (live && k == 0) {
-    const double work = s.psrf[ipn], ph0 = L2(s.ph, ipn, 0);
+  const int is = blockIdx.x * COLS + k;      // lane k of the first wavefront: column k's sums
+  if (c == 0 && k < COLS && is < nip) {
+    const double work = s.psrf[is], ph0 = L2(s.ph, is, 0);
     double ps = 0.;
     for (int k0 = (nvl - 1) / CHN * CHN; k0 >= 0; k0 -= CHN) {
       double d[CHN];
 #pragma unroll
-      for (int j = 0; j < CHN; j++) d[j] = sh_dp[c][k0 + j];
+      for (int j = 0; j < CHN; j++) d[j] = sh_dp[k][k0 + j];
 #pragma unroll
       for (int j = CHN - 1; j >= 0; j--) {
         if (k0 + j >= nvl) continue;
         ps = k0 + j == nvl - 1 ? d[j] : ps + d[j];
       }
     }
-    s.psrf[ipn] = ps;
-    if (its > 0) s.ptdcy[(size_t)(its % 2) * nip + ipn] = ps - work;
+    s.psrf[is] = ps;
+    if (its > 0) s.ptdcy[(size_t)(its % 2) * nip + is] = ps - work;
     double mp = 0., thm = 0.;
     for (int k0 = 0; k0 < nvl; k0 += CHN) {
       double e[CHN], t[CHN];
 #pragma unroll
       for (int j = 0; j < CHN; j++) {
-        e[j] = sh_ex[c][k0 + j];
-        t[j] = sh_th[c][k0 + j];
+        e[j] = sh_ex[k][k0 + j];
+        t[j] = sh_th[k][k0 + j];
       }
 #pragma unroll
       for (int j = 0; j < CHN; j++) {
@@ -650,7 +655,7 @@ __global__ void __launch_bounds__(256) k_hystat(DevGrid g, DevState s, double *m
         t[j] = mp;
       }
 #pragma unroll
-      for (int j = 0; j < CHN; j++) sh_mp[c][k0 + j] = t[j];
+      for (int j = 0; j < CHN; j++) sh_mp[k][k0 + j] = t[j];
     }
   }
   __syncthreads();
