@@ -8,6 +8,7 @@
 // is a cell-level kernel.  Loop orders and operation orders are those of the
 // reference.  Columns a land/sea mask marks as land are left as they are.
 #include "fimhip_internal.h"
+#include "div_by.h"
 #include "fim_pow.h"
 
 #include <stdlib.h>
@@ -235,14 +236,15 @@ __device__ __forceinline__ bool absorbs(double t, double bound) {
 // increase (zold/znew = +-x).
 struct PcwGeom {
   double f, fl, fn, dz;
-  double rf, rfn, dx;   // FAST only: 1/(f+1e-22), 1/(fn+1e-22), the flux slab fraction
+  double rf, rfn, dx;   // 1/(f+1e-22), 1/(fn+1e-22), the flux slab fraction (the slab's part of its layer)
+  double ds, rds;       // not FAST: the slab and its reciprocal
 };
 template <bool FAST>
 __device__ __forceinline__ PcwGeom pcwise_geom(int kk, const double *xold, const double *xnew, int lane) {
   const bool up = xold[0] < xold[kk];
   auto zo = [&](int k) { return up ? xold[k] : -xold[k]; };
   auto zn = [&](int k) { return up ? xnew[k] : -xnew[k]; };
-  PcwGeom g{0., 0., 0., 0., 0., 0., 0.};
+  PcwGeom g{};
   if (lane < kk) {
     g.f = dmax(0., zo(lane + 1) - zo(lane));
     g.fn = dmax(0., zn(lane + 1) - zn(lane));
@@ -255,6 +257,15 @@ __device__ __forceinline__ PcwGeom pcwise_geom(int kk, const double *xold, const
     const double fc = g.dz > 0. ? g.f : g.fl;
     const double adz = fabs(g.dz);
     g.dx = fc > 0. ? dmin(fc, adz) / fc : 0.;
+  } else {
+    // what the fields of a column share of their divisions (the fields'
+    // quotients from these have a division's own rounding: div_by)
+    g.rf = div_rcp(g.f + 1.e-22);
+    g.rfn = div_rcp(g.fn + 1.e-22);
+    const double fc = g.dz > 0. ? g.f : g.fl, adz = fabs(g.dz);
+    g.ds = dmin(0. + fc, adz) - dmin(0., adz);
+    g.dx = g.ds / fc;
+    g.rds = div_rcp(g.ds);
   }
   return g;
 }
@@ -282,7 +293,7 @@ __device__ double pcwise_w(int kk, const PcwGeom &gm, double a, int lane) {
     } else {
       const double t = a * f;
       fin = absorbs(t, bnd);
-      v = fin ? (FAST ? t * gm.rf : t / (f + small)) : a;
+      v = fin ? (FAST ? t * gm.rf : div_by(t, f + small, gm.rf)) : a;
     }
     while (wany(!fin)) {
       const double vu = w_dn1(v);
@@ -304,7 +315,7 @@ __device__ double pcwise_w(int kk, const PcwGeom &gm, double a, int lane) {
     } else {
       const double t = a2 * f;
       fin = absorbs(t, bnd);
-      w = fin ? (FAST ? t * gm.rf : t / (f + small)) : a2;
+      w = fin ? (FAST ? t * gm.rf : div_by(t, f + small, gm.rf)) : a2;
     }
     while (wany(!fin)) {
       const double wd = w_up1(w);
@@ -336,28 +347,18 @@ __device__ double pcwise_w(int kk, const PcwGeom &gm, double a, int lane) {
         else if (dz < 0. && gm.fl > 0.) vf = -dz * (wl + bl * .5 * (1. - dx));
       }
     } else if (live && lane >= 1) {
-      double slab = 0., amount = 0.;
-      const double dz = gm.dz;
+      const double dz = gm.dz, dx = gm.dx;
+      double amount = 0., fc = 0.;
       if (dz > 0.) {
-        const double fc = f;                       // fco(layer lane)
-        if (fc > 0.) {
-          double dslab = dmin(slab + fc, dz) - dmin(slab, dz);
-          double dx = dslab / fc;
-          double fcdx = w + b * .5 * (dx - 1.) + 0. * (.25 - dx * (.5 - dx * (1. / 3.)));
-          amount = amount + fcdx * dslab;
-          slab = slab + dslab;
-        }
+        fc = f;                                    // fco(layer lane)
+        const double fcdx = w + b * .5 * (dx - 1.) + 0. * (.25 - dx * (.5 - dx * (1. / 3.)));
+        amount = amount + fcdx * gm.ds;
       } else if (dz < 0.) {
-        const double fc = gm.fl;                   // fco(layer lane - 1)
-        if (fc > 0.) {
-          double dslab = dmin(slab + fc, -dz) - dmin(slab, -dz);
-          double dx = dslab / fc;
-          double fcdx = wl + bl * .5 * (1. - dx) + 0. * (.25 - dx * (.5 - dx * (1. / 3.)));
-          amount = amount + fcdx * dslab;
-          slab = slab + dslab;
-        }
+        fc = gm.fl;                                // fco(layer lane - 1)
+        const double fcdx = wl + bl * .5 * (1. - dx) + 0. * (.25 - dx * (.5 - dx * (1. / 3.)));
+        amount = amount + fcdx * gm.ds;
       }
-      if (slab != 0.) vf = -dz * amount / slab;
+      if (fc > 0. && gm.ds != 0.) vf = div_by(-dz * amount, gm.ds, gm.rds);
     }
   }
   double vhi = w_dn1(vf);
@@ -366,7 +367,7 @@ __device__ double pcwise_w(int kk, const PcwGeom &gm, double a, int lane) {
   double y = 0.;
   if (live) {
     const double amount = w * f - (vhi - vlo);
-    y = FAST ? (amount + w * small) * gm.rfn : (amount + w * small) / (gm.fn + small);
+    y = FAST ? (amount + w * small) * gm.rfn : div_by(amount + w * small, gm.fn + small, gm.rfn);
   }
   return y;
 }
@@ -621,41 +622,62 @@ __global__ void __launch_bounds__(64 * HW) k_regrid_w(HybCols<V> s, const StepCt
 // k_remap_theta (one thread per column, as k_regrid_tail; G6 x 50, FP64:
 // 440 us with both on lane 0, 216 us for the three kernels): the remapped
 // theta goes to thbuf and the layer depths in p**(kappa+1),
-// max(pk1new(k)-pk1new(k+1), pk1new(1)*1e-6), to exsmo.
+// max(pk1new(k)-pk1new(k+1), pk1new(1)*1e-6), to exsmo.  Bound by its FP64
+// instructions; with the 65th interface's pow in one wavefront of the block and
+// the fields' divisions by reciprocals of the geometry: FP64, G7 x 64 layers,
+// 580 -> 563 us; G6 x 50, 144 -> 138 us.
 template <typename V>
 __global__ void __launch_bounds__(64 * HW) k_remap_w(HybCols<V> s, const StepCtl *ctl, int its) {
   __shared__ double sh[HW][7][LMAX];
   const int ncol = s.ncol, nvl = s.nvl, nvlp1 = nvl + 1, ntra = s.ntra;
   const int lane = threadIdx.x, c = threadIdx.y;
   const int col = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * HW + c));
-  if (col >= ncol) return;
-  if (s.wet && !ldc(s.wet, col)) {    // land: no remap
+  bool act = col < ncol;
+  if (act && s.wet && !ldc(s.wet, col)) {    // land: no remap
     for (int k = lane; k < nvlp1; k += 64) L2(s.sdot, col, k) = 0.;
-    return;
+    act = false;
   }
   if (ctl) its = load_ctl(ctl).its;
   double *prcol = sh[c][0], *pk1col = sh[c][1], *exnew = sh[c][2], *prnew = sh[c][3], *pk1new = sh[c][4],
          *th1 = sh[c][5], *exold = sh[c][6];
+  // FP32 state: the plain-double pow (a few ulp) instead of the correctly rounded one
   const double small = 1.e-6;
-  for (int k = lane; k < nvlp1; k += 64) {
-    const double eo = L2(s.ex, col, k);
-    const double p = L2(s.pr, col, k);
-    exold[k] = eo;
-    prcol[k] = p;
-    exnew[k] = L2(s.exsmo, col, k);
-    pk1col[k] = eo * p / CP;
+  auto pres = [](double e) { return P1000 * (sizeof(V) < sizeof(double) ? fim_pow_fast(e / CP, CP / RD) : fim_pow(e / CP, CP / RD)); };
+  if (act) {
+    for (int k = lane; k < nvlp1; k += 64) {
+      const double eo = L2(s.ex, col, k);
+      const double p = L2(s.pr, col, k);
+      exold[k] = eo;
+      prcol[k] = p;
+      exnew[k] = L2(s.exsmo, col, k);
+      pk1col[k] = eo * p / CP;
+    }
+    wsync();
+    for (int k = lane; k < nvlp1; k += 64) {
+      double e = exnew[k];
+      if (its > 0) e = SLAK * e + (1. - SLAK) * exold[k];
+      if (k >= 1 && k <= nvlp1 - 2) e = dmax(.0001 * exold[k] + .9999 * exold[k + 1], dmin(.0001 * exold[k] + .9999 * exold[k - 1], e));
+      exnew[k] = e;
+      if (k < 64) {
+        const double pn = pres(e);
+        prnew[k] = pn;
+        pk1new[k] = e * pn / CP;
+      }
+    }
   }
-  wsync();
-  for (int k = lane; k < nvlp1; k += 64) {
-    double e = exnew[k];
-    if (its > 0) e = SLAK * e + (1. - SLAK) * exold[k];
-    if (k >= 1 && k <= nvlp1 - 2) e = dmax(.0001 * exold[k] + .9999 * exold[k + 1], dmin(.0001 * exold[k] + .9999 * exold[k - 1], e));
-    exnew[k] = e;
-    // FP32 state: the plain-double pow (a few ulp) instead of the correctly rounded one
-    const double pn = P1000 * (sizeof(V) < sizeof(double) ? fim_pow_fast(e / CP, CP / RD) : fim_pow(e / CP, CP / RD));
-    prnew[k] = pn;
-    pk1new[k] = e * pn / CP;
+  if (nvlp1 > 64) {
+    // the 65th interface of the block's columns: lane j of the first wavefront
+    // takes column j's (in each wavefront by itself the pow is a second pass
+    // for one lane; a column without work has a value nobody reads)
+    __syncthreads();
+    if (c == 0 && lane < HW) {
+      const double e = sh[lane][2][64], pn = pres(e);
+      sh[lane][3][64] = pn;
+      sh[lane][4][64] = e * pn / CP;
+    }
+    __syncthreads();
   }
+  if (!act) return;
   wsync();
   for (int k = lane; k < nvl; k += 64) C2(s.dp, col, k) = prnew[k] - prnew[k + 1];
   wsync();

@@ -30,6 +30,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "div_by.h"
 #include "hycom_edges.h"
 
 namespace fimhip {
@@ -78,19 +79,6 @@ __device__ __forceinline__ UV col_total2(double (*buf)[LPC + 1], double u, doubl
   wave_sync();
   return r;
 }
-// n / s from r = 1 / s, with the division's own rounding: two corrections by
-// the exact remainder (Markstein 1990: with r the nearest to 1/s, the second
-// one, from a quotient within one unit, ends on the nearest).  s is a
-// thickness in pascals (1e-3 to 1e9); outside the range in which every
-// remainder is a normal number, and for 0, inf and NaN, it divides.
-__device__ __forceinline__ double div_by(double n, double s, double r) {
-  double q = n * r;
-  q = __builtin_fma(__builtin_fma(-q, s, n), r, q);
-  q = __builtin_fma(__builtin_fma(-q, s, n), r, q);
-  if (!(fabs(n) > 1.e-200 && fabs(n) < 1.e200)) q = n / s;
-  return q;
-}
-
 // EDGES: the edge values are the public arrays' (an uploaded state);
 // otherwise they are formed here from the cells, from the values
 // fimhip_ocn_edgvar saw (dpe the mid-time thickness; the velocities have not
@@ -414,7 +402,7 @@ __global__ void __launch_bounds__(256) hyc_mom_upd(HycGrid g, HycState s, HycEdg
   sx[cc][1][k] = vn;
   sx[cc][2][k] = qq;
   sx[cc][3][k] = slab;
-  sx[cc][4][k] = 1. / slab;
+  sx[cc][4][k] = div_rcp(slab);
   wave_sync();
   if (k < 2) {
     double *x = sx[cc][k];
