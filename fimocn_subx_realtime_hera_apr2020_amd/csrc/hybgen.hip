@@ -871,17 +871,18 @@ __global__ void __launch_bounds__(64) k_remap_inflate(HybCols<V> s, double extop
 }
 
 // one exchange of the theta redistribution of remap_1d (hybgen.F90:515-789,
-// final loop): layers p (tha, depth dplo) and p+1 (thb, dpup)
-__device__ __forceinline__ void theta_pair(double &tha, double &thb, double dplo, double dpup, double tlo,
-                                           double tup) {
+// final loop): layers p (tha, depth dplo) and p+1 (thb, dpup), with the depths'
+// reciprocals, which do not wait for the sweep (a division in its chain would)
+__device__ __forceinline__ void theta_pair(double &tha, double &thb, double dplo, double dpup, double rlo, double rup,
+                                           double tlo, double tup) {
   const double devilo = (tha - tlo) * dplo;
   const double deviup = (thb - tup) * dpup;
-  if (deviup > 0. && devilo < 0.) {
-    tha = tha + dmin(deviup, -devilo) / dplo;
-    thb = thb - dmin(deviup, -devilo) / dpup;
-  } else if (deviup < 0. && devilo > 0.) {
-    tha = tha - dmin(devilo, -deviup) / dplo;
-    thb = thb + dmin(devilo, -deviup) / dpup;
+  const bool down = deviup > 0. && devilo < 0.;      // from the upper layer to the lower
+  if (down || (deviup < 0. && devilo > 0.)) {
+    const double m = down ? dmin(deviup, -devilo) : dmin(devilo, -deviup);
+    const double qa = div_by(m, dplo, rlo), qb = div_by(m, dpup, rup);
+    tha = down ? tha + qa : tha - qa;
+    thb = down ? thb - qb : thb + qb;
   }
 }
 
@@ -892,7 +893,8 @@ __device__ __forceinline__ void theta_pair(double &tha, double &thb, double dplo
 // reads 16 levels of 4 columns), the sweep works on one chunk in registers and
 // carries the upper layer of the pair that straddles two chunks, and the
 // result goes back to column-major tracer 1 through an LDS tile, so every
-// global access is coalesced.
+// global access is coalesced.  Bound by the sweep's latency: without a division
+// in its chain, FP64, G3 x 64 layers, 32 -> 25 us, G7 93 -> 84 us.
 template <int NVL, bool FULL, typename V>
 __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
   constexpr int CH = 16;
@@ -902,7 +904,7 @@ __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
   const int NCH = (nvl + CH - 1) / CH;   // the top chunk may be a part of one
   const int lane = threadIdx.x, c0 = blockIdx.x * 64;
   const int sl = lane & 15, sj = lane >> 4;
-  double cth = 0., cdl = 0.;   // level k0+CH (the chunk above): theta still to be finalised, layer depth
+  double cth = 0., cdl = 0., crd = 0.;   // level k0+CH (the chunk above): theta still to be finalised, layer depth
 #pragma unroll 1
   for (int ch = NCH - 1; ch >= 0; ch--) {
     const int k0 = ch * CH;
@@ -915,27 +917,29 @@ __global__ void __launch_bounds__(64) k_remap_theta(HybCols<V> s) {
       sdl[sl][c] = L2(s.exsmo, cc, lev);
     }
     wsync();
-    double th[CH], dl[CH];
+    double th[CH], dl[CH], rd[CH];
 #pragma unroll
     for (int j = 0; j < CH; j++) {
       th[j] = sth[j][lane];
       dl[j] = sdl[j][lane];
+      rd[j] = div_rcp(dl[j]);
     }
     if (ch < NCH - 1) {   // the pair (k0+CH-1, k0+CH) finishes level k0+CH
-      theta_pair(th[CH - 1], cth, dl[CH - 1], cdl, ldc(s.thetac, k0 + CH - 1), ldc(s.thetac, k0 + CH));
+      theta_pair(th[CH - 1], cth, dl[CH - 1], cdl, rd[CH - 1], crd, ldc(s.thetac, k0 + CH - 1), ldc(s.thetac, k0 + CH));
       sout[CH][lane] = (V)cth;
     }
 #pragma unroll
     for (int j = CH - 2; j >= 0; j--) {
       if (k0 + j < 1) break;
       if (!FULL && k0 + j + 1 > nvl - 1) continue;
-      theta_pair(th[j], th[j + 1], dl[j], dl[j + 1], ldc(s.thetac, k0 + j), ldc(s.thetac, k0 + j + 1));
+      theta_pair(th[j], th[j + 1], dl[j], dl[j + 1], rd[j], rd[j + 1], ldc(s.thetac, k0 + j), ldc(s.thetac, k0 + j + 1));
     }
     // levels k0+1 .. k0+CH-1 are final; k0 is carried (final in the bottom chunk)
 #pragma unroll
     for (int j = 0; j < CH; j++) sout[j][lane] = (V)th[j];
     cth = th[0];
     cdl = dl[0];
+    crd = rd[0];
     wsync();
     // store levels k0+1 .. k0+CH (16 levels of 4 columns per instruction), and level 0 at the bottom
     const int lev = k0 + 1 + sl;
