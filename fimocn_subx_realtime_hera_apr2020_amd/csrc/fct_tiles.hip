@@ -1,5 +1,6 @@
-// The tracer flux-corrected transport of a step in one kernel (the batched
-// mixed-precision form): trcadv1-3 (trcadv_compute.F90:19-315) together with
+// Kernels over patches of cells for the batched mixed-precision form's tracer
+// transport: the first two stages of the chain (k_e_trcadv12, below), and the
+// whole flux-corrected transport of a step in one kernel: trcadv1-3 (trcadv_compute.F90:19-315) together with
 // the least-squares edge reconstructions of tracers 2..ntra that edgvar3
 // forms for them (edgvar3.F90:65-163), without any intermediate array in HBM.
 //
@@ -18,9 +19,9 @@
 // with a block barrier between stages.  A ring's values are recomputed by
 // each patch that needs them, so a cell's results in rings 1-2 exist in
 // several blocks but are written to HBM only by the block whose core holds
-// the cell.  Every operation is the one the three-kernel chain performs
-// (kernels_ens.hip), in the same order, so the results are bit-identical to
-// it; in particular each edge's flux is formed from the same operands on
+// the cell.  Every operation is the one the chain of k_e_trcadv12 and
+// k_e_trcadv3 (kernels_ens.hip) performs, in the same order, so the results are
+// bit-identical to it; in particular each edge's flux is formed from the same operands on
 // both sides and the tracer mass still cancels exactly across every edge.
 //
 // The block reads the tracer and tracer mass of cells that other blocks

@@ -159,19 +159,22 @@ extern "C" int fimhip_create(const fimhip_grid_desc *gd, int device, fimhip_ctx 
   // ---- state and work arrays
   const size_t cz = (size_t)nip * nvl, lz = (size_t)nip * (nvl + 1), ez = (size_t)nip * NPP * nvl;
   DevState &s = c->s;
-  struct { double **p; size_t n; } arrs[] = {
+  const Arena::Arr arrs[] = {
       {&s.us, cz}, {&s.vs, cz}, {&s.dp, cz}, {&s.pr, lz}, {&s.ex, lz}, {&s.ph, lz}, {&s.mp, cz},
       {&s.tr, cz * ntra}, {&s.trdp, cz * ntra}, {&s.u_tdcy, 3 * cz}, {&s.v_tdcy, 3 * cz},
       {&s.dp_tdcy, 3 * cz}, {&s.dpl_tdcy, 3 * cz}, {&s.trc_tdcy, 3 * cz * ntra}, {&s.trl_tdcy, 3 * cz * ntra},
       {&s.massfx, 3 * ez}, {&s.ws, cz}, {&s.relvor, cz}, {&s.sdot, lz}, {&s.psrf, (size_t)nip},
       {&s.ptdcy, 2 * (size_t)nip}, {&s.u_edg, ez}, {&s.v_edg, ez}, {&s.dp_edg, ez}, {&s.lp_edg, ez},
-      {&s.mont_edg, ez}, {&s.uvsq_edg, ez}, {&s.trc_edg, ez * ntra}, {&s.antifx, ez}, {&s.delp_lo, cz},
+      {&s.mont_edg, ez}, {&s.uvsq_edg, ez}, {&s.trc_edg, ez * ntra}};
+  const Arena::Arr work[] = {
+      {&s.antifx, ez}, {&s.delp_lo, cz},
       {&s.r_plus, cz}, {&s.r_mnus, cz}, {&s.antiflx, ez * ntra}, {&s.trcr_lo, cz * ntra},
       {&s.trmax, cz * ntra}, {&s.trmin, cz * ntra}, {&s.tr_rp, cz * ntra}, {&s.tr_rm, cz * ntra},
       {&s.u2, cz}, {&s.v2, cz}, {&s.exsmo, lz}, {&s.thbuf, cz}, {&s.vn, ez}, {&s.bke, ez}, {&s.pgx, cz},
       {&s.pgy, cz}, {&s.dp_alt, cz}, {&s.pr_alt, lz}, {&s.mp_alt, cz}, {&s.tr_alt, cz * ntra}};
   for (auto &a : arrs)
     if ((r = c->arena.alloc(a.p, a.n))) { fimhip_destroy(c); return r; }
+  if ((r = c->arena.alloc_all(work))) { fimhip_destroy(c); return r; }
   // patches of 44 cells, smaller where those would leave CUs without a block
   // (trcadv1 at G3 x 4 tracers: 25 us with 44, 12 us with 12; at G4 29 and 28)
   const int core = (int)std::max(12LL, (long long)nip * ntra / 600);
@@ -842,20 +845,38 @@ extern "C" int fimhip_sync(fimhip_ctx *c) {
 
 // globsum: fixed-order block partials (cells strided by the grid), summed in
 // block order, so the result is reproducible run to run.  One block's partial
-// of sum q: area*dp (q = 0) or area*dp*tr_q over its cells.
+// of sum q: area*dp (q = 0) or area*dp*tr_q over its cells, a thread per cell
+// adding its column in level order.  The block reads 16 levels of its 256
+// cells at a time side by side and hands the products over in LDS (each thread
+// reading its own column, 512 bytes from the next: G7 x 64 layers x 4 tracers
+// took 750 us, this 252; G3 129 and 70, most of it the sums in blocks of their
+// own).
+constexpr int GSUM_CH = 16;
 
 __device__ __forceinline__ double gsum_block(const double *area, const double *dp, const double *tq, bool with_tr,
-                                             int nip, int nvl, double *sh) {
+                                             int nip, int nvl, double (*sv)[257]) {
   double acc = 0.;
-  for (int ipn = blockIdx.x * 256 + threadIdx.x; ipn < nip; ipn += gridDim.x * 256) {
+  for (int c0 = blockIdx.x * 256; c0 < nip; c0 += gridDim.x * 256) {
     double col = 0.;
-    for (int k = 0; k < nvl; k++) {
-      double v = area[ipn] * dp[(size_t)ipn * nvl + k];
-      if (with_tr) v = v * tq[(size_t)ipn * nvl + k];
-      col = col + v;
+    for (int k0 = 0; k0 < nvl; k0 += GSUM_CH) {
+      const int kn = min(GSUM_CH, nvl - k0), lev = threadIdx.x % GSUM_CH;
+#pragma unroll
+      for (int i = 0; i < GSUM_CH; i++) {
+        const int j = threadIdx.x / GSUM_CH + i * (256 / GSUM_CH), ipn = c0 + j;
+        if (ipn < nip && lev < kn) {
+          double v = area[ipn] * dp[(size_t)ipn * nvl + k0 + lev];
+          if (with_tr) v = v * tq[(size_t)ipn * nvl + k0 + lev];
+          sv[lev][j] = v;
+        }
+      }
+      __syncthreads();
+      if (c0 + (int)threadIdx.x < nip)
+        for (int k = 0; k < kn; k++) col = col + sv[k][threadIdx.x];
+      __syncthreads();
     }
-    acc = acc + col;
+    if (c0 + (int)threadIdx.x < nip) acc = acc + col;
   }
+  double *sh = sv[0];
   sh[threadIdx.x] = acc;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -867,22 +888,20 @@ __device__ __forceinline__ double gsum_block(const double *area, const double *d
   return r;
 }
 
-__global__ void __launch_bounds__(256) k_globsum(DevGrid g, DevState s, const double *trb, int ntrb,
-                                                 double *part) {
-  __shared__ double sh[256];
-  const int nip = g.nip, nvl = g.nvl, ntra = g.ntra;
-  for (int q = 0; q <= ntra + ntrb; q++) {
-    const double *tq = q > ntra ? trb + (size_t)(q - 1 - ntra) * nip * nvl : s.tr + (size_t)(q > 0 ? q - 1 : 0) * nip * nvl;
-    const double r = gsum_block(g.area, s.dp, tq, q > 0, nip, nvl, sh);
-    if (threadIdx.x == 0) part[(size_t)q * gridDim.x + blockIdx.x] = r;
-  }
+// sum q = blockIdx.y
+__global__ void __launch_bounds__(256) k_globsum(DevGrid g, DevState s, const double *trb, double *part) {
+  __shared__ double sv[GSUM_CH][257];
+  const int nip = g.nip, nvl = g.nvl, ntra = g.ntra, q = blockIdx.y;
+  const double *tq = q > ntra ? trb + (size_t)(q - 1 - ntra) * nip * nvl : s.tr + (size_t)(q > 0 ? q - 1 : 0) * nip * nvl;
+  const double r = gsum_block(g.area, s.dp, tq, q > 0, nip, nvl, sv);
+  if (threadIdx.x == 0) part[(size_t)q * gridDim.x + blockIdx.x] = r;
 }
 
 extern "C" int fimhip_globsum(fimhip_ctx *c, double *mass, double *trtot) {
   if (!c || !mass) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
   const int nq = c->ntra + c->cb.ntrb;
-  k_globsum<<<c->gsum_blocks, 256, 0, c->stream>>>(c->g, c->s, c->cb.trb, c->cb.ntrb, c->gsum_partial);
+  k_globsum<<<dim3(c->gsum_blocks, 1 + nq), 256, 0, c->stream>>>(c->g, c->s, c->cb.trb, c->gsum_partial);
   std::vector<double> h((size_t)c->gsum_blocks * (1 + nq));
   HIPCHK(hipMemcpyAsync(h.data(), c->gsum_partial, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   TRY(finish(c));
@@ -910,10 +929,10 @@ static std::mutex g_scratch_mu;
 
 __global__ void __launch_bounds__(256) k_globsum_dev(const double *area, const double *dp, const double *tr, int nip,
                                                      int nvl, int nq1, double *part) {
-  __shared__ double sh[256];
+  __shared__ double sv[GSUM_CH][257];
   for (int q = 0; q < nq1; q++) {
     const double *tq = tr + (size_t)(q > 0 ? q - 1 : 0) * nip * nvl;
-    const double r = gsum_block(area, dp, tq, q > 0, nip, nvl, sh);
+    const double r = gsum_block(area, dp, tq, q > 0, nip, nvl, sv);
     if (threadIdx.x == 0) part[(size_t)q * GSUM_BLOCKS + blockIdx.x] = r;
   }
 }

@@ -43,6 +43,23 @@ struct Arena {
   }
   template <class T>
   int alloc(T **p, size_t n) { return raw((void **)p, n * sizeof(T)); }
+  // several arrays of doubles in one allocation, at staggered offsets too (one
+  // allocation each takes a small instance longer to create than its step)
+  struct Arr { double **p; size_t n; };
+  template <size_t N>
+  int alloc_all(const Arr (&arrs)[N]) {
+    constexpr size_t stagger = 4352 / sizeof(double);
+    size_t total = 0;
+    for (auto &a : arrs) total += (a.n + 31) / 32 * 32 + stagger;
+    double *w = nullptr;
+    const int r = alloc(&w, total);
+    if (r) return r;
+    for (auto &a : arrs) {
+      *a.p = w;
+      w += (a.n + 31) / 32 * 32 + stagger;
+    }
+    return 0;
+  }
   template <class T>
   int upload(T **p, const T *h, size_t n) {
     int r = alloc(p, n);

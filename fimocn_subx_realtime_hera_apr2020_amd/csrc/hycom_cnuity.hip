@@ -653,25 +653,27 @@ extern "C" int fimhip_ocn_create(const fimhip_grid_desc *gd, const double *rprox
   const size_t cz = (size_t)nip * kdm, ez = cz * NPP;
   HycState &s = o->s;
   double *um, *vm, *un, *vn, *dpe;
-  struct { double **p; size_t n; } arrs[] = {
+  const Arena::Arr arrs[] = {
       {&um, ez}, {&vm, ez}, {&un, ez}, {&vn, ez}, {&dpe, ez}, {&s.dp, 2 * cz}, {&s.pres, (size_t)nip * (kdm + 1)},
-      {&s.massflx, ez}, {&s.mssfx_avg, ez}, {&s.antiflx, ez}, {&s.vnm, ez}, {&s.vnn, ez}, {&s.dp_lo, cz},
-      {&s.dpc, cz}, {&s.dpr, cz}, {&s.flxplus, cz}, {&s.flxmnus, cz}, {&s.rplus, cz}, {&s.rmnus, cz},
-      {&s.del2p, cz}, {&s.dptmp, cz}, {&s.brat, cz}, {&s.clippd, (size_t)nip * NPP}, {&s.clippb, (size_t)nip * NPP},
-      {&s.rpbot, (size_t)nip}, {&s.rpbotb, (size_t)nip}, {&s.aux, (size_t)nip}, {&s.dpe, cz},
-      {&s.pbe, (size_t)nip}, {&s.p0e, (size_t)nip}, {&o->pres_f, (size_t)nip * (kdm + 1)},
+      {&s.massflx, ez}, {&s.mssfx_avg, ez},
       // the edge interpolation's inputs and outputs
       {&o->ed.uclin, 2 * cz}, {&o->ed.vclin, 2 * cz}, {&o->ed.uclin_alt, 2 * cz}, {&o->ed.vclin_alt, 2 * cz},
       {&o->ed.utrop, (size_t)nip * 3}, {&o->ed.vtrop, (size_t)nip * 3},
       {&o->ed.geop, (size_t)nip * (kdm + 1)}, {&o->ed.montg, cz}, {&o->ed.spcifv, cz},
       {&o->ed.pr_edg, (size_t)nip * NPP * (kdm + 1)}, {&o->ed.geop_edg, ez}, {&o->ed.mont_edg, ez},
       {&o->ed.uvsq_edg, ez}, {&o->ed.spcv_edg, ez},
-      // the momentum equation's forcing and work arrays
+      // the momentum equation's forcing
       {&o->mo.taux, (size_t)nip}, {&o->mo.tauy, (size_t)nip}, {&o->mo.ustarb, (size_t)nip},
-      {&o->mo.drag, (size_t)nip}, {&o->mo.dpbot, (size_t)nip}, {&o->mo.d4u, cz}, {&o->mo.d4v, cz},
-      {&o->mo.gradx, cz}, {&o->mo.grady, cz}, {&o->mo.relvor, cz}, {&o->mo.visc, cz},
       // the tracers and density the transport and the grid generator share
       {&o->tr.temp, cz}, {&o->tr.saln, cz}, {&o->hy.dens, cz}};
+  const Arena::Arr work[] = {
+      {&s.vnm, ez}, {&s.vnn, ez}, {&s.antiflx, ez}, {&s.dp_lo, cz}, {&s.dpc, cz}, {&s.dpr, cz}, {&s.flxplus, cz},
+      {&s.flxmnus, cz}, {&s.rplus, cz}, {&s.rmnus, cz}, {&s.del2p, cz}, {&s.dptmp, cz}, {&s.brat, cz}, {&s.dpe, cz},
+      {&o->mo.d4u, cz}, {&o->mo.d4v, cz}, {&o->mo.gradx, cz}, {&o->mo.grady, cz}, {&o->mo.relvor, cz},
+      {&o->mo.visc, cz}, {&o->pres_f, (size_t)nip * (kdm + 1)}, {&s.clippd, (size_t)nip * NPP},
+      {&s.clippb, (size_t)nip * NPP}, {&s.rpbot, (size_t)nip}, {&s.rpbotb, (size_t)nip}, {&s.aux, (size_t)nip},
+      {&s.pbe, (size_t)nip}, {&s.p0e, (size_t)nip}, {&o->mo.drag, (size_t)nip}, {&o->mo.dpbot, (size_t)nip}};
+  if ((r = o->arena.alloc_all(work))) { fimhip_ocn_destroy(o); return r; }
   for (auto &a : arrs)
     if ((r = o->arena.alloc(a.p, a.n))) { fimhip_ocn_destroy(o); return r; }
   s.um = um; s.vm = vm; s.un = un; s.vn = vn; s.dpm_edg = dpe;
