@@ -509,7 +509,7 @@ def test_restart_round_trip_then_steps_match_checker_bitwise(case, tmp_path):
 @pytest.mark.parametrize("flux_scheme,ntrb", [(1, 0), (2, 2)])
 def test_forty_layers_steps_match_checker_bitwise(oracle_lib, flux_scheme, ntrb):
     """40 layers (the kernels' paths for nvl below the wavefront width):
-    start-up plus 9 full steps identical to the checker."""
+    start-up plus 9 full steps identical to the oracle."""
     from fimocn_subx_realtime_hera_apr2020_amd import fimhip
     from helpers import seeded_case
     O = oracle_lib
@@ -728,7 +728,7 @@ def test_ragged_layer_counts_match_checker_bitwise(oracle_lib, nvl):
     """Layer counts at the edges of the column kernels' 16-level chunks
     (hybgen's and fct3d's serial sweeps, one thread per column): start-up plus
     6 full steps with class-B transport every 2 steps, identical to the
-    checker."""
+    oracle."""
     from fimocn_subx_realtime_hera_apr2020_amd import fimhip
     from helpers import seeded_case
     O = oracle_lib
