@@ -37,14 +37,15 @@ struct Arena;
 // neighbours 4-5 and its edge count (8 bits each); the neighbours' indices of
 // the shared edges, proxs (4 bits each).  The local indices are set for
 // rings 0-2 only.
-constexpr int CORE_ROW = 108;
+// words of trcadv12's core rows and where their parts begin (k_core_rows in
+// fct_tiles.hip)
+constexpr int CR_NBR = 36, CR_ST = 72, CR_NB = 90, CORE_ROW = 96;
 struct EnsTiles {
   int npatch;
   const int *off;      // (npatch + 1) first tile cell of each patch
   const int4 *cnt;     // (npatch) n0, n1, n2, n3
   const int4 *ent;
-  const int *core_row; // (CORE_ROW, nip), see k_core_rows in fct_tiles.hip
-  bool cyclic;         // every cell's slots run around it in the same sense
+  const int *core_row; // (CORE_ROW, nip)
   int r_max, lo_max;   // most cells of a patch in rings 0-1 and 0-2
 };
 

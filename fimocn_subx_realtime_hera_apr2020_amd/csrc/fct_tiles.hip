@@ -28,7 +28,6 @@
 // update in the same launch, so the kernel reads one buffer and writes the
 // other of a pair (the instance alternates them every step).
 #include <algorithm>
-#include <type_traits>
 #include <vector>
 
 #include "ens_internal.h"
@@ -205,12 +204,10 @@ __device__ __forceinline__ float fct_theta_edge(float thi, float thx, float tht,
   return (2.f * (thi + thx) + ta + tb) * (1.f / 6.f);
 }
 
-// The donor-cell value of an edge with mass flux m out of the cell: the
-// low-order flux is m * upwind, and the antidiffusive flux m * (te - upwind),
-// each one rounding on both sides of the edge (the reference forms
-// .5*((m+|m|)*t - (|m|-m)*tx), the same product, and the difference of the two
-// fluxes).
-__device__ __forceinline__ float fct_upwind(float m, float ti, float tx) { return m >= 0.f ? ti : tx; }
+// The low-order (donor-cell) flux of an edge with mass flux m out of the cell.
+__device__ __forceinline__ float fct_low(float m, float ti, float tx) {
+  return .5f * ((m + fabsf(m)) * ti - (fabsf(m) - m) * tx);
+}
 
 __device__ __forceinline__ float fct_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
@@ -287,14 +284,17 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
   for (int e = 0; e < NP; e++) v[e] = Str[l[e] * 64 + lane];
   const float rar = ldc(g.rarea, cell);
   const float a1 = (float)c.ab1, a2 = (float)c.ab2, a3 = (float)c.ab3;
-  float acc = 0.f, mx = ti, mn = ti;
+  float acc = 0.f, mx = ti, mn = ti, fl[NP];
 #pragma unroll
   for (int e = 0; e < NP; e++) {
     mx = fmaxf(mx, v[e]);
     mn = fminf(mn, v[e]);
   }
 #pragma unroll
-  for (int e = 0; e < NP; e++) acc = acc + m[e] * fct_upwind(m[e], ti, v[e]);
+  for (int e = 0; e < NP; e++) {
+    fl[e] = fct_low(m[e], ti, v[e]);
+    acc = acc + fl[e];
+  }
   const float tlo = -acc * rar;
   const float lo = tdp0 + a1 * tlo + a2 * tlo_of + a3 * tlo_vof;
   mx = fmaxf(0.f, mx);
@@ -319,9 +319,9 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
     for (int j = 0; j < NP; j++) d[j] = v[j] - ti;
 #pragma unroll
     for (int e = 0; e < NP; e++) {
-      float ac = 0.f;      // both cells' sums start at the shared edge's slot
+      float ac = 0.f;
 #pragma unroll
-      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[(e + j) % NP], FHF(cell, e, (e + j) % NP), ac);
+      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[j], FHF(cell, e, j), ac);
       const float eo = ti + ac;
       const int4 ex = Sent[l[e]];
       const int xcell = uni(ex.x), xs = uni(eslot(en, e)), xnp = uni(enp(ex));
@@ -329,8 +329,7 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
       float ax = 0.f;
 #pragma unroll
       for (int j = 0; j < NPP; j++) {
-        const int jj = xs + j < xnp ? xs + j : xs + j - xnp;
-        if (j < xnp) ax = __builtin_fmaf(Str[uni(lnb(ex, jj)) * 64 + lane] - tx, FHF(xcell, xs, jj), ax);
+        if (j < xnp) ax = __builtin_fmaf(Str[uni(lnb(ex, j)) * 64 + lane] - tx, FHF(xcell, xs, j), ax);
       }
       const float en_ = tx + ax;
       te[e] = .5f * (eo + en_);
@@ -339,7 +338,7 @@ __device__ __forceinline__ void fct_stage_a(const EnsGrid &g, const EnsState &s,
   float sp = 0.f, sm = 0.f;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
-    const float a = m[e] * (te[e] - fct_upwind(m[e], ti, v[e]));
+    const float a = m[e] * te[e] - fl[e];
     a_out[e] = a;
     sp = sp - fminf(0.f, a);
     sm = sm + fmaxf(0.f, a);
@@ -607,8 +606,6 @@ void ens_launch_trc_fct(int tile, const EnsGrid &g, const EnsState &s, hipStream
 //    vector load, a cell ahead, and are handed out by v_readlane: as scalar
 //    loads they missed the scalar cache and each batch waited about 1500
 //    cycles (9.0 ms);
-//  * of a neighbour's six stencil cells three are in registers (the cell
-//    itself and the two cells at the edge's ends);
 //  * the mass fluxes and tendencies are loaded two cells ahead;
 //  * every tracer and member of a patch runs in turn on one XCD, whose L2
 //    then holds the patch's rows and mass fluxes (8.0 ms in block order);
@@ -672,7 +669,7 @@ __device__ __forceinline__ float tile_lo(const StepCtl &c, const int4 &en, int i
   for (int e = 0; e < NP; e++) {
     mx = fmaxf(mx, v[e]);
     mn = fminf(mn, v[e]);
-    acc = acc + in.m[e] * fct_upwind(in.m[e], ti, v[e]);
+    acc = acc + fct_low(in.m[e], ti, v[e]);
   }
   const float tlo = -acc * rar;
   const float lo = in.tdp0 + a1 * tlo + a2 * in.lo_of + a3 * in.lo_vof;
@@ -685,8 +682,13 @@ __device__ __forceinline__ int row_i(const int2 &row, int w) {
   return __builtin_amdgcn_readlane(w & 1 ? row.y : row.x, w >> 1);
 }
 __device__ __forceinline__ float row_f(const int2 &row, int w) { return __int_as_float(row_i(row, w)); }
+// i-th 16-bit field from word w0
+__device__ __forceinline__ int row_h(const int2 &row, int w0, int i) {
+  const int p = row_i(row, w0 + (i >> 1));
+  return i & 1 ? (p >> 16) & 0xffff : p & 0xffff;
+}
 
-template <int NP, bool CYC>
+template <int NP>
 __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, const StepCtl &c, int cell, int i, int t,
                                           int col, size_t toff, int k, float area, const int2 &row, const TileInB &in,
                                           const float *Str, const float *Slo) {
@@ -695,7 +697,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   const float dp = (float)in.dp;
   const float ti = Str[i * 64 + k], lo = Slo[i * 64 + k];
 #pragma unroll
-  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, 102 + e) & ~1, k);
+  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, CR_NB + e) & ~3, k);
   if (t == 0) {
 #pragma unroll
     for (int e = 0; e < NP; e++) {
@@ -710,14 +712,11 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
     for (int e = 0; e < NP; e++) {
       float ac = 0.f, ax = 0.f;
 #pragma unroll
-      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[(e + j) % NP], row_f(row, e * NPP + (e + j) % NP), ac);
-      ax = -d[e] * row_f(row, 36 + e * NPP);
+      for (int j = 0; j < NP; j++) ac = __builtin_fmaf(d[j], row_f(row, e * NPP + j), ac);
 #pragma unroll
-      for (int r = 1; r < NPP; r++) {
-        const float n = CYC && r == 1 ? v[(e + NP - 1) % NP]
-                        : CYC && r == NPP - 1 ? v[(e + 1) % NP]
-                                              : lds_at(Str, row_i(row, 72 + e * (NPP - 1) + r - 1), k);
-        ax = __builtin_fmaf(n - v[e], row_f(row, 36 + e * NPP + r), ax);
+      for (int j = 0; j < NPP; j++) {
+        const float n = lds_at(Str, row_h(row, CR_ST, e * NPP + j), k) - v[e];
+        if (j < NPP - 1 || !(row_i(row, CR_NB + e) & 2)) ax = __builtin_fmaf(n, row_f(row, CR_NBR + e * NPP + j), ax);
       }
       te[e] = .5f * ((ti + ac) + (v[e] + ax));
     }
@@ -726,8 +725,8 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
 #pragma unroll
   for (int e = 0; e < NP; e++) {
     const float m = in.m[e];
-    const float a = m * (te[e] - fct_upwind(m, ti, v[e]));
-    if (row_i(row, 102 + e) & 1) __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
+    const float a = m * te[e] - fct_low(m, ti, v[e]);
+    if (row_i(row, CR_NB + e) & 1) __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
     sp = sp - fminf(0.f, a);
     sm = sm + fmaxf(0.f, a);
     mx = fmaxf(mx, v[e]);
@@ -737,7 +736,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   mn = fminf(fmaxf(0.f, mn), lo);
 #pragma unroll
   for (int e = 0; e < NP; e++) {
-    const float x = lds_at(Slo, row_i(row, 102 + e) & ~1, k);
+    const float x = lds_at(Slo, row_i(row, CR_NB + e) & ~3, k);
     mx = fmaxf(mx, x);
     mn = fminf(mn, x);
   }
@@ -752,7 +751,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qm * fct_rcp(fmaxf(sm, 1.e-11f)))), &TRV(s.tr_rm, col));
 }
 
-template <int NW, bool SWZ, bool CYC>
+template <int NW, bool SWZ>
 __global__ void __launch_bounds__(64 * NW) k_e_trcadv12(EnsGrid g, EnsState s) {
   extern __shared__ float lds[];       // the tracer of rings 0-2, the low-order tracer of rings 0-1
   const int nvl = g.d.nvl, nip = g.d.nip, ncol = s.ncol, ntra = g.d.ntra;
@@ -825,8 +824,8 @@ __global__ void __launch_bounds__(64 * NW) k_e_trcadv12(EnsGrid g, EnsState s) {
     const int2 nrow = load_row(j + 1);
     const float area = lane_f(arl, j);
     if (live) {
-      if (((z >> 16) & 0xff) == 6) tile_flux<6, CYC>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
-      else tile_flux<5, CYC>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
+      if (((z >> 16) & 0xff) == 6) tile_flux<6>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
+      else tile_flux<5>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
     }
     cb = nb;
     row = nrow;
@@ -839,52 +838,39 @@ void ens_launch_trcadv12(int tile, const EnsGrid &g, const EnsState &s, hipStrea
   const int np = g.ptiles.npatch, tm = g.d.ntra * s.members;
   const dim3 swz((np + 7) / 8 * 8 * tm), lin(np * tm);
   const size_t sh = (size_t)(g.ptiles.lo_max + g.ptiles.r_max) * 64 * sizeof(float);
-  auto run = [&](auto cyc) {
-    constexpr bool C = decltype(cyc)::value;
-    switch (tile & 5) {
-      case 0: k_e_trcadv12<8, false, C><<<lin, dim3(64, 8), sh, st>>>(g, s); break;
-      case 1: k_e_trcadv12<16, false, C><<<lin, dim3(64, 16), sh, st>>>(g, s); break;
-      case 4: k_e_trcadv12<8, true, C><<<swz, dim3(64, 8), sh, st>>>(g, s); break;
-      default: k_e_trcadv12<16, true, C><<<swz, dim3(64, 16), sh, st>>>(g, s); break;
-    }
-  };
-  if (g.ptiles.cyclic) run(std::true_type{});
-  else run(std::false_type{});
+  switch (tile & 5) {
+    case 0: k_e_trcadv12<8, false><<<lin, dim3(64, 8), sh, st>>>(g, s); break;
+    case 1: k_e_trcadv12<16, false><<<lin, dim3(64, 16), sh, st>>>(g, s); break;
+    case 4: k_e_trcadv12<8, true><<<swz, dim3(64, 8), sh, st>>>(g, s); break;
+    default: k_e_trcadv12<16, true><<<swz, dim3(64, 16), sh, st>>>(g, s); break;
+  }
 }
 
 // Per cell, as the core of its patch, what the two-sided reconstructions of
 // its edges need, one row of CORE_ROW words that a wavefront reads with one
-// load and hands out lane by lane: 0-35 the cell's own coefficients (edge,
-// stencil cell), 36-71 the neighbours' of the shared edges, each sum starting
-// at the shared edge's slot, 72-101 the LDS byte offsets (256 per tile cell)
-// of the neighbours' stencil cells after the first (which is the cell itself),
-// 102-107 those of the neighbours, with bit 0 set where the cell stores the
-// edge's antidiffusive flux (it has the lower index).  A pentagon's missing stencil cell is the
-// neighbour itself with coefficient 0, before the last.  Clears *cyclic unless
-// the slots of all cells run around them in one sense: then the second and
-// last cells of a neighbour's stencil are the cell's own neighbours of slots
-// e-1 and e+1.  One block per patch, one thread per core cell and edge.
-__global__ void __launch_bounds__(256) k_core_rows(EnsGrid g, EnsTiles ts, int *rows, int *cyclic) {
+// load and hands out lane by lane: the cell's own coefficients (edge, stencil
+// cell), the neighbours' of the shared edges, both in the order of the
+// stencil's slots, from CR_ST on the LDS byte offsets (256 per tile cell; 16
+// bits) of the neighbours' stencil cells, and from CR_NB on those of the
+// neighbours, with bit 0 set where the cell stores the edge's antidiffusive
+// flux (it has the lower index) and bit 1 where the neighbour is a pentagon,
+// whose missing stencil cell is the neighbour itself with coefficient 0.  One
+// block per patch, one thread per core cell and edge.
+__global__ void __launch_bounds__(256) k_core_rows(EnsGrid g, EnsTiles ts, int *rows) {
   const int p = blockIdx.x, n0 = ts.cnt[p].x;
   const int4 *ent = ts.ent + ts.off[p];
   for (int q = threadIdx.x; q < n0 * NPP; q += blockDim.x) {
     const int e = q % NPP;
     const int4 en = ent[q / NPP];
-    const int c = en.x, np = enp(en), l = lnb(en, e);
+    const int c = en.x, l = lnb(en, e);
     const int4 ex = ent[l];
     const int x = ex.x, nx = enp(ex), xs = eslot(en, e);
     int *row = rows + (size_t)c * CORE_ROW;
-    row[102 + e] = 256 * l | (c < x);
-    for (int r = 0; r < NPP; r++) {
-      row[e * NPP + r] = __float_as_int(g.hfcoef[((size_t)c * NPP + e) * NPP + r]);
-      const bool in = nx == NPP || r != NPP - 2;
-      const int j = (xs + (r < NPP - 1 ? r : nx - 1)) % nx;
-      row[36 + e * NPP + r] = in ? __float_as_int(g.hfcoef[((size_t)x * NPP + xs) * NPP + j]) : 0;
-      if (r > 0) row[72 + e * (NPP - 1) + r - 1] = 256 * (in ? lnb(ex, j) : l);
-      const int want = r == 1 ? (e + np - 1) % np : (e + 1) % np;
-      if (e < np && (r == 1 || r == NPP - 1) &&
-          g.d.prox[(size_t)x * NPP + j] != g.d.prox[(size_t)c * NPP + want])
-        *cyclic = 0;
+    row[CR_NB + e] = 256 * l | (nx < NPP ? 2 : 0) | (c < x);
+    for (int j = 0; j < NPP; j++) {
+      row[e * NPP + j] = __float_as_int(g.hfcoef[((size_t)c * NPP + e) * NPP + j]);
+      row[CR_NBR + e * NPP + j] = j < nx ? __float_as_int(g.hfcoef[((size_t)x * NPP + xs) * NPP + j]) : 0;
+      ((unsigned short *)(row + CR_ST))[e * NPP + j] = (unsigned short)(256 * (j < nx ? lnb(ex, j) : l));
     }
   }
 }
@@ -896,16 +882,12 @@ int ens_make_core(Arena &a, const TileHost &t, EnsGrid &g) {
     d.r_max = std::max(d.r_max, c[1]);
     d.lo_max = std::max(d.lo_max, c[2]);
   }
-  int *rows = nullptr, *flag = nullptr, cyclic = 1;
-  int r;
-  if ((r = a.alloc(&rows, (size_t)g.d.nip * CORE_ROW)) || (r = a.upload(&flag, std::vector<int>(1, 1)))) return r;
-  k_core_rows<<<d.npatch, 256, 0, a.stream>>>(g, d, rows, flag);
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(&cyclic, flag, sizeof cyclic, hipMemcpyDeviceToHost, a.stream) != hipSuccess ||
-      hipStreamSynchronize(a.stream) != hipSuccess)
-    return FIMHIP_EHIP;
+  int *rows = nullptr;
+  const int r = a.alloc(&rows, (size_t)g.d.nip * CORE_ROW);
+  if (r) return r;
+  k_core_rows<<<d.npatch, 256, 0, a.stream>>>(g, d, rows);
+  if (hipGetLastError() != hipSuccess) return FIMHIP_EHIP;
   d.core_row = rows;
-  d.cyclic = cyclic != 0;
   return FIMHIP_OK;
 }
 

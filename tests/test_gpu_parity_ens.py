@@ -9,12 +9,14 @@ and the FP32 Kahan-compensated sums must agree with the FP64 sums."""
 import numpy as np
 import pytest
 
+from golden import make_ens_bits
 from helpers import rel_l2
 
 pytestmark = pytest.mark.gpu
 
 NVL, NTRA, DT = 64, 4, 240.0
 FLAGS = 1 | 2          # wind noise + member perturbations
+SUMS = ("mass", "totals", "mass32", "totals32")
 
 # relative-L2 bounds of the FP32 form against FP64 after 96 full steps at
 # G5 x 64 (dt = 240 s), about 5x the errors measured on MI355X (us 2.0e-4,
@@ -771,3 +773,17 @@ def test_tracer_transport_on_grids_with_other_slot_orders(seed):
     for n in out[0]:
         assert rel_l2(out[1][n], out[0][n]) < 1e-6, n
         assert np.array_equal(out[1][n], out[2][n]), n
+
+
+@pytest.mark.parametrize("case", list(make_ens_bits.CASES))
+def test_results_keep_their_bits(case):
+    """Every field of the batched form has the recorded bits: the FP32 sums
+    and differences of the tracer transport are formed in one order, whatever
+    kernels form them."""
+    import json
+    print("case: %s" % case, flush=True)
+    with open(make_ens_bits.FILE) as f:
+        want = json.load(f)[case]
+    got = make_ens_bits.digests(case)
+    assert set(got) == set(want)
+    assert [n for n in got if got[n] != want[n] and n not in SUMS] == []
