@@ -880,82 +880,87 @@ __device__ __forceinline__ KPair kp_merge(KPair a, KPair b) {  // a + b, compens
   return r;
 }
 
-// One wavefront per column, lane = level, four tracers (and with the first
-// four the mass) per pass over the thickness, each lane its own partial sums
-// over the columns of its wavefront.  Bound by memory: one read of the
-// thickness and the tracers.  (A thread per column, one sum a pass, read 256
-// bytes apart and the thickness once per tracer: 8 members x G7 x 64 layers x
-// 4 tracers took 10.7 ms, this takes 0.43.)
-template <int NT>
-__device__ __forceinline__ void e_globsum_pass(const EnsGrid &g, const EnsState &s, int t0, bool mass, double (&a)[NT + 1],
-                                               KPair (&kp)[NT + 1]) {
-  const int nip = g.d.nip, nvl = g.d.nvl, ntra = g.d.ntra, ncol = s.ncol;
-  const int k = threadIdx.x & 63, m = blockIdx.y;
-  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  if (k >= nvl) return;
-  constexpr int UN = 2;      // columns in flight
-  const int stride = gridDim.x * 4;
-  for (int i0 = blockIdx.x * 4 + w; i0 < nip; i0 += UN * stride) {
-    double dp[UN];
-    float tr[UN][NT];
-#pragma unroll
-    for (int u = 0; u < UN; u++) {
-      const int col = m * nip + min(i0 + u * stride, nip - 1);
-      dp[u] = EC(s.dp, col, k);
-#pragma unroll
-      for (int j = 0; j < NT; j++) tr[u][j] = ETR(s.tr, min(t0 + j, ntra - 1), col, k);
-    }
-#pragma unroll
-    for (int u = 0; u < UN; u++) {
-      const int ipn = i0 + u * stride;
-      if (ipn >= nip) break;
-      const double v = ldc(g.d.area, ipn) * dp[u];
-      const float vf = GF(area, ipn) * (float)dp[u];
-      if (mass) {
-        a[NT] = a[NT] + v;
-        kp[NT] = kp_add(kp[NT], vf);
-      }
-#pragma unroll
-      for (int j = 0; j < NT; j++) {
-        a[j] = a[j] + v * (double)tr[u][j];
-        kp[j] = kp_add(kp[j], vf * tr[u][j]);
-      }
-    }
-  }
-}
+// A thread per column, adding its levels in order, then its columns, then the
+// block's threads in a tree: the sums' order is fixed.  blockIdx.z takes NT
+// tracers, the first also the mass.  A block reads 16 levels of its 256 columns
+// side by side and hands them over in LDS (each thread reading its own column,
+// 256 bytes from the next, one sum after another: 8 members x G7 x 64 layers x 4
+// tracers took 10.7 ms, this takes 1.03, at 2.6 TB/s; 16 x G5 1.08 and 0.28).
+// Bound by memory: the thickness once per NT tracers and the tracers once, and
+// two blocks of it fit a CU.
+constexpr int GS_NT = 2;
 __global__ void __launch_bounds__(256) k_e_globsum(EnsGrid g, EnsState s, double *p64, float *p32) {
-  __shared__ double sh[256];
-  __shared__ float shs[256], shc[256];
-  const int ntra = g.d.ntra, m = blockIdx.y, nb = gridDim.x;
-  constexpr int NT = 4;
-  for (int t0 = 0; t0 < ntra; t0 += NT) {
-    double a[NT + 1] = {};
-    KPair kp[NT + 1] = {};
-    e_globsum_pass<NT>(g, s, t0, t0 == 0, a, kp);
+  constexpr int NT = GS_NT, CH = 16;
+  __shared__ double sdp[CH][257];
+  __shared__ float str[NT][CH][257];
+  const int nip = g.d.nip, nvl = g.d.nvl, ntra = g.d.ntra, ncol = s.ncol;
+  const int m = blockIdx.y, nb = gridDim.x, t0 = blockIdx.z * NT, tid = threadIdx.x;
+  const bool mass = t0 == 0;
+  double acc[NT + 1] = {};           // [NT]: the mass
+  KPair kp[NT + 1] = {};
+  for (int c0 = blockIdx.x * 256; c0 < nip; c0 += nb * 256) {
+    const int ipn = c0 + tid;
+    const double ar = ipn < nip ? g.d.area[ipn] : 0.;
+    const float arf = ipn < nip ? g.area[ipn] : 0.f;
+    double cs[NT + 1] = {};
+    for (int k0 = 0; k0 < nvl; k0 += CH) {
+      const int kn = min(CH, nvl - k0), lev = tid % CH;
+      __syncthreads();
 #pragma unroll
-    for (int j = 0; j <= NT; j++) {
-      const int q = j == NT ? 0 : t0 + j + 1;      // 0: the mass
-      if (q > ntra || (j == NT && t0 > 0)) continue;
-      sh[threadIdx.x] = a[j];
-      shs[threadIdx.x] = kp[j].s;
-      shc[threadIdx.x] = kp[j].c;
-      __syncthreads();
-      for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-          sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + w];
-          KPair r = kp_merge(KPair{shs[threadIdx.x], shc[threadIdx.x]}, KPair{shs[threadIdx.x + w], shc[threadIdx.x + w]});
-          shs[threadIdx.x] = r.s;
-          shc[threadIdx.x] = r.c;
+      for (int i = 0; i < CH; i++) {
+        const int j = tid / CH + i * (256 / CH), col = m * nip + c0 + j;
+        if (c0 + j < nip && lev < kn) {
+          sdp[lev][j] = EC(s.dp, col, k0 + lev);
+#pragma unroll
+          for (int t = 0; t < NT; t++) str[t][lev][j] = ETR(s.tr, min(t0 + t, ntra - 1), col, k0 + lev);
         }
-        __syncthreads();
-      }
-      if (threadIdx.x == 0) {
-        const size_t o = ((size_t)m * (ntra + 1) + q) * nb + blockIdx.x;
-        p64[o] = sh[0];
-        p32[2 * o] = shs[0];
-        p32[2 * o + 1] = shc[0];
       }
       __syncthreads();
+      if (ipn < nip)
+        for (int k = 0; k < kn; k++) {
+          const double dp = sdp[k][tid], v = ar * dp;
+          const float vf = arf * (float)dp;
+          if (mass) {
+            cs[NT] = cs[NT] + v;
+            kp[NT] = kp_add(kp[NT], vf);
+          }
+#pragma unroll
+          for (int t = 0; t < NT; t++) {
+            const float tr = str[t][k][tid];
+            cs[t] = cs[t] + v * (double)tr;
+            kp[t] = kp_add(kp[t], vf * tr);
+          }
+        }
+    }
+    if (ipn < nip)
+#pragma unroll
+      for (int t = 0; t <= NT; t++) acc[t] = acc[t] + cs[t];
+  }
+  double *sh = sdp[0];
+  float *shs = str[0][0], *shc = str[0][1];
+#pragma unroll
+  for (int t = 0; t <= NT; t++) {
+    const int q = t == NT ? 0 : t0 + t + 1;      // 0: the mass
+    if (q > ntra || (t == NT && !mass)) continue;
+    __syncthreads();
+    sh[tid] = acc[t];
+    shs[tid] = kp[t].s;
+    shc[tid] = kp[t].c;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if (tid < w) {
+        sh[tid] = sh[tid] + sh[tid + w];
+        const KPair r = kp_merge(KPair{shs[tid], shc[tid]}, KPair{shs[tid + w], shc[tid + w]});
+        shs[tid] = r.s;
+        shc[tid] = r.c;
+      }
+      __syncthreads();
+    }
+    if (tid == 0) {
+      const size_t o = ((size_t)m * (ntra + 1) + q) * nb + blockIdx.x;
+      p64[o] = sh[0];
+      p32[2 * o] = shs[0];
+      p32[2 * o + 1] = shc[0];
     }
   }
 }
@@ -1033,7 +1038,7 @@ void ens_launch_narrow(const double *src, float *dst, size_t n, size_t stride, i
 }
 void ens_launch_globsum(const EnsGrid &g, const EnsState &s, double *part64, float *part32, int nblocks,
                         hipStream_t st) {
-  k_e_globsum<<<dim3(nblocks, s.members), 256, 0, st>>>(g, s, part64, part32);
+  k_e_globsum<<<dim3(nblocks, s.members, (g.d.ntra + GS_NT - 1) / GS_NT), 256, 0, st>>>(g, s, part64, part32);
 }
 
 }  // namespace fimhip
