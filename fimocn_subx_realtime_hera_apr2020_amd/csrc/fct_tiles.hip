@@ -677,7 +677,10 @@ __device__ __forceinline__ float tile_lo(const StepCtl &c, const int4 &en, int i
   return tlo;
 }
 
-// word w of a core row that the wavefront holds two words a lane
+// word w of a core row that the wavefront holds two words a lane.  Every lane
+// stays active from the load of a row to its last word (lanes above the column
+// compute on level 0's values and store nothing): a copy of the row's register
+// that the compiler makes while some lanes are off would lose their words.
 __device__ __forceinline__ int row_i(const int2 &row, int w) {
   return __builtin_amdgcn_readlane(w & 1 ? row.y : row.x, w >> 1);
 }
@@ -690,8 +693,8 @@ __device__ __forceinline__ int row_h(const int2 &row, int w0, int i) {
 
 template <int NP>
 __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, const StepCtl &c, int cell, int i, int t,
-                                          int col, size_t toff, int k, float area, const int2 &row, const TileInB &in,
-                                          const float *Str, const float *Slo) {
+                                          int col, size_t toff, int k, bool live, float area, const int2 &row,
+                                          const TileInB &in, const float *Str, const float *Slo) {
   const int nvl = g.d.nvl, ncol = s.ncol;
   float v[NP], te[NP];
   const float dp = (float)in.dp;
@@ -724,29 +727,35 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   float sp = 0.f, sm = 0.f, mx = ti, mn = ti;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
-    const float m = in.m[e];
-    const float a = m * te[e] - fct_low(m, ti, v[e]);
-    if (row_i(row, CR_NB + e) & 1) __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
-    sp = sp - fminf(0.f, a);
-    sm = sm + fmaxf(0.f, a);
     mx = fmaxf(mx, v[e]);
     mn = fminf(mn, v[e]);
   }
   mx = fmaxf(fmaxf(0.f, mx), lo);
   mn = fminf(fmaxf(0.f, mn), lo);
+  int lower = 0;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
     const float x = lds_at(Slo, row_i(row, CR_NB + e) & ~3, k);
     mx = fmaxf(mx, x);
     mn = fminf(mn, x);
+    lower |= (row_i(row, CR_NB + e) & 1) << e;
+  }
+#pragma unroll
+  for (int e = 0; e < NP; e++) {
+    const float m = in.m[e];
+    const float a = m * te[e] - fct_low(m, ti, v[e]);
+    if (((lower >> e) & 1) && live) __builtin_nontemporal_store(a, &s.antiflx[(((size_t)t * ncol + col) * NPP + e) * nvl + k]);
+    sp = sp - fminf(0.f, a);
+    sm = sm + fmaxf(0.f, a);
   }
   mx = fmaxf(0.f, mx);
   mn = fmaxf(0.f, mn);
-  __builtin_nontemporal_store(mx, &TRV(s.trmax, col));
-  __builtin_nontemporal_store(mn, &TRV(s.trmin, col));
   const float a2 = (float)c.ab2, a3 = (float)c.ab3, ra1 = (float)(1. / c.ab1) * area;
   const float qp = ((mx - lo) * dp - (a2 * fminf(0.f, in.to) + a3 * fmaxf(0.f, in.tv))) * ra1;
   const float qm = ((lo - mn) * dp + (a2 * fmaxf(0.f, in.to) + a3 * fminf(0.f, in.tv))) * ra1;
+  if (!live) return;
+  __builtin_nontemporal_store(mx, &TRV(s.trmax, col));
+  __builtin_nontemporal_store(mn, &TRV(s.trmin, col));
   __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qp * fct_rcp(fmaxf(sp, 1.e-11f)))), &TRV(s.tr_rp, col));
   __builtin_nontemporal_store(fmaxf(0.f, fminf(1.f, qm * fct_rcp(fmaxf(sm, 1.e-11f)))), &TRV(s.tr_rm, col));
 }
@@ -823,10 +832,8 @@ __global__ void __launch_bounds__(64 * NW) k_e_trcadv12(EnsGrid g, EnsState s) {
     const TileInB nb = load_b(j + 1);
     const int2 nrow = load_row(j + 1);
     const float area = lane_f(arl, j);
-    if (live) {
-      if (((z >> 16) & 0xff) == 6) tile_flux<6>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
-      else tile_flux<5>(g, s, c, cell, i, t, base + cell, toff, k, area, row, cb, Str, Slo);
-    }
+    if (((z >> 16) & 0xff) == 6) tile_flux<6>(g, s, c, cell, i, t, base + cell, toff, k, live, area, row, cb, Str, Slo);
+    else tile_flux<5>(g, s, c, cell, i, t, base + cell, toff, k, live, area, row, cb, Str, Slo);
     cb = nb;
     row = nrow;
   }

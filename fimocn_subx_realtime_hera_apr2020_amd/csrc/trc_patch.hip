@@ -46,7 +46,11 @@ __device__ __forceinline__ int lnb(const int4 &en, int e) {
 }
 __device__ __forceinline__ int enp(const int4 &en) { return (en.z >> 16) & 0xff; }
 
-struct Row { int a, b, c; };         // word 64 i + lane in the i-th
+// word 64 i + lane in the i-th.  Every lane stays active from the load of a
+// row to its last word (lanes above the column compute on level 0's values and
+// store nothing): a copy of a row's register that the compiler makes while some
+// lanes are off would lose their words.
+struct Row { int a, b, c; };
 __device__ __forceinline__ int row_i(const Row &r, int w) {
   return __builtin_amdgcn_readlane(w < 64 ? r.a : w < 128 ? r.b : r.c, w & 63);
 }
@@ -87,12 +91,13 @@ __global__ void __launch_bounds__(256) k_patch_rows(DevGrid g, EnsTiles ts, int 
   }
 }
 
-// One core cell: its row is here, its stencil's tracer in LDS.  A pentagon
+// One core cell: its row is here, its stencil's tracer in LDS; lane: of the
+// wavefront, k: its level, or 0 above the column (live).  A pentagon
 // neighbour's sixth stencil value is the neighbour's own (difference 0) with
 // coefficient 0, and PENT keeps it out of the sum.
 template <int NP, bool THETA>
-__device__ __forceinline__ void flux_col(const DevGrid &g, const DevState &s, const AB &ab, int t, int cell, int i, int k,
-                                         double rar, int pent, const Row &row, const double *Str) {
+__device__ __forceinline__ void flux_col(const DevGrid &g, const DevState &s, const AB &ab, int t, int cell, int i, int lane,
+                                         int k, bool live, double rar, int pent, const Row &row, const double *Str) {
   const int nip = g.nip, nvl = g.nvl;
   const int nf = ab.nf - 1, of = ab.of - 1, vof = ab.vof - 1;
   const size_t csz = (size_t)nip * nvl;
@@ -107,10 +112,10 @@ __device__ __forceinline__ void flux_col(const DevGrid &g, const DevState &s, co
   const double dpc = dmax(1.e-11, C2(s.dp, cell, k));
   const double td = C2(s.trdp + t * csz, cell, k), tlof = TAB(s.trl_tdcy, t, of, cell, k);
   const double tlov = TAB(s.trl_tdcy, t, vof, cell, k);
-  const double ti = Str[i * 64 + k];
+  const double ti = Str[i * 64 + lane];
   double v[NP], te[NP];
 #pragma unroll
-  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_h(row, R_NB, e), k);
+  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_h(row, R_NB, e), lane);
   if (THETA) {
 #pragma unroll
     for (int e = 0; e < NP; e++) te[e] = (2. * (ti + v[e]) + v[(e + NP - 1) % NP] + v[(e + 1) % NP]) * (1. / 6.);
@@ -122,25 +127,31 @@ __device__ __forceinline__ void flux_col(const DevGrid &g, const DevState &s, co
       for (int j = 0; j < NP; j++) own = own + (v[j] - ti) * row_d(row, R_OWN + 2 * (e * NPP + j));
 #pragma unroll
       for (int j = 0; j < NPP; j++) {
-        const double q = (lds_at(Str, row_h(row, R_ST, e * NPP + j), k) - v[e]) * row_d(row, R_NBR + 2 * (e * NPP + j));
+        const double q = (lds_at(Str, row_h(row, R_ST, e * NPP + j), lane) - v[e]) * row_d(row, R_NBR + 2 * (e * NPP + j));
         if (j < NPP - 1 || !((pent >> e) & 1)) oth = oth + q;
       }
       te[e] = 0.5 * (own + oth);
+      // formed here, not in the branch of the live lanes below, to which the
+      // compiler would move the arithmetic and keep all the row's words
+      asm volatile("" : "+v"(te[e]));
     }
   }
-  double acc = 0., sp = 0., sm = 0., mx = ti, mn = ti;
+  double af[NP], acc = 0., sp = 0., sm = 0., mx = ti, mn = ti;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
     const double flx_hi = m[e] * te[e];
     const double fl = 0.5 * ((m[e] + fabs(m[e])) * ti - (mx_[e] + fabs(mx_[e])) * v[e]);
     const double a = flx_hi - fl;
-    __builtin_nontemporal_store(a, &E3(s.antiflx + t * csz * NPP, cell, e, k));
+    af[e] = a;
     sp = sp - dmin(0., a);
     sm = sm + dmax(0., a);
     acc = acc + fl;
     mx = dmax(mx, v[e]);
     mn = dmin(mn, v[e]);
   }
+  if (!live) return;
+#pragma unroll
+  for (int e = 0; e < NP; e++) __builtin_nontemporal_store(af[e], &E3(s.antiflx + t * csz * NPP, cell, e, k));
   const double tlo = -acc * rar;
   __builtin_nontemporal_store(tlo, &TAB(s.trl_tdcy, t, nf, cell, k));
   const double trcdp_lo = td + ab.ab1 * tlo + ab.ab2 * tlof + ab.ab3 * tlov;
@@ -153,13 +164,15 @@ __device__ __forceinline__ void flux_col(const DevGrid &g, const DevState &s, co
 
 template <bool THETA>
 __device__ __forceinline__ void flux_cells(const DevGrid &g, const DevState &s, const EnsTiles &ts, const AB &ab, int t,
-                                           const int4 &ev, double rarl, int w, int n0, int k, const double *Str) {
+                                           const int4 &ev, double rarl, int w, int n0, int lane,
+                                           const double *Str) {
   const int jl = (n0 - 1 - w) / NW;
   auto load_row = [&](int j) {
-    const int *r = ts.core_row + (size_t)__builtin_amdgcn_readlane(ev.x, min(j, jl)) * ROWP + k;
+    const int *r = ts.core_row + (size_t)__builtin_amdgcn_readlane(ev.x, min(j, jl)) * ROWP + lane;
     return Row{r[0], r[64], r[128]};
   };
-  const bool live = k < g.nvl;
+  const bool live = lane < g.nvl;
+  const int k = live ? lane : 0;
   Row row = load_row(0);
   for (int i = w, j = 0; i < n0; i += NW, j++) {
     const Row nrow = load_row(j + 1);
@@ -167,10 +180,8 @@ __device__ __forceinline__ void flux_cells(const DevGrid &g, const DevState &s, 
     const long long b = __double_as_longlong(rarl);
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, j), hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), j);
     const double rar = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-    if (live) {
-      if (((z >> 16) & 0xff) == 6) flux_col<6, THETA>(g, s, ab, t, cell, i, k, rar, (z >> 24) & 0x3f, row, Str);
-      else flux_col<5, THETA>(g, s, ab, t, cell, i, k, rar, (z >> 24) & 0x3f, row, Str);
-    }
+    if (((z >> 16) & 0xff) == 6) flux_col<6, THETA>(g, s, ab, t, cell, i, lane, k, live, rar, (z >> 24) & 0x3f, row, Str);
+    else flux_col<5, THETA>(g, s, ab, t, cell, i, lane, k, live, rar, (z >> 24) & 0x3f, row, Str);
     row = nrow;
   }
 }
