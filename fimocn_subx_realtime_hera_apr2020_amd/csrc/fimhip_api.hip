@@ -331,14 +331,16 @@ extern "C" long long fimhip_field_size(const fimhip_ctx *c, int f) {
 }
 
 // edgvar1's edge fields of the last fimhip_step (u_edg, v_edg, lp_edg,
-// mont_edg, uvsq_edg and trc_edg)
-static void form_edges(fimhip_ctx *c) {
-  if (!c->edges_due) return;
-  c->edges_due = false;
+// mont_edg, uvsq_edg and trc_edg); they stay due if a launch is refused
+static int form_edges(fimhip_ctx *c) {
+  if (!c->edges_due) return 0;
   DevState t = c->s;
   t.us = c->start.us; t.vs = c->start.vs; t.pr = c->start.pr; t.mp = c->start.mp; t.tr = c->start.tr;
   launch_edgvar1(c->g, t, c->stream);
   if (c->ntra > 1) step_own_edges(c->g, t, 1, c->ntra, c->stream);
+  HIPCHK(hipGetLastError());
+  c->edges_due = false;
+  return 0;
 }
 static bool edge_field(int f) {
   return f == FIMHIP_U_EDG || f == FIMHIP_V_EDG || f == FIMHIP_LP_EDG || f == FIMHIP_MONT_EDG ||
@@ -346,12 +348,13 @@ static bool edge_field(int f) {
 }
 // before field f is written (f < 0: any field): after a step of the transport
 // alone the winds and the Montgomery potential are still those of its start
-static void before_write(fimhip_ctx *c, int f) {
-  if (!c->edges_due) return;
+static int before_write(fimhip_ctx *c, int f) {
+  if (!c->edges_due) return 0;
   const DevState &s = c->s;
   const bool us = c->start.us == s.us, vs = c->start.vs == s.vs, mp = c->start.mp == s.mp;
   if (f < 0 ? us || vs || mp : edge_field(f) || (f == FIMHIP_US && us) || (f == FIMHIP_VS && vs) || (f == FIMHIP_MP && mp))
-    form_edges(c);
+    return form_edges(c);
+  return 0;
 }
 
 static int h2d(fimhip_ctx *c, int f, const double *h) {
@@ -400,9 +403,8 @@ static int ab_out(fimhip_ctx *c, int f, double *h) { return ab_slot(c, f, h, c->
 extern "C" int fimhip_upload(fimhip_ctx *c, int f, const double *h) {
   if (!c || f < 0 || f >= FIMHIP_NFIELDS) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  before_write(c, f);
-  int r = h2d(c, f, h);
-  if (r) return r;
+  int r = before_write(c, f);
+  if (r || (r = h2d(c, f, h))) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -410,9 +412,8 @@ extern "C" int fimhip_upload(fimhip_ctx *c, int f, const double *h) {
 extern "C" int fimhip_download(fimhip_ctx *c, int f, double *h) {
   if (!c || f < 0 || f >= FIMHIP_NFIELDS) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  if (edge_field(f)) form_edges(c);
-  int r = d2h(c, f, h);
-  if (r) return r;
+  int r = edge_field(f) ? form_edges(c) : 0;
+  if (r || (r = d2h(c, f, h))) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -435,7 +436,7 @@ extern "C" int fimhip_edgvar1_r8(fimhip_ctx *c, int its, const double *u_vel, co
   (void)its; (void)delp; (void)exner; (void)geop; (void)dp_edg; (void)geop_edg;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_US, u_vel)); TRY(h2d(c, FIMHIP_VS, v_vel)); TRY(h2d(c, FIMHIP_PR, pres));
   TRY(h2d(c, FIMHIP_MP, montg)); TRY(h2d(c, FIMHIP_TR, tracr));
   // trc_edg is intent(out) for tracer 1 only; the other tracers pass through
@@ -456,7 +457,7 @@ extern "C" int fimhip_edgvar3_r8(fimhip_ctx *c, int its, const double *u_vel, co
   (void)u_edg; (void)v_edg; (void)lp_edg; (void)geop_edg; (void)mont_edg; (void)uvsq_edg;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_DP, delp)); TRY(h2d(c, FIMHIP_TR, tracr));
   TRY(h2d(c, FIMHIP_TRC_EDG, trc_edg));   // tracer 1 edges pass through
   launch_edgvar3(c->g, c->s, c->stream);
@@ -472,7 +473,7 @@ extern "C" int fimhip_cnuity_r8(fimhip_ctx *c, int its, const double *u_velo, co
   (void)its; (void)timing;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_US, u_velo)); TRY(h2d(c, FIMHIP_VS, v_velo)); TRY(h2d(c, FIMHIP_U_EDG, u_edg));
   TRY(h2d(c, FIMHIP_V_EDG, v_edg)); TRY(h2d(c, FIMHIP_DP_EDG, dp_edg)); TRY(h2d(c, FIMHIP_LP_EDG, lp_edg));
   TRY(h2d(c, FIMHIP_DP, delp)); TRY(h2d(c, FIMHIP_PR, pres)); TRY(h2d(c, FIMHIP_EX, exner));
@@ -492,7 +493,7 @@ extern "C" int fimhip_mass_adv_r8(fimhip_ctx *c, int its, const double *u_velo, 
   (void)its; (void)timing;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_US, u_velo)); TRY(h2d(c, FIMHIP_VS, v_velo)); TRY(h2d(c, FIMHIP_U_EDG, u_edg));
   TRY(h2d(c, FIMHIP_V_EDG, v_edg)); TRY(h2d(c, FIMHIP_DP_EDG, dp_edg)); TRY(h2d(c, FIMHIP_LP_EDG, lp_edg));
   TRY(h2d(c, FIMHIP_DP, delp)); TRY(h2d(c, FIMHIP_PR, pres)); TRY(h2d(c, FIMHIP_EX, exner));
@@ -510,7 +511,7 @@ extern "C" int fimhip_transp0_r8(fimhip_ctx *c, int its, double *cumufx, const d
   (void)its;
   if (!c || c->cb.ntrb < 1) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_DP, dp3d));
   launch_transp0(c->g, c->s, c->cb, c->stream);
   TRY(d2h(c, FIMHIP_CUMUFX, cumufx)); TRY(d2h(c, FIMHIP_DPINIT, dpinit));
@@ -522,7 +523,7 @@ extern "C" int fimhip_transp1_r8(fimhip_ctx *c, int its, int nf, int of, int vof
   (void)its;
   if (!c || c->cb.ntrb < 1 || nf < 1 || nf > 3 || of < 1 || of > 3 || vof < 1 || vof > 3) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_CUMUFX, cumufx)); TRY(h2d(c, FIMHIP_MASSFX, massfx));
   launch_transp1(c->g, c->s, c->cb, AB{nf, of, vof, adbash1, adbash2, adbash3}, c->stream);
   TRY(d2h(c, FIMHIP_CUMUFX, cumufx));
@@ -534,7 +535,7 @@ extern "C" int fimhip_transp2_r8(fimhip_ctx *c, int its, double *tracr, const do
   (void)its; (void)timing;
   if (!c || c->cb.ntrb < 1 || !tracr) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   const size_t tz = (size_t)c->nip * c->nvl * c->cb.ntrb;
   double *trb_host = tracr + (size_t)c->nip * c->nvl * c->ntra;
   HIPCHK(hipMemcpyAsync(c->cb.trb, trb_host, tz * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -550,7 +551,7 @@ extern "C" int fimhip_trcadv_r8(fimhip_ctx *c, int its, const double *trcr_edg, 
   (void)its; (void)timing;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_TRC_EDG, trcr_edg)); TRY(h2d(c, FIMHIP_TR, tracr)); TRY(h2d(c, FIMHIP_TRDP, trcdp));
   TRY(ab_in(c, FIMHIP_TRC_TDCY, trc_tdcy)); TRY(ab_in(c, FIMHIP_TRL_TDCY, trclo_tdcy));
   TRY(ab_nf_in(c, FIMHIP_MASSFX, massfx)); TRY(h2d(c, FIMHIP_DP, delp));
@@ -567,7 +568,7 @@ extern "C" int fimhip_momtum_r8(fimhip_ctx *c, int its, double *u_velo, double *
   (void)its; (void)geop_edg;
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_US, u_velo)); TRY(h2d(c, FIMHIP_VS, v_velo)); TRY(h2d(c, FIMHIP_EX, exner));
   TRY(h2d(c, FIMHIP_U_EDG, u_edg)); TRY(h2d(c, FIMHIP_V_EDG, v_edg)); TRY(h2d(c, FIMHIP_TRC_EDG, trcr_edg));
   TRY(h2d(c, FIMHIP_MONT_EDG, mont_edg)); TRY(h2d(c, FIMHIP_UVSQ_EDG, uvsq_edg));
@@ -584,7 +585,7 @@ extern "C" int fimhip_hybgen_r8(fimhip_ctx *c, int its, const double *targt, dou
   (void)timing;
   if (!c || !targt) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   HIPCHK(hipMemcpyAsync((void *)c->g.thetac, targt, c->nvl * sizeof(double), hipMemcpyHostToDevice, c->stream));
   TRY(h2d(c, FIMHIP_US, us3d)); TRY(h2d(c, FIMHIP_VS, vs3d)); TRY(h2d(c, FIMHIP_TR, tr3d));
   TRY(h2d(c, FIMHIP_EX, ex3d)); TRY(h2d(c, FIMHIP_DP, dp3d)); TRY(h2d(c, FIMHIP_PR, pr3d));
@@ -599,7 +600,7 @@ extern "C" int fimhip_hystat_r8(fimhip_ctx *c, int its, double *ph3d, const doub
                                 const double *dp3d, double *tr3d, double *trdp, double *psrf, double *ptdcy) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  form_edges(c);
+  TRY(form_edges(c));
   TRY(h2d(c, FIMHIP_PH, ph3d)); TRY(h2d(c, FIMHIP_EX, ex3d)); TRY(h2d(c, FIMHIP_DP, dp3d));
   TRY(h2d(c, FIMHIP_TR, tr3d)); TRY(h2d(c, FIMHIP_PSRF, psrf)); TRY(h2d(c, FIMHIP_PTDCY, ptdcy));
   launch_hystat(c->g, c->s, its, c->stream);
@@ -785,7 +786,7 @@ extern "C" int fimhip_transp2_r4(fimhip_ctx *c, int its, float *tracr, float *cu
 extern "C" int fimhip_init_state(fimhip_ctx *c, int init_hybgen) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  before_write(c, -1);
+  TRY(before_write(c, -1));
   launch_trdp(c->g, c->s, c->stream);
   if (init_hybgen) {
     launch_hybgen(c->g, c->s, 0, c->stream);
@@ -1060,7 +1061,7 @@ int synth_into(int nip, int nvl, int ntra, const double *lat, const double *lon,
 extern "C" int fimhip_synth_device(fimhip_ctx *c, unsigned long long seed, int member, int flags) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  before_write(c, -1);
+  TRY(before_write(c, -1));
   return synth_into(c->nip, c->nvl, c->ntra, c->lat.data(), c->lon.data(), seed, member, flags, c->s, c->stream);
 }
 
