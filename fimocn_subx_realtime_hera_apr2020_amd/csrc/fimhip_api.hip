@@ -330,10 +330,16 @@ extern "C" long long fimhip_field_size(const fimhip_ctx *c, int f) {
   return FIMHIP_EINVAL;
 }
 
+struct TimerScope {
+  explicit TimerScope(KTimer *t) { g_ktimer = t; }
+  ~TimerScope() { g_ktimer = nullptr; }
+};
+
 // edgvar1's edge fields of the last fimhip_step (u_edg, v_edg, lp_edg,
 // mont_edg, uvsq_edg and trc_edg); they stay due if a launch is refused
 static int form_edges(fimhip_ctx *c) {
   if (!c->edges_due) return 0;
+  const TimerScope scope(c->kt);
   DevState t = c->s;
   t.us = c->start.us; t.vs = c->start.vs; t.pr = c->start.pr; t.mp = c->start.mp; t.tr = c->start.tr;
   launch_edgvar1(c->g, t, c->stream);
@@ -346,14 +352,18 @@ static bool edge_field(int f) {
   return f == FIMHIP_U_EDG || f == FIMHIP_V_EDG || f == FIMHIP_LP_EDG || f == FIMHIP_MONT_EDG ||
          f == FIMHIP_UVSQ_EDG || f == FIMHIP_TRC_EDG;
 }
-// before field f is written (f < 0: any field): after a step of the transport
-// alone the winds and the Montgomery potential are still those of its start
+// Before field f is written from outside the step.  After a step of the
+// transport alone the winds and the Montgomery potential are still those of its
+// start, from which the due edge fields are formed: a field that is written
+// whole goes to its other buffer instead (forming the edge fields for it would
+// cost a third of such a step, and most callers never ask for them).
 static int before_write(fimhip_ctx *c, int f) {
   if (!c->edges_due) return 0;
-  const DevState &s = c->s;
-  const bool us = c->start.us == s.us, vs = c->start.vs == s.vs, mp = c->start.mp == s.mp;
-  if (f < 0 ? us || vs || mp : edge_field(f) || (f == FIMHIP_US && us) || (f == FIMHIP_VS && vs) || (f == FIMHIP_MP && mp))
-    return form_edges(c);
+  if (edge_field(f)) return form_edges(c);
+  DevState &s = c->s;
+  if (f == FIMHIP_US && s.us == c->start.us) std::swap(s.us, s.u2);
+  if (f == FIMHIP_VS && s.vs == c->start.vs) std::swap(s.vs, s.v2);
+  if (f == FIMHIP_MP && s.mp == c->start.mp) std::swap(s.mp, s.mp_alt);
   return 0;
 }
 
@@ -403,6 +413,7 @@ static int ab_out(fimhip_ctx *c, int f, double *h) { return ab_slot(c, f, h, c->
 extern "C" int fimhip_upload(fimhip_ctx *c, int f, const double *h) {
   if (!c || f < 0 || f >= FIMHIP_NFIELDS) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  if (!h || !*field_ptr(c, f)) return FIMHIP_EINVAL;
   int r = before_write(c, f);
   if (r || (r = h2d(c, f, h))) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -786,7 +797,8 @@ extern "C" int fimhip_transp2_r4(fimhip_ctx *c, int its, float *tracr, float *cu
 extern "C" int fimhip_init_state(fimhip_ctx *c, int init_hybgen) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  TRY(before_write(c, -1));
+  if (init_hybgen && (c->start.us == c->s.us || c->start.vs == c->s.vs)) TRY(form_edges(c));   // moved in place
+  TRY(before_write(c, FIMHIP_MP));
   launch_trdp(c->g, c->s, c->stream);
   if (init_hybgen) {
     launch_hybgen(c->g, c->s, 0, c->stream);
@@ -810,10 +822,7 @@ extern "C" int fimhip_init_state(fimhip_ctx *c, int init_hybgen) {
 extern "C" int fimhip_step(fimhip_ctx *c, int its, int mode) {
   if (!c || its < 1 || (mode != 0 && mode != 1)) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  struct TimerScope {
-    explicit TimerScope(KTimer *t) { g_ktimer = t; }
-    ~TimerScope() { g_ktimer = nullptr; }
-  } scope(c->kt);
+  const TimerScope scope(c->kt);
   ab_rotate(c->ab, its, c->dt);
   const DevState &s = c->s;
   c->start = {s.us, s.vs, s.pr, s.mp, s.tr};
@@ -1061,8 +1070,14 @@ int synth_into(int nip, int nvl, int ntra, const double *lat, const double *lon,
 extern "C" int fimhip_synth_device(fimhip_ctx *c, unsigned long long seed, int member, int flags) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  TRY(before_write(c, -1));
-  return synth_into(c->nip, c->nvl, c->ntra, c->lat.data(), c->lon.data(), seed, member, flags, c->s, c->stream);
+  // winds that the due edge fields are formed from stay in their buffers
+  DevState &s = c->s, d = s;
+  if (c->edges_due && s.us == c->start.us) d.us = s.u2;
+  if (c->edges_due && s.vs == c->start.vs) d.vs = s.v2;
+  TRY(synth_into(c->nip, c->nvl, c->ntra, c->lat.data(), c->lon.data(), seed, member, flags, d, c->stream));
+  if (d.us != s.us) std::swap(s.us, s.u2);
+  if (d.vs != s.vs) std::swap(s.vs, s.v2);
+  return FIMHIP_OK;
 }
 
 extern "C" int fimhip_profile(fimhip_ctx *c, int on) {

@@ -803,3 +803,47 @@ def test_edge_fields_formed_when_asked_for(oracle_lib, mode, flux_scheme, nvl):
             same_edges(m)
         finally:
             m.close()
+
+
+def test_winds_written_each_step_form_no_edge_fields(oracle_lib):
+    """A transport driven by winds from outside (uploaded, or seeded again,
+    before each step) forms no edge field that nobody asks for, and those
+    that are asked for are the last step's."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip
+    from helpers import seeded_case
+    O = oracle_lib
+    g, st, th, ds = seeded_case(3)
+    o = O.OracleRun(O.grid_arrays(g, NVL, DT, th, ds), NVL, NTRA, DT, pow_kind=1)
+    o.load(st)
+    o.init(True)
+    m = fimhip.Model(g, NVL, NTRA, DT, th, ds)
+    live = (np.arange(6)[None, :] < g.nprox[:, None])[:, :, None]
+    try:
+        m.load(st)
+        m.init_state(True)
+        m.profile(True)
+        us, vs, mp = m.download("us"), m.download("vs"), m.download("mp")
+        for its in range(1, 5):
+            o.step(its, 1)
+            m.step(its, 1)
+            for f, a in (("us", us), ("vs", vs), ("mp", mp)):
+                w = a * (1. + .01 * its)
+                o.a[f][...] = w.reshape(o.a[f].shape)
+                m.upload(f, w)
+            if its == 3:
+                m.upload("us", us * (1. + .01 * its))      # twice in a row
+        assert m.profile_report()["k_edgvar1"][0] == 4
+        for f in ("dp", "pr", "tr", "trdp", "us", "vs", "mp"):
+            assert _same(m.download(f), o.a[f]), f
+        for f in ("u_edg", "v_edg", "lp_edg", "mont_edg", "uvsq_edg"):
+            assert _same(m.download(f) * live, o.a[f].reshape(m.shape(f)) * live), f
+        assert m.profile_report()["k_edgvar1"][0] == 5
+        m.step(5, 1)
+        m.synth(seed=3)
+        m.init_state(False)
+        assert m.profile_report()["k_edgvar1"][0] == 6
+        o.step(5, 1)
+        for f in ("u_edg", "v_edg", "lp_edg", "mont_edg", "uvsq_edg"):
+            assert _same(m.download(f) * live, o.a[f].reshape(m.shape(f)) * live), f
+    finally:
+        m.close()
