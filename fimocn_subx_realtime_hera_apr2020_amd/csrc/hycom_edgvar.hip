@@ -424,6 +424,9 @@ static int edg_launch(fimhip_ocn *o, int leapm, int leapn) {
   o->e_leapm = leapm;
   o->e_leapn = leapn;
   o->e_dp_old = o->e_uv_old = false;
+  HycEdg &ed = o->ed;
+  ed.uclin_e = ed.uclin; ed.vclin_e = ed.vclin; ed.utrop_e = ed.utrop; ed.vtrop_e = ed.vtrop;
+  ed.montg_e = ed.montg; ed.spcifv_e = ed.spcifv;
   HIPCHK(hipGetLastError());
   return FIMHIP_OK;
 }
@@ -432,12 +435,13 @@ template <int LPC>
 static void form_kernels(fimhip_ocn *o) {
   const HycGrid &g = o->g;
   const HycState &s = o->s;
-  const HycEdg &ed = o->ed;
+  HycEdg ed = o->ed;
+  ed.utrop = ed.utrop_e; ed.vtrop = ed.vtrop_e; ed.montg = ed.montg_e; ed.spcifv = ed.spcifv_e;
   hipStream_t st = o->stream;
   const dim3 grid(ocn_blocks(o, LPC)), blk(256);
   const size_t cz = (size_t)o->nip * o->kdm, om = (o->e_leapm - 1) * cz, on = (o->e_leapn - 1) * cz;
   const double *dpm = o->e_dp_old ? s.dpe : s.dp + om;
-  const double *u = o->e_uv_old ? ed.uclin_alt : ed.uclin, *v = o->e_uv_old ? ed.vclin_alt : ed.vclin;
+  const double *u = ed.uclin_e, *v = ed.vclin_e;
   KT_LAUNCH("hyc_uvedge", st, hyc_uvedge<LPC><<<grid, blk, 0, st>>>(g, ed, u + om, v + om, o->e_leapm, s.um, s.vm, dpm,
                                                                     s.p0e, o->pres_f, ed.uvsq_edg));
   KT_LAUNCH("hyc_uvedge", st, hyc_uvedge<LPC><<<grid, blk, 0, st>>>(g, ed, u + on, v + on, o->e_leapn, s.un, s.vn,

@@ -534,7 +534,7 @@ static int hyb_launch(fimhip_ocn *o, int leap, int with_tracers) {
   if (with_tracers && o->tr.numtr <= 0) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
   // the thickness and the velocities are written in place
-  if (!o->e_dp_old || !o->e_uv_old) {
+  if (!o->e_dp_old || o->ed.uclin == o->ed.uclin_e || o->ed.vclin == o->ed.vclin_e) {
     const int r = ocn_form_edges(o);
     if (r) return r;
   }

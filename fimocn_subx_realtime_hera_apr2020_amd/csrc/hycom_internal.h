@@ -146,6 +146,10 @@ __device__ __forceinline__ double col_sums6(double (*buf)[LPC + 1], const double
 struct HycEdg {
   double *uclin, *vclin, *utrop, *vtrop, *geop, *montg, *spcifv;
   double *uclin_alt, *vclin_alt;   // momtum writes the new velocities here and the pairs are swapped
+  // the inputs as the last edge interpolation saw them: these arrays or, once
+  // the host has uploaded others since, their other buffers
+  double *uclin_e, *vclin_e, *utrop_e, *vtrop_e, *montg_e, *spcifv_e;
+  double *utrop_alt, *vtrop_alt, *montg_alt, *spcifv_alt;   // allocated by the first such upload
   double *pr_edg, *geop_edg, *mont_edg, *uvsq_edg, *spcv_edg;
 };
 
@@ -210,7 +214,7 @@ struct fimhip_ocn {
   // of them is asked for, from the values of that call:
   bool edges_due = false;            // the public edge arrays are older than the last edgvar
   int e_leapm = 0, e_leapn = 0;      // its levels
-  bool e_dp_old = false;             // cnuity has run since: its mid-time thickness is in s.dpe
+  bool e_dp_old = false;             // the thickness has changed since: the mid-time one is kept in s.dpe
   bool e_uv_old = false;             // momtum has run since: its velocities are in the alt pair
   bool alt_stale = false;            // the alt pair's land values miss an upload
   double *pres_f = nullptr;          // (kdm+1,nip) interfaces of the forming
@@ -225,8 +229,8 @@ double *ocn_field(fimhip_ocn *o, int f, size_t *n);
 // the public edge arrays, if they are due (hycom_edgvar.hip)
 int ocn_form_edges(fimhip_ocn *o);
 // a whole field to or from the host on the instance's stream, with the edge
-// arrays formed first where the transfer would read them or replace what they
-// are formed from
+// arrays formed first where the transfer would read or replace one; an input
+// they are formed from goes to its other buffer
 int ocn_put(fimhip_ocn *o, int f, const double *h);
 int ocn_get(fimhip_ocn *o, int f, double *h);
 // blocks of a launch over all cells with LPC lanes per column (a multiple of 8)

@@ -81,8 +81,8 @@ __device__ __forceinline__ UV col_total2(double (*buf)[LPC + 1], double u, doubl
 }
 // EDGES: the edge values are the public arrays' (an uploaded state);
 // otherwise they are formed here from the cells, from the values
-// fimhip_ocn_edgvar saw (dpe the mid-time thickness; the velocities have not
-// changed since), which costs less than storing and reading five edge arrays.
+// fimhip_ocn_edgvar saw (dpe the mid-time thickness, the arrays named _e; the
+// velocities have not changed since), which costs less than storing and reading five edge arrays.
 // Bound by memory (six cell arrays gathered at the neighbours) and, nearly as
 // much, by the FP64 expressions of the edges: cells away from the coast run
 // them without the coast's selections.
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256, 4) hyc_mom_pgf(HycGrid g, HycState s, Hyc
                          : 0.;
   }
   double tv = 0., bv = 0.;
-  if (!EDGES && k < 2 * NC) tv = (k < NC ? ed.utrop : ed.vtrop)[(k % NC == 0 ? i : g.prox[i * NPP + k % NC - 1]) * 3 + leapm - 1];
+  if (!EDGES && k < 2 * NC) tv = (k < NC ? ed.utrop_e : ed.vtrop_e)[(k % NC == 0 ? i : g.prox[i * NPP + k % NC - 1]) * 3 + leapm - 1];
   if (!EDGES && k < NPP) bv = s.pbe[g.prox[i * NPP + k]];
   const double di = live ? HC(s.dp + on, i, k) : 0., dm = live ? HC(s.dp + om, i, k) : 0.;
   const double de = !EDGES && live ? HC(dpe, i, k) : 0.;
@@ -260,12 +260,12 @@ __global__ void __launch_bounds__(256, 4) hyc_mom_pgf(HycGrid g, HycState s, Hyc
         }
       } else {
         double PB[NPP], M[NPP], SV[NPP], nm[NPP], ns[NPP];
-        const double mi = HC(ed.montg, i, k), svi = HC(ed.spcifv, i, k);
+        const double mi = HC(ed.montg_e, i, k), svi = HC(ed.spcifv_e, i, k);
 #pragma unroll
         for (int e = 0; e < NPP; e++) {
           PB[e] = sbot[cc][e];
-          M[e] = HC(ed.montg, nb[e], k);
-          SV[e] = HC(ed.spcifv, nb[e], k);
+          M[e] = HC(ed.montg_e, nb[e], k);
+          SV[e] = HC(ed.spcifv_e, nb[e], k);
         }
         sidewall(cj, de, pr.pe, PB, mi, M, svi, SV, nm, ns);
         __builtin_amdgcn_sched_barrier(0);
@@ -465,13 +465,13 @@ static int mom_launch(fimhip_ocn *o, int leapm, int leapn) {
   if (leapm < 1 || leapm > 2 || leapn < 1 || leapn > 2 || leapm == leapn) return FIMHIP_EINVAL;
   if (!(o->mo.batrop > 0.)) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
-  // a second momtum since the edge interpolation, or one at other levels, is
-  // one on the arrays themselves
-  if (o->e_uv_old || leapm != o->e_leapm) {
+  HycEdg &ed = o->ed;
+  // a second momtum since the edge interpolation, one at other levels, or one
+  // on other velocities, is one on the arrays themselves
+  if (o->e_uv_old || leapm != o->e_leapm || ed.uclin != ed.uclin_e || ed.vclin != ed.vclin_e) {
     const int r = ocn_form_edges(o);
     if (r) return r;
   }
-  HycEdg &ed = o->ed;
   if (o->alt_stale) {       // land keeps its velocities: the other pair needs them too
     const size_t n = 2 * (size_t)o->nip * o->kdm * sizeof(double);
     HIPCHK(hipMemcpyAsync(ed.uclin_alt, ed.uclin, n, hipMemcpyDeviceToDevice, o->stream));

@@ -678,3 +678,58 @@ def test_edge_arrays_formed_when_asked_for(oracle_lib, then, janjic, kdm):
             assert _same(o.download(n), h.e[n]), n
     finally:
         o.close()
+
+
+@pytest.mark.parametrize("at", ["before edgvar", "before cnuity", "before momtum", "after momtum", "each"])
+def test_inputs_uploaded_each_step_form_no_edge_arrays(oracle_lib, at):
+    """A host that uploads the edge interpolation's inputs once a step pays for
+    no edge array that nobody asks for; the step uses, and a download gives,
+    the values that fimhip_ocn_edgvar saw."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, ocean
+    print("case: G3 x 24, inputs uploaded %s" % at, flush=True)
+    g = _grid(3)
+    case = ocean.hycom_ocean_case(g, kdm=24, seed=11, numtr=1)
+    h = oracle_lib.HycomCnuity(g, case)
+    o = fimhip.Ocean(g, 24, case["wet"], case["dtleap"])
+    try:
+        o.set_momtum(case["batrop"], case["veldff"], case["smagcf"])
+        for n in fimhip.OCN_MOMTUM_FIELDS:
+            o.upload(n, case[n])
+        o.profile(True)
+        places = ("before edgvar", "before cnuity", "before momtum", "after momtum")
+
+        def host(place, st):
+            if at not in (place, "each"):
+                return
+            for j, n in enumerate(("utrop", "vtrop", "montg", "spcifv")):
+                if at == "each" and (j + st) % 4 != places.index(place):
+                    continue
+                h.e[n][...] = (1. + 1e-4 * st) * np.asarray(case[n]).reshape(h.e[n].shape)
+                o.upload(n, h.e[n])
+
+        h.edgvar(g, 2, 1, False)
+        o.step_edgvar(2, 1)
+        for st in range(1, 7):
+            m = 1 + st % 2
+            n = 3 - m
+            host(places[0], st)
+            h.edgvar(g, m, n, False)
+            o.step_edgvar(m, n)
+            host(places[1], st)
+            assert h.step(st, m, n) == 0
+            o.step(st, m, n)
+            host(places[2], st)
+            h.momtum(g, m, n, False)
+            o.step_momtum(m, n)
+            host(places[3], st)
+        ran = o.profile_report()
+        assert "hyc_edgint_full" not in ran and "hyc_uvedge" not in ran and ran["hyc_vnorm"][0] == 7
+        for n in ARRAYS:
+            assert _same(o.download(n), h.a[n]), n
+        for n in ("uclin", "vclin", "ustarb", "utrop", "vtrop", "montg", "spcifv"):
+            assert _same(o.download(n), h.e[n]), n
+        got = {n: o.download(n) for n in EDG_CHECK[:5] + tuple(h.EDG_OUT)}
+        got["pres"] = o.download("pres")
+        _edg_same(h, got, at)
+    finally:
+        o.close()
