@@ -191,11 +191,12 @@ __global__ void __launch_bounds__(256, 5) hyc_vnorm(HycGrid g, HycState s, HycEd
 }
 
 // the public edge velocities of leapfrog level 'slot' from the velocities uc,
-// vc; with dpm, the interfaces of that thickness into pres (index 0 unused)
+// vc; with dpm, the interfaces of that thickness from the top one, p0[i * p0s],
+// into pres (whose top interface stays) and, with pbe, its bottom
 template <int LPC>
 __global__ void __launch_bounds__(256) hyc_uvedge(HycGrid g, HycEdg ed, const double *uc, const double *vc, int slot,
-                                                  double *ue, double *ve, const double *dpm, const double *p0e,
-                                                  double *pres, double *uvsq) {
+                                                  double *ue, double *ve, const double *dpm, const double *p0,
+                                                  int p0s, double *pres, double *pbe, double *uvsq) {
   __shared__ double sh[256 / LPC][LPC + 1];
   __shared__ double tab[256 / LPC][VT_SVE];     // the cell's cs then sn, (4,6) each
   const int kdm = g.kdm, nip = g.nip;
@@ -229,8 +230,9 @@ __global__ void __launch_bounds__(256) hyc_uvedge(HycGrid g, HycEdg ed, const do
     vx[e] = wx ? b : H_LAND;
   }
   if (dpm && wi) {
-    const double p = col_pres(sh[c.cc], live ? HC(dpm, i, k) : 0., p0e[i], k, kdm);
+    const double p = col_pres(sh[c.cc], live ? HC(dpm, i, k) : 0., p0[(size_t)i * p0s], k, kdm);
     if (live) pres[(size_t)i * (kdm + 1) + k + 1] = p;
+    if (pbe && k == kdm - 1) pbe[i] = p;
   }
 #pragma unroll
   for (int q = 0; q < NRL; q++)
@@ -407,53 +409,65 @@ static void edg_kernels(fimhip_ocn *o, int leapm, int leapn) {
   hipStream_t st = o->stream;
   const dim3 grid(ocn_blocks(o, LPC)), blk(256);
   const double *dpm = s.dp + (size_t)(leapm - 1) * o->nip * o->kdm;
-  if (o->janjic) KT_LAUNCH("hyc_janjic", st, hyc_janjic<LPC><<<grid, blk, 0, st>>>(g, s, ed));
   KT_LAUNCH("hyc_vnorm", st, hyc_vnorm<LPC><<<grid, blk, 0, st>>>(g, s, ed, leapm, leapn));
   KT_LAUNCH("hyc_edgint", st, (hyc_edgint<LPC, false><<<grid, blk, 0, st>>>(g, s, ed, dpm, nullptr)));
 }
 
-// bclin_edgvar on the device-resident arrays (hycom_edgvar.F90:128-478)
-static int edg_launch(fimhip_ocn *o, int leapm, int leapn) {
-  if (leapm < 1 || leapm > 2 || leapn < 1 || leapn > 2 || leapm == leapn) return FIMHIP_EINVAL;
-  HIPCHK(hipSetDevice(o->device));
-  g_ktimer = o->kt;
-  if (o->kdm <= 32) edg_kernels<32>(o, leapm, leapn);
-  else edg_kernels<64>(o, leapm, leapn);
-  g_ktimer = nullptr;
-  o->edges_due = true;
-  o->e_leapm = leapm;
-  o->e_leapn = leapn;
-  o->e_dp_old = o->e_uv_old = false;
-  HycEdg &ed = o->ed;
-  ed.uclin_e = ed.uclin; ed.vclin_e = ed.vclin; ed.utrop_e = ed.utrop; ed.vtrop_e = ed.vtrop;
-  ed.montg_e = ed.montg; ed.spcifv_e = ed.spcifv;
-  HIPCHK(hipGetLastError());
-  return FIMHIP_OK;
-}
-
+// the public edge arrays of the instance's current values (now), or of those
+// that the last hyc_vnorm saw
 template <int LPC>
-static void form_kernels(fimhip_ocn *o) {
+static void form_kernels(fimhip_ocn *o, int leapm, int leapn, bool now) {
   const HycGrid &g = o->g;
   const HycState &s = o->s;
   HycEdg ed = o->ed;
+  ed.uclin = ed.uclin_e; ed.vclin = ed.vclin_e;
   ed.utrop = ed.utrop_e; ed.vtrop = ed.vtrop_e; ed.montg = ed.montg_e; ed.spcifv = ed.spcifv_e;
   hipStream_t st = o->stream;
   const dim3 grid(ocn_blocks(o, LPC)), blk(256);
-  const size_t cz = (size_t)o->nip * o->kdm, om = (o->e_leapm - 1) * cz, on = (o->e_leapn - 1) * cz;
-  const double *dpm = o->e_dp_old ? s.dpe : s.dp + om;
-  const double *u = ed.uclin_e, *v = ed.vclin_e;
-  KT_LAUNCH("hyc_uvedge", st, hyc_uvedge<LPC><<<grid, blk, 0, st>>>(g, ed, u + om, v + om, o->e_leapm, s.um, s.vm, dpm,
-                                                                    s.p0e, o->pres_f, ed.uvsq_edg));
-  KT_LAUNCH("hyc_uvedge", st, hyc_uvedge<LPC><<<grid, blk, 0, st>>>(g, ed, u + on, v + on, o->e_leapn, s.un, s.vn,
-                                                                    nullptr, nullptr, nullptr, nullptr));
-  KT_LAUNCH("hyc_edgint_full", st, (hyc_edgint<LPC, true><<<grid, blk, 0, st>>>(g, s, ed, dpm, o->pres_f)));
+  const size_t cz = (size_t)o->nip * o->kdm, om = (leapm - 1) * cz, on = (leapn - 1) * cz;
+  const double *dpm = !now && o->e_dp_old ? s.dpe : s.dp + om;
+  double *pres = now ? s.pres : o->pres_f;
+  KT_LAUNCH("hyc_uvedge", st, hyc_uvedge<LPC><<<grid, blk, 0, st>>>(g, ed, ed.uclin + om, ed.vclin + om, leapm, s.um, s.vm,
+                                                                    dpm, now ? s.pres : s.p0e, now ? o->kdm + 1 : 1,
+                                                                    pres, now ? s.pbe : nullptr, ed.uvsq_edg));
+  KT_LAUNCH("hyc_uvedge", st, hyc_uvedge<LPC><<<grid, blk, 0, st>>>(g, ed, ed.uclin + on, ed.vclin + on, leapn, s.un, s.vn,
+                                                                    nullptr, nullptr, 0, nullptr, nullptr, nullptr));
+  KT_LAUNCH("hyc_edgint_full", st, (hyc_edgint<LPC, true><<<grid, blk, 0, st>>>(g, s, ed, dpm, pres)));
+}
+
+template <int LPC>
+static void janjic_kernel(fimhip_ocn *o) {
+  const dim3 grid(ocn_blocks(o, LPC)), blk(256);
+  KT_LAUNCH("hyc_janjic", o->stream, hyc_janjic<LPC><<<grid, blk, 0, o->stream>>>(o->g, o->s, o->ed));
+}
+
+// bclin_edgvar on the device-resident arrays (hycom_edgvar.F90:128-478); full:
+// with the public edge arrays at once, for a caller that takes them all
+static int edg_launch(fimhip_ocn *o, int leapm, int leapn, bool full) {
+  if (leapm < 1 || leapm > 2 || leapn < 1 || leapn > 2 || leapm == leapn) return FIMHIP_EINVAL;
+  HIPCHK(hipSetDevice(o->device));
+  HycEdg &ed = o->ed;
+  ed.uclin_e = ed.uclin; ed.vclin_e = ed.vclin; ed.utrop_e = ed.utrop; ed.vtrop_e = ed.vtrop;
+  ed.montg_e = ed.montg; ed.spcifv_e = ed.spcifv;
+  const bool l32 = o->kdm <= 32;
+  g_ktimer = o->kt;
+  if (o->janjic) l32 ? janjic_kernel<32>(o) : janjic_kernel<64>(o);
+  if (full) l32 ? form_kernels<32>(o, leapm, leapn, true) : form_kernels<64>(o, leapm, leapn, true);
+  else l32 ? edg_kernels<32>(o, leapm, leapn) : edg_kernels<64>(o, leapm, leapn);
+  g_ktimer = nullptr;
+  o->edges_due = !full;
+  o->e_leapm = leapm;
+  o->e_leapn = leapn;
+  o->e_dp_old = o->e_uv_old = false;
+  HIPCHK(hipGetLastError());
+  return FIMHIP_OK;
 }
 
 int ocn_form_edges(fimhip_ocn *o) {
   if (!o->edges_due) return FIMHIP_OK;
   g_ktimer = o->kt;
-  if (o->kdm <= 32) form_kernels<32>(o);
-  else form_kernels<64>(o);
+  if (o->kdm <= 32) form_kernels<32>(o, o->e_leapm, o->e_leapn, false);
+  else form_kernels<64>(o, o->e_leapm, o->e_leapn, false);
   g_ktimer = nullptr;
   o->edges_due = false;
   HIPCHK(hipGetLastError());
@@ -470,7 +484,7 @@ extern "C" int fimhip_ocn_set_janjic(fimhip_ocn *o, int on) {
 // profile report that follows waits for it
 extern "C" int fimhip_ocn_edgvar(fimhip_ocn *o, int leapm, int leapn) {
   if (!o) return FIMHIP_EINVAL;
-  return edg_launch(o, leapm, leapn);
+  return edg_launch(o, leapm, leapn, false);
 }
 
 extern "C" int fimhip_ocn_edgvar_r8(fimhip_ocn *o, int nstep, int leapm, int leapn, const double *uclin,
@@ -493,7 +507,7 @@ extern "C" int fimhip_ocn_edgvar_r8(fimhip_ocn *o, int nstep, int leapm, int lea
   int r = 0;
   for (int j = 0; j < nin; j++)
     if ((r = ocn_put(o, fi[j], in[j]))) return r;
-  if ((r = edg_launch(o, leapm, leapn))) return r;
+  if ((r = edg_launch(o, leapm, leapn, true))) return r;
   double *outp[] = {pres, um_edg, vm_edg, un_edg, vn_edg, dp_edg, pr_edg, mont_edg, uvsq_edg, spcv_edg, geop_edg};
   const int fo[] = {FIMHIP_OCN_PRES, FIMHIP_OCN_UM_EDG, FIMHIP_OCN_VM_EDG, FIMHIP_OCN_UN_EDG, FIMHIP_OCN_VN_EDG,
                     FIMHIP_OCN_DPM_EDG, FIMHIP_OCN_PR_EDG, FIMHIP_OCN_MONT_EDG, FIMHIP_OCN_UVSQ_EDG,

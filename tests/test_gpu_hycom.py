@@ -733,3 +733,41 @@ def test_inputs_uploaded_each_step_form_no_edge_arrays(oracle_lib, at):
         _edg_same(h, got, at)
     finally:
         o.close()
+
+
+@pytest.mark.parametrize("before", ["nothing", "resident"])
+def test_edgvar_dropin_forms_each_array_once(oracle_lib, before):
+    """The drop-in takes every edge array, so it forms them directly; what the
+    resident edge interpolation forms for the steps alone is not formed
+    beside them.  The resident steps that follow use its arrays."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, ocean
+    print("case: G3 x 40, edgvar drop-in after %s" % before, flush=True)
+    g = _grid(3)
+    case = ocean.hycom_ocean_case(g, kdm=40, seed=23, numtr=1)
+    h = oracle_lib.HycomCnuity(g, case)
+    o = fimhip.Ocean(g, 40, case["wet"], case["dtleap"])
+    try:
+        o.set_momtum(case["batrop"], case["veldff"], case["smagcf"])
+        for n in fimhip.OCN_MOMTUM_FIELDS:
+            o.upload(n, case[n])
+        if before == "resident":
+            o.step_edgvar(2, 1)
+        a = {n: np.ascontiguousarray(case[n], np.float64).copy() for n in fimhip.OCN_EDGVAR_FIELDS}
+        o.profile(True)
+        h.edgvar(g, 2, 1, False)
+        o.edgvar(1, 2, 1, a["uclin"], a["vclin"], a["utrop"], a["vtrop"], a["dp"], a["pres"], a["geop"], a["montg"],
+                 a["spcifv"], a["um_edg"], a["vm_edg"], a["un_edg"], a["vn_edg"], a["dpm_edg"], a["pr_edg"],
+                 a["geop_edg"], a["mont_edg"], a["uvsq_edg"], a["spcv_edg"])
+        ran = {n: v[0] for n, v in o.profile_report().items()}
+        assert ran == {"hyc_uvedge": 2, "hyc_edgint_full": 1}
+        _edg_same(h, a, before)
+        assert h.step(1, 2, 1) == 0
+        o.step(1, 2, 1)
+        h.momtum(g, 2, 1, False)
+        o.step_momtum(2, 1)
+        for n in ARRAYS:
+            assert _same(o.download(n), h.a[n]), n
+        for n in ("uclin", "vclin", "ustarb"):
+            assert _same(o.download(n), h.e[n]), n
+    finally:
+        o.close()
