@@ -59,7 +59,8 @@ struct fimhip_ctx {
   // or before something else writes what they are formed from.
   bool edges_due = false;
   struct { double *us, *vs, *pr, *mp, *tr; } start{};
-  EnsTiles tiles{};                  // patches of trcadv1 in fimhip_step
+  HostGrid hg;                       // neighbour tables, until the patches are built
+  EnsTiles tiles{};                  // patches of trcadv1 in fimhip_step (step_prepare)
 };
 
 // dyn_init.F90:125 taper for smoo_coeff
@@ -165,20 +166,22 @@ extern "C" int fimhip_create(const fimhip_grid_desc *gd, int device, fimhip_ctx 
       {&s.dp_tdcy, 3 * cz}, {&s.dpl_tdcy, 3 * cz}, {&s.trc_tdcy, 3 * cz * ntra}, {&s.trl_tdcy, 3 * cz * ntra},
       {&s.massfx, 3 * ez}, {&s.ws, cz}, {&s.relvor, cz}, {&s.sdot, lz}, {&s.psrf, (size_t)nip},
       {&s.ptdcy, 2 * (size_t)nip}, {&s.u_edg, ez}, {&s.v_edg, ez}, {&s.dp_edg, ez}, {&s.lp_edg, ez},
-      {&s.mont_edg, ez}, {&s.uvsq_edg, ez}, {&s.trc_edg, ez * ntra}};
+      {&s.trc_edg, ez * ntra}};      // mont_edg, uvsq_edg: need_edges
   const Arena::Arr work[] = {
       {&s.antifx, ez}, {&s.delp_lo, cz},
       {&s.r_plus, cz}, {&s.r_mnus, cz}, {&s.antiflx, ez * ntra}, {&s.trcr_lo, cz * ntra},
       {&s.trmax, cz * ntra}, {&s.trmin, cz * ntra}, {&s.tr_rp, cz * ntra}, {&s.tr_rm, cz * ntra},
-      {&s.u2, cz}, {&s.v2, cz}, {&s.exsmo, lz}, {&s.thbuf, cz}, {&s.vn, ez}, {&s.bke, ez}, {&s.pgx, cz},
-      {&s.pgy, cz}, {&s.dp_alt, cz}, {&s.pr_alt, lz}, {&s.mp_alt, cz}, {&s.tr_alt, cz * ntra}};
+      {&s.u2, cz}, {&s.v2, cz}, {&s.exsmo, lz}, {&s.thbuf, cz}};
   for (auto &a : arrs)
     if ((r = c->arena.alloc(a.p, a.n))) { fimhip_destroy(c); return r; }
   if ((r = c->arena.alloc_all(work))) { fimhip_destroy(c); return r; }
-  // patches of 44 cells, smaller where those would leave CUs without a block
-  // (trcadv1 at G3 x 4 tracers: 25 us with 44, 12 us with 12; at G4 29 and 28)
-  const int core = (int)std::max(12LL, (long long)nip * ntra / 600);
-  if ((r = patch_tables(c->arena, hg, c->g, core, c->tiles))) { fimhip_destroy(c); return r; }
+  s.vn = s.u_edg;
+  s.bke = s.v_edg;
+  s.pgx = s.lp_edg;
+  s.pgy = s.lp_edg + cz;
+  c->hg.prox.swap(hg.prox);
+  c->hg.proxs.swap(hg.proxs);
+  c->hg.nprox.swap(hg.nprox);
   c->gsum_blocks = GSUM_BLOCKS;
   if ((r = c->arena.alloc(&c->gsum_partial, (size_t)c->gsum_blocks * (1 + ntra)))) { fimhip_destroy(c); return r; }
   if (hipStreamSynchronize(c->stream) != hipSuccess) { fimhip_destroy(c); return FIMHIP_EHIP; }
@@ -330,6 +333,35 @@ extern "C" long long fimhip_field_size(const fimhip_ctx *c, int f) {
   return FIMHIP_EINVAL;
 }
 
+// What fimhip_step needs beyond the routines on host arrays, built by the first
+// call of the device-resident path: an instance that only serves the routines
+// pays for none of it.
+static int step_prepare(fimhip_ctx *c) {
+  if (c->tiles.npatch) return 0;
+  const size_t cz = (size_t)c->nip * c->nvl, lz = (size_t)c->nip * (c->nvl + 1);
+  DevState &s = c->s;
+  int r;
+  if (!s.pr_alt && (r = c->arena.alloc(&s.pr_alt, lz))) return r;
+  if (!s.mp_alt && (r = c->arena.alloc(&s.mp_alt, cz))) return r;
+  // patches of 44 cells, smaller where those would leave CUs without a block
+  // (trcadv1 at G3 x 4 tracers: 25 us with 44, 12 us with 12; at G4 29 and 28)
+  const int core = (int)std::max(12LL, (long long)c->nip * c->ntra / 600);
+  EnsTiles t{};
+  if ((r = patch_tables(c->arena, c->hg, c->g, core, t))) return r;
+  c->tiles = t;
+  c->hg = HostGrid{};
+  return 0;
+}
+// mont_edg and uvsq_edg, which a step alone never holds
+static int need_edges(fimhip_ctx *c) {
+  const size_t ez = (size_t)c->nip * NPP * c->nvl;
+  DevState &s = c->s;
+  int r;
+  if (!s.mont_edg && (r = c->arena.alloc(&s.mont_edg, ez))) return r;
+  if (!s.uvsq_edg && (r = c->arena.alloc(&s.uvsq_edg, ez))) return r;
+  return 0;
+}
+
 struct TimerScope {
   explicit TimerScope(KTimer *t) { g_ktimer = t; }
   ~TimerScope() { g_ktimer = nullptr; }
@@ -339,6 +371,8 @@ struct TimerScope {
 // mont_edg, uvsq_edg and trc_edg); they stay due if a launch is refused
 static int form_edges(fimhip_ctx *c) {
   if (!c->edges_due) return 0;
+  const int r = need_edges(c);
+  if (r) return r;
   const TimerScope scope(c->kt);
   DevState t = c->s;
   t.us = c->start.us; t.vs = c->start.vs; t.pr = c->start.pr; t.mp = c->start.mp; t.tr = c->start.tr;
@@ -369,6 +403,10 @@ static int before_write(fimhip_ctx *c, int f) {
 
 static int h2d(fimhip_ctx *c, int f, const double *h) {
   if (!h) return FIMHIP_EINVAL;
+  if (f == FIMHIP_MONT_EDG || f == FIMHIP_UVSQ_EDG) {
+    const int r = need_edges(c);
+    if (r) return r;
+  }
   double **p = field_ptr(c, f);
   if (!*p) return FIMHIP_EINVAL;     // class-B fields before fimhip_set_class_b
   HIPCHK(hipMemcpyAsync(*p, h, fimhip_field_size(c, f) * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -376,6 +414,10 @@ static int h2d(fimhip_ctx *c, int f, const double *h) {
 }
 static int d2h(fimhip_ctx *c, int f, double *h) {
   if (!h) return FIMHIP_EINVAL;
+  if (f == FIMHIP_MONT_EDG || f == FIMHIP_UVSQ_EDG) {
+    const int r = need_edges(c);
+    if (r) return r;
+  }
   double **p = field_ptr(c, f);
   if (!*p) return FIMHIP_EINVAL;
   HIPCHK(hipMemcpyAsync(h, *p, fimhip_field_size(c, f) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -413,7 +455,7 @@ static int ab_out(fimhip_ctx *c, int f, double *h) { return ab_slot(c, f, h, c->
 extern "C" int fimhip_upload(fimhip_ctx *c, int f, const double *h) {
   if (!c || f < 0 || f >= FIMHIP_NFIELDS) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
-  if (!h || !*field_ptr(c, f)) return FIMHIP_EINVAL;
+  if (!h) return FIMHIP_EINVAL;
   int r = before_write(c, f);
   if (r || (r = h2d(c, f, h))) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -452,6 +494,7 @@ extern "C" int fimhip_edgvar1_r8(fimhip_ctx *c, int its, const double *u_vel, co
   TRY(h2d(c, FIMHIP_MP, montg)); TRY(h2d(c, FIMHIP_TR, tracr));
   // trc_edg is intent(out) for tracer 1 only; the other tracers pass through
   TRY(h2d(c, FIMHIP_TRC_EDG, trc_edg));
+  TRY(need_edges(c));
   launch_edgvar1(c->g, c->s, c->stream);
   TRY(d2h(c, FIMHIP_U_EDG, u_edg)); TRY(d2h(c, FIMHIP_V_EDG, v_edg)); TRY(d2h(c, FIMHIP_LP_EDG, lp_edg));
   TRY(d2h(c, FIMHIP_MONT_EDG, mont_edg)); TRY(d2h(c, FIMHIP_UVSQ_EDG, uvsq_edg));
@@ -797,6 +840,7 @@ extern "C" int fimhip_transp2_r4(fimhip_ctx *c, int its, float *tracr, float *cu
 extern "C" int fimhip_init_state(fimhip_ctx *c, int init_hybgen) {
   if (!c) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  TRY(step_prepare(c));
   if (init_hybgen && (c->start.us == c->s.us || c->start.vs == c->s.vs)) TRY(form_edges(c));   // moved in place
   TRY(before_write(c, FIMHIP_MP));
   launch_trdp(c->g, c->s, c->stream);
@@ -822,6 +866,8 @@ extern "C" int fimhip_init_state(fimhip_ctx *c, int init_hybgen) {
 extern "C" int fimhip_step(fimhip_ctx *c, int its, int mode) {
   if (!c || its < 1 || (mode != 0 && mode != 1)) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(c->device));
+  const int r = step_prepare(c);
+  if (r) return r;
   const TimerScope scope(c->kt);
   ab_rotate(c->ab, its, c->dt);
   const DevState &s = c->s;

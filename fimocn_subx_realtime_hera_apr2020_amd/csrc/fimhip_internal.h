@@ -67,11 +67,12 @@ struct DevState {
   double *antiflx, *trcr_lo, *trmax, *trmin, *tr_rp, *tr_rm;   // per tracer
   double *u2, *v2, *exsmo, *thbuf;
   // the device-resident step: the normal edge wind, Montgomery potential plus
-  // kinetic energy on the edges, the edge-pressure line integrals, and the
-  // buffers that alternate with dp, pr, mp and tr, so that the values of a
-  // step's start stay until the next step
+  // kinetic energy on the edges and the edge-pressure line integrals, in
+  // u_edg, v_edg and lp_edg, whose own values are formed on demand; and the
+  // buffers that alternate with pr and mp (dp alternates with delp_lo, tr with
+  // trcr_lo), so that the values of a step's start stay until the next step
   double *vn, *bke, *pgx, *pgy;
-  double *dp_alt, *pr_alt, *mp_alt, *tr_alt;
+  double *pr_alt, *mp_alt;
 };
 
 // Class-B tracer transport state (transp3d.F90, fct3d.F90): the tracers

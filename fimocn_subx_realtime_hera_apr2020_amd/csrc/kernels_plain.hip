@@ -889,7 +889,8 @@ __global__ void __launch_bounds__(256) k_s_cnuity3(DevGrid g, DevState s, AB ab)
   __builtin_nontemporal_store(dmax(0., dmin(1., q_mnus / dmax(pm, thshld))), &C2(s.r_mnus, ipn, k));
 }
 
-// cnuity4 + cnuity5; the thickness and pressure go to their other buffers
+// cnuity4 + cnuity5; the pressure goes to its other buffer, the thickness to
+// that of the low-order thickness, which cnuity3 was the last to read
 template <int NP>
 __device__ __forceinline__ void s_cnuity4_col(const DevGrid &g, const DevState &s, const AB &ab, int ipn, int k,
                                               double &dpn, double &lt) {
@@ -917,7 +918,7 @@ __device__ __forceinline__ void s_cnuity4_col(const DevGrid &g, const DevState &
   const double dtn = lo + at;
   __builtin_nontemporal_store(dtn, &AB3(s.dp_tdcy, nf, ipn, k));
   dpn = dp0 + ab.ab1 * dtn + ab.ab2 * to + ab.ab3 * tv;
-  __builtin_nontemporal_store(dpn, &C2(s.dp_alt, ipn, k));
+  __builtin_nontemporal_store(dpn, &C2(s.delp_lo, ipn, k));
   lt = (ab.ab1 * dtn + ab.ab2 * to + ab.ab3 * tv) / g.dt;
 }
 __global__ void __launch_bounds__(256) k_s_cnuity45(DevGrid g, DevState s, AB ab) {
@@ -1031,7 +1032,7 @@ __device__ __forceinline__ void s_massadv2_col(const DevGrid &g, const DevState 
   __builtin_nontemporal_store(dtn, &AB3(s.dp_tdcy, nf, ipn, k));
   const double d = dp0 + ab.ab1 * dtn + ab.ab2 * to + ab.ab3 * tv;
   dpn = dmax(d, 0.0);
-  __builtin_nontemporal_store(dpn, &C2(s.dp_alt, ipn, k));
+  __builtin_nontemporal_store(dpn, &C2(s.delp_lo, ipn, k));
   lt = (ab.ab1 * dtn + ab.ab2 * to + ab.ab3 * tv) / g.dt;
 }
 __global__ void __launch_bounds__(256) k_s_massadv2(DevGrid g, DevState s, AB ab) {
@@ -1103,8 +1104,9 @@ __global__ void __launch_bounds__(256) k_s_trcadv2(DevGrid g, DevState s, AB ab)
   }
 }
 
-// trcadv3; the tracer goes to its other buffer, the tracer mass (TRDP) only
-// where hystat does not form it again
+// trcadv3; the tracer goes to the buffer of the low-order tracer, which trcadv2
+// was the last to read, the tracer mass (TRDP) only where hystat does not form it
+// again
 template <int NP, bool TRDP>
 __device__ __forceinline__ void s_trcadv3_col(const DevGrid &g, const DevState &s, const AB &ab, int ipn, int k) {
   const int nip = g.nip, nvl = g.nvl, ntra = g.ntra;
@@ -1133,7 +1135,7 @@ __device__ __forceinline__ void s_trcadv3_col(const DevGrid &g, const DevState &
     __builtin_nontemporal_store(tt, &TAB(s.trc_tdcy, t, nf, ipn, k));
     const double tdp = td + ab.ab1 * tt + ab.ab2 * to + ab.ab3 * tv;
     if (TRDP) __builtin_nontemporal_store(tdp, &C2(s.trdp + t * csz, ipn, k));
-    __builtin_nontemporal_store(dmax(mn, dmin(mx, tdp / dpc)), &C2(s.tr_alt + t * csz, ipn, k));
+    __builtin_nontemporal_store(dmax(mn, dmin(mx, tdp / dpc)), &C2(s.trcr_lo + t * csz, ipn, k));
   }
 }
 template <bool TRDP>
@@ -1274,7 +1276,7 @@ void step_continuity(const DevGrid &g, DevState &s, const AB &ab, bool mass_adv,
     KT_LAUNCH("k_cnuity3", st, k_s_cnuity3<<<gr, bl, 0, st>>>(g, s, ab));
     KT_LAUNCH("k_cnuity45", st, k_s_cnuity45<<<gr, bl, 0, st>>>(g, s, ab));
   }
-  swap_ptr(s.dp, s.dp_alt);
+  swap_ptr(s.dp, s.delp_lo);
   swap_ptr(s.pr, s.pr_alt);
 }
 // Rows of the tracer kernels' grid: one (every tracer of a column in one
@@ -1288,7 +1290,7 @@ void step_tracers(const DevGrid &g, DevState &s, const EnsTiles &ts, const AB &a
   KT_LAUNCH("k_trcadv2", st, k_s_trcadv2<<<gr, bl, 0, st>>>(g, s, ab));
   if (last) KT_LAUNCH("k_trcadv3", st, k_s_trcadv3<true><<<gr, bl, 0, st>>>(g, s, ab));
   else KT_LAUNCH("k_trcadv3", st, k_s_trcadv3<false><<<gr, bl, 0, st>>>(g, s, ab));
-  swap_ptr(s.tr, s.tr_alt);
+  swap_ptr(s.tr, s.trcr_lo);
 }
 void step_momtum(const DevGrid &g, DevState &s, const double *theta_start, const AB &ab, hipStream_t st) {
   KT_LAUNCH("k_momtum", st, k_s_momtum<<<col_grid(g.nip), col_block(), 0, st>>>(g, s, theta_start, ab));

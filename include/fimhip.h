@@ -176,7 +176,8 @@ enum {
    (tracers 2..ntra) hold each cell's own reconstructions (the step's readers
    form the two-sided averages), except that DP_EDG holds mass_adv's final
    edge depths under flux_conserv_schm = 2.  The step does not store the
-   others and TRC_EDG; they are formed when they are downloaded. */
+   others and TRC_EDG; they are formed when they are downloaded (MONT_EDG and
+   UVSQ_EDG are allocated when they are first needed). */
 /* number of doubles of a field */
 long long fimhip_field_size(const fimhip_ctx *ctx, int field);
 int fimhip_upload(fimhip_ctx *ctx, int field, const double *host);
@@ -188,7 +189,9 @@ int fimhip_init_state(fimhip_ctx *ctx, int init_hybgen);
 /* one dynamics step on the device, asynchronous: mode 0 = DYN_1(its) then
  * DYN_2(its) (abstart, edgvar1, edgvar3, cnuity, trcadv, momtum, hybgen,
  * hystat: dyn_run.F90:119-425); mode 1 = transport only (abstart, edgvar1,
- * edgvar3, cnuity, trcadv) */
+ * edgvar3, cnuity, trcadv).  The first fimhip_init_state or fimhip_step on an
+ * instance builds the tables that only the step needs (FIMHIP_ENOMEM if they do
+ * not fit: nothing has changed). */
 int fimhip_step(fimhip_ctx *ctx, int its, int mode);
 /* the namelist switch flux_conserv_schm (fimnamelist.F90; dyn_run.F90:377-386)
  * for fimhip_step: 1 = cnuity (FCT, the default), 2 = mass_adv */

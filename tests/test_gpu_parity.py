@@ -847,3 +847,35 @@ def test_winds_written_each_step_form_no_edge_fields(oracle_lib):
             assert _same(m.download(f) * live, o.a[f].reshape(m.shape(f)) * live), f
     finally:
         m.close()
+
+
+def test_device_memory_of_an_instance_stays_that_of_its_arrays():
+    """Per cell and layer a plain instance holds 89 + 25 ntra FP64 values (the
+    fields of fimhip_field_size and the routines' work arrays) and the grid's
+    tables: what the device-resident step needs beyond the routines' arrays
+    shares their memory or takes the place of edge fields that only a caller
+    who asks for them gets allocated."""
+    import torch
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, state
+    g = fimhip.icos_grid(6)
+    th, ds = state.vertical_tables(64)
+    ntra, cell = 4, 8 * 64 * g.nip
+    print("case: G6 x 64 x %d tracers, device memory" % ntra, flush=True)
+    arrays = (89 + 25 * ntra) * cell
+    tables = 8 * 160 * g.nip + (64 << 20)      # metrics, neighbours, HIP's allocation granularity
+    free = lambda: torch.cuda.mem_get_info()[0]   # noqa: E731
+    start = free()
+    m = fimhip.Model(g, 64, ntra, 60.0, th, ds)
+    try:
+        m.synth(seed=1)
+        m.init_state(False)
+        assert start - free() < arrays + tables
+        m.step(1, 0)
+        m.step(2, 1)
+        m.sync()
+        assert start - free() < arrays + tables
+        m.download("mont_edg")
+        # the buffers of pr and mp, the patches' tables (1 KB a cell)
+        assert start - free() < arrays + 2.1 * cell + 1024 * g.nip + tables
+    finally:
+        m.close()
