@@ -652,16 +652,14 @@ extern "C" int fimhip_ocn_create(const fimhip_grid_desc *gd, const double *rprox
   o->mo.smagcf = 0.3;              // fimnamelist.F90:253
   const size_t cz = (size_t)nip * kdm, ez = cz * NPP;
   HycState &s = o->s;
-  double *um, *vm, *un, *vn, *dpe;
   const Arena::Arr arrs[] = {
-      {&um, ez}, {&vm, ez}, {&un, ez}, {&vn, ez}, {&dpe, ez}, {&s.dp, 2 * cz}, {&s.pres, (size_t)nip * (kdm + 1)},
+      {&s.dpm_edg, ez}, {&s.dp, 2 * cz}, {&s.pres, (size_t)nip * (kdm + 1)},
       {&s.massflx, ez}, {&s.mssfx_avg, ez},
-      // the edge interpolation's inputs and outputs
+      // the edge interpolation's inputs and outputs (the others: ocn_need_edges)
       {&o->ed.uclin, 2 * cz}, {&o->ed.vclin, 2 * cz}, {&o->ed.uclin_alt, 2 * cz}, {&o->ed.vclin_alt, 2 * cz},
       {&o->ed.utrop, (size_t)nip * 3}, {&o->ed.vtrop, (size_t)nip * 3},
       {&o->ed.geop, (size_t)nip * (kdm + 1)}, {&o->ed.montg, cz}, {&o->ed.spcifv, cz},
-      {&o->ed.pr_edg, (size_t)nip * NPP * (kdm + 1)}, {&o->ed.geop_edg, ez}, {&o->ed.mont_edg, ez},
-      {&o->ed.uvsq_edg, ez}, {&o->ed.spcv_edg, ez},
+      {&o->ed.geop_edg, ez},
       // the momentum equation's forcing
       {&o->mo.taux, (size_t)nip}, {&o->mo.tauy, (size_t)nip}, {&o->mo.ustarb, (size_t)nip},
       // the tracers and density the transport and the grid generator share
@@ -676,7 +674,6 @@ extern "C" int fimhip_ocn_create(const fimhip_grid_desc *gd, const double *rprox
   if ((r = o->arena.alloc_all(work))) { fimhip_ocn_destroy(o); return r; }
   for (auto &a : arrs)
     if ((r = o->arena.alloc(a.p, a.n))) { fimhip_ocn_destroy(o); return r; }
-  s.um = um; s.vm = vm; s.un = un; s.vn = vn; s.dpm_edg = dpe;
   if ((r = o->arena.alloc(&s.flag, 1))) { fimhip_ocn_destroy(o); return r; }
   if (hipStreamSynchronize(o->stream) != hipSuccess) { fimhip_ocn_destroy(o); return FIMHIP_EHIP; }
   *out = o;
@@ -744,8 +741,20 @@ extern "C" int fimhip_ocn_sync(fimhip_ocn *o) {
 extern "C" long long fimhip_ocn_field_size(const fimhip_ocn *o, int f) {
   if (!o) return FIMHIP_EINVAL;
   size_t n = 0;
-  if (!ocn_field(const_cast<fimhip_ocn *>(o), f, &n)) return FIMHIP_EINVAL;
-  return (long long)n;
+  (void)ocn_field(const_cast<fimhip_ocn *>(o), f, &n);
+  return n ? (long long)n : FIMHIP_EINVAL;
+}
+
+int ocn_need_edges(fimhip_ocn *o) {
+  const size_t ez = (size_t)o->nip * o->kdm * NPP;
+  const Arena::Arr arrs[] = {{&o->s.um, ez}, {&o->s.vm, ez}, {&o->s.un, ez}, {&o->s.vn, ez},
+                             {&o->ed.pr_edg, (size_t)o->nip * NPP * (o->kdm + 1)}, {&o->ed.mont_edg, ez},
+                             {&o->ed.uvsq_edg, ez}, {&o->ed.spcv_edg, ez}};
+  for (auto &a : arrs) {
+    const int r = *a.p ? FIMHIP_OK : o->arena.alloc(a.p, a.n);
+    if (r) return r;
+  }
+  return FIMHIP_OK;
 }
 
 // an edge array that fimhip_ocn_edgvar leaves to be formed
@@ -792,9 +801,10 @@ static int before_put(fimhip_ocn *o, int f, size_t n) {
 
 int ocn_put(fimhip_ocn *o, int f, const double *h) {
   size_t n = 0;
-  if (!ocn_field(o, f, &n)) return FIMHIP_EINVAL;
-  const int r = before_put(o, f, n);
+  int r = lazy_edge(f) ? ocn_need_edges(o) : FIMHIP_OK;
   if (r) return r;
+  if (!ocn_field(o, f, &n)) return FIMHIP_EINVAL;
+  if ((r = before_put(o, f, n))) return r;
   HIPCHK(hipMemcpyAsync(ocn_field(o, f, &n), h, n * sizeof(double), hipMemcpyHostToDevice, o->stream));
   if (f == FIMHIP_OCN_UCLIN || f == FIMHIP_OCN_VCLIN) o->alt_stale = true;
   return FIMHIP_OK;
@@ -802,12 +812,12 @@ int ocn_put(fimhip_ocn *o, int f, const double *h) {
 
 int ocn_get(fimhip_ocn *o, int f, double *h) {
   size_t n = 0;
+  if (lazy_edge(f)) {
+    int r = ocn_need_edges(o);
+    if (r || (r = ocn_form_edges(o))) return r;
+  }
   const double *d = ocn_field(o, f, &n);
   if (!d) return FIMHIP_EINVAL;
-  if (lazy_edge(f)) {
-    const int r = ocn_form_edges(o);
-    if (r) return r;
-  }
   HIPCHK(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, o->stream));
   return FIMHIP_OK;
 }
@@ -862,6 +872,10 @@ static int ocn_launch(fimhip_ocn *o, int nstep, int leapm, int leapn) {
   // second step, or another level, is a step on the arrays themselves
   if (o->e_dp_old || leapm != o->e_leapm) {
     const int r = ocn_form_edges(o);
+    if (r) return r;
+  }
+  if (!o->edges_due) {
+    const int r = ocn_need_edges(o);
     if (r) return r;
   }
   HIPCHK(hipMemsetAsync(o->s.flag, 0, sizeof(int), o->stream));

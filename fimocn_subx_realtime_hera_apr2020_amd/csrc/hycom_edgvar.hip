@@ -446,6 +446,10 @@ static void janjic_kernel(fimhip_ocn *o) {
 static int edg_launch(fimhip_ocn *o, int leapm, int leapn, bool full) {
   if (leapm < 1 || leapm > 2 || leapn < 1 || leapn > 2 || leapm == leapn) return FIMHIP_EINVAL;
   HIPCHK(hipSetDevice(o->device));
+  if (full) {
+    const int r = ocn_need_edges(o);
+    if (r) return r;
+  }
   HycEdg &ed = o->ed;
   ed.uclin_e = ed.uclin; ed.vclin_e = ed.vclin; ed.utrop_e = ed.utrop; ed.vtrop_e = ed.vtrop;
   ed.montg_e = ed.montg; ed.spcifv_e = ed.spcifv;
@@ -465,6 +469,8 @@ static int edg_launch(fimhip_ocn *o, int leapm, int leapn, bool full) {
 
 int ocn_form_edges(fimhip_ocn *o) {
   if (!o->edges_due) return FIMHIP_OK;
+  const int r = ocn_need_edges(o);
+  if (r) return r;
   g_ktimer = o->kt;
   if (o->kdm <= 32) form_kernels<32>(o, o->e_leapm, o->e_leapn, false);
   else form_kernels<64>(o, o->e_leapm, o->e_leapn, false);

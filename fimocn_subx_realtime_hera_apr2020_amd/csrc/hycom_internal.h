@@ -223,9 +223,12 @@ struct fimhip_ocn {
   fimhip::KTimer *kt = nullptr;              // non-null while profiling
 };
 
-// the device array of a FIMHIP_OCN_* field and its element count; nullptr for
-// a field the instance does not have
+// the device array of a FIMHIP_OCN_* field and its element count (0 for a
+// field the instance does not have); nullptr also for a public edge array that
+// is not allocated yet
 double *ocn_field(fimhip_ocn *o, int f, size_t *n);
+// allocates the public edge arrays that the resident steps do without
+int ocn_need_edges(fimhip_ocn *o);
 // the public edge arrays, if they are due (hycom_edgvar.hip)
 int ocn_form_edges(fimhip_ocn *o);
 // a whole field to or from the host on the instance's stream, with the edge

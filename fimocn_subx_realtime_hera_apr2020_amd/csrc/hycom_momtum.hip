@@ -472,6 +472,10 @@ static int mom_launch(fimhip_ocn *o, int leapm, int leapn) {
     const int r = ocn_form_edges(o);
     if (r) return r;
   }
+  if (!o->edges_due) {
+    const int r = ocn_need_edges(o);
+    if (r) return r;
+  }
   if (o->alt_stale) {       // land keeps its velocities: the other pair needs them too
     const size_t n = 2 * (size_t)o->nip * o->kdm * sizeof(double);
     HIPCHK(hipMemcpyAsync(ed.uclin_alt, ed.uclin, n, hipMemcpyDeviceToDevice, o->stream));

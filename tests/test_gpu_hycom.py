@@ -771,3 +771,35 @@ def test_edgvar_dropin_forms_each_array_once(oracle_lib, before):
             assert _same(o.download(n), h.e[n]), n
     finally:
         o.close()
+
+
+def test_device_memory_of_the_resident_ocean_stays_that_of_its_arrays():
+    """Per cell and layer the ocean held 106 FP64 values when every edge array
+    was stored; an instance whose steps leave them to be formed holds fewer,
+    and the edge arrays come when one is asked for."""
+    import torch
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip, ocean
+    g = _grid(6)
+    kdm = 32
+    case = ocean.hycom_ocean_case(g, kdm=kdm, seed=5, numtr=1)
+    cell, tables = 8 * kdm * g.nip, 8 * 160 * g.nip + (64 << 20)
+    print("case: G6 x %d, device memory" % kdm, flush=True)
+    free = lambda: torch.cuda.mem_get_info()[0]   # noqa: E731
+    start = free()
+    o = fimhip.Ocean(g, kdm, case["wet"], case["dtleap"])
+    try:
+        o.set_momtum(case["batrop"], case["veldff"], case["smagcf"])
+        for n in ("dp", "pres", "uclin", "vclin", "utrop", "vtrop", "geop", "montg", "spcifv", "massflx", "mssfx_avg"):
+            o.upload(n, case[n])
+        for st in (1, 2):
+            o.upload("montg", case["montg"])
+            o.step_edgvar(1 + st % 2, 2 - st % 2)
+            o.step(st, 1 + st % 2, 2 - st % 2)
+            o.step_momtum(1 + st % 2, 2 - st % 2)
+        o.sync()
+        used = start - free()
+        assert used < 90 * cell + tables
+        e = o.download("pr_edg")
+        assert np.isfinite(e).all() and start - free() > used + 40 * cell
+    finally:
+        o.close()
