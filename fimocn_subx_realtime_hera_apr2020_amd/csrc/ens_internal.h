@@ -92,8 +92,11 @@ constexpr int ENS_NTILES = 8;                       // cols {1,2,4,8} x swizzle 
 inline int tile_cols(int t) { return 1 << (t & 3); }
 inline bool tile_swz(int t) { return (t >> 2) & 1; }
 
+// The numbers are part of the interface (fimhip_ens_set_tile).  trcadv12 has the
+// number of the trcadv1 it took the place of; trcadv2's is kept, without a
+// kernel, so that the numbers after it stay.
 enum EnsKernel {
-  EK_EDGVAR1 = 0, EK_EDGVAR3, EK_CNUITY12, EK_CNUITY3, EK_CNUITY45, EK_TRCADV12, EK_TRCADV3,
+  EK_EDGVAR1 = 0, EK_EDGVAR3, EK_CNUITY12, EK_CNUITY3, EK_CNUITY45, EK_TRCADV12, EK_TRCADV2_NONE, EK_TRCADV3,
   EK_MOMTUM, EK_HYSTAT, EK_MASSADV1, EK_MASSADV2, EK_TRCFCT, EK_NKERNELS
 };
 extern const char *const ens_kernel_names[EK_NKERNELS];

@@ -14,7 +14,7 @@ namespace fimhip {
 
 const char *const ens_kernel_names[EK_NKERNELS] = {
     "e_edgvar1", "e_edgvar3", "e_cnuity12", "e_cnuity3", "e_cnuity45",
-    "e_trcadv12", "e_trcadv3", "e_momtum", "e_hystat", "e_massadv1", "e_massadv2", "e_trc_fct"};
+    "e_trcadv12", "e_trcadv2", "e_trcadv3", "e_momtum", "e_hystat", "e_massadv1", "e_massadv2", "e_trc_fct"};
 
 #define EC(a, col, k) (a)[(size_t)(col) * nvl + (k)]
 #define EL(a, col, k) (a)[(size_t)(col) * nvlp1 + (k)]

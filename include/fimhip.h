@@ -331,7 +331,10 @@ int fimhip_ens_download(fimhip_ens *ens, int member, int field, double *host);
  * mass32/trtot32 (may be NULL) from FP32 Kahan-compensated sums */
 int fimhip_ens_globsum(fimhip_ens *ens, double *mass, double *trtot, double *mass32, double *trtot32);
 /* launch shapes: kernel k in 0..fimhip_ens_kernel_count()-1, tile 0..7 =
- * (1,2,4,8 columns per block) x (XCD-contiguous block order off/on) */
+ * (1,2,4,8 columns per block) x (XCD-contiguous block order off/on); of
+ * e_trcadv12's tile bit 0 chooses 8 or 16 wavefronts per block, bit 1 is not
+ * used and bit 2 is the block order; e_trcadv2 has no kernel (e_trcadv12 does
+ * its work) and keeps its number.  No tile changes a result. */
 int fimhip_ens_kernel_count(void);
 const char *fimhip_ens_kernel_name(int kernel);
 int fimhip_ens_set_tile(fimhip_ens *ens, int kernel, int tile);

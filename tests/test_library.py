@@ -81,3 +81,18 @@ def test_state_generator_is_batch_invariant():
         assert np.array_equal(a[k][:100], b[k])
     c = state.make_state(g.lat, g.lon, 64, 4, wind_noise=True, perturb=True, member=4)
     assert not np.array_equal(a["us"], c["us"])
+
+
+def test_kernel_numbers_of_the_launch_shapes_stay():
+    """fimhip_ens_set_tile takes a kernel's number, and launch shapes are kept
+    by number or name: a kernel that goes leaves its number behind."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip
+    lib = fimhip.load_library()
+    names = [lib.fimhip_ens_kernel_name(k).decode() for k in range(lib.fimhip_ens_kernel_count())]
+    assert names == ["e_edgvar1", "e_edgvar3", "e_cnuity12", "e_cnuity3", "e_cnuity45", "e_trcadv12", "e_trcadv2",
+                     "e_trcadv3", "e_momtum", "e_hystat", "e_massadv1", "e_massadv2", "e_trc_fct"]
+    set_to = {}
+    shape = type("Shape", (), dict(kernel_names=lambda self: names, h=None, lib=type("Lib", (), dict(
+        fimhip_ens_set_tile=staticmethod(lambda h, k, t: set_to.update({k: t}) or 0)))()))()
+    fimhip.Ensemble.set_tiles(shape, {"e_trcadv1": 5, "e_trcadv2": 3, "e_momtum": 6})
+    assert set_to == {5: 5, 6: 3, 8: 6}
