@@ -632,6 +632,7 @@ extern "C" int fimhip_ens_autotune(fimhip_ens *e, int mode, int reps, double *ti
     best[f].assign(EK_NKERNELS, 1e30);
     tab[f].assign(nt, std::numeric_limits<double>::quiet_NaN());
     pick[f].assign(e->tile, e->tile + EK_NKERNELS);
+    std::fill_n(tab[f].begin() + EK_TRCADV2_NONE * ENS_NTILES, ENS_NTILES, 0.);      // no kernel, no time
     for (int t = 0; t < ENS_NTILES; t++) {
       for (int k = 0; k < EK_NKERNELS; k++) e->tile[k] = t;
       KTimer kt;

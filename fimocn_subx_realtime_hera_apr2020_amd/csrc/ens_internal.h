@@ -130,6 +130,8 @@ constexpr TileLimits TRC64_LIMITS = {2, 44, 80, 120, 120}; // the FP64 step's tr
 constexpr TileLimits FCT_LIMITS = {3, FCT_CORE_MAX, FCT_R_MAX, FCT_LO_MAX, FCT_TILE_MAX};
 int ens_build_tiles(const HostGrid &h, int nip, const TileLimits &lim, TileHost &out);
 int ens_upload_tiles(Arena &a, const TileHost &t, EnsTiles &d);
+// marks in t's core cells the edges whose neighbour is a pentagon
+void patch_pentagons(const HostGrid &h, TileHost &t);
 // the FP64 step's patches of at most 'core' cells and their rows (trc_patch.hip)
 int patch_tables(Arena &a, const HostGrid &h, const DevGrid &g, int core, EnsTiles &ts);
 void launch_patch_trcadv1(const DevGrid &g, const DevState &s, const EnsTiles &ts, const AB &ab, hipStream_t st);

@@ -133,16 +133,19 @@ int ens_upload_tiles(Arena &a, const TileHost &t, EnsTiles &d) {
 // The patch tables of a grid, for inspection: sizes[0] = number of patches,
 // sizes[1] = number of tile-cell entries; cnt (4 per patch: n0..n3) and ent
 // (4 per entry, see EnsTiles) are written when not NULL and large enough.
-extern "C" int fimhip_ens_patches(const fimhip_grid_desc *gd, int *sizes, int *cnt, long long cnt_len, int *ent,
-                                  long long ent_len) {
+extern "C" int fimhip_patches(const fimhip_grid_desc *gd, int form, int core, int *sizes, int *cnt, long long cnt_len,
+                              int *ent, long long ent_len) {
   using namespace fimhip;
-  if (!gd || !sizes || gd->nip < 12 || !gd->nprox || !gd->prox || !gd->proxs || !gd->lat || !gd->lon || !gd->area)
+  if (form < 0 || form > 2 || core < 0 || !gd || !sizes || gd->nip < 12 || !gd->nprox || !gd->prox || !gd->proxs || !gd->lat || !gd->lon || !gd->area)
     return FIMHIP_EINVAL;
   HostGrid h;
   int r = host_grid_prepare(gd, h);
   if (r) return r;
   TileHost t;
-  if ((r = ens_build_tiles(h, gd->nip, FCT_LIMITS, t))) return r;
+  TileLimits lim = form == 0 ? FCT_LIMITS : form == 1 ? TRC_LIMITS : TRC64_LIMITS;
+  if (core > 0) lim.core = std::min(core, lim.core);
+  if ((r = ens_build_tiles(h, gd->nip, lim, t))) return r;
+  if (form == 2) patch_pentagons(h, t);
   sizes[0] = (int)t.cnt.size();
   sizes[1] = (int)t.ent.size();
   if (cnt) {
@@ -156,6 +159,10 @@ extern "C" int fimhip_ens_patches(const fimhip_grid_desc *gd, int *sizes, int *c
       for (int j = 0; j < 4; j++) ent[4 * i + j] = t.ent[i][j];
   }
   return FIMHIP_OK;
+}
+extern "C" int fimhip_ens_patches(const fimhip_grid_desc *gd, int *sizes, int *cnt, long long cnt_len, int *ent,
+                                  long long ent_len) {
+  return fimhip_patches(gd, 0, 0, sizes, cnt, cnt_len, ent, ent_len);
 }
 
 namespace fimhip {

@@ -216,17 +216,20 @@ __global__ void __launch_bounds__(64 * NW) k_p_trcadv1(DevGrid g, DevState s, En
 
 }  // namespace
 
-int patch_tables(Arena &a, const HostGrid &h, const DevGrid &g, int core, EnsTiles &ts) {
-  TileHost t;
-  int r = ens_build_tiles(h, g.nip, {2, std::min(core, TRC64_LIMITS.core), TRC64_LIMITS.r, TRC64_LIMITS.lo, TRC64_LIMITS.tile}, t);
-  if (r) return r;
-  // per core cell and edge, whether the neighbour is a pentagon (bits 24-29 of the third word)
+void patch_pentagons(const HostGrid &h, TileHost &t) {
   for (size_t p = 0; p < t.cnt.size(); p++)
     for (int i = 0; i < t.cnt[p][0]; i++) {
       auto &en = t.ent[t.off[p] + i];
       for (int e = 0; e < NPP; e++)
         if (h.nprox[h.prox[(size_t)en[0] * NPP + e]] != NPP) en[2] |= 1 << (24 + e);
     }
+}
+
+int patch_tables(Arena &a, const HostGrid &h, const DevGrid &g, int core, EnsTiles &ts) {
+  TileHost t;
+  int r = ens_build_tiles(h, g.nip, {2, std::min(core, TRC64_LIMITS.core), TRC64_LIMITS.r, TRC64_LIMITS.lo, TRC64_LIMITS.tile}, t);
+  if (r) return r;
+  patch_pentagons(h, t);
   if ((r = ens_upload_tiles(a, t, ts))) return r;
   ts.lo_max = 0;
   for (auto &c : t.cnt) ts.lo_max = std::max(ts.lo_max, c[2]);

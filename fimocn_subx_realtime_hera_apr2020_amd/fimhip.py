@@ -45,7 +45,7 @@ EXPORTS = ["fimhip_create", "fimhip_destroy", "fimhip_abstart", "fimhip_set_ab",
            "fimhip_ens_globsum",
            "fimhip_ens_kernel_count", "fimhip_ens_kernel_name", "fimhip_ens_set_tile", "fimhip_ens_get_tile",
            "fimhip_ens_autotune", "fimhip_ens_profile", "fimhip_ens_profile_report",
-           "fimhip_globsum_noalloc", "fimhip_ens_set_fused", "fimhip_ens_get_fused", "fimhip_ens_patches",
+           "fimhip_globsum_noalloc", "fimhip_ens_set_fused", "fimhip_ens_get_fused", "fimhip_ens_patches", "fimhip_patches",
            "fimhip_ens_set_wet", "fimhip_ls_pseudo_inverse",
            "fimhip_ocn_create", "fimhip_ocn_destroy", "fimhip_ocn_cnuity_r8", "fimhip_ocn_cnuity",
            "fimhip_ocn_field_size", "fimhip_ocn_upload", "fimhip_ocn_download", "fimhip_ocn_mass",
@@ -151,6 +151,8 @@ def load_library() -> ct.CDLL:
     lib.fimhip_ens_set_wet.argtypes = [vp, ct.c_int, _PI]
     lib.fimhip_ls_pseudo_inverse.argtypes = [ct.POINTER(ct.c_float), ct.c_int, ct.POINTER(ct.c_float)]
     lib.fimhip_ens_patches.argtypes = [ct.POINTER(GridDesc), _PI, _PI, ct.c_longlong, _PI, ct.c_longlong]
+    lib.fimhip_patches.argtypes = [ct.POINTER(GridDesc), ct.c_int, ct.c_int, _PI, _PI, ct.c_longlong, _PI,
+                                   ct.c_longlong]
     lib.fimhip_ens_set_flux_scheme.argtypes = [vp, ct.c_int]
     lib.fimhip_ens_set_class_b.argtypes = [vp, ct.c_int, ct.c_int]
     lib.fimhip_ens_load_class_b.argtypes = [vp, ct.c_int, _PD]
@@ -306,15 +308,21 @@ def ens_patches(grid: _glvl.Grid, nvl: int = 64):
     (cnt, ent) with cnt (npatch, 4) the cumulative ends of each patch's core
     and rings 1-3 in its entries, ent (nentries, 4) each entry's 0-based cell
     and packed local neighbour indices."""
+    return patches(grid, 0, 0, nvl)
+
+
+def patches(grid: _glvl.Grid, form: int, core: int = 0, nvl: int = 64):
+    """The patch partition of a form of the tracer transport (fimhip_patches),
+    as ens_patches returns it."""
     import numpy as _np
     lib = load_library()
     gd, keep = _grid_desc(grid, nvl, 1, 60.0, _np.zeros(nvl), _np.zeros(nvl))
     sz = (ct.c_int * 2)()
-    _chk(lib.fimhip_ens_patches(ct.byref(gd), sz, None, 0, None, 0), "ens_patches")
+    _chk(lib.fimhip_patches(ct.byref(gd), form, core, sz, None, 0, None, 0), "patches")
     cnt = _np.zeros((sz[0], 4), _np.int32)
     ent = _np.zeros((sz[1], 4), _np.int32)
-    _chk(lib.fimhip_ens_patches(ct.byref(gd), sz, cnt.ctypes.data_as(_PI), cnt.size, ent.ctypes.data_as(_PI),
-                                ent.size), "ens_patches")
+    _chk(lib.fimhip_patches(ct.byref(gd), form, core, sz, cnt.ctypes.data_as(_PI), cnt.size, ent.ctypes.data_as(_PI),
+                            ent.size), "patches")
     return cnt, ent
 
 

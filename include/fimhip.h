@@ -312,6 +312,13 @@ int fimhip_ens_set_wet(fimhip_ens *ens, int member, const int *wet);
  * when given with room (len in ints).  Host only. */
 int fimhip_ens_patches(const fimhip_grid_desc *grid, int *sizes, int *cnt, long long cnt_len, int *ent,
                        long long ent_len);
+/* the same for form 0 (as fimhip_ens_patches), 1 (the batched form's trcadv12)
+ * or 2 (the FP64 step's trcadv1) and cores of at most 'core' cells (0: the
+ * form's limit).  Forms 1 and 2 have two rings (the fourth count is the third),
+ * and their local indices are set for the core and ring 1; form 2 marks in bits
+ * 24-29 of a core cell's third word the edges whose neighbour is a pentagon. */
+int fimhip_patches(const fimhip_grid_desc *grid, int form, int core, int *sizes, int *cnt, long long cnt_len, int *ent,
+                   long long ent_len);
 /* flux_conserv_schm for the steps that follow (dyn_run.F90:377-386): 1 = FCT
  * cnuity (default), 2 = mass_adv (massadv.F90:21-160), with the edge's normal
  * wind taken from its lower-index cell so the FP32 mass fluxes still cancel */

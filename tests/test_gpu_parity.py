@@ -879,3 +879,32 @@ def test_device_memory_of_an_instance_stays_that_of_its_arrays():
         assert start - free() < arrays + 2.1 * cell + 1024 * g.nip + tables
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("seed,mode,flux_scheme,nvl", [(None, 1, 1, 64), (3, 1, 1, 40), (3, 0, 2, 64)])
+def test_steps_on_grids_with_other_slot_orders_match_checker_bitwise(oracle_lib, seed, mode, flux_scheme, nvl):
+    """The patches' rows hold each neighbour's stencil in the neighbour's own
+    slot order: with every cell's slots reversed (seed None), or each cell's
+    turned and started at random, the steps have the oracle's bits."""
+    from fimocn_subx_realtime_hera_apr2020_amd import fimhip
+    from helpers import seeded_case
+    from test_gpu_parity_ens import _turned
+    O = oracle_lib
+    g, st, th, ds = seeded_case(3, nvl=nvl)
+    g = _turned(g, seed)
+    o = O.OracleRun(O.grid_arrays(g, nvl, DT, th, ds), nvl, NTRA, DT, pow_kind=1, flux_scheme=flux_scheme)
+    o.load(st)
+    o.init(True)
+    m = fimhip.Model(g, nvl, NTRA, DT, th, ds)
+    try:
+        m.set_flux_scheme(flux_scheme)
+        m.load(st)
+        m.init_state(True)
+        for its in range(1, 5):
+            o.step(its, mode)
+            m.step(its, mode)
+        m.sync()
+        for f in ("us", "vs", "dp", "pr", "ex", "tr", "trdp", "ws"):
+            assert _same(m.download(f), o.a[f]), f
+    finally:
+        m.close()
