@@ -349,7 +349,7 @@ int fimhip_ens_get_tile(const fimhip_ens *ens, int kernel);
 /* time every tile of every kernel over reps steps and keep each kernel's
  * fastest, for both forms of the tracer transport, and keep the faster form;
  * advances the state (reload it afterwards); times may be NULL or receive
- * kernel_count x 8 mean milliseconds */
+ * kernel_count x 8 mean milliseconds (e_trcadv2's are e_trcadv12's) */
 int fimhip_ens_autotune(fimhip_ens *ens, int mode, int reps, double *times);
 int fimhip_ens_profile(fimhip_ens *ens, int on);
 int fimhip_ens_profile_report(fimhip_ens *ens, char *buf, int len);
