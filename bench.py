@@ -1075,6 +1075,29 @@ def cpu_schemes(o, m, grid, a, th, ds, fimhip, O, threads, ntrb=8):
             "cores": threads, "kind": "port"}
 
 
+def headline(out):
+    """The report's headline, short enough for the tail of a log (every leg in
+    full goes to stderr): each leg by its time, seven digits."""
+    legs = ("plain_fp64", "ensemble", "uneven_batch", "hycom", "accuracy_96", "cpu_baseline")
+    plain, _, uneven, hyc, acc, cpu = [out.get(k) for k in legs]
+    line = {k: v for k, v in out.items() if k not in legs}
+    line["config"] = {k: v for k, v in out["config"].items() if k != "dt_note"}
+    line["roofline"] = {k: v for k, v in out["roofline"].items() if k in ("bound", "achieved", "peak", "unit", "frac",
+                                                                          "traffic")}
+    line["plain_fp64_ms"] = plain and plain["ms_per_step"]
+    line["uneven_batch_ms"] = uneven and uneven["mixed"]["ms_per_step"]
+    line["hycom_ms"] = hyc and {k: v["ms_per_step"] for k, v in hyc.items() if isinstance(v, dict) and "ms_per_step" in v}
+    line["accuracy_rel_l2_max"] = acc and max(acc["rel_l2_vs_fp64"].values())
+    line["cpu_value"] = cpu and cpu["value"]
+
+    def short(x):
+        if isinstance(x, float):
+            return float("%.7g" % x)
+        return {k: short(v) for k, v in x.items()} if isinstance(x, dict) else x
+
+    return short(line)
+
+
 def main():
     a = parse()
     if a.dt is None:        # module_control.F90:214-220 (SubdivNum = 2 at every level)
@@ -1156,7 +1179,8 @@ def main():
         "plain_fp64": plain, "ensemble": ens, "uneven_batch": uneven, "hycom": hyc,
         "accuracy_96": acc, "cpu_baseline": cpu,
     }
-    print(json.dumps(out))
+    print("detail: " + json.dumps(out), file=sys.stderr, flush=True)
+    print(json.dumps(headline(out)), flush=True)
 
 
 if __name__ == "__main__":

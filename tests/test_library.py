@@ -96,3 +96,28 @@ def test_kernel_numbers_of_the_launch_shapes_stay():
         fimhip_ens_set_tile=staticmethod(lambda h, k, t: set_to.update({k: t}) or 0)))()))()
     fimhip.Ensemble.set_tiles(shape, {"e_trcadv1": 5, "e_trcadv2": 3, "e_momtum": 6})
     assert set_to == {5: 5, 6: 3, 8: 6}
+
+
+def test_bench_prints_a_line_that_a_logs_tail_holds():
+    """Whatever the legs report, the line has the headline's keys and fits into
+    2000 characters."""
+    import json
+    import sys
+    sys.path.insert(0, ROOT)
+    import bench
+    leg = {"value": 1.0 / 3, "ms_per_step": 2.0 / 3, "kernels": {"k%d" % i: {"ms": 1.0 / 7} for i in range(200)}}
+    out = {"metric": "m" * 70, "value": 1e10 / 3, "unit": "u", "n_gpus": 1, "steps": 20, "warmup": 5, "ms_per_step": 1.0 / 3,
+           "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32+f64", "data": "d" * 60,
+           "config": {"workload": "w" * 170, "dt_note": "n" * 200, "nip": 163842},
+           "roofline": {"bound": "hbm", "achieved": 1.0 / 3, "frac": 1.0 / 7, "kernels": leg["kernels"]},
+           "dominant_kernel": {"kernel": "e_trcadv12", "mean_launch_ms": 1.0 / 3}, "speedup_vs_plain_fp64": 2.0 / 3,
+           "plain_fp64": leg, "ensemble": leg, "uneven_batch": {"mixed": leg, "fp64": leg},
+           "hycom": dict({"n%d" % i: leg for i in range(6)}, workload="w"),
+           "accuracy_96": {"rel_l2_vs_fp64": {"us": 1e-4 / 3, "vs": 2e-4 / 3}}, "cpu_baseline": leg}
+    for drop in ((), ("plain_fp64", "uneven_batch", "hycom", "accuracy_96", "cpu_baseline")):
+        line = bench.headline({k: None if k in drop else v for k, v in out.items()})
+        assert len(json.dumps(line)) < 1900
+        for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+                  "vs_baseline", "dtype", "data", "config"):
+            assert k in line, k
+        assert line["value"] == 3333333000.0 and line["config"]["nip"] == 163842
