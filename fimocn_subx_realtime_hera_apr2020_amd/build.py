@@ -21,7 +21,7 @@ SOURCES = ["fimhip_api.hip", "kernels_plain.hip", "trc_patch.hip", "transp3d.hip
            "hycom_edgvar.hip", "hycom_momtum.hip", "hycom_transp.hip", "hycom_hybgen.hip"]
 HOST_SOURCES = ["grid.cpp", "lsq_svd.cpp"]      # host-only C++ (g++)
 HEADERS = ["fimhip_internal.h", "fim_pow.h", "fim_pow_tables.h", "synth.h", "host_common.h", "ens_internal.h",
-           "hycom_internal.h"]
+           "hycom_internal.h", "hycom_edges.h", "div_by.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("FIMHIP_ARCH", "gfx950")

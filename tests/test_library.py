@@ -121,3 +121,10 @@ def test_bench_prints_a_line_that_a_logs_tail_holds():
                   "vs_baseline", "dtype", "data", "config"):
             assert k in line, k
         assert line["value"] == 3333333000.0 and line["config"]["nip"] == 163842
+
+
+def test_incremental_build_sees_every_header():
+    """A source is compiled again when a header is newer than its object: the
+    list of headers is the folder's."""
+    from fimocn_subx_realtime_hera_apr2020_amd import build
+    assert sorted(build.HEADERS) == sorted(f for f in os.listdir(build.CSRC) if f.endswith(".h"))
