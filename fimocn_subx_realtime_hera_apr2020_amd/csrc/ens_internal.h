@@ -30,13 +30,18 @@ namespace fimhip {
 struct HostGrid;
 struct Arena;
 
-// Patches of cells for the fused tracer FCT (fct_tiles.hip): per patch the
-// cumulative ends n0..n3 of its core and three neighbour rings in its list
-// of tile cells, and per tile cell an entry of four ints: the cell index;
+// Patches of cells with their neighbour rings, of three kernels: the fused
+// tracer FCT (three rings) and trcadv12 (two; both fct_tiles.hip) of the batched
+// form, and the FP64 step's trcadv1 (two; trc_patch.hip).  Per patch the
+// cumulative ends n0..n3 of its core and rings in its list of tile cells (with
+// two rings n3 is n2), and per tile cell an entry of four ints: the cell index;
 // the local indices in the tile of its neighbours 0-3 (8 bits each); of
 // neighbours 4-5 and its edge count (8 bits each); the neighbours' indices of
-// the shared edges, proxs (4 bits each).  The local indices are set for
-// rings 0-2 only.
+// the shared edges, proxs (4 bits each).  The local indices are set for all but
+// the last ring (0 there).  In the FP64 tables bits 24-29 of a core cell's third
+// int mark the edges whose neighbour is a pentagon.  core_row: per core cell
+// what the two-ring kernels hand out lane by lane, CORE_ROW words a cell in
+// trcadv12's format (k_core_rows), ROWP in the FP64 trcadv1's (k_patch_rows).
 // words of trcadv12's core rows and where their parts begin (k_core_rows in
 // fct_tiles.hip)
 constexpr int CR_NBR = 36, CR_ST = 72, CR_NB = 90, CORE_ROW = 96;
@@ -45,7 +50,7 @@ struct EnsTiles {
   const int *off;      // (npatch + 1) first tile cell of each patch
   const int4 *cnt;     // (npatch) n0, n1, n2, n3
   const int4 *ent;
-  const int *core_row; // (CORE_ROW, nip)
+  const int *core_row; // not the fused FCT's
   int r_max, lo_max;   // most cells of a patch in rings 0-1 and 0-2
 };
 

@@ -22,7 +22,6 @@ const char *const ens_kernel_names[EK_NKERNELS] = {
 #define EAB(a, sl, col, k) (a)[((size_t)(sl) * ncol + (col)) * nvl + (k)]
 #define ETR(a, t, col, k) (a)[((size_t)(t) * ncol + (col)) * nvl + (k)]
 #define ETAB(a, t, sl, col, k) (a)[(((size_t)(t) * 3 + (sl)) * ncol + (col)) * nvl + (k)]
-#define ETE(a, t, col, e, k) (a)[(((size_t)(t) * ncol + (col)) * NPP + (e)) * nvl + (k)]
 #define GPROX(i, e) ldc(g.d.prox, (i) * NPP + (e))
 #define GPROXS(i, e) ldc(g.d.proxs, (i) * NPP + (e))
 #define FCS(i, e, j) ldc(g.cs, ((i) * NPP + (e)) * 4 + (j))

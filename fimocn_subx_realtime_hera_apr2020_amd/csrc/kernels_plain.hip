@@ -701,7 +701,7 @@ __global__ void __launch_bounds__(256) k_trdp(DevGrid g, DevState s) {
 // passes through memory between them.  The kernels are bound by HBM traffic
 // (4-5.5 TB/s), so each is written to move fewer bytes, up to momtum about
 // 2340 B per cell-level and step for 4 tracers against 3560 B with the
-// kernels above (G7 x 64: 7.1 ms a step against 9.36 ms):
+// kernels above (G7 x 64: 6.8 ms a step against 9.3 ms):
 //  * k_edgvar1 stores the normal edge wind, the sum of Montgomery potential
 //    and kinetic energy, the two line integrals of the edge pressure and the
 //    vorticity: 15 values instead of 36;
@@ -714,8 +714,8 @@ __global__ void __launch_bounds__(256) k_trdp(DevGrid g, DevState s) {
 //    trcadv2 forms trcadv1's bounds again from the tracer; trcadv3 does not
 //    store the tracer mass where hystat forms it again.
 // Every load of a stage is issued before its first use, with the edge loops
-// unrolled per cell shape.  The values of the step's start (u2, v2 and the
-// other buffers of dp, pr, mp, tr) stay until the next step, so the edge
+// unrolled per cell shape.  The values of the step's start (in u2, v2, trcr_lo
+// and the other buffers of pr and mp) stay until the next step, so the edge
 // fields a caller may download are formed from them when asked for.
 
 template <int NP, bool MOM>
