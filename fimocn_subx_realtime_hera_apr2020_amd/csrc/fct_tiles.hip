@@ -707,7 +707,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   const float dp = (float)in.dp;
   const float ti = Str[i * 64 + k], lo = Slo[i * 64 + k];
 #pragma unroll
-  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, CR_NB + e) & ~3, k);
+  for (int e = 0; e < NP; e++) v[e] = lds_at(Str, row_i(row, CR_NB + e) & ~1, k);
   if (t == 0) {
 #pragma unroll
     for (int e = 0; e < NP; e++) {
@@ -726,7 +726,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
 #pragma unroll
       for (int j = 0; j < NPP; j++) {
         const float n = lds_at(Str, row_h(row, CR_ST, e * NPP + j), k) - v[e];
-        if (j < NPP - 1 || !(row_i(row, CR_NB + e) & 2)) ax = __builtin_fmaf(n, row_f(row, CR_NBR + e * NPP + j), ax);
+        ax = __builtin_fmaf(n, row_f(row, CR_NBR + e * NPP + j), ax);      // (0 * 0 for a pentagon's missing cell)
       }
       te[e] = .5f * ((ti + ac) + (v[e] + ax));
     }
@@ -742,7 +742,7 @@ __device__ __forceinline__ void tile_flux(const EnsGrid &g, const EnsState &s, c
   int lower = 0;
 #pragma unroll
   for (int e = 0; e < NP; e++) {
-    const float x = lds_at(Slo, row_i(row, CR_NB + e) & ~3, k);
+    const float x = lds_at(Slo, row_i(row, CR_NB + e) & ~1, k);
     mx = fmaxf(mx, x);
     mn = fminf(mn, x);
     lower |= (row_i(row, CR_NB + e) & 1) << e;
@@ -867,8 +867,9 @@ void ens_launch_trcadv12(int tile, const EnsGrid &g, const EnsState &s, hipStrea
 // stencil's slots, from CR_ST on the LDS byte offsets (256 per tile cell; 16
 // bits) of the neighbours' stencil cells, and from CR_NB on those of the
 // neighbours, with bit 0 set where the cell stores the edge's antidiffusive
-// flux (it has the lower index) and bit 1 where the neighbour is a pentagon,
-// whose missing stencil cell is the neighbour itself with coefficient 0.  One
+// flux (it has the lower index).  A pentagon's missing stencil cell is the
+// pentagon itself with coefficient 0: its term adds 0.  (Leaving the term out
+// by a flag took trcadv12 from 6.86 to 6.97 ms at 8 members x G7 x 64.)  One
 // block per patch, one thread per core cell and edge.
 __global__ void __launch_bounds__(256) k_core_rows(EnsGrid g, EnsTiles ts, int *rows) {
   const int p = blockIdx.x, n0 = ts.cnt[p].x;
@@ -880,7 +881,7 @@ __global__ void __launch_bounds__(256) k_core_rows(EnsGrid g, EnsTiles ts, int *
     const int4 ex = ent[l];
     const int x = ex.x, nx = enp(ex), xs = eslot(en, e);
     int *row = rows + (size_t)c * CORE_ROW;
-    row[CR_NB + e] = 256 * l | (nx < NPP ? 2 : 0) | (c < x);
+    row[CR_NB + e] = 256 * l | (c < x);
     for (int j = 0; j < NPP; j++) {
       row[e * NPP + j] = __float_as_int(g.hfcoef[((size_t)c * NPP + e) * NPP + j]);
       row[CR_NBR + e * NPP + j] = j < nx ? __float_as_int(g.hfcoef[((size_t)x * NPP + xs) * NPP + j]) : 0;
