@@ -603,12 +603,14 @@ void ens_launch_trc_fct(int tile, const EnsGrid &g, const EnsState &s, hipStream
 // transport have the same bits.
 //
 // What bounds it: HBM traffic, 256 B per cell-level for 4 tracers plus the
-// halo, half of it writes, at 4.4 TB/s (a large copy reaches 4.75).  As
-// three kernels (edgvar3's reconstructions stored and read back, the
-// low-order tracer stored, the mass flux read twice) it moved 620 B.  8
-// members x G7 x 64 x 4 tracers: 9.75 -> 6.7 ms; 16 x G5: 1.20 -> 0.87 ms; G6
-// with 20 tracers: 1.65 -> 1.07 ms; 3 x G4 x 38 x 3 tracers: 42 -> 40 us.
-// What got it there:
+// halo, half of it writes: 53 GB for 16 members x G7 x 64 by the counters (1.23
+// times its own bytes; their fetch side is uncertain by 20 %) in 13.4 ms, 4.0
+// TB/s (a large copy reaches 4.75).  As three kernels (edgvar3's
+// reconstructions stored and read back, the low-order tracer stored, the mass
+// flux read twice) it moved 620 B.  8 members x G7 x 64 x 4 tracers: 9.75 ->
+// 6.85 ms; 16 x G5: 1.20 -> 0.90 ms; G6 with 20 tracers: 1.65 -> 1.08 ms; 3 x G4
+// x 38 x 3 tracers: 42 -> 45 us, in one launch instead of three.
+// What got it there (each measured when the kernel took 7.2 ms):
 //  * the cells' coefficients and stencil offsets come one row per cell by a
 //    vector load, a cell ahead, and are handed out by v_readlane: as scalar
 //    loads they missed the scalar cache and each batch waited about 1500
